@@ -211,7 +211,7 @@ int rp_hip_fill_scaled(void* ptr, const void* scalar_dev, double scale, size_t s
 int rp_hip_convert(void* dst, int dst_dtype, const void* src, int src_dtype, size_t size);
 
 /* The backward of y = x . w + b for 2-D operands in one call: dx [m, k] = dy . w^T, dw [k, n] = x^T . dy,
- * db [n] = column sums of dy (rows added top to bottom, as rp_hip_reduce_rows).  dy [m, n] is dense; x [m, k], w [k, n],
+ * db [n] = column sums of dy (as rp_hip_reduce_rows).  dy [m, n] is dense; x [m, k], w [k, n],
  * dx and dw carry (row, column) strides in elements; any of dx, dw, db may be NULL; accumulate_* = 1 adds to what the
  * output holds.  Same values, bit for bit, as two rp_hip_gemm_strided_batched calls with the transposes as swapped
  * strides (backward_matmul_fn, ops/ops.c:6759-6814) and rp_hip_reduce_rows; for small float32 layers (the
@@ -222,7 +222,8 @@ int rp_hip_linear_backward(void* dx, void* dw, void* db, const void* dy, const v
                            int accumulate_dx, int accumulate_dw, int accumulate_db, int dtype);
 
 /* Bias gradient of Linear on the device: grad [rows, cols] dense -> out [cols],
- * each column summed top to bottom in fp32 (fp64 for float64).  Stands in for
+ * each column summed in fp32 (fp64 for float64): up to 256 rows top to bottom, more
+ * rows as runs of 64, four runs to a chunk, each level top to bottom.  Stands in for
  * the device->host->device round trip of reduce_grad_to_shape
  * (ops/ops.c:6970-7101) in the [rows, cols] -> [cols] case. */
 int rp_hip_reduce_rows(void* out, const void* grad, int rows, int cols, int accumulate, int dtype);

@@ -1,0 +1,73 @@
+// Column sums of a dense [rows, cols] matrix (the bias gradient of a Linear layer), shared by rp_hip_reduce_rows and the
+// one-launch backward of small layers so that both leave the same bits.
+//
+// The order is fixed.  Up to 256 rows are added top to bottom in the accumulate type, the reference's own order
+// (ops/ops.c:7027-7086).  More rows are cut into chunks of 256 and those into runs of 64: the rows of a run, the runs of a
+// chunk and the chunks are each added top to bottom (the error bound is that of a sum of 68 + rows / 256 terms instead
+// of one of rows terms, and four waves add at a time).
+//
+// What bounds it is not the arithmetic but how many loads are in flight: a thread that walks its column with
+// sixteen loads at a time spends a memory round trip per sixteen rows (1024 x 1024 in bf16 took 23 us).  256 threads
+// therefore fetch a tile of WIDTH bytes times ROWS rows at once, 16 bytes per load and all of them in flight together,
+// park it in LDS, and the rows are added out of LDS, a column per lane.
+#pragma once
+#include "rp_common.h"
+
+#include <cstring>
+
+namespace rp {
+
+constexpr int COLSUM_CHUNK = 256, COLSUM_RUN = 64;
+
+template <typename T, int WIDTH, int ROWS>
+struct ColumnTile {
+    static constexpr int COLS = WIDTH / (int)sizeof(T), VEC = 16 / (int)sizeof(T);
+    static constexpr int VPR = WIDTH / 16, RPP = 256 / VPR, NV = ROWS / RPP;         // vectors per row, rows per pass of 256 threads, passes
+    static constexpr size_t BYTES = (size_t)WIDTH * ROWS;
+    typedef __attribute__((ext_vector_type(4))) unsigned int vec_t;
+    vec_t v[NV];
+    // rows from r0 on (zeros from r1 on), columns from c0 on
+    __device__ __forceinline__ void load(const T* grad, int r0, int r1, int c0, int cols, int t) {
+        const int c = c0 + (t % VPR) * VEC;
+#pragma unroll
+        for (int i = 0; i < NV; i++) {
+            const int r = r0 + t / VPR + RPP * i;
+            v[i] = vec_t{0, 0, 0, 0};
+            if (r >= r1) continue;
+            const T* p = grad + (size_t)r * cols + c;
+            if (c + VEC <= cols) memcpy(&v[i], p, 16);           // at any alignment of whole elements
+            else {
+                T e[VEC];
+                memset(e, 0, 16);
+#pragma unroll
+                for (int k = 0; k < VEC; k++) if (c + k < cols) e[k] = p[k];
+                memcpy(&v[i], e, 16);
+            }
+        }
+    }
+    __device__ __forceinline__ void store(T* lds, int t) const {
+#pragma unroll
+        for (int i = 0; i < NV; i++) *(vec_t*)(lds + (size_t)(t / VPR + RPP * i) * COLS + (t % VPR) * VEC) = v[i];
+    }
+    // s + the first n rows from lds on, top to bottom, sixteen rows read ahead of the ones being added (adding the zeros
+    // past the last row changes nothing: s is never -0)
+    static __device__ __forceinline__ typename traits<T>::acc add(typename traits<T>::acc s, const T* lds, int col, int n) {
+        constexpr int U = 16;
+        static_assert(ROWS % U == 0, "whole groups of rows");
+        T x[U], next[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) x[u] = lds[u * COLS + col];
+        for (int r = 0; r < n; r += U) {
+            const int ahead = r + U < n ? r + U : r;
+#pragma unroll
+            for (int u = 0; u < U; u++) next[u] = lds[(ahead + u) * COLS + col];
+#pragma unroll
+            for (int u = 0; u < U; u++) s += widen(x[u]);
+#pragma unroll
+            for (int u = 0; u < U; u++) x[u] = next[u];
+        }
+        return s;
+    }
+};
+
+}  // namespace rp

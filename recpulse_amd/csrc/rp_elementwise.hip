@@ -4,7 +4,7 @@
 // on-device bias gradient and cross-entropy.  16-bit dtypes compute in fp32
 // and narrow once with the reference's rounding, like the reference's host
 // path (functional/functional.c:10-56).
-#include "rp_common.h"
+#include "rp_column_sums.h"
 
 #include <cfloat>
 
@@ -524,30 +524,98 @@ __global__ void sum_dim_kernel(T* out, const T* x, size_t outer, size_t dim, siz
     }
 }
 
-// Linear's bias gradient: out[j] = sum_i grad[i, j], rows added top to bottom
-// in the accumulate type — the order the reference's host loop produces
-// (ops/ops.c:7048-7061).  Threads of a block own adjacent columns, so every
-// row read is one coalesced segment.
-template <typename T>
-__global__ void reduce_rows_kernel(T* out, const T* g, int rows, int cols, int accumulate) {
+// Linear's bias gradient: out[j] = sum_i grad[i, j] in the order of rp_column_sums.h.  A block is 1 to 4 groups of 256 threads, a group owns one chunk of WIDTH bytes' worth
+// of columns.  Up to 1024 rows the groups meet in LDS and the block finishes; beyond that every group is a block of its
+// own that leaves its chunk's sums in `partials` [chunk][cols], and column_sums_finish_kernel adds them (one block walking
+// more rows has one tile of loads in flight at a time; 8192 x 8192 then keeps 128 of the 256 CUs busy).
+// WIDTH: 64 in the first case, where blocks are few and a CU's own bandwidth counts, whole cache lines in the second.
+template <typename T, int WIDTH>
+__global__ void __launch_bounds__(1024) column_sums_kernel(T* out, typename traits<T>::acc* partials, const T* grad, int rows, int cols, int accumulate) {
     using A = typename traits<T>::acc;
-    int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= cols) return;
-    A s = 0;
-    const T* p = g + j;
-    int i = 0;
-    constexpr int U = 16;                       // independent loads in flight; the adds stay in row order
-    for (; i + U <= rows; i += U) {
-        A v[U];
-#pragma unroll
-        for (int u = 0; u < U; u++) v[u] = widen(p[(size_t)(i + u) * cols]);
-#pragma unroll
-        for (int u = 0; u < U; u++) s += v[u];
+    using Tile = ColumnTile<T, WIDTH, COLSUM_CHUNK>;
+    constexpr int COLS = Tile::COLS;
+    extern __shared__ __attribute__((aligned(16))) unsigned char colsum_lds[];
+    const int t = threadIdx.x & 255, group = threadIdx.x >> 8, groups = blockDim.x >> 8;
+    const int chunk = blockIdx.y * groups + group, r0 = chunk * COLSUM_CHUNK;
+    const int r1 = r0 + COLSUM_CHUNK < rows ? r0 + COLSUM_CHUNK : rows;
+    const int c0 = blockIdx.x * COLS;
+    T* tile = (T*)(colsum_lds + group * Tile::BYTES);
+    {
+        Tile regs;
+        regs.load(grad, r0, r1, c0, cols, t);
+        regs.store(tile, t);
     }
-    for (; i < rows; i++) s += widen(p[(size_t)i * cols]);
+    __syncthreads();
+    // rows <= COLSUM_CHUNK: the group's first wave adds all of them; otherwise each of its four waves adds a run
+    const int lane = t & 63, wave = t >> 6, runs = rows <= COLSUM_CHUNK ? 1 : COLSUM_CHUNK / COLSUM_RUN;
+    const int first = wave * COLSUM_RUN, mine = runs == 1 ? r1 - r0 : (r1 - r0 - first < COLSUM_RUN ? r1 - r0 - first : COLSUM_RUN);
+    A s = 0;
+    if (wave < runs && lane < COLS && mine > 0) s = Tile::add(s, tile + first * COLS, lane, mine);
+    __syncthreads();                                    // the tiles have been read: their LDS carries the runs' sums now
+    A* parts = (A*)colsum_lds + (size_t)group * (COLSUM_CHUNK / COLSUM_RUN) * COLS;
+    if (wave < runs && lane < COLS) parts[wave * COLS + lane] = s;
+    __syncthreads();
+    if (t >= COLS) return;                              // (no barrier after this point)
+    const int j = c0 + t;
+    if (j >= cols) return;
+    if (partials) {
+        for (int q = 1; q < runs; q++) s += parts[q * COLS + t];
+        partials[(size_t)chunk * cols + j] = s;
+        return;
+    }
+    if (group > 0) return;
+    s = 0;
+    for (int g = 0; g < groups; g++) {
+        const A* p = (const A*)colsum_lds + (size_t)g * (COLSUM_CHUNK / COLSUM_RUN) * COLS + t;
+        A c = p[0];
+        for (int q = 1; q < runs; q++) c += p[q * COLS];
+        s += c;
+    }
     T r = narrow<T>(s);
     if (accumulate) r = narrow<T>(widen(out[j]) + widen(r));
     out[j] = r;
+}
+
+template <typename T>
+__global__ void __launch_bounds__(64) column_sums_finish_kernel(T* out, const typename traits<T>::acc* partials, int chunks, int cols, int accumulate) {
+    using A = typename traits<T>::acc;
+    const int j = blockIdx.x * 64 + threadIdx.x;
+    if (j >= cols) return;
+    A s = 0;
+    int i = 0;
+    constexpr int U = 32;                               // independent loads in flight; the adds stay in chunk order
+    for (; i + U <= chunks; i += U) {
+        A v[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) v[u] = partials[(size_t)(i + u) * cols + j];
+#pragma unroll
+        for (int u = 0; u < U; u++) s += v[u];
+    }
+    for (; i < chunks; i++) s += partials[(size_t)i * cols + j];
+    T r = narrow<T>(s);
+    if (accumulate) r = narrow<T>(widen(out[j]) + widen(r));
+    out[j] = r;
+}
+
+template <typename T>
+static int launch_column_sums(T* out, const T* grad, int rows, int cols, int accumulate) {
+    using A = typename traits<T>::acc;
+    const int chunks = (rows + COLSUM_CHUNK - 1) / COLSUM_CHUNK;
+    if (chunks <= 4) {
+        using Tile = ColumnTile<T, 64, COLSUM_CHUNK>;
+        hipLaunchKernelGGL((column_sums_kernel<T, 64>), dim3((cols + Tile::COLS - 1) / Tile::COLS), dim3(256 * chunks), chunks * Tile::BYTES, current_stream(),
+                           out, (A*)nullptr, grad, rows, cols, accumulate);
+        return check_launch("column_sums_kernel") ? 0 : -1;
+    }
+    if (chunks > 65535) { set_error("rp_hip_reduce_rows: too many rows (%d)", rows); return -1; }
+    void* ws = nullptr;
+    if (rp_hip_malloc(&ws, (size_t)chunks * cols * sizeof(A)) != 0) return -1;
+    using Tile = ColumnTile<T, 128, COLSUM_CHUNK>;
+    hipLaunchKernelGGL((column_sums_kernel<T, 128>), dim3((cols + Tile::COLS - 1) / Tile::COLS, chunks), dim3(256), Tile::BYTES, current_stream(), out, (A*)ws, grad, rows, cols, accumulate);
+    hipLaunchKernelGGL(column_sums_finish_kernel<T>, dim3((cols + 63) / 64), dim3(64), 0, current_stream(), out, (const A*)ws, chunks, cols, accumulate);
+    const bool ok = check_launch("column_sums_kernel");
+    rp_hip_free(ws);                                    // back to the pool while the kernels are still queued: safe for later work on this stream
+    return ok ? 0 : -1;
 }
 
 // ---- cross-entropy ----------------------------------------------------------------------
@@ -944,10 +1012,8 @@ int rp_hip_convert(void* dst, int dst_dtype, const void* src, int src_dtype, siz
 
 int rp_hip_reduce_rows(void* out, const void* grad, int rows, int cols, int accumulate, int dtype) {
     RP_REQUIRE(out && grad && rows > 0 && cols > 0, "rp_hip_reduce_rows");
-    unsigned blocks = (unsigned)((cols + 63) / 64);
-    RP_DISPATCH_DTYPE(dtype, hipLaunchKernelGGL(reduce_rows_kernel<T>, dim3(blocks), dim3(64), 0, current_stream(),
-                                               (T*)out, (const T*)grad, rows, cols, accumulate));
-    return check_launch("reduce_rows_kernel") ? 0 : -1;
+    RP_DISPATCH_DTYPE(dtype, return launch_column_sums<T>((T*)out, (const T*)grad, rows, cols, accumulate));
+    return -1;
 }
 
 int rp_hip_cross_entropy_mean(void* loss_out, void* grad_logits, const void* logits, const int* targets,

@@ -6,6 +6,7 @@
 // fixed order of additions, up to about a thousand workgroups in flight.  Operands are read straight from global
 // memory with any strides (16-byte loads along k where k is the unit-stride axis); nothing is staged, every value is
 // used once per workgroup.
+#include "rp_column_sums.h"
 #include "rp_gemm.h"
 
 namespace rp {
@@ -13,16 +14,34 @@ namespace rp {
 typedef __attribute__((ext_vector_type(4))) float f32x4t_t;
 
 // MFMA step j of a 16-deep chunk uses k = chunk + 4*(lane / 16) + j for the four k slots: a permutation of k that both
-// operands share, chosen so that a lane's four values are consecutive in k.
+// operands share, chosen so that a lane's four values are consecutive in k.  p points at the lane's first value.
 template <bool VEC>
-__device__ __forceinline__ void tiny_load4(float (&v)[4], const float* p, long long k_stride, int k0, int k_end) {
-    if (VEC && k0 + 4 <= k_end) {
-        const f32x4t_t x = *(const f32x4t_t*)(p + k0);
-        v[0] = x[0]; v[1] = x[1]; v[2] = x[2]; v[3] = x[3];
-    } else {
+__device__ __forceinline__ f32x4t_t tiny_load4(const float* p, long long k_stride) {
+    if (VEC) return *(const f32x4t_t*)p;
+    return f32x4t_t{p[0], p[k_stride], p[2 * k_stride], p[3 * k_stride]};
+}
+// the same with zeros from k_end on
+__device__ __forceinline__ f32x4t_t tiny_load4_masked(const float* p, long long k_stride, int k0, int k_end) {
+    f32x4t_t v;
 #pragma unroll
-        for (int j = 0; j < 4; j++) v[j] = (k0 + j < k_end) ? p[(long long)(k0 + j) * k_stride] : 0.f;
+    for (int j = 0; j < 4; j++) v[j] = (k0 + j < k_end) ? p[(long long)j * k_stride] : 0.f;
+    return v;
+}
+
+// U whole chunks from chunk c on: all of their loads are requested before the first is multiplied
+template <bool A_VEC, bool B_VEC, int U>
+__device__ __forceinline__ void tiny_chunks(f32x4t_t& acc, const float* ap, const float* bp, long long a_ks, long long b_ks, int c, int kq) {
+    f32x4t_t a[U], b[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+        const long long k0 = 16 * (c + u) + 4 * kq;
+        a[u] = tiny_load4<A_VEC>(ap + k0 * a_ks, a_ks);
+        b[u] = tiny_load4<B_VEC>(bp + k0 * b_ks, b_ks);
     }
+#pragma unroll
+    for (int u = 0; u < U; u++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u][j], b[u][j], acc, 0, 0, 0);
 }
 
 // One 16 x 16 tile of C_z (tile row tm, tile column tn) by the 256 threads of a workgroup; red: 3 x 256 floats of LDS.
@@ -38,30 +57,34 @@ __device__ __forceinline__ void tiny_tile(const GemmArgs& g, int z, int tm, int 
     const float* ap = (const float*)g.A + (long long)z * g.a_bs + (long long)row * g.a_rs;
     const float* bp = (const float*)g.B + (long long)z * g.b_bs + (long long)col * g.b_cs;
 
-    // chunks of 16 k, a contiguous quarter of them per wave
+    // chunks of 16 k, a contiguous quarter of them per wave.  Every batch of loads is one memory round trip, which is most
+    // of what such a product costs: up to eight chunks (64 values per lane) go in one batch.
     const int chunks = (g.k + 15) / 16, per_wave = (chunks + 3) / 4;
     const int c_begin = wave * per_wave, c_end = c_begin + per_wave < chunks ? c_begin + per_wave : chunks;
+    const int whole = g.k / 16 < c_end ? g.k / 16 : c_end;         // chunks before this one are not cut off by the end of k
     f32x4t_t acc = {0.f, 0.f, 0.f, 0.f};
-    int c = c_begin;
-    for (; c + 2 <= c_end; c += 2) {                 // two chunks at a time: sixteen values in flight per lane
-        float a0[4], b0[4], a1[4], b1[4];
-        const int k0 = 16 * c + 4 * kq, k1 = k0 + 16;
-        tiny_load4<A_VEC>(a0, ap, g.a_cs, k0, g.k);
-        tiny_load4<B_VEC>(b0, bp, g.b_rs, k0, g.k);
-        tiny_load4<A_VEC>(a1, ap, g.a_cs, k1, g.k);
-        tiny_load4<B_VEC>(b1, bp, g.b_rs, k1, g.k);
-#pragma unroll
-        for (int j = 0; j < 4; j++) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a0[j], b0[j], acc, 0, 0, 0);
-#pragma unroll
-        for (int j = 0; j < 4; j++) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a1[j], b1[j], acc, 0, 0, 0);
+    f32x4t_t a_tail = {0.f, 0.f, 0.f, 0.f}, b_tail = {0.f, 0.f, 0.f, 0.f};
+    const bool cut = c_end == chunks && c_begin < chunks && g.k % 16 != 0;
+    if (cut) {                                                     // the cut-off chunk: requested first, multiplied last
+        const int k0 = 16 * (chunks - 1) + 4 * kq;
+        a_tail = tiny_load4_masked(ap + (long long)k0 * g.a_cs, g.a_cs, k0, g.k);
+        b_tail = tiny_load4_masked(bp + (long long)k0 * g.b_rs, g.b_rs, k0, g.k);
     }
-    if (c < c_end) {
-        float a0[4], b0[4];
-        const int k0 = 16 * c + 4 * kq;
-        tiny_load4<A_VEC>(a0, ap, g.a_cs, k0, g.k);
-        tiny_load4<B_VEC>(b0, bp, g.b_rs, k0, g.k);
+    int c = c_begin;
+    for (; c + 8 <= whole; c += 8) tiny_chunks<A_VEC, B_VEC, 8>(acc, ap, bp, g.a_cs, g.b_rs, c, kq);
+    switch (whole - c) {                                           // (negative when the wave has no whole chunk)
+        case 7: tiny_chunks<A_VEC, B_VEC, 7>(acc, ap, bp, g.a_cs, g.b_rs, c, kq); break;
+        case 6: tiny_chunks<A_VEC, B_VEC, 6>(acc, ap, bp, g.a_cs, g.b_rs, c, kq); break;
+        case 5: tiny_chunks<A_VEC, B_VEC, 5>(acc, ap, bp, g.a_cs, g.b_rs, c, kq); break;
+        case 4: tiny_chunks<A_VEC, B_VEC, 4>(acc, ap, bp, g.a_cs, g.b_rs, c, kq); break;
+        case 3: tiny_chunks<A_VEC, B_VEC, 3>(acc, ap, bp, g.a_cs, g.b_rs, c, kq); break;
+        case 2: tiny_chunks<A_VEC, B_VEC, 2>(acc, ap, bp, g.a_cs, g.b_rs, c, kq); break;
+        case 1: tiny_chunks<A_VEC, B_VEC, 1>(acc, ap, bp, g.a_cs, g.b_rs, c, kq); break;
+        default: break;
+    }
+    if (cut) {
 #pragma unroll
-        for (int j = 0; j < 4; j++) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a0[j], b0[j], acc, 0, 0, 0);
+        for (int j = 0; j < 4; j++) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a_tail[j], b_tail[j], acc, 0, 0, 0);
     }
 
     // the four partial tiles meet in LDS and are added in wave order
@@ -100,9 +123,10 @@ static bool tiny_a_vec(const GemmArgs& g) { return g.a_cs == 1 && g.a_rs % 4 == 
 static bool tiny_b_vec(const GemmArgs& g) { return g.b_rs == 1 && g.b_cs % 4 == 0 && g.b_bs % 4 == 0 && ((uintptr_t)g.B & 15) == 0; }
 
 // The backward of a small Linear layer in one launch: the tiles of dX = dY . W^T, then the tiles of dW = X^T . dY, then
-// the column sums of dY for db (one thread per column, rows added top to bottom as reduce_rows does).  Every block
+// the column sums of dY for db (in reduce_rows' order).  Every block
 // does what it would have done in three separate launches, so the bits are the same; what goes away is two launch
 // latencies, which is most of the time of such a layer.  Either GEMM or the sums may be absent (zero tiles / blocks).
+constexpr int DB_WIDTH = 64;            // bytes of a row that one workgroup sums
 struct ColumnSums {
     float* out;
     const float* grad;       // [rows, cols], dense
@@ -122,26 +146,36 @@ __device__ __forceinline__ void tiny_tile_any(const GemmArgs& g, bool a_vec, boo
     else tiny_tile_of<false, false>(g, tile, red);
 }
 
-__global__ void __launch_bounds__(256) linear_backward_tiny32_kernel(GemmArgs gx, GemmArgs gw, ColumnSums db, int tiles_x, int tiles_w, int vec_flags) {
-    __shared__ float red[3][256];
-    const int b = blockIdx.x;
-    if (b < tiles_x) { tiny_tile_any(gx, vec_flags & 1, vec_flags & 2, b, red); return; }
-    if (b < tiles_x + tiles_w) { tiny_tile_any(gw, vec_flags & 4, vec_flags & 8, b - tiles_x, red); return; }
-    const int j = (b - tiles_x - tiles_w) * 256 + threadIdx.x;
-    if (j >= db.cols) return;
-    float s = 0.f;
-    const float* p = db.grad + j;
-    int i = 0;
-    constexpr int U = 16;                       // independent loads in flight; the adds stay in row order
-    for (; i + U <= db.rows; i += U) {
-        float v[U];
-#pragma unroll
-        for (int u = 0; u < U; u++) v[u] = p[(size_t)(i + u) * db.cols];
-#pragma unroll
-        for (int u = 0; u < U; u++) s += v[u];
+__global__ void __launch_bounds__(256) linear_backward_tiny32_kernel(GemmArgs gx, GemmArgs gw, ColumnSums db, int tiles_x, int blocks_db, int vec_flags) {
+    constexpr int DB_ROWS = 128;
+    using Tile = ColumnTile<float, DB_WIDTH, DB_ROWS>;
+    __shared__ __attribute__((aligned(16))) float tile[DB_ROWS * Tile::COLS];       // column sums; the GEMM tiles meet in its first 3 KB
+    float (*red)[256] = (float (*)[256])tile;
+    const int b = (int)blockIdx.x - blocks_db;           // the column sums go first: their chain of additions is the longest of any workgroup
+    if (b >= 0 && b < tiles_x) { tiny_tile_any(gx, vec_flags & 1, vec_flags & 2, b, red); return; }
+    if (b >= 0) { tiny_tile_any(gw, vec_flags & 4, vec_flags & 8, b - tiles_x, red); return; }
+    // column sums in the order of rp_column_sums.h, a chunk in two tiles of 128 rows: the next tile is on its way while
+    // the wave adds this one (a whole chunk per tile would cost every workgroup of the launch twice the LDS)
+    constexpr int COLS = Tile::COLS;
+    const int t = threadIdx.x, c0 = (int)blockIdx.x * COLS, j = c0 + t;
+    const bool serial = db.rows <= COLSUM_CHUNK;
+    float total = 0.f, s = 0.f;
+    Tile regs;
+    regs.load(db.grad, 0, db.rows, c0, db.cols, t);
+    for (int r = 0; r < db.rows; r += DB_ROWS) {
+        regs.store(tile, t);
+        __syncthreads();
+        if (r + DB_ROWS < db.rows) regs.load(db.grad, r + DB_ROWS, db.rows, c0, db.cols, t);
+        if (t < COLS) {
+            const int n = db.rows - r < DB_ROWS ? db.rows - r : DB_ROWS;
+            if (serial) s = Tile::add(s, tile, t, n);
+            else
+                for (int q = 0; q < n; q += COLSUM_RUN) s += Tile::add(0.f, tile + q * COLS, t, n - q < COLSUM_RUN ? n - q : COLSUM_RUN);
+            if ((r + DB_ROWS) % COLSUM_CHUNK == 0 || r + DB_ROWS >= db.rows) { total += s; s = 0.f; }
+        }
+        __syncthreads();
     }
-    for (; i < db.rows; i++) s += p[(size_t)i * db.cols];
-    db.out[j] = db.accumulate ? db.out[j] + s : s;
+    if (t < COLS && j < db.cols) db.out[j] = db.accumulate ? db.out[j] + total : total;
 }
 
 // gx / gw: batch 1, fp32, each taken by the tiny kernel on its own (the caller checks); m == 0 marks an absent GEMM,
@@ -149,11 +183,11 @@ __global__ void __launch_bounds__(256) linear_backward_tiny32_kernel(GemmArgs gx
 int launch_linear_backward_tiny(const GemmArgs& gx, const GemmArgs& gw, void* db, const void* dy, int rows, int cols, int accumulate_db) {
     const int tiles_x = gx.m > 0 ? ((gx.m + 15) / 16) * ((gx.n + 15) / 16) : 0;
     const int tiles_w = gw.m > 0 ? ((gw.m + 15) / 16) * ((gw.n + 15) / 16) : 0;
-    const int blocks_db = db ? (cols + 255) / 256 : 0;
+    const int blocks_db = db ? (cols + DB_WIDTH / 4 - 1) / (DB_WIDTH / 4) : 0;
     if (tiles_x + tiles_w + blocks_db == 0) return 0;
     ColumnSums cs{(float*)db, (const float*)dy, rows, db ? cols : 0, accumulate_db};
     const int flags = (gx.m > 0 && tiny_a_vec(gx) ? 1 : 0) | (gx.m > 0 && tiny_b_vec(gx) ? 2 : 0) | (gw.m > 0 && tiny_a_vec(gw) ? 4 : 0) | (gw.m > 0 && tiny_b_vec(gw) ? 8 : 0);
-    hipLaunchKernelGGL(linear_backward_tiny32_kernel, dim3(tiles_x + tiles_w + blocks_db), dim3(256), 0, current_stream(), gx, gw, cs, tiles_x, tiles_w, flags);
+    hipLaunchKernelGGL(linear_backward_tiny32_kernel, dim3(tiles_x + tiles_w + blocks_db), dim3(256), 0, current_stream(), gx, gw, cs, tiles_x, blocks_db, flags);
     return check_launch("linear_backward_tiny32_kernel") ? 0 : -1;
 }
 

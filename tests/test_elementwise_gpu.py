@@ -121,6 +121,32 @@ def test_reduce_rows_matches_reference_order_bit_exact(dt):
         capi.check(L().rp_hip_reduce_rows(do.ptr, dg.ptr, rows, cols, 1, dt), "reduce_rows")
         assert np.array_equal(do.numpy(), oracle.add(want, want, dt))
 
+@pytest.mark.parametrize("dt", ALL, ids=lambda d: NAMES[d])
+@pytest.mark.parametrize("rows", [255, 257, 1024, 1025, 2600])
+def test_reduce_rows_beyond_one_chunk_bit_exact(dt, rows):
+    """Runs of 64 rows, four of them to a chunk of 256, every level added top to bottom: one block up to 1024 rows, a
+    finishing launch beyond.  Columns on both sides of a 128-byte tile, and a width that leaves the rows unaligned."""
+    rng = np.random.default_rng(46)
+    for cols in (1, 63, 128, 261):
+        g = rand_storage(rng, (rows, cols), dt)
+        dg, do = Dev(g, dt), Dev.empty((cols,), dt)
+        capi.check(L().rp_hip_reduce_rows(do.ptr, dg.ptr, rows, cols, 0, dt), "reduce_rows")
+        acc = np.float64 if dt == F64 else np.float32
+        wide = oracle.to_f64(g, dt).astype(acc)                 # exact: every storage value is a float32
+        total = np.zeros(cols, acc)
+        for r0 in range(0, rows, 256):
+            chunk = np.zeros(cols, acc)
+            for q0 in range(r0, min(r0 + 256, rows), 64 if rows > 256 else 256):
+                run = np.zeros(cols, acc)
+                for row in wide[q0:min(q0 + (64 if rows > 256 else 256), r0 + 256)]:
+                    run += row
+                chunk += run
+            total += chunk
+        want = oracle.to_storage(total.astype(np.float64), dt)
+        assert np.array_equal(do.numpy(), want)
+        capi.check(L().rp_hip_reduce_rows(do.ptr, dg.ptr, rows, cols, 1, dt), "reduce_rows")
+        assert np.array_equal(do.numpy(), oracle.add(want, want, dt))
+
 
 @pytest.mark.parametrize("dt", ALL, ids=lambda d: NAMES[d])
 def test_fill_and_convert(dt):
