@@ -44,6 +44,7 @@ struct Plan {
     int bm, bn;
     bool a_mc, b_mc, edge;
     const char* name;
+    bool ragged = false;      // rows that are no whole number of 16-byte vectors, or start at any element (16-bit MFMA kernels)
 };
 
 constexpr int SK_MAX_M = 8;           // rows the skinny kernel takes

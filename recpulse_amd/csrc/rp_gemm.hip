@@ -59,10 +59,20 @@ static void choose_tile16(Plan& p, int batch, int m, int k, int n) {
     p.edge = (m % p.bm) || (n % p.bn) || (k % M16_BK);
 }
 
+// Tile of the fp32 / fp64 MFMA kernel.
+static void choose_tile_wide(Plan& p, int batch, int m, int k, int n, int dtype) {
+    p.fam = FAM_MFMAW;
+    const long long tiles128 = (long long)((m + 127) / 128) * ((n + 127) / 128) * batch;
+    // a 128 x 128 tile over a 64-wide output would compute and fetch half of it for nothing
+    if (m > 64 && n > 64 && tiles128 >= cu_tiles() / 2) { p.bm = 128; p.bn = 128; p.name = (dtype == RP_DTYPE_FLOAT32) ? "mfma32_128x128" : "mfma64_128x128"; }
+    else { p.bm = 64; p.bn = 64; p.name = (dtype == RP_DTYPE_FLOAT32) ? "mfma32_64x64" : "mfma64_64x64"; }
+    p.edge = (m % p.bm) || (n % p.bn) || (k % (dtype == RP_DTYPE_FLOAT32 ? 32 : 16));
+}
+
 // Decide the kernel family and tile from shapes and strides alone (pointer
 // alignment is checked by the caller, which may still fall back to generic).
 static Plan make_plan(int batch, int m, int k, int n, long long a_rs, long long a_cs, long long b_rs, long long b_cs,
-                      long long c_rs, long long c_cs, long long a_bs, long long b_bs, int dtype, bool allow_direct = true) {
+                      long long c_rs, long long c_cs, long long a_bs, long long b_bs, int dtype, bool allow_direct = true, bool bases_aligned = true) {
     Plan p{FAM_GENERIC, 64, 64, false, false, true, "generic"};
     if (path_disabled("mfma")) return p;
     const int vec = 16 / (int)dtype_size(dtype);                // elements per 16-byte vector
@@ -72,7 +82,7 @@ static Plan make_plan(int batch, int m, int k, int n, long long a_rs, long long 
     bool a_mc = (a_rs == 1) && (a_cs % vec == 0) && (m % vec == 0);
     bool b_mc = (b_cs == 1) && (b_rs % vec == 0) && (n % vec == 0);
     bool b_kc = (b_rs == 1) && (b_cs % vec == 0) && (k % vec == 0);
-    bool batch_ok = (batch == 1) || ((a_bs % vec == 0) && (b_bs % vec == 0));
+    bool batch_ok = bases_aligned && ((batch == 1) || ((a_bs % vec == 0) && (b_bs % vec == 0)));
 
     // the MFMA kernels address a tile with 32-bit byte offsets from a 64-bit tile pointer
     const long long max_stride = 1ll << 22;
@@ -97,7 +107,7 @@ static Plan make_plan(int batch, int m, int k, int n, long long a_rs, long long 
     }
     // VALU skinny: few rows, row-major B, enough columns and depth to be worth streaming
     const int valu_rows = (dtype == RP_DTYPE_FLOAT32) ? SK_MAX_M : 4;
-    if (batch == 1 && dtype != RP_DTYPE_FLOAT64 && m <= valu_rows && b_mc && n >= 64 * vec && (long long)k * n >= (1ll << 20) &&
+    if (batch_ok && batch == 1 && dtype != RP_DTYPE_FLOAT64 && m <= valu_rows && b_mc && n >= 64 * vec && (long long)k * n >= (1ll << 20) &&
         (n + 64 * vec - 1) / (64 * vec) <= SK_MAX_GROUPS) {
         p.fam = FAM_SKINNY; p.name = "skinny"; p.b_mc = true;
         return p;
@@ -145,6 +155,28 @@ static Plan make_plan(int batch, int m, int k, int n, long long a_rs, long long 
         p.fam = FAM_PIPE32K; p.bm = 128; p.bn = 64; p.a_mc = !a_kc; p.b_mc = !b_kc; p.edge = (m % 128) || n != 64; p.name = "pipe32k_128x64";
         return p;
     }
+    if (!mfma_ok && strides_ok && !path_disabled("ragged")) {
+        // Rows that are no whole number of 16-byte vectors or start anywhere: the MFMA kernels' ragged variants.  They need a
+        // vector's worth of elements along the unit-stride axis and rows that do not overlap.  Outputs of less than two
+        // 64 x 64 tiles between small operands stay on the generic kernel, which splits their k over the chip (a handful of
+        // MFMA workgroups would walk it slab by slab).
+        const bool ak = a_cs == 1 && k >= vec && (a_rs >= k || m == 1), am = a_rs == 1 && m >= vec && (a_cs >= m || k == 1);
+        const bool bn = b_cs == 1 && n >= vec && (b_rs >= n || k == 1), bk = b_rs == 1 && k >= vec && (b_cs >= k || n == 1);
+        const bool worth = (long long)m * n * batch >= 8192 || (long long)k * n >= (1 << 18) || (long long)m * k >= (1 << 18);
+        if ((ak || am) && (bn || bk) && worth) {
+            p.ragged = true;
+            p.a_mc = !ak;
+            p.b_mc = bn;
+            if (!is16) {
+                choose_tile_wide(p, batch, m, k, n, dtype);
+            } else if (few_rows && n >= 256 && k >= 1024 && (long long)k * n >= (1ll << 22)) {
+                p.fam = FAM_MFMA16_SKINNY; p.bm = 32; p.bn = 128; p.edge = true; p.name = "mfma16_skinny_32x128";
+            } else {
+                choose_tile16(p, batch, m, k, n);
+            }
+            return p;
+        }
+    }
     if (!mfma_ok) return p;
     p.a_mc = !a_kc;             // when both qualify (extent-1 corner cases) keep the row-major reading
     p.b_mc = b_mc;
@@ -152,12 +184,7 @@ static Plan make_plan(int batch, int m, int k, int n, long long a_rs, long long 
     if (is16) {
         choose_tile16(p, batch, m, k, n);
     } else {
-        p.fam = FAM_MFMAW;
-        long long tiles128 = (long long)((m + 127) / 128) * ((n + 127) / 128) * batch;
-        // a 128 x 128 tile over a 64-wide output would compute and fetch half of it for nothing
-        if (m > 64 && n > 64 && tiles128 >= cu_tiles() / 2) { p.bm = 128; p.bn = 128; p.name = (dtype == RP_DTYPE_FLOAT32) ? "mfma32_128x128" : "mfma64_128x128"; }
-        else { p.bm = 64; p.bn = 64; p.name = (dtype == RP_DTYPE_FLOAT32) ? "mfma32_64x64" : "mfma64_64x64"; }
-        p.edge = (m % p.bm) || (n % p.bn) || (k % (dtype == RP_DTYPE_FLOAT32 ? 32 : 16));
+        choose_tile_wide(p, batch, m, k, n, dtype);
     }
     return p;
 }
@@ -186,7 +213,8 @@ static int run_gemm(const GemmArgs& g, int dtype) {
         if (direct32_takes(g)) { g_last_kernel = p.name; return launch_direct32(g); }
         p = make_plan(g.batch, g.m, g.k, g.n, g.a_rs, g.a_cs, g.b_rs, g.b_cs, g.c_rs, g.c_cs, g.a_bs, g.b_bs, dtype, false);     // base pointers or spans it cannot address
     }
-    if (p.fam != FAM_GENERIC && p.fam != FAM_TINY && !(aligned16(g.A) && aligned16(g.B))) { p.fam = FAM_GENERIC; p.name = "generic"; }
+    if (p.fam != FAM_GENERIC && p.fam != FAM_TINY && !p.ragged && !(aligned16(g.A) && aligned16(g.B)))
+        p = make_plan(g.batch, g.m, g.k, g.n, g.a_rs, g.a_cs, g.b_rs, g.b_cs, g.c_rs, g.c_cs, g.a_bs, g.b_bs, dtype, false, false);
     g_last_kernel = p.name;
     switch (p.fam) {
         case FAM_MFMA16:

@@ -1,8 +1,19 @@
-// bf16 / fp16 MFMA GEMM, 256 x 256 block tile (2 x 2 waves).
-#include "rp_gemm_mfma16_kernel.h"
+// bf16 / fp16 MFMA GEMM, 256 x 256 block tile: selection across its translation units (each kernel of this tile compiles
+// for about twenty seconds).
+#include "rp_gemm.h"
 
 namespace rp {
 
-int launch_mfma16_256(const GemmArgs& g, const Plan& p, int dtype) { return m16_launch_tile_dtype<256, 256, 2>(g, p, dtype); }
+int launch_mfma16_256_bf16(const GemmArgs& g, const Plan& p);
+int launch_mfma16_256_ragged_bf16(const GemmArgs& g, const Plan& p);
+int launch_mfma16_256_f16(const GemmArgs& g, const Plan& p);
+int launch_mfma16_256_ragged_f16(const GemmArgs& g, const Plan& p);
+
+int launch_mfma16_256(const GemmArgs& g, const Plan& p, int dtype) {
+    if (dtype == RP_DTYPE_BFLOAT16) return p.ragged ? launch_mfma16_256_ragged_bf16(g, p) : launch_mfma16_256_bf16(g, p);
+    if (dtype == RP_DTYPE_FLOAT16) return p.ragged ? launch_mfma16_256_ragged_f16(g, p) : launch_mfma16_256_f16(g, p);
+    set_error("mfma16 GEMM: unsupported dtype %d", dtype);
+    return -1;
+}
 
 }  // namespace rp

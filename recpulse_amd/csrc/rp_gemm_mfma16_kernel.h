@@ -140,7 +140,23 @@ struct FragMap {
     }
 };
 
-template <typename T, int BM, int BN, int WGM, bool A_MC, bool B_MC, bool EDGE, bool SPLITK>
+// EDGE: what of the tile may hang over the problem.
+enum { M16_WHOLE = 0, M16_EDGE = 1, M16_RAGGED = 2 };
+// M16_WHOLE: nothing.  M16_EDGE: m, n or k end inside a tile, in whole 16-byte vectors.  M16_RAGGED: anywhere, and rows may
+// start at any element (16-byte loads are issued at 2-byte alignment, which the memory path takes).  There a vector may
+// straddle the end of its row.  Past the end of a free axis that is harmless (the neighbouring row's values land in rows
+// or columns of the tile that are never stored), past the end of k it is not, and past the operand's last element it
+// would leave the buffer.  Both can only happen in the last slab, so there a straddling vector is loaded `pull` elements
+// further back, where it ends with the row, and shifted into place (zeros behind it) on its way to LDS.
+// Requires at least 8 elements along the unit-stride axis, and rows (or k rows) that do not overlap.
+//
+// `v` with its elements (16 bits each) moved down by `pull` < 8
+__device__ __forceinline__ u32x4_t m16_pull_shift(u32x4_t v, int pull) {
+    return __builtin_bit_cast(u32x4_t, __builtin_bit_cast(unsigned __int128, v) >> (16 * pull));
+}
+typedef unsigned int u32x4_any_t __attribute__((ext_vector_type(4), aligned(2)));       // a 16-byte vector at any element
+
+template <typename T, int BM, int BN, int WGM, bool A_MC, bool B_MC, int EDGE, bool SPLITK>
 __global__ void __launch_bounds__(256) gemm_mfma16_kernel(GemmArgs g, int tiles_m, int tiles_n, float* partials, int k_per_split, int sched_total) {
     constexpr int WGN = 4 / WGM;
     constexpr int WM = BM / WGM, WN = BN / WGN;       // wave patch
@@ -209,6 +225,7 @@ __global__ void __launch_bounds__(256) gemm_mfma16_kernel(GemmArgs g, int tiles_
     // Per-thread piece offsets (bytes from the slab pointer).  The buffer descriptor ends at the operand's last
     // element, which zero-fills rows past the free extent (KC) or k past the end (MC); the other axis of each
     // layout is masked explicitly by swapping in an offset no descriptor covers.
+    constexpr int BACK = EDGE == M16_RAGGED ? 16 : 0;        // the descriptors start this many bytes early, so that pulled-back offsets stay positive
     uint32_t a_goff[NA], b_goff[NB];
     int a_r0, a_kk0, b_r0, b_kk0;
     MapA::coords0(t, a_r0, a_kk0);
@@ -216,13 +233,13 @@ __global__ void __launch_bounds__(256) gemm_mfma16_kernel(GemmArgs g, int tiles_
 #pragma unroll
     for (int i = 0; i < NA; i++) {
         int r = a_r0 + (A_MC ? 0 : i * MapA::PIECE_ROWS), kk = a_kk0 + (A_MC ? i * MapA::PIECE_ROWS : 0);
-        a_goff[i] = (uint32_t)(((long long)r * a_fs + (long long)kk * a_ks) * 2);
+        a_goff[i] = (uint32_t)(((long long)r * a_fs + (long long)kk * a_ks) * 2) + BACK;
         if (EDGE && A_MC && m0 + r >= g.m) a_goff[i] = BUFFER_OOB;
     }
 #pragma unroll
     for (int i = 0; i < NB; i++) {
         int r = b_r0 + (B_MC ? 0 : i * MapB::PIECE_ROWS), kk = b_kk0 + (B_MC ? i * MapB::PIECE_ROWS : 0);
-        b_goff[i] = (uint32_t)(((long long)r * b_fs + (long long)kk * b_ks) * 2);
+        b_goff[i] = (uint32_t)(((long long)r * b_fs + (long long)kk * b_ks) * 2) + BACK;
         if (EDGE && B_MC && n0 + r >= g.n) b_goff[i] = BUFFER_OOB;
         if (n_segmented) {
             const int j = n0 + r, seg = j / g.seg_n, c = j - seg * g.seg_n;
@@ -243,12 +260,20 @@ __global__ void __launch_bounds__(256) gemm_mfma16_kernel(GemmArgs g, int tiles_
 
     u32x4_t ra[NA], rb[NB];
     const int nslabs = (kend - kbeg + M16_BK - 1) / M16_BK;
+    // M16_RAGGED: how many elements of this thread's vectors stick out of their row in the last slab (0: none or all)
+    int a_pull = 0, b_pull = 0;
+    if constexpr (EDGE == M16_RAGGED) {
+        const int klast = kend - kbeg - (nslabs - 1) * M16_BK;
+        const int a_in = A_MC ? g.m - m0 - a_r0 : klast - a_kk0, b_in = B_MC ? g.n - n0 - b_r0 : klast - b_kk0;
+        a_pull = a_in > 0 && a_in < 8 ? 8 - a_in : 0;
+        b_pull = b_in > 0 && b_in < 8 ? 8 - b_in : 0;
+    }
     __amdgpu_buffer_rsrc_t a_rsrc, b_rsrc;
     int kleft = 0;        // k still in range counted from the slab the descriptors point at (EDGE, KC operands)
 
     auto point_at_slab = [&](int k0) {
-        a_rsrc = buffer_rsrc(a_slab, EDGE ? (long long)(a_end - a_slab) : 0x7fffffffll);
-        b_rsrc = buffer_rsrc(b_slab, EDGE ? (long long)(b_end - b_slab) : 0x7fffffffll);
+        a_rsrc = buffer_rsrc(a_slab - BACK, EDGE ? (long long)(a_end - a_slab) + BACK : 0x7fffffffll);
+        b_rsrc = buffer_rsrc(b_slab - BACK, EDGE ? (long long)(b_end - b_slab) + BACK : 0x7fffffffll);
         kleft = kend - kbeg - k0;
     };
     // Without edges piece i sits a uniform number of bytes after piece 0: one lane offset per operand plus a scalar
@@ -262,6 +287,7 @@ __global__ void __launch_bounds__(256) gemm_mfma16_kernel(GemmArgs g, int tiles_
         } else {
             uint32_t off = a_goff[i];
             if (!A_MC && a_kk0 >= kleft) off = BUFFER_OOB;
+            if (EDGE == M16_RAGGED && kleft <= M16_BK) off -= 2 * a_pull;
             ra[i] = __builtin_amdgcn_raw_buffer_load_b128(a_rsrc, (int)off, 0, 0);
         }
     };
@@ -272,15 +298,18 @@ __global__ void __launch_bounds__(256) gemm_mfma16_kernel(GemmArgs g, int tiles_
         } else {
             uint32_t off = b_goff[i];
             if (!B_MC && b_kk0 >= kleft) off = BUFFER_OOB;
+            if (EDGE == M16_RAGGED && kleft <= M16_BK) off -= 2 * b_pull;
             rb[i] = __builtin_amdgcn_raw_buffer_load_b128(b_rsrc, (int)off, 0, 0);
         }
     };
-    auto store_piece_a = [&](uint16_t* stage, auto ic) {
+    auto store_piece_a = [&](uint16_t* stage, auto ic, auto last_tag) {
         constexpr int i = decltype(ic)::value;
+        if constexpr (EDGE == M16_RAGGED && decltype(last_tag)::value) ra[i] = m16_pull_shift(ra[i], a_pull);
         *(u32x4_t*)(stage + a_wr0 + i * MapA::LDS_STEP) = ra[i];
     };
-    auto store_piece_b = [&](uint16_t* stage, auto ic) {
+    auto store_piece_b = [&](uint16_t* stage, auto ic, auto last_tag) {
         constexpr int i = decltype(ic)::value;
+        if constexpr (EDGE == M16_RAGGED && decltype(last_tag)::value) rb[i] = m16_pull_shift(rb[i], b_pull);
         *(u32x4_t*)(stage + b_wr0 + i * MapB::LDS_STEP) = rb[i];
     };
 
@@ -312,8 +341,12 @@ __global__ void __launch_bounds__(256) gemm_mfma16_kernel(GemmArgs g, int tiles_
     static_for<0, NA>([&](auto ic) { load_piece_a(ic); });
     static_for<0, NB>([&](auto ic) { load_piece_b(ic); });
     if (tile_id != first_slot) __syncthreads();            // the previous tile's epilogue has read its staged rows out of LDS
-    static_for<0, NA>([&](auto ic) { store_piece_a(smem, ic); });
-    static_for<0, NB>([&](auto ic) { store_piece_b(smem, ic); });
+    auto store_first = [&](auto last_tag) {
+        static_for<0, NA>([&](auto ic) { store_piece_a(smem, ic, last_tag); });
+        static_for<0, NB>([&](auto ic) { store_piece_b(smem, ic, last_tag); });
+    };
+    if (EDGE == M16_RAGGED && nslabs == 1) store_first(std::true_type{});
+    else store_first(std::false_type{});
     a_slab += a_step;
     advance_b();
     if (nslabs > 1) {
@@ -327,10 +360,10 @@ __global__ void __launch_bounds__(256) gemm_mfma16_kernel(GemmArgs g, int tiles_
     static_for<0, RD_A + RD_B>([&](auto rc) { read_item(smem, I0{}, I0{}, rc); });
 
     // Pieces of both operands in one list: 0 .. NA-1 are A's, NA .. NA+NB-1 are B's.
-    auto store_piece = [&](uint16_t* stage, auto pc) {
+    auto store_piece = [&](uint16_t* stage, auto pc, auto last_tag) {
         constexpr int p = decltype(pc)::value;
-        if constexpr (p < NA) store_piece_a(stage, std::integral_constant<int, p>{});
-        else store_piece_b(stage, std::integral_constant<int, p - NA>{});
+        if constexpr (p < NA) store_piece_a(stage, std::integral_constant<int, p>{}, last_tag);
+        else store_piece_b(stage, std::integral_constant<int, p - NA>{}, last_tag);
     };
     auto load_piece = [&](auto pc) {
         constexpr int p = decltype(pc)::value;
@@ -346,6 +379,7 @@ __global__ void __launch_bounds__(256) gemm_mfma16_kernel(GemmArgs g, int tiles_
                      const uint16_t* rd_stage, uint16_t* wr_stage) {
         constexpr int MSLOT = decltype(mslotc)::value;
         constexpr bool DO_READ = decltype(readc)::value, WR = decltype(wrc)::value, LD = decltype(ldc)::value;
+        constexpr std::integral_constant<bool, WR && !LD> last{};            // what is written to LDS is the last slab: no further one is requested
         constexpr int P0 = decltype(p0c)::value, NP = decltype(p1c)::value - P0;
         constexpr int NR = DO_READ ? RD_A + RD_B : 0;
         static_for<0, NMFMA>([&](auto qc) {
@@ -375,7 +409,7 @@ __global__ void __launch_bounds__(256) gemm_mfma16_kernel(GemmArgs g, int tiles_
                 }
                 if constexpr (j == 1 || j == 3) {
                     constexpr int p = P0 + i * PPR + (j == 3 ? 1 : 0);
-                    if constexpr (WR && (j == 1 || PPR == 2) && p < P0 + NP) store_piece(wr_stage, std::integral_constant<int, p>{});
+                    if constexpr (WR && (j == 1 || PPR == 2) && p < P0 + NP) store_piece(wr_stage, std::integral_constant<int, p>{}, last);
                 }
                 if constexpr (j == 4 || j == 5) {
                     constexpr int p = P0 + i * PPR + (j == 5 ? 1 : 0);
@@ -390,7 +424,7 @@ __global__ void __launch_bounds__(256) gemm_mfma16_kernel(GemmArgs g, int tiles_
                 constexpr int D = NMFMA - 1;
                 if constexpr (q < D) {
                     static_for<P0 + (NP * q) / D, P0 + (NP * (q + 1)) / D>([&](auto pc) {
-                        if constexpr (WR) store_piece(wr_stage, pc);
+                        if constexpr (WR) store_piece(wr_stage, pc, last);
                     });
                 }
                 if constexpr (q > 0) {
@@ -400,7 +434,7 @@ __global__ void __launch_bounds__(256) gemm_mfma16_kernel(GemmArgs g, int tiles_
                 }
             } else {
                 static_for<P0 + (NP * q) / NMFMA, P0 + (NP * (q + 1)) / NMFMA>([&](auto pc) {
-                    if constexpr (WR) store_piece(wr_stage, pc);
+                    if constexpr (WR) store_piece(wr_stage, pc, last);
                     if constexpr (LD) load_piece(pc);
                 });
             }
@@ -535,6 +569,20 @@ __global__ void __launch_bounds__(256) gemm_mfma16_kernel(GemmArgs g, int tiles_
                     memcpy(&o, out, 16);
                 }
                 __builtin_nontemporal_store(o, (u32x4_t*)(crow + gn_out));  // written once, never re-read: keep it out of the way of the operand panels in L2
+            } else if (EDGE && g.c_cs == 1 && gn + 8 <= g.n) {
+                // rows of C that start at any element: the same vector, unaligned (a plain store: the L2 joins the
+                // partial cache lines of neighbouring lanes and rows)
+                u32x4_t o = staged;
+                if (accum) {
+                    T y[8], old[8], out[8];
+                    const u32x4_t was = *(const u32x4_any_t*)(crow + gn);
+                    memcpy(y, &staged, 16);
+                    memcpy(old, &was, 16);
+#pragma unroll
+                    for (int e = 0; e < 8; e++) out[e] = narrow<T>(widen(old[e]) + widen(y[e]));
+                    memcpy(&o, out, 16);
+                }
+                *(u32x4_any_t*)(crow + gn) = o;
             } else {
                 T y[8];
                 memcpy(y, &staged, 16);
@@ -572,9 +620,13 @@ __global__ void __launch_bounds__(256) gemm_mfma16_kernel(GemmArgs g, int tiles_
             for (int r = erow; r < WM; r += RPS) {
                 const int gm = m0 + wm0 + r;
                 if (EDGE && gm >= g.m) break;
-                // n is a multiple of 8 on this path, so the 8 columns are all in or all out
-                if (!EDGE || gn + 8 <= g.n) {
-                    float* prow = partials + (((long long)z * gridDim.z + blockIdx.z) * g.m + gm) * g.n + gn;
+                float* prow = partials + (((long long)z * gridDim.z + blockIdx.z) * g.m + gm) * g.n + gn;
+                if (EDGE == M16_RAGGED) {
+                    const float* src = region + r * EP + ecol;
+                    if (gn + 8 <= g.n) memcpy(prow, src, 32);
+                    else
+                        for (int e = 0; e < 8 && gn + e < g.n; e++) prow[e] = src[e];
+                } else if (!EDGE || gn + 8 <= g.n) {          // n is a multiple of 8, so the 8 columns are all in or all out
                     *(f32x4_t*)prow = *(const f32x4_t*)(region + r * EP + ecol);
                     *(f32x4_t*)(prow + 4) = *(const f32x4_t*)(region + r * EP + ecol + 4);
                 }
@@ -585,7 +637,7 @@ __global__ void __launch_bounds__(256) gemm_mfma16_kernel(GemmArgs g, int tiles_
 }
 
 // Launch one instantiation.  nsplit > 1 selects the split-k variant: partials must hold batch * nsplit * m * n floats.
-template <typename T, int BM, int BN, int WGM, bool A_MC, bool B_MC, bool EDGE, bool SPLITK>
+template <typename T, int BM, int BN, int WGM, bool A_MC, bool B_MC, int EDGE, bool SPLITK>
 static int m16_launch(const GemmArgs& g, float* partials, int nsplit, int k_per_split) {
     int tiles_m = (g.m + BM - 1) / BM, tiles_n = (g.n + BN - 1) / BN;
     const int sched_total = scheduled_grid(tiles_m, tiles_n);
@@ -604,18 +656,19 @@ static int m16_launch(const GemmArgs& g, float* partials, int nsplit, int k_per_
 }
 
 // Layout and edge dispatch for one tile shape (no split-k).
+template <typename T, int BM, int BN, int WGM, int EDGE>
+static int m16_launch_layout(const GemmArgs& g, const Plan& p) {
+    if (!p.a_mc && p.b_mc) return m16_launch<T, BM, BN, WGM, false, true, EDGE, false>(g, nullptr, 1, 0);
+    if (!p.a_mc && !p.b_mc) return m16_launch<T, BM, BN, WGM, false, false, EDGE, false>(g, nullptr, 1, 0);
+    if (p.a_mc && p.b_mc) return m16_launch<T, BM, BN, WGM, true, true, EDGE, false>(g, nullptr, 1, 0);
+    return m16_launch<T, BM, BN, WGM, true, false, EDGE, false>(g, nullptr, 1, 0);
+}
+
 template <typename T, int BM, int BN, int WGM>
 static int m16_launch_tile(const GemmArgs& g, const Plan& p) {
-    if (p.edge) {
-        if (!p.a_mc && p.b_mc) return m16_launch<T, BM, BN, WGM, false, true, true, false>(g, nullptr, 1, 0);
-        if (!p.a_mc && !p.b_mc) return m16_launch<T, BM, BN, WGM, false, false, true, false>(g, nullptr, 1, 0);
-        if (p.a_mc && p.b_mc) return m16_launch<T, BM, BN, WGM, true, true, true, false>(g, nullptr, 1, 0);
-        return m16_launch<T, BM, BN, WGM, true, false, true, false>(g, nullptr, 1, 0);
-    }
-    if (!p.a_mc && p.b_mc) return m16_launch<T, BM, BN, WGM, false, true, false, false>(g, nullptr, 1, 0);
-    if (!p.a_mc && !p.b_mc) return m16_launch<T, BM, BN, WGM, false, false, false, false>(g, nullptr, 1, 0);
-    if (p.a_mc && p.b_mc) return m16_launch<T, BM, BN, WGM, true, true, false, false>(g, nullptr, 1, 0);
-    return m16_launch<T, BM, BN, WGM, true, false, false, false>(g, nullptr, 1, 0);
+    if (p.ragged) return m16_launch_layout<T, BM, BN, WGM, M16_RAGGED>(g, p);
+    if (p.edge) return m16_launch_layout<T, BM, BN, WGM, M16_EDGE>(g, p);
+    return m16_launch_layout<T, BM, BN, WGM, M16_WHOLE>(g, p);
 }
 
 template <int BM, int BN, int WGM>

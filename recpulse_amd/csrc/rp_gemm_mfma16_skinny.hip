@@ -10,18 +10,18 @@
 
 namespace rp {
 
-template <typename T>
+template <typename T, int EDGE>
 static int launch_skinny16_t(const GemmArgs& g, const Plan& p, float* partials, int nsplit, int k_per_split) {
     constexpr int BM = 32, BN = 128, WGM = 1;
-    if (!p.a_mc && p.b_mc) return m16_launch<T, BM, BN, WGM, false, true, true, true>(g, partials, nsplit, k_per_split);
-    if (!p.a_mc && !p.b_mc) return m16_launch<T, BM, BN, WGM, false, false, true, true>(g, partials, nsplit, k_per_split);
-    if (p.a_mc && p.b_mc) return m16_launch<T, BM, BN, WGM, true, true, true, true>(g, partials, nsplit, k_per_split);
-    return m16_launch<T, BM, BN, WGM, true, false, true, true>(g, partials, nsplit, k_per_split);
+    if (!p.a_mc && p.b_mc) return m16_launch<T, BM, BN, WGM, false, true, EDGE, true>(g, partials, nsplit, k_per_split);
+    if (!p.a_mc && !p.b_mc) return m16_launch<T, BM, BN, WGM, false, false, EDGE, true>(g, partials, nsplit, k_per_split);
+    if (p.a_mc && p.b_mc) return m16_launch<T, BM, BN, WGM, true, true, EDGE, true>(g, partials, nsplit, k_per_split);
+    return m16_launch<T, BM, BN, WGM, true, false, EDGE, true>(g, partials, nsplit, k_per_split);
 }
 
 int launch_mfma16_skinny(const GemmArgs& g, const Plan& p, int dtype) {
     if (dtype != RP_DTYPE_BFLOAT16 && dtype != RP_DTYPE_FLOAT16) { set_error("mfma16 skinny GEMM: unsupported dtype %d", dtype); return -1; }
-    if (!p.a_mc && p.b_mc && stream128_takes(g)) return launch_stream128(g, dtype);
+    if (!p.ragged && !p.a_mc && p.b_mc && stream128_takes(g)) return launch_stream128(g, dtype);
     constexpr int BN = 128;
     const int tiles = ((g.n + BN - 1) / BN) * ((g.m + 31) / 32) * g.batch;
     // about three blocks per CU in flight, each split at least four slabs deep
@@ -33,8 +33,9 @@ int launch_mfma16_skinny(const GemmArgs& g, const Plan& p, int dtype) {
     void* ws = nullptr;
     if (gemm_workspace(&ws, (size_t)g.batch * nsplit * g.m * g.n * sizeof(float)) != 0) return -1;
     int rc;
-    if (dtype == RP_DTYPE_BFLOAT16) rc = launch_skinny16_t<bf16_t>(g, p, (float*)ws, nsplit, k_per_split);
-    else rc = launch_skinny16_t<f16_t>(g, p, (float*)ws, nsplit, k_per_split);
+    const bool bf = dtype == RP_DTYPE_BFLOAT16;
+    if (p.ragged) rc = bf ? launch_skinny16_t<bf16_t, M16_RAGGED>(g, p, (float*)ws, nsplit, k_per_split) : launch_skinny16_t<f16_t, M16_RAGGED>(g, p, (float*)ws, nsplit, k_per_split);
+    else rc = bf ? launch_skinny16_t<bf16_t, M16_EDGE>(g, p, (float*)ws, nsplit, k_per_split) : launch_skinny16_t<f16_t, M16_EDGE>(g, p, (float*)ws, nsplit, k_per_split);
     if (rc == 0) rc = launch_splitk_combine(g, (const float*)ws, nsplit, g.m, dtype);
     gemm_workspace_release(ws);          // back to the pool while the kernels are still queued: safe for later work on this stream; held with the graph while one is being recorded
     return rc;

@@ -28,10 +28,16 @@ template <> struct mfmaw_cfg<double> {
     static __device__ __forceinline__ int acc_row(int v, int lane) { return 4 * v + (lane >> 4); }
 };
 
+// What of a tile may hang over the problem: nothing; m, n or k ending inside it in whole 16-byte vectors; or ending
+// anywhere, with rows that start at any element.  In the last case a vector that straddles the end of its row (of k, or of
+// the free axis) is loaded `pull` elements further back, so that it ends with the row, and shifted into place with zeros
+// behind it on its way to LDS.  It takes at least a vector's worth of elements along the unit-stride axis.
+enum { MW_WHOLE = 0, MW_EDGE = 1, MW_RAGGED = 2 };
+
 // One operand's slab traffic, a 16-byte piece per thread at a time: piece i of thread t covers V consecutive
 // elements along the operand's unit-stride axis.  LDS is k-major, [BK][ROWS + PAD]; a KC piece (V consecutive k
 // of one row) is transposed on the way in with V scalar writes.
-template <typename T, int ROWS, bool MC, bool EDGE>
+template <typename T, int ROWS, bool MC, int EDGE>
 struct MwSlab {
     using cfg = mfmaw_cfg<T>;
     static constexpr int V = cfg::VEC, NP = ROWS * cfg::BK / V / 256, PITCH = ROWS + cfg::PAD;
@@ -46,7 +52,19 @@ struct MwSlab {
         int r, kk;
         coords(t, i, r, kk);
         if (EDGE && !((row0 + r < free_extent) && (k0 + kk < k_extent))) return uint4{0u, 0u, 0u, 0u};
-        return load_at(base + (long long)(row0 + r) * free_stride + (long long)(k0 + kk) * k_stride);
+        return load_at(base + (long long)(row0 + r) * free_stride + (long long)(k0 + kk) * k_stride - pull(row0, k0, free_extent, k_extent, t, i));
+    }
+    static __device__ __forceinline__ int pull(int row0, int k0, int free_extent, int k_extent, int t, int i) {
+        if (EDGE != MW_RAGGED || (MC ? row0 + ROWS <= free_extent : k0 + cfg::BK <= k_extent)) return 0;       // (uniform: no vector of this slab straddles)
+        int r, kk;
+        coords(t, i, r, kk);
+        const int in = MC ? free_extent - row0 - r : k_extent - k0 - kk;
+        return in > 0 && in < V ? V - in : 0;
+    }
+    // a piece on its way to LDS: straddling vectors into place
+    static __device__ __forceinline__ uint4 settle(uint4 raw, int row0, int k0, int free_extent, int k_extent, int t, int i) {
+        if (EDGE != MW_RAGGED || (MC ? row0 + ROWS <= free_extent : k0 + cfg::BK <= k_extent)) return raw;
+        return __builtin_bit_cast(uint4, __builtin_bit_cast(unsigned __int128, raw) >> (8 * (int)sizeof(T) * pull(row0, k0, free_extent, k_extent, t, i)));
     }
     // the same piece with the offset of its free index given (a free axis that is a list of segments)
     static __device__ __forceinline__ uint4 load_free_at(const T* base, long long free_offset, long long k_stride, int row0, int k0,
@@ -97,7 +115,7 @@ __host__ __device__ constexpr size_t mw_smem_bytes(int bm, int bn) {
     return loop > epi ? loop : epi;
 }
 
-template <typename T, int BM, int BN, bool A_MC, bool B_MC, bool EDGE, bool SPLITK>
+template <typename T, int BM, int BN, bool A_MC, bool B_MC, int EDGE, bool SPLITK>
 __global__ void __launch_bounds__(256, 2) gemm_mfmaw_kernel(GemmArgs g, int tiles_m, int tiles_n, float* partials, int k_per_split) {
     using cfg = mfmaw_cfg<T>;
     constexpr int MT = cfg::MT, BK = cfg::BK, NKS = BK / cfg::KS;
@@ -162,10 +180,10 @@ __global__ void __launch_bounds__(256, 2) gemm_mfmaw_kernel(GemmArgs g, int tile
             regs[p] = SlabB::load(base, b_fs, b_ks, n0, k0, g.n, klen, t, p - NA);
         }
     };
-    auto store_piece = [&](auto pc, T* stage) {
+    auto store_piece = [&](auto pc, T* stage, int k0) {
         constexpr int p = decltype(pc)::value;
-        if constexpr (p < NA) SlabA::store(stage, regs[p], t, p);
-        else SlabB::store(stage + A_ELEMS, regs[p], t, p - NA);
+        if constexpr (p < NA) SlabA::store(stage, SlabA::settle(regs[p], m0, k0, g.m, klen, t, p), t, p);
+        else SlabB::store(stage + A_ELEMS, SlabB::settle(regs[p], n0, k0, g.n, klen, t, p - NA), t, p - NA);
     };
 
     const int lf = lane % MT, lk = lane / MT;         // lane's free index and k index inside one MFMA
@@ -180,7 +198,7 @@ __global__ void __launch_bounds__(256, 2) gemm_mfmaw_kernel(GemmArgs g, int tile
 
     // prologue: slab 0 into stage 0, slab 1 into registers, fragments(0) of slab 0
     static_for<0, NP_ALL>([&](auto pc) { load_piece(pc, 0); });
-    static_for<0, NP_ALL>([&](auto pc) { store_piece(pc, smem); });
+    static_for<0, NP_ALL>([&](auto pc) { store_piece(pc, smem, 0); });
     if (nslabs > 1) static_for<0, NP_ALL>([&](auto pc) { load_piece(pc, BK); });
     __syncthreads();
     read_frags(smem, 0, 0);
@@ -200,7 +218,7 @@ __global__ void __launch_bounds__(256, 2) gemm_mfmaw_kernel(GemmArgs g, int tile
                 constexpr int P0 = (NP_ALL * ks) / (NKS - 1), P1 = (NP_ALL * (ks + 1)) / (NKS - 1);
                 if constexpr (NEXT) {
                     static_for<P0, P1>([&](auto pc) {
-                        store_piece(pc, other);
+                        store_piece(pc, other, (s + 1) * BK);
                         if constexpr (NEXT2) load_piece(pc, (s + 2) * BK);
                     });
                 }
@@ -263,8 +281,15 @@ __global__ void __launch_bounds__(256, 2) gemm_mfmaw_kernel(GemmArgs g, int tile
             T vals[V];
             memcpy(vals, &raw, 16);
             if constexpr (SPLITK) {
-                // fp32 partial tile [split][m][n]; n is a multiple of 4 on this path, so the vector is wholly in or out
-                if (!EDGE || gn + V <= g.n) *(uint4*)(partials + (((long long)z * gridDim.z + blockIdx.z) * g.m + gm) * g.n + gn) = raw;
+                // fp32 partial tile [split][m][n]; unless ragged n is a multiple of 4, so the vector is wholly in or out
+                float* prow = partials + (((long long)z * gridDim.z + blockIdx.z) * g.m + gm) * g.n + gn;
+                if (EDGE == MW_RAGGED) {
+                    if (gn + V <= g.n) memcpy(prow, &raw, 16);
+                    else
+                        for (int e = 0; e < V; e++) if (gn + e < g.n) prow[e] = (float)vals[e];
+                } else if (!EDGE || gn + V <= g.n) {
+                    *(uint4*)prow = raw;
+                }
                 continue;
             }
             T* crow = C + (long long)gm * g.c_rs;
@@ -281,6 +306,12 @@ __global__ void __launch_bounds__(256, 2) gemm_mfmaw_kernel(GemmArgs g, int tile
                 uint4 o;
                 memcpy(&o, out, 16);
                 *(uint4*)(crow + gn_out) = o;
+            } else if (EDGE && g.c_cs == 1 && gn + V <= g.n) {          // rows of C that start at any element: the same vector, unaligned
+                T old[V], out[V];
+                if (accum) memcpy(old, crow + gn, 16);
+#pragma unroll
+                for (int e = 0; e < V; e++) out[e] = finish<T>(vals[e], has_bias, bv[e], accum, accum ? old[e] : (T)0);
+                memcpy(crow + gn, out, 16);
             } else {
 #pragma unroll
                 for (int e = 0; e < V; e++) {
@@ -431,7 +462,7 @@ static int mw_launch_shortk(const GemmArgs& g, bool edge) {
     return launch(gemm_mfmaw_shortk_kernel<T, BM, BN, A_MC, B_MC, false>);
 }
 
-template <typename T, int BM, int BN, bool A_MC, bool B_MC, bool EDGE, bool SPLITK>
+template <typename T, int BM, int BN, bool A_MC, bool B_MC, int EDGE, bool SPLITK>
 static int mw_launch(const GemmArgs& g, dim3 grid, int tiles_m, int tiles_n, float* partials, int k_per_split) {
     constexpr size_t smem = mw_smem_bytes<T>(BM, BN);
     auto kern = gemm_mfmaw_kernel<T, BM, BN, A_MC, B_MC, EDGE, SPLITK>;
@@ -441,27 +472,29 @@ static int mw_launch(const GemmArgs& g, dim3 grid, int tiles_m, int tiles_n, flo
 }
 
 template <typename T, int BM, int BN, bool A_MC, bool B_MC>
-static int launch_mfmaw_edge(const GemmArgs& g, bool edge, float* partials, int nsplit, int k_per_split) {
+static int launch_mfmaw_edge(const GemmArgs& g, const Plan& p, float* partials, int nsplit, int k_per_split) {
     int tiles_m = (g.m + BM - 1) / BM, tiles_n = (g.n + BN - 1) / BN;
     if (nsplit > 1) {
-        if constexpr (sizeof(T) == 4) {           // split-k partials are fp32; always the predicated variant
+        if constexpr (sizeof(T) == 4) {           // split-k partials are fp32; always a predicated variant
             dim3 grid(scheduled_grid(tiles_m, tiles_n), g.batch, nsplit);
-            return mw_launch<T, BM, BN, A_MC, B_MC, true, true>(g, grid, tiles_m, tiles_n, partials, k_per_split);
+            if (p.ragged) return mw_launch<T, BM, BN, A_MC, B_MC, MW_RAGGED, true>(g, grid, tiles_m, tiles_n, partials, k_per_split);
+            return mw_launch<T, BM, BN, A_MC, B_MC, MW_EDGE, true>(g, grid, tiles_m, tiles_n, partials, k_per_split);
         }
         set_error("mfmaw GEMM: split-k is fp32 only");
         return -1;
     }
     dim3 grid(scheduled_grid(tiles_m, tiles_n), g.batch);
-    if (edge) return mw_launch<T, BM, BN, A_MC, B_MC, true, false>(g, grid, tiles_m, tiles_n, nullptr, 0);
-    return mw_launch<T, BM, BN, A_MC, B_MC, false, false>(g, grid, tiles_m, tiles_n, nullptr, 0);
+    if (p.ragged) return mw_launch<T, BM, BN, A_MC, B_MC, MW_RAGGED, false>(g, grid, tiles_m, tiles_n, nullptr, 0);
+    if (p.edge) return mw_launch<T, BM, BN, A_MC, B_MC, MW_EDGE, false>(g, grid, tiles_m, tiles_n, nullptr, 0);
+    return mw_launch<T, BM, BN, A_MC, B_MC, MW_WHOLE, false>(g, grid, tiles_m, tiles_n, nullptr, 0);
 }
 
 template <typename T, int BM, int BN>
 static int launch_mfmaw_layout(const GemmArgs& g, const Plan& p, float* partials, int nsplit, int k_per_split) {
-    if (!p.a_mc && p.b_mc) return launch_mfmaw_edge<T, BM, BN, false, true>(g, p.edge, partials, nsplit, k_per_split);
-    if (!p.a_mc && !p.b_mc) return launch_mfmaw_edge<T, BM, BN, false, false>(g, p.edge, partials, nsplit, k_per_split);
-    if (p.a_mc && p.b_mc) return launch_mfmaw_edge<T, BM, BN, true, true>(g, p.edge, partials, nsplit, k_per_split);
-    return launch_mfmaw_edge<T, BM, BN, true, false>(g, p.edge, partials, nsplit, k_per_split);
+    if (!p.a_mc && p.b_mc) return launch_mfmaw_edge<T, BM, BN, false, true>(g, p, partials, nsplit, k_per_split);
+    if (!p.a_mc && !p.b_mc) return launch_mfmaw_edge<T, BM, BN, false, false>(g, p, partials, nsplit, k_per_split);
+    if (p.a_mc && p.b_mc) return launch_mfmaw_edge<T, BM, BN, true, true>(g, p, partials, nsplit, k_per_split);
+    return launch_mfmaw_edge<T, BM, BN, true, false>(g, p, partials, nsplit, k_per_split);
 }
 
 template <typename T>
@@ -471,7 +504,7 @@ static int launch_mfmaw_t(const GemmArgs& g, const Plan& p) {
     // is split the same way while all its tiles together leave CUs idle.
     int nsplit = 1, k_per_split = 0;
     constexpr int BK = mfmaw_cfg<T>::BK;
-    if (sizeof(T) == 4 && p.bm == 64 && g.n % 4 == 0 && g.seg_k == 0 && g.seg_n == 0 && g.c_fold_from == 0 && !g.bias_by_row) {   // (segments and the folded store: never split)
+    if (sizeof(T) == 4 && p.bm == 64 && (g.n % 4 == 0 || p.ragged) && g.seg_k == 0 && g.seg_n == 0 && g.c_fold_from == 0 && !g.bias_by_row) {   // (segments and the folded store: never split)
         int tiles = ((g.m + 63) / 64) * ((g.n + 63) / 64) * g.batch;
         int want = (256 + tiles - 1) / tiles, deep = g.k / (2 * BK);
         nsplit = want < deep ? want : deep;
@@ -492,7 +525,7 @@ static int launch_mfmaw_t(const GemmArgs& g, const Plan& p) {
 
 int launch_mfmaw(const GemmArgs& g, const Plan& p, int dtype) {
     // fp32, k of at most two slabs, at least 128 tiles of 128 x 128: the resident, cross-tile pipelined kernel
-    if (dtype == RP_DTYPE_FLOAT32 && p.bm == 128 && g.k <= 2 * mfmaw_cfg<float>::BK && !path_disabled("shortk") && g.seg_k == 0 && g.seg_n == 0 && g.c_fold_from == 0 && !g.bias_by_row) {
+    if (dtype == RP_DTYPE_FLOAT32 && !p.ragged && p.bm == 128 && g.k <= 2 * mfmaw_cfg<float>::BK && !path_disabled("shortk") && g.seg_k == 0 && g.seg_n == 0 && g.c_fold_from == 0 && !g.bias_by_row) {
         const bool edge = p.edge || g.k != 2 * mfmaw_cfg<float>::BK;
         if (!p.a_mc && p.b_mc) return mw_launch_shortk<float, 128, 128, false, true>(g, edge);
         if (!p.a_mc && !p.b_mc) return mw_launch_shortk<float, 128, 128, false, false>(g, edge);

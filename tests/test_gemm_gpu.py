@@ -540,6 +540,58 @@ def test_wide_tiles_for_outputs_of_at_most_64_rows():
                c_init=None if c0 is None else np.ascontiguousarray(c0[:, cols]), accumulate=epilogue)
 
 
+RAGGED_SHAPES = [  # (batch, m, k, n, kernel): every 16-bit tile, k of one slab and its tails, free axes that end 1 .. 7 past a vector
+    (1, 1000, 9, 9, "mfma16_64x64"), (1, 131, 8, 65, "mfma16_64x64"), (1, 203, 63, 129, "mfma16_64x64"), (3, 121, 65, 71, "mfma16_64x64"),
+    (1, 199, 391, 137, "mfma16_64x64"), (1, 1450, 127, 1403, "mfma16_128x128"), (130, 33, 77, 261, "mfma16_64x128"), (66, 35, 1025, 305, "mfma16_64x256"),
+    (1, 3000, 259, 2821, "mfma16_256x256"), (1, 5, 4099, 1027, "mfma16_skinny_32x128"), (1, 33, 4102, 1035, "mfma16_skinny_32x128")]
+
+
+RAGGED_WIDE_SHAPES = [  # the same for fp32 (with and without a k split) and fp64
+    (F32, 1, 600, 33, 517, "mfma32_64x64"), (F32, 1, 530, 261, 527, "mfma32_64x64"), (F32, 70, 65, 7, 71, "mfma32_64x64"), (F32, 1, 1450, 67, 1403, "mfma32_128x128"),
+    (F64, 1, 131, 5, 67, "mfma64_64x64"), (F64, 3, 121, 65, 71, "mfma64_64x64"), (F64, 1, 1450, 33, 1403, "mfma64_128x128")]
+
+
+@pytest.mark.parametrize("layout", LAYOUTS)
+@pytest.mark.parametrize("dt,batch,m,k,n,kernel", [(dt,) + shape for dt in HALF for shape in RAGGED_SHAPES] + RAGGED_WIDE_SHAPES)
+def test_ragged_rows(dt, batch, m, k, n, kernel, layout):
+    """Rows at any element and of any length on the MFMA kernels.  The operands are slices of NaN-filled arrays that end
+    with the operand's last element, so a value taken from outside the slice shows; integers, so the bits are known."""
+    rng = np.random.default_rng(46)
+    fill = oracle.to_storage(np.full(1, np.nan), dt)[0]
+    es = capi.DTYPE_SIZE[dt]
+
+    def operand(rows, cols):                       # [batch, rows, cols], pitch cols + 3, everything around it NaN, nothing after it
+        flat = np.full(1 + batch * rows * (cols + 3) - 3, fill)
+        view = np.lib.stride_tricks.as_strided(flat[1:], (batch, rows, cols), (rows * (cols + 3) * es, (cols + 3) * es, es))
+        vals = rng.integers(-2, 3, (batch, rows, cols)).astype(np.float64)
+        view[...] = oracle.to_storage(vals, dt)
+        return capi.DeviceBuffer.from_numpy(flat), vals, (rows * (cols + 3), cols + 3, 1)
+
+    da, a64, a_st = operand(m, k) if layout[0] == "n" else operand(k, m)
+    db, b64, b_st = operand(k, n) if layout[1] == "n" else operand(n, k)
+    if layout[0] == "t":
+        a64, a_st = a64.transpose(0, 2, 1), (a_st[0], a_st[2], a_st[1])
+    if layout[1] == "t":
+        b64, b_st = b64.transpose(0, 2, 1), (b_st[0], b_st[2], b_st[1])
+    exact = np.matmul(a64, b64)
+    bias = oracle.to_storage(rng.integers(-2, 3, n).astype(np.float64), dt)
+    dbias = capi.DeviceBuffer.from_numpy(bias)
+    pitch = n + 5
+    c0 = oracle.to_storage(rng.integers(-2, 3, (batch, m, pitch)).astype(np.float64), dt)
+    for with_bias, accumulate in ((False, False), (True, True)):
+        dc = capi.DeviceBuffer.from_numpy(c0)
+        capi.gemm(dc.at(es), da.at(es), db.at(es), dbias.ptr if with_bias else None, batch, m, k, n, a_st, b_st, (m * pitch, pitch, 1), accumulate, dt)
+        assert capi.last_gemm_kernel() == ("generic" if layout[0] == "t" and m < 8 else kernel)      # fewer than a vector of rows to load along
+        want = oracle.to_storage(exact, dt)
+        if with_bias:
+            want = oracle.to_storage(oracle.to_f64(want, dt) + oracle.to_f64(bias, dt), dt)
+        expect = c0.reshape(-1).copy()
+        inner = np.lib.stride_tricks.as_strided(expect[1:], (batch, m, n), (m * pitch * es, pitch * es, es))
+        inner[...] = oracle.to_storage(oracle.to_f64(inner.copy(), dt) + oracle.to_f64(want, dt), dt) if accumulate else want
+        assert np.array_equal(dc.to_numpy(c0.dtype, (expect.size,)), expect)      # C, and nothing around it
+        dc.free()
+
+
 @pytest.mark.parametrize("dt", ALL, ids=lambda d: NAMES[d])
 def test_linear_backward_in_one_call(dt):
     """rp_hip_linear_backward against two GEMM calls with swapped strides and rp_hip_reduce_rows: the same bits,
