@@ -607,11 +607,13 @@ static int launch_column_sums(T* out, const T* grad, int rows, int cols, int acc
                            out, (A*)nullptr, grad, rows, cols, accumulate);
         return check_launch("column_sums_kernel") ? 0 : -1;
     }
-    if (chunks > 65535) { set_error("rp_hip_reduce_rows: too many rows (%d)", rows); return -1; }
     void* ws = nullptr;
     if (rp_hip_malloc(&ws, (size_t)chunks * cols * sizeof(A)) != 0) return -1;
     using Tile = ColumnTile<T, 128, COLSUM_CHUNK>;
-    hipLaunchKernelGGL((column_sums_kernel<T, 128>), dim3((cols + Tile::COLS - 1) / Tile::COLS, chunks), dim3(256), Tile::BYTES, current_stream(), out, (A*)ws, grad, rows, cols, accumulate);
+    constexpr int MOST = 65535;                         // chunks one launch can hold
+    for (int c = 0; c < chunks; c += MOST)
+        hipLaunchKernelGGL((column_sums_kernel<T, 128>), dim3((cols + Tile::COLS - 1) / Tile::COLS, chunks - c < MOST ? chunks - c : MOST), dim3(256), Tile::BYTES, current_stream(),
+                           out, (A*)ws + (size_t)c * cols, grad + (size_t)c * COLSUM_CHUNK * cols, rows - c * COLSUM_CHUNK, cols, accumulate);
     hipLaunchKernelGGL(column_sums_finish_kernel<T>, dim3((cols + 63) / 64), dim3(64), 0, current_stream(), out, (const A*)ws, chunks, cols, accumulate);
     const bool ok = check_launch("column_sums_kernel");
     rp_hip_free(ws);                                    // back to the pool while the kernels are still queued: safe for later work on this stream

@@ -147,35 +147,39 @@ __device__ __forceinline__ void tiny_tile_any(const GemmArgs& g, bool a_vec, boo
 }
 
 __global__ void __launch_bounds__(256) linear_backward_tiny32_kernel(GemmArgs gx, GemmArgs gw, ColumnSums db, int tiles_x, int blocks_db, int vec_flags) {
-    constexpr int DB_ROWS = 128;
+    constexpr int DB_ROWS = COLSUM_CHUNK;
     using Tile = ColumnTile<float, DB_WIDTH, DB_ROWS>;
-    __shared__ __attribute__((aligned(16))) float tile[DB_ROWS * Tile::COLS];       // column sums; the GEMM tiles meet in its first 3 KB
+    __shared__ __attribute__((aligned(16))) float tile[DB_ROWS * Tile::COLS];       // column sums (16 KB: eight workgroups still share a CU); the GEMM tiles meet in its first 3 KB
     float (*red)[256] = (float (*)[256])tile;
     const int b = (int)blockIdx.x - blocks_db;           // the column sums go first: their chain of additions is the longest of any workgroup
     if (b >= 0 && b < tiles_x) { tiny_tile_any(gx, vec_flags & 1, vec_flags & 2, b, red); return; }
     if (b >= 0) { tiny_tile_any(gw, vec_flags & 4, vec_flags & 8, b - tiles_x, red); return; }
-    // column sums in the order of rp_column_sums.h, a chunk in two tiles of 128 rows: the next tile is on its way while
-    // the wave adds this one (a whole chunk per tile would cost every workgroup of the launch twice the LDS)
+    // column sums in the order of rp_column_sums.h, a chunk of 256 rows per tile: the next one is on its way while the first
+    // wave adds this one.  Its 64 lanes are 16 columns times the four runs of a chunk, so the runs are added side by side
+    // (one after another, with two tiles a chunk, 768 rows took 3 us longer).
     constexpr int COLS = Tile::COLS;
-    const int t = threadIdx.x, c0 = (int)blockIdx.x * COLS, j = c0 + t;
-    const bool serial = db.rows <= COLSUM_CHUNK;
-    float total = 0.f, s = 0.f;
+    static_assert(COLS * (COLSUM_CHUNK / COLSUM_RUN) == 64, "one wave adds the runs of a chunk");
+    const int t = threadIdx.x, c0 = (int)blockIdx.x * COLS, col = t % COLS, run = t / COLS;
+    float total = 0.f;
     Tile regs;
     regs.load(db.grad, 0, db.rows, c0, db.cols, t);
     for (int r = 0; r < db.rows; r += DB_ROWS) {
         regs.store(tile, t);
         __syncthreads();
         if (r + DB_ROWS < db.rows) regs.load(db.grad, r + DB_ROWS, db.rows, c0, db.cols, t);
-        if (t < COLS) {
-            const int n = db.rows - r < DB_ROWS ? db.rows - r : DB_ROWS;
-            if (serial) s = Tile::add(s, tile, t, n);
-            else
-                for (int q = 0; q < n; q += COLSUM_RUN) s += Tile::add(0.f, tile + q * COLS, t, n - q < COLSUM_RUN ? n - q : COLSUM_RUN);
-            if ((r + DB_ROWS) % COLSUM_CHUNK == 0 || r + DB_ROWS >= db.rows) { total += s; s = 0.f; }
+        if (db.rows <= COLSUM_CHUNK) {
+            if (t < COLS) total = Tile::add(0.f, tile, col, db.rows);
+        } else if (t < 64) {
+            const int n = db.rows - r - run * COLSUM_RUN;
+            const float s = n > 0 ? Tile::add(0.f, tile + run * COLSUM_RUN * COLS, col, n < COLSUM_RUN ? n : COLSUM_RUN) : 0.f;
+            float chunk = 0.f;
+#pragma unroll
+            for (int q = 0; q < COLSUM_CHUNK / COLSUM_RUN; q++) chunk += __shfl(s, q * COLS + col);       // (a run past the last row adds nothing)
+            total += chunk;
         }
         __syncthreads();
     }
-    if (t < COLS && j < db.cols) db.out[j] = db.accumulate ? db.out[j] + total : total;
+    if (t < COLS && c0 + col < db.cols) db.out[c0 + col] = db.accumulate ? db.out[c0 + col] + total : total;
 }
 
 // gx / gw: batch 1, fp32, each taken by the tiny kernel on its own (the caller checks); m == 0 marks an absent GEMM,
