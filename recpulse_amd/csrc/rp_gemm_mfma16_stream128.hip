@@ -80,7 +80,7 @@ template <> struct s8_ops<f16_t> {
 };
 
 template <typename T, int MR>
-__global__ void __launch_bounds__(256) gemm_stream128_kernel(GemmArgs g, float* partials, int groups, int nsplit, int* arrivals, int local) {
+__global__ void __launch_bounds__(256) gemm_stream128_kernel(GemmArgs g, float* partials, int groups, int nsplit, int pitch, int* arrivals, int local) {
     constexpr int NF = MR / 16;                                           // A fragments (16 rows each)
     constexpr int RS = S8_RS, S8_ROUND = S8_STEP * RS;                    // steps and k rows of a round
     extern __shared__ __attribute__((aligned(16))) float red[];          // [S8_WAVES][MR][S8_PITCH]
@@ -203,7 +203,7 @@ __global__ void __launch_bounds__(256) gemm_stream128_kernel(GemmArgs g, float* 
     // accumulator register v of tile (f, c) holds row 16f + 4q + v at column 8j + c: a lane's 8 residues of one row are
     // 8 adjacent columns, two 16-byte stores at consecutive addresses across the lanes of a row
     const SplitkOutput<T> out(g);
-    const __amdgpu_buffer_rsrc_t part_rsrc = buffer_rsrc(partials, partials ? (long long)nsplit * g.m * g.n * 4 : 0);
+    const __amdgpu_buffer_rsrc_t part_rsrc = buffer_rsrc(partials, partials ? (long long)nsplit * g.m * pitch * 4 : 0);
 #pragma unroll
     for (int f = 0; f < NF; f++)
 #pragma unroll
@@ -235,12 +235,12 @@ __global__ void __launch_bounds__(256) gemm_stream128_kernel(GemmArgs g, float* 
     if (!arrivals) {
 #pragma unroll
         for (int i = 0; i < NQ; i++)
-            if (qlive[i]) *(f32x4_t*)(partials + ((long long)split * g.m + qrow[i]) * g.n + qcol[i]) = sum[i];
+            if (qlive[i]) *(f32x4_t*)(partials + ((long long)split * g.m + qrow[i]) * pitch + qcol[i]) = sum[i];
         return;
     }
     int part_off[NQ];                                    // (dead quads: an offset beyond the buffer, the store is dropped)
 #pragma unroll
-    for (int i = 0; i < NQ; i++) part_off[i] = qlive[i] ? (int)((((long long)split * g.m + qrow[i]) * g.n + qcol[i]) * 4) : (int)BUFFER_OOB;
+    for (int i = 0; i < NQ; i++) part_off[i] = qlive[i] ? (int)((((long long)split * g.m + qrow[i]) * pitch + qcol[i]) * 4) : (int)BUFFER_OOB;
     if (local) {
 #pragma unroll
         for (int i = 0; i < NQ; i++) __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, sum[i]), part_rsrc, part_off[i], 0, 0);
@@ -251,22 +251,22 @@ __global__ void __launch_bounds__(256) gemm_stream128_kernel(GemmArgs g, float* 
 
     // ---- single-launch finish: the last block of this column group to arrive adds all splits ----
     if (!splitk_arrive(arrivals + group, nsplit, local != 0, &arrived_last)) return;
-    splitk_finish_window<T, S8_COLS, MR / 8, 4>(g, out, part_rsrc, nsplit, 0, g.m, n0, local != 0, arrivals + group);
+    splitk_finish_window<T, S8_COLS, MR / 8, 4>(g, out, part_rsrc, nsplit, pitch, 0, g.m, n0, local != 0, arrivals + group);
 }
 
 template <typename T, int MR>
-static int launch_stream128_mr(const GemmArgs& g, float* partials, int groups, int nsplit, int* arrivals, int local) {
+static int launch_stream128_mr(const GemmArgs& g, float* partials, int groups, int nsplit, int pitch, int* arrivals, int local) {
     constexpr size_t smem = (size_t)S8_WAVES * MR * S8_PITCH * sizeof(float);
     auto kern = gemm_stream128_kernel<T, MR>;
     if (smem > 64 * 1024 && !check_hip(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem), "hipFuncSetAttribute")) return -1;
-    hipLaunchKernelGGL(kern, dim3(8 * ((groups + 7) / 8) * nsplit), dim3(256), smem, current_stream(), g, partials, groups, nsplit, arrivals, local);
+    hipLaunchKernelGGL(kern, dim3(8 * ((groups + 7) / 8) * nsplit), dim3(256), smem, current_stream(), g, partials, groups, nsplit, pitch, arrivals, local);
     return check_launch("gemm_stream128_kernel") ? 0 : -1;
 }
 
 template <typename T>
-static int launch_stream128_t(const GemmArgs& g, float* partials, int groups, int nsplit, int* arrivals, int local) {
-    if (g.m <= 16) return launch_stream128_mr<T, 16>(g, partials, groups, nsplit, arrivals, local);
-    return launch_stream128_mr<T, 32>(g, partials, groups, nsplit, arrivals, local);
+static int launch_stream128_t(const GemmArgs& g, float* partials, int groups, int nsplit, int pitch, int* arrivals, int local) {
+    if (g.m <= 16) return launch_stream128_mr<T, 16>(g, partials, groups, nsplit, pitch, arrivals, local);
+    return launch_stream128_mr<T, 32>(g, partials, groups, nsplit, pitch, arrivals, local);
 }
 
 // k splits for an output of n columns: one block per CU (a wave per SIMD), each at least two passes of its waves deep
@@ -295,19 +295,24 @@ bool stream128_takes(const GemmArgs& g) { return g.a_cs == 1 && g.b_cs == 1 && s
 int launch_stream128(const GemmArgs& g, int dtype) {
     const int groups = (g.n + S8_COLS - 1) / S8_COLS;
     const int nsplit = stream128_nsplit(g.k, g.n);
-    const size_t part_bytes = (size_t)nsplit * g.m * g.n * sizeof(float);
-    void* ws = nullptr;
-    if (nsplit > 1 && gemm_workspace(&ws, part_bytes) != 0) return -1;
+    // Exchanged inside an XCD, the partial rows of a column group must not share cache lines with another group's (see
+    // splitk_finish_window): their pitch is then a whole number of strips.  Where that does not fit the array of the entry
+    // point that allocates nothing, they are exchanged at device scope, in rows of n.
+    const size_t dense_bytes = (size_t)nsplit * g.m * g.n * sizeof(float), strip_bytes = (size_t)nsplit * g.m * groups * S8_COLS * sizeof(float);
     int* arrivals = nullptr;
     if (nsplit > 1) {
         bool failed = false;
-        arrivals = splitk_arrival_counters(groups, part_bytes, &failed);
-        if (failed) { gemm_workspace_release(ws); return -1; }
+        arrivals = splitk_arrival_counters(groups, strip_bytes, &failed);
+        if (failed) return -1;
     }
-    const int local = arrivals && workgroups_share_xcd_by_residue() ? 1 : 0;
+    const bool room = !noalloc_active() || strip_bytes <= RP_HIP_NOALLOC_WORKSPACE_BYTES;
+    const int local = arrivals && room && workgroups_share_xcd_by_residue() ? 1 : 0;
+    const int pitch = local ? groups * S8_COLS : g.n;
+    void* ws = nullptr;
+    if (nsplit > 1 && gemm_workspace(&ws, local ? strip_bytes : dense_bytes) != 0) return -1;
     int rc;
-    if (dtype == RP_DTYPE_BFLOAT16) rc = launch_stream128_t<bf16_t>(g, (float*)ws, groups, nsplit, arrivals, local);
-    else rc = launch_stream128_t<f16_t>(g, (float*)ws, groups, nsplit, arrivals, local);
+    if (dtype == RP_DTYPE_BFLOAT16) rc = launch_stream128_t<bf16_t>(g, (float*)ws, groups, nsplit, pitch, arrivals, local);
+    else rc = launch_stream128_t<f16_t>(g, (float*)ws, groups, nsplit, pitch, arrivals, local);
     if (rc == 0 && nsplit > 1 && !arrivals) rc = launch_splitk_combine(g, (const float*)ws, nsplit, g.m, dtype);
     if (ws) gemm_workspace_release(ws);          // back to the pool while the kernels are still queued: safe for later work on this stream; held with the graph while one is being recorded
     return rc;

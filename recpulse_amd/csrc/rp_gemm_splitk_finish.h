@@ -74,7 +74,7 @@ __device__ __forceinline__ bool splitk_arrive(int* counter, int nsplit, bool loc
     return *flag;
 }
 
-// The block that arrived last adds the fp32 partials [split][g.m][g.n] of rows m0 .. m_end-1 and COLS columns from n0 in
+// The block that arrived last adds the fp32 partials [split][g.m][pitch] of rows m0 .. m_end-1 and COLS columns from n0 in
 // split order (so the result does not depend on which block that is), runs the epilogue and leaves the counter at
 // zero for the next launch.  QN quads per thread and pass; the loads of U splits of all of a thread's quads are in
 // flight together (QN * U * 4 registers, which count against the calling kernel's occupancy): their offsets are all
@@ -82,11 +82,13 @@ __device__ __forceinline__ bool splitk_arrive(int* counter, int nsplit, bool loc
 // branch per load the compiler puts waits between them, and the finish takes a memory round trip per load).  (Plain
 // loads of the partials cannot hit stale lines of this CU's vector cache: it fills on the CU's own loads only and
 // starts every launch empty, and the one block of a launch that reads a tile's partials reads them here for the first
-// time.)
+// time.  That holds only while no other block's tile has a share in the same cache lines: two blocks that finish on one
+// CU would otherwise meet in them, the second reading the line as the first found it.  So in the local form a tile's rows
+// must start and end on cache lines: a pitch of whole strips.)
 template <typename T, int COLS, int QN, int U_SPLITS, bool LOCAL>
 __device__ __forceinline__ void splitk_finish_window_scope(const GemmArgs& g, const SplitkOutput<T>& out, __amdgpu_buffer_rsrc_t part_rsrc, int nsplit,
-                                                           int m0, int m_end, int n0, int* counter) {
-    const long long split_stride = (long long)g.m * g.n;
+                                                           int pitch, int m0, int m_end, int n0, int* counter) {
+    const long long split_stride = (long long)g.m * pitch;
     constexpr int QPR = COLS / 4;                        // quads per row of the window
     constexpr int RPP = 256 * QN / QPR;                  // rows per pass
     for (int r0 = m0; r0 < m_end; r0 += RPP) {
@@ -98,7 +100,7 @@ __device__ __forceinline__ void splitk_finish_window_scope(const GemmArgs& g, co
             const int idx = threadIdx.x + 256 * q;
             row[q] = r0 + idx / QPR; col[q] = n0 + (idx % QPR) * 4;
             live[q] = row[q] < m_end && col[q] < g.n;    // n is a multiple of 4 here, so a quad is wholly in or out
-            at[q] = live[q] ? ((long long)row[q] * g.n + col[q]) * 4 : (long long)BUFFER_OOB;      // bytes; dead quads read zeros
+            at[q] = live[q] ? ((long long)row[q] * pitch + col[q]) * 4 : (long long)BUFFER_OOB;      // bytes; dead quads read zeros
         }
         f32x4_t sum[QN];
 #pragma unroll
@@ -134,10 +136,10 @@ __device__ __forceinline__ void splitk_finish_window_scope(const GemmArgs& g, co
 }
 
 template <typename T, int COLS, int QN, int U_SPLITS = 8>
-__device__ __forceinline__ void splitk_finish_window(const GemmArgs& g, const SplitkOutput<T>& out, __amdgpu_buffer_rsrc_t part_rsrc, int nsplit,
+__device__ __forceinline__ void splitk_finish_window(const GemmArgs& g, const SplitkOutput<T>& out, __amdgpu_buffer_rsrc_t part_rsrc, int nsplit, int pitch,
                                                      int m0, int m_end, int n0, bool local, int* counter) {
-    if (local) splitk_finish_window_scope<T, COLS, QN, U_SPLITS, true>(g, out, part_rsrc, nsplit, m0, m_end, n0, counter);
-    else splitk_finish_window_scope<T, COLS, QN, U_SPLITS, false>(g, out, part_rsrc, nsplit, m0, m_end, n0, counter);
+    if (local) splitk_finish_window_scope<T, COLS, QN, U_SPLITS, true>(g, out, part_rsrc, nsplit, pitch, m0, m_end, n0, counter);
+    else splitk_finish_window_scope<T, COLS, QN, U_SPLITS, false>(g, out, part_rsrc, nsplit, pitch, m0, m_end, n0, counter);
 }
 
 }  // namespace rp
