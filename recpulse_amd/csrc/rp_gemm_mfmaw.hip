@@ -523,6 +523,10 @@ static int launch_mfmaw_t(const GemmArgs& g, const Plan& p) {
     return rc;
 }
 
+// fp32 on the bf16 matrix cores (rp_gemm_split32.hip)
+bool split32_takes(const GemmArgs& g, const Plan& p);
+int launch_split32(const GemmArgs& g, const Plan& p);
+
 int launch_mfmaw(const GemmArgs& g, const Plan& p, int dtype) {
     // fp32, k of at most two slabs, at least 128 tiles of 128 x 128: the resident, cross-tile pipelined kernel
     if (dtype == RP_DTYPE_FLOAT32 && !p.ragged && p.bm == 128 && g.k <= 2 * mfmaw_cfg<float>::BK && !path_disabled("shortk") && g.seg_k == 0 && g.seg_n == 0 && g.c_fold_from == 0 && !g.bias_by_row) {
@@ -532,6 +536,7 @@ int launch_mfmaw(const GemmArgs& g, const Plan& p, int dtype) {
         if (p.a_mc && p.b_mc) return mw_launch_shortk<float, 128, 128, true, true>(g, edge);
         return mw_launch_shortk<float, 128, 128, true, false>(g, edge);
     }
+    if (dtype == RP_DTYPE_FLOAT32 && split32_takes(g, p)) return launch_split32(g, p);
     if (dtype == RP_DTYPE_FLOAT32) return launch_mfmaw_t<float>(g, p);
     if (dtype == RP_DTYPE_FLOAT64) return launch_mfmaw_t<double>(g, p);
     set_error("mfmaw GEMM: unsupported dtype %d", dtype);

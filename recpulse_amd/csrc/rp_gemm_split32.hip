@@ -1,0 +1,344 @@
+// fp32 GEMM on the bf16 matrix cores: every fp32 value as the exact sum of three bf16 values.
+//
+// The fp32 MFMA runs 128 multiply-adds per cycle and CU, the bf16 MFMA sixteen times as many.  x = h + m + l with h = bf16(x),
+// m = bf16(x - h), l = x - h - m is exact (8 + 8 + 8 significant bits, each with its own sign, cover 24), so
+//   a b = ah bh + (ah bm + am bh) + (am bm + ah bl + al bh) + [am bl + al bm + al bl]
+// where the bracket is at most 2^-25 |a b|, under the rounding of a single fp32 product, and is left out: six bf16 MFMAs (whose
+// products are exact in fp32) of 32 cycles per k-step of 16 stand in for eight fp32 MFMAs of 64.  The five small products
+// go to an accumulator of their own, and the two meet once, in the epilogue: the large one then rounds once per 16 k instead
+// of once per product or two.  2-norm error against 64 bits, N(0,1) values, this kernel / the fp32 MFMA kernel: k = 67
+// 5.1e-8 / 1.5e-7, 256 8.9e-8 / 2.9e-7, 1024 1.9e-7 / 5.7e-7, 4096 4.0e-7 / 1.15e-6, the same in every layout; uniform values
+// in [0, 1) 0.35 - 0.45 of it; values spread over 2^+-30 equal it within 10 % either way at k <= 128 and are 0.85 of it at 4096.
+//
+// What the split cannot hold: infinities, NaN and values that round to bf16 infinity (their m and l become NaN, so every
+// output they touch is NaN, here or in a finite dot product that overflowed), and values below 2^-110, whose last bits fall
+// below the smallest bf16 subnormal.  The tile looks for both - non-finite accumulators at the end, the smallest non-zero
+// magnitude while it splits - and, if it met one, is computed again with fp32 MFMAs (the whole workgroup together).  So
+// the results for such inputs are the ones the fp32 kernel gives; they cost the sum of both.
+//
+// Shape: 128 x 128 tile, 4 waves of 64 x 64, k slab 32.  A slab is fetched to registers as fp32 (16 values of either operand
+// per thread), split there and written to LDS as rows of [32 h | 32 m | 32 l]; all four operand layouts leave the same
+// rows, so the multiplying half is common to them.  Fragment reads per MFMA are half those of a plain bf16 kernel (twelve for
+// 24 MFMAs).  LDS holds one slab (52 KB): two workgroups share a CU.  The next slab is requested at the start of this one's
+// 48 MFMAs and split between those of the second half, two values after one or two MFMAs (splitting between the two barriers
+// instead: 4096^3 788 us against 745, 2048^3 162 against 129).
+//
+// What bounds it: 52 % of the cycles are MFMA-busy, at a clock of 1.9 GHz and less that the power limit leaves.  4096^3: 750 -
+// 800 us where the fp32 MFMAs take 1 050 - 1 170; 2048^3 128 against 160; 3001 x 1027 x 2049 101 against 225.
+#include "rp_gemm.h"
+
+namespace rp {
+
+namespace {
+
+constexpr int S32_BK = 32;
+constexpr int S32_PITCH = 3 * S32_BK + 8;           // 16-bit elements per LDS row: 16 rows of ds_read_b128 cover all banks once
+
+typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2_t;
+
+// The smallest non-zero magnitude met so far, in the terms of a pair of bf16 values: 2 |h| - 1 as a 16-bit integer orders
+// magnitudes, with zero above all others; the two halves run separately.
+typedef __attribute__((ext_vector_type(2))) unsigned short u16x2_t;
+__device__ __forceinline__ uint32_t s32_least(uint32_t so_far, uint32_t h) {
+    uint32_t key;
+    asm("v_pk_mad_u16 %0, %1, %2, %3" : "=v"(key) : "v"(h), "s"(0x00020002u), "v"(0xFFFFFFFFu));
+    return __builtin_bit_cast(uint32_t, __builtin_elementwise_min(__builtin_bit_cast(u16x2_t, so_far), __builtin_bit_cast(u16x2_t, key)));
+}
+constexpr uint32_t S32_LEAST = ((127u - 110u) << 8) - 1u;           // the key of 2^-110
+
+__device__ __forceinline__ uint32_t s32_pack(float a, float b) {
+    const bf16x2_t v = {(__bf16)a, (__bf16)b};                        // one packed conversion, round to nearest even
+    return __builtin_bit_cast(uint32_t, v);
+}
+
+// two values -> their h, m and l pairs
+__device__ __forceinline__ void s32_split2(float x0, float x1, uint32_t& h, uint32_t& m, uint32_t& l) {
+    h = s32_pack(x0, x1);
+    const float r0 = x0 - __uint_as_float(h << 16), r1 = x1 - __uint_as_float(h & 0xFFFF0000u);
+    m = s32_pack(r0, r1);
+    l = s32_pack(r0 - __uint_as_float(m << 16), r1 - __uint_as_float(m & 0xFFFF0000u));
+}
+
+// One operand's slab traffic.  A thread holds four vectors of four values along the unit-stride axis.
+//   KC (unit stride along k): vector i is row t / 8 + 32 i, k 4 (t % 8) .. + 3.
+//   MC (unit stride along the free axis): vector i is k 4 (t % 8) + i, rows 4 (t / 8) .. + 3: a 4 x 4 block, transposed in
+//   registers; eight lanes span the slab's k (64 bytes of an LDS row), a wave reads whole 128-byte lines of eight k rows at a time.
+// EDGE: extents and row starts of any size (otherwise the tile and all slabs are whole).  A vector that straddles the end of its
+// row is fetched `pull` elements further back, where it ends with the row, and shifted into place.
+template <int ROWS, bool MC, bool EDGE>
+struct S32Slab {
+    static_assert(ROWS * S32_BK == 256 * 16, "16 values per thread");
+    u32x4_t v[4];
+    u32x2_t planes[4][3];         // rows' h, m and l
+    int r0, kk0;                  // first free index and k of vector 0
+    uint32_t goff[EDGE ? 4 : 1];  // byte offset of the vectors from the slab pointer
+    int step;                     // bytes between vectors
+    int pull;                     // MC: elements the vectors stick out of the free axis
+    const char* slab;
+    const char* end;
+    long long slab_step;
+    __device__ __forceinline__ void init(const float* base, long long free_stride, long long k_stride, int row0, int free_extent, int k, int t) {
+        r0 = MC ? 4 * (t / 8) : t / 8;
+        kk0 = 4 * (t % 8);
+        slab = (const char*)(base + (long long)row0 * free_stride);
+        end = (const char*)(base + (long long)(free_extent - 1) * free_stride + (long long)(k - 1) * k_stride + 1);
+        slab_step = (long long)S32_BK * k_stride * 4;
+        step = (int)((MC ? k_stride : 32 * free_stride) * 4);
+        pull = 0;
+        if (EDGE && MC) {
+            const int in = free_extent - row0 - r0;
+            pull = in > 0 && in < 4 ? 4 - in : 0;
+        }
+#pragma unroll
+        for (int i = 0; i < (EDGE ? 4 : 1); i++) {
+            const int r = r0 + (MC ? 0 : 32 * i), kk = kk0 + (MC ? i : 0);
+            goff[i] = (uint32_t)(((long long)r * free_stride + (long long)kk * k_stride) * 4) + (EDGE ? 16 : 0);
+            if (EDGE && row0 + r >= free_extent) goff[i] = BUFFER_OOB;
+        }
+    }
+    // the slab `slab` points at, of which kleft k are in range; then on to the next one
+    __device__ __forceinline__ void load(int kleft) {
+        if constexpr (!EDGE) {
+            const __amdgpu_buffer_rsrc_t rsrc = buffer_rsrc(slab, 0x7fffffffll);
+#pragma unroll
+            for (int i = 0; i < 4; i++) v[i] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)goff[0], i * step, 0);
+        } else {
+            const __amdgpu_buffer_rsrc_t rsrc = buffer_rsrc(slab - 16, (long long)(end - slab) + 16);      // starts early: pulled-back offsets stay positive
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const int in = kleft - kk0 - (MC ? i : 0);
+                const int back = MC ? pull : (in > 0 && in < 4 ? 4 - in : 0);
+                v[i] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, in > 0 ? (int)(goff[i] - 4 * back) : (int)BUFFER_OOB, 0, 0);
+            }
+        }
+        slab += slab_step;
+    }
+    // straddling vectors into place (kleft: of the slab that was loaded)
+    __device__ __forceinline__ void settle(int kleft) {
+        if constexpr (EDGE) {
+            const int in = kleft - kk0;
+            const int back = MC ? pull : (in > 0 && in < 4 ? 4 - in : 0);
+            if (__builtin_amdgcn_ballot_w64(back != 0) == 0) return;
+#pragma unroll
+            for (int i = 0; i < 4; i++) v[i] = __builtin_bit_cast(u32x4_t, __builtin_bit_cast(unsigned __int128, v[i]) >> (32 * back));
+        }
+    }
+    __device__ __forceinline__ float at(int i, int e) const { return __uint_as_float(v[i][e]); }
+    // unit u = 0 .. 7 of the split: two values of row u / 2 of the thread's four
+    template <int U>
+    __device__ __forceinline__ void split(uint32_t& least) {
+        constexpr int j = U / 2, p = U % 2;
+        const float x0 = MC ? at(2 * p, j) : at(j, 2 * p), x1 = MC ? at(2 * p + 1, j) : at(j, 2 * p + 1);
+        uint32_t h, m, l;
+        s32_split2(x0, x1, h, m, l);
+        least = s32_least(least, h);
+        planes[j][0][p] = h; planes[j][1][p] = m; planes[j][2][p] = l;
+    }
+    __device__ __forceinline__ void split_all(uint32_t& least) {
+        static_for<0, 8>([&](auto u) { split<decltype(u)::value>(least); });
+    }
+    __device__ __forceinline__ void store(uint16_t* lds) const {
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            uint16_t* row = lds + (r0 + (MC ? j : 32 * j)) * S32_PITCH + kk0;
+#pragma unroll
+            for (int q = 0; q < 3; q++) *(u32x2_t*)(row + q * S32_BK) = planes[j][q];
+        }
+    }
+    // the slab as fp32, k-major [32][ROWS + 4], for the fp32 MFMAs
+    __device__ __forceinline__ void store_plain(float* lds) const {
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            if (MC) *(u32x4_t*)(lds + (kk0 + i) * (ROWS + 4) + r0) = v[i];
+            else
+#pragma unroll
+                for (int e = 0; e < 4; e++) lds[(kk0 + e) * (ROWS + 4) + r0 + 32 * i] = at(i, e);
+        }
+    }
+};
+
+}  // namespace
+
+template <bool A_MC, bool B_MC, bool EDGE>
+__global__ void __launch_bounds__(256, 2) gemm_split32_kernel(GemmArgs g, int tiles_m, int tiles_n) {
+    constexpr int BM = 128, BN = 128, TM = 2, TN = 2;
+    __shared__ __attribute__((aligned(16))) uint16_t lds[(BM + BN) * S32_PITCH];
+    static_assert(sizeof(lds) >= (size_t)S32_BK * (BM + 4 + BN + 4) * 4, "room for the fp32 slab");
+    const TileCoord tc = schedule_tile(blockIdx.x, tiles_m, tiles_n);
+    if (!tc.valid) return;
+    const int z = blockIdx.y, m0 = tc.tm * BM, n0 = tc.tn * BN;
+    const int t = threadIdx.x, lane = t & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int wm0 = (wave >> 1) * 64, wn0 = (wave & 1) * 64;
+    const float* A = (const float*)g.A + (long long)z * g.a_bs;
+    const float* B = (const float*)g.B + (long long)z * g.b_bs;
+    uint16_t* const a_lds = lds;
+    uint16_t* const b_lds = lds + BM * S32_PITCH;
+    const int nslabs = (g.k + S32_BK - 1) / S32_BK;
+
+    f32x16_t big[TM][TN], small[TM][TN];
+    auto clear = [&](f32x16_t (&acc)[TM][TN]) {
+#pragma unroll
+        for (int i = 0; i < TM; i++)
+#pragma unroll
+            for (int j = 0; j < TN; j++)
+#pragma unroll
+                for (int v = 0; v < 16; v++) acc[i][j][v] = 0.f;
+    };
+    clear(big);
+    clear(small);
+    uint32_t least = 0xFFFFFFFFu;
+    {
+        S32Slab<BM, A_MC, EDGE> sa;
+        S32Slab<BN, B_MC, EDGE> sb;
+        sa.init(A, g.a_rs, g.a_cs, m0, g.m, g.k, t);
+        sb.init(B, g.b_cs, g.b_rs, n0, g.n, g.k, t);
+        sa.load(g.k);
+        sb.load(g.k);
+        // lane's fragment of MFMA tile i: row 32 i + lane % 32, k 8 (lane / 32) .. + 7 of a step of 16
+        const uint16_t* const a_fr = a_lds + (wm0 + (lane & 31)) * S32_PITCH + 8 * (lane >> 5);
+        const uint16_t* const b_fr = b_lds + (wn0 + (lane & 31)) * S32_PITCH + 8 * (lane >> 5);
+        sa.settle(g.k);
+        sb.settle(g.k);
+        sa.split_all(least);
+        sb.split_all(least);
+        sa.store(a_lds);
+        sb.store(b_lds);
+        __syncthreads();
+        // one slab: 48 MFMAs; the next one is requested at its start and split between the MFMAs of its second half
+        auto step = [&](int kleft, auto next_tag) {
+            constexpr bool NEXT = decltype(next_tag)::value;
+            if constexpr (NEXT) {
+                sa.load(kleft - S32_BK);
+                sb.load(kleft - S32_BK);
+            }
+            static_for<0, 2>([&](auto ksc) {
+                constexpr int ks = decltype(ksc)::value;
+                bf16x8_t af[TM][3], bf[TN][3];
+#pragma unroll
+                for (int p = 0; p < 3; p++) {
+#pragma unroll
+                    for (int i = 0; i < TM; i++) af[i][p] = *(const bf16x8_t*)(a_fr + 32 * i * S32_PITCH + p * S32_BK + 16 * ks);
+#pragma unroll
+                    for (int j = 0; j < TN; j++) bf[j][p] = *(const bf16x8_t*)(b_fr + 32 * j * S32_PITCH + p * S32_BK + 16 * ks);
+                }
+                if constexpr (NEXT && ks == 1) {
+                    sa.settle(kleft - S32_BK);
+                    sb.settle(kleft - S32_BK);
+                }
+                static_for<0, 24>([&](auto qc) {
+                    constexpr int q = decltype(qc)::value, i = (q / TN) % TM, j = q % TN, prod = q / (TM * TN);
+                    constexpr int PA[6] = {0, 0, 1, 1, 0, 2}, PB[6] = {0, 1, 0, 1, 2, 0};
+                    f32x16_t& acc = prod == 0 ? big[i][j] : small[i][j];
+                    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[i][PA[prod]], bf[j][PB[prod]], acc, 0, 0, 0);
+                    if constexpr (NEXT && ks == 1) {
+                        static_for<16 * q / 24, 16 * (q + 1) / 24>([&](auto uc) {
+                            constexpr int u = decltype(uc)::value;
+                            if constexpr (u < 8) sa.template split<u>(least);
+                            else sb.template split<u - 8>(least);
+                        });
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                });
+            });
+            if constexpr (NEXT) {
+                __syncthreads();
+                sa.store(a_lds);
+                sb.store(b_lds);
+            }
+            __syncthreads();
+        };
+        int kleft = g.k;
+        for (; kleft > S32_BK; kleft -= S32_BK) step(kleft, std::true_type{});
+        step(kleft, std::false_type{});
+    }
+    bool redo = (least & 0xFFFFu) < S32_LEAST || (least >> 16) < S32_LEAST;
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++)
+#pragma unroll
+            for (int v = 0; v < 16; v++) {
+                big[i][j][v] += small[i][j][v];
+                redo |= !(fabsf(big[i][j][v]) <= 3.402823466e38f);
+            }
+
+    const int lf = lane & 31, lk = lane >> 5;
+    if (__syncthreads_or(redo)) {
+        float* const ap = (float*)lds;
+        float* const bp = ap + S32_BK * (BM + 4);
+        clear(big);
+        S32Slab<BM, A_MC, EDGE> sa;
+        S32Slab<BN, B_MC, EDGE> sb;
+        sa.init(A, g.a_rs, g.a_cs, m0, g.m, g.k, t);
+        sb.init(B, g.b_cs, g.b_rs, n0, g.n, g.k, t);
+        for (int s = 0; s < nslabs; s++) {
+            const int kleft = g.k - s * S32_BK;
+            sa.load(kleft);
+            sb.load(kleft);
+            sa.settle(kleft);
+            sb.settle(kleft);
+            sa.store_plain(ap);
+            sb.store_plain(bp);
+            __syncthreads();
+            for (int kk = lk; kk < S32_BK; kk += 2) {
+                float af[TM], bf[TN];
+#pragma unroll
+                for (int i = 0; i < TM; i++) af[i] = ap[kk * (BM + 4) + wm0 + 32 * i + lf];
+#pragma unroll
+                for (int j = 0; j < TN; j++) bf[j] = bp[kk * (BN + 4) + wn0 + 32 * j + lf];
+#pragma unroll
+                for (int i = 0; i < TM; i++)
+#pragma unroll
+                    for (int j = 0; j < TN; j++) big[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(af[i], bf[j], big[i][j], 0, 0, 0);
+            }
+            __syncthreads();
+        }
+    }
+
+    // straight from the accumulators: a store instruction is 32 adjacent columns of two rows
+    float* C = (float*)g.C + (long long)z * g.c_bs;
+    const float* bias = (const float*)g.bias;
+    const bool has_bias = bias != nullptr, accum = g.accumulate != 0;
+#pragma unroll
+    for (int j = 0; j < TN; j++) {
+        const int gn = n0 + wn0 + 32 * j + lf;
+        const bool col_ok = !EDGE || gn < g.n;
+        const float bv = has_bias && col_ok ? bias[gn] : 0.f;
+#pragma unroll
+        for (int i = 0; i < TM; i++)
+#pragma unroll
+            for (int v = 0; v < 16; v++) {
+                const int gm = m0 + wm0 + 32 * i + 8 * (v / 4) + 4 * lk + (v % 4);
+                if (EDGE && !(col_ok && gm < g.m)) continue;
+                float* pc = C + (long long)gm * g.c_rs + (long long)gn * g.c_cs;
+                *pc = finish<float>(big[i][j][v], has_bias, bv, accum, accum ? *pc : 0.f);
+            }
+    }
+}
+
+template <bool A_MC, bool B_MC>
+static int launch_split32_layout(const GemmArgs& g, bool edge) {
+    const int tiles_m = (g.m + 127) / 128, tiles_n = (g.n + 127) / 128;
+    const dim3 grid(scheduled_grid(tiles_m, tiles_n), g.batch);
+    if (edge) hipLaunchKernelGGL((gemm_split32_kernel<A_MC, B_MC, true>), grid, dim3(256), 0, current_stream(), g, tiles_m, tiles_n);
+    else hipLaunchKernelGGL((gemm_split32_kernel<A_MC, B_MC, false>), grid, dim3(256), 0, current_stream(), g, tiles_m, tiles_n);
+    return check_launch("gemm_split32_kernel") ? 0 : -1;
+}
+
+// Every fp32 product that the 128 x 128 tile is right for and whose k is not one or two slabs of whole vectors (those have a
+// kernel that pipelines across tiles).  With the 64 x 64 tile a slab's split would take longer than its MFMAs.  Segmented
+// operands and the convolution's epilogue options stay with the fp32 MFMA kernel.
+bool split32_takes(const GemmArgs& g, const Plan& p) {
+    return p.bm == 128 && g.seg_k == 0 && g.seg_n == 0 && g.c_fold_from == 0 && !g.bias_by_row && !path_disabled("split32");
+}
+
+int launch_split32(const GemmArgs& g, const Plan& p) {
+    const bool edge = p.ragged || g.m % 128 || g.n % 128 || g.k % S32_BK;
+    if (!p.a_mc && p.b_mc) return launch_split32_layout<false, true>(g, edge);
+    if (!p.a_mc && !p.b_mc) return launch_split32_layout<false, false>(g, edge);
+    if (p.a_mc && p.b_mc) return launch_split32_layout<true, true>(g, edge);
+    return launch_split32_layout<true, false>(g, edge);
+}
+
+}  // namespace rp

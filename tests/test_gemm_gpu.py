@@ -972,3 +972,69 @@ def test_fp32_short_reduction_integers_bit_exact():
         b = b if layout[1] == "n" else b.transpose(0, 2, 1)
         got = device_gemm(a, b, F32)
         assert np.array_equal(got, np.matmul(a.astype(np.float64), b.astype(np.float64)).astype(np.float32)), layout
+
+
+# fp32 tiles of 128 x 128 run on the bf16 matrix cores with every value split in three.  Shapes: whole tiles and slabs of 32;
+# k one past and one short of a slab, free axes one past and one short of a tile, k of less than a slab, a batch.
+SPLIT32_SHAPES = [(1, 1408, 96, 1536), (1, 1409, 97, 1535), (1, 1407, 95, 1537), (1, 1500, 7, 1500), (1, 1411, 1029, 1404), (2, 1024, 68, 1160)]
+
+
+@pytest.mark.parametrize("layout", LAYOUTS)
+@pytest.mark.parametrize("batch,m,k,n", SPLIT32_SHAPES)
+def test_split32_is_as_close_as_fp32_sums(batch, m, k, n, layout):
+    """Against float64.  Every step of 16 k rounds the running sum once (2^-24 of it at most, of random sign), two more
+    roundings join the small products and the bias; a plane of either operand left out would cost 2^-18 and more."""
+    rng = np.random.default_rng(47)
+
+    def operand(rows, cols, transposed):
+        x = rng.normal(0, 1, (batch, rows, cols)).astype(np.float32)
+        return (x, capi.DeviceBuffer.from_numpy(np.ascontiguousarray(x.transpose(0, 2, 1))), (rows * cols, 1, rows)) if transposed else (x, capi.DeviceBuffer.from_numpy(x), (rows * cols, cols, 1))
+
+    a, da, a_st = operand(m, k, layout[0] == "t")
+    b, db, b_st = operand(k, n, layout[1] == "t")
+    bias, c0 = rng.normal(0, 1, n).astype(np.float32), rng.normal(0, 1, (batch, m, n)).astype(np.float32)
+    exact = np.matmul(a.astype(np.float64), b.astype(np.float64))
+    dbias = capi.DeviceBuffer.from_numpy(bias)
+    for with_bias, accumulate in ((False, False), (True, True)):
+        dc = capi.DeviceBuffer.from_numpy(c0)
+        capi.gemm(dc.ptr, da.ptr, db.ptr, dbias.ptr if with_bias else None, batch, m, k, n, a_st, b_st, (m * n, n, 1), accumulate, F32)
+        assert capi.last_gemm_kernel() == "mfma32_128x128"
+        want = exact + (bias if with_bias else 0.0) + (c0 if accumulate else 0.0)
+        got = dc.to_numpy(np.float32, (batch, m, n)).astype(np.float64)
+        assert np.linalg.norm(got - want) <= 2.0 ** -24 * (np.sqrt(k / 16) + 4) * np.linalg.norm(want)
+        dc.free()
+
+
+@pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan, np.finfo(np.float32).max, -np.finfo(np.float32).max, 2.0 ** -105, 2.0 ** -111, 2.0 ** -120])
+@pytest.mark.parametrize("m,k,n", [(1408, 96, 1536), (1411, 99, 1405)])
+def test_split32_values_that_do_not_split(m, k, n, value):
+    """Infinities, NaN, magnitudes that round to bf16 infinity and magnitudes whose last bits bf16 cannot hold: a tile that meets
+    one is computed with fp32 MFMAs.  One row of A is `value` times N(0, 1) where that is tiny (fp32 sums of k products then
+    bound the row's error by itself; the smallest stays a normal number, the fp32 MFMA takes subnormals as zero), otherwise
+    `value` stands in two places."""
+    rng = np.random.default_rng(48)
+    a, b = rng.normal(0, 1, (m, k)).astype(np.float32), rng.normal(0, 1, (k, n)).astype(np.float32)
+    tiny = abs(value) < 1
+    if tiny:
+        a[5] = (rng.normal(0, 1, k) * value).astype(np.float32)
+        b *= np.float32(2.0 ** 60)
+    else:
+        a[5, 7] = value
+        b[k - 1, n - 2] = value
+    dc, da, db = capi.DeviceBuffer(m * n * 4), capi.DeviceBuffer.from_numpy(a), capi.DeviceBuffer.from_numpy(b)
+    capi.gemm(dc.ptr, da.ptr, db.ptr, None, 1, m, k, n, (0, k, 1), (0, n, 1), (0, n, 1), False, F32)
+    assert capi.last_gemm_kernel() == "mfma32_128x128"
+    got = dc.to_numpy(np.float32, (m, n))
+    with np.errstate(all="ignore"):
+        want = np.matmul(a.astype(np.float64), b.astype(np.float64))
+        as32 = want.astype(np.float32)
+    assert np.array_equal(np.isnan(got), np.isnan(as32)) and np.array_equal(np.isinf(got), np.isinf(as32))
+    there = np.isinf(as32)
+    assert np.array_equal(got[there], as32[there])
+    for rows in (slice(5, 6), slice(0, 5), slice(6, m)):
+        w, g = want[rows], got[rows].astype(np.float64)
+        keep = np.isfinite(as32[rows])
+        keep[:, n - 2] &= tiny                             # (one huge value sets the scale of that column's errors)
+        if not tiny and rows.start == 5:
+            continue
+        assert np.linalg.norm((g - w)[keep]) <= 2.0 ** -24 * (np.sqrt(k) + 4) * np.linalg.norm(w[keep])
