@@ -3,7 +3,7 @@
 // The reference composes attention from op_matmul, op_mul_scalar, op_softmax and op_matmul
 // (ops/ops.c:6816-6884, 6022-6086, 5721-5788), which streams the [S, S] score and probability matrices through
 // memory four times; at 512 x 512 per head they outweigh Q, K, V and O eight to one.  Here a workgroup owns 128 query
-// rows of one head (a wave 32 of them) and walks the keys 32 at a time:
+// rows of one head (a wave 32 of them) and walks the keys 32 or 64 at a time:
 //
 //   S^T tile   = K_blk (32 keys x D) * Q_w^T (D x 32 queries)        MFMA 32x32x16, fp32 accumulate
 //   online softmax on S^T: in this orientation a lane owns ONE query (its column) and 16 keys (its registers), so the
@@ -44,23 +44,87 @@ template <typename T> __device__ __forceinline__ s16x8_t pack8(const float* x) {
     return __builtin_bit_cast(s16x8_t, w);
 }
 
+// SPLIT (small grids): the workgroup owns 32 rows instead of 128, its four waves take every fourth block of 32 of the axis
+// that is walked, and the four partial results meet in LDS at the end.  A wave stages its own blocks, in LDS of its own: a
+// wave's LDS operations are executed in order, so there is one stage and no barrier; this keeps the compiler's order too.
+__device__ __forceinline__ void attn_wave_order() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+constexpr int attn_max(int a, int b) { return a > b ? a : b; }
+template <int D> constexpr int AT_PART = D + 4;                                     // LDS pitch of a row of a partial result in floats
+template <int D> constexpr int attn_parts_bytes() { return 4 * 32 * AT_PART<D> * 4; }
+
+// A wave's 32 x D partial result (lane = row c, registers 4*v4 .. + 3 of tile dt: columns 32*dt + 8*v4 + 4h ..) to its place
+template <int D>
+__device__ __forceinline__ void attn_put_part(float* parts, int wave, int h, int c, const f32x16_t (&acc)[D / 32]) {
+    float* row = parts + (wave * 32 + c) * AT_PART<D>;
+#pragma unroll
+    for (int dt = 0; dt < D / 32; dt++)
+#pragma unroll
+        for (int v4 = 0; v4 < 4; v4++)
+            *(f32x4_t*)(row + 32 * dt + 8 * v4 + 4 * h) = f32x4_t{acc[dt][4 * v4], acc[dt][4 * v4 + 1], acc[dt][4 * v4 + 2], acc[dt][4 * v4 + 3]};
+}
+// Thread t writes columns (t % 8) * D/8 .. of row t / 8: the four partial results, weighted, in wave order
 template <typename T, int D>
-__global__ void __launch_bounds__(256, D <= 64 ? 3 : 1) attention_fwd16_kernel(AttnArgs g) {
+__device__ __forceinline__ void attn_add_parts(T* out, const float* parts, const float (&weight)[4]) {
+    const float* p = parts + (threadIdx.x / 8) * AT_PART<D> + (threadIdx.x % 8) * (D / 8);
+#pragma unroll
+    for (int i = 0; i < D / 8; i += 4) {
+        f32x4_t sum = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int w = 0; w < 4; w++) {
+            const f32x4_t v = *(const f32x4_t*)(p + w * 32 * AT_PART<D> + i);
+#pragma unroll
+            for (int e = 0; e < 4; e++) sum[e] = fmaf(v[e], weight[w], sum[e]);
+        }
+        T o[4];
+#pragma unroll
+        for (int e = 0; e < 4; e++) o[e] = narrow<T>(sum[e]);
+        uint2 w2;
+        memcpy(&w2, o, 8);
+        *(uint2*)(out + (threadIdx.x % 8) * (D / 8) + i) = w2;
+    }
+}
+
+// The larger of this lane's value and that of the lane 32 away
+__device__ __forceinline__ float attn_pair_max(float x) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+
+template <int D, bool SPLIT, int NB>
+constexpr int attn_fwd_lds_bytes() {
+    constexpr int blocks = (SPLIT ? 4 : 2) * 32 * NB * (m16_mc_pitch(D) + D + 8) * 2;
+    return SPLIT ? attn_max(blocks, attn_parts_bytes<D>() + 2 * 4 * 32 * 4) : blocks;
+}
+
+// A step is 32 NB keys.  At d = 128 two workgroups share a CU, at d <= 64 three.  bf16, one wave's 32 queries, before (32 keys a
+// step; at d = 128 one workgroup per CU) and after (64 keys; the running maximum, its exchange and the rescaling of O^T come
+// half as often, and so do the barriers): [192, 512, 512, d] 20.4 -> 17.0, 27.8 -> 25.0 and 68.6 -> 40.8 us for d = 32, 64, 128;
+// [8, 4096, 4096, 64] 86 -> 60 us.  What bounds it is the softmax arithmetic (sixteen exponentials of a quarter rate beside
+// eight MFMAs per 32 x 32 scores at d = 64), not memory.
+template <typename T, int D, bool SPLIT, int NB>
+__global__ void __launch_bounds__(256, D > 64 || SPLIT ? 2 : 3) attention_fwd16_kernel(AttnArgs g) {
     static_assert(D % 32 == 0 && D <= 128, "head dimension: a multiple of 32 up to 128");
     constexpr int KS = D / 16;              // k-steps of the first product
     constexpr int DT = D / 32;              // 32-row tiles of O^T
     constexpr int VP = m16_mc_pitch(D);     // LDS pitch of a V row in elements, the GEMM kernels' conflict-free one for this read pattern
-    constexpr int VPIECES = AT_KEYS * D / 8 / 256 > 0 ? AT_KEYS * D / 8 / 256 : 1;      // 16-byte pieces of a V block per thread
+    constexpr int KEYS = 32 * NB;           // keys per step
+    constexpr int LANES = SPLIT ? 64 : 256; // threads that stage a block
+    constexpr int VPIECES = KEYS * D / 8 / LANES > 0 ? KEYS * D / 8 / LANES : 1;      // 16-byte pieces of a V block per thread
     constexpr int RP = D + 8;               // LDS pitch of a K row in elements: 16 bytes past a multiple of 128, so that ds_read_b128 of 16 rows is conflict-free
-    __shared__ __attribute__((aligned(16))) uint16_t vlds[2][AT_KEYS * VP];
-    __shared__ __attribute__((aligned(16))) uint16_t klds[2][AT_KEYS * RP];
+    extern __shared__ __attribute__((aligned(16))) uint16_t fwd_lds[];
+    uint16_t (*vlds)[KEYS * VP] = (uint16_t (*)[KEYS * VP])fwd_lds;                                         // [stage, or wave]
+    uint16_t (*klds)[KEYS * RP] = (uint16_t (*)[KEYS * RP])(fwd_lds + (SPLIT ? 4 : 2) * KEYS * VP);
+    const int tid = SPLIT ? threadIdx.x & 63 : threadIdx.x;
 
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int h = lane >> 5, c = lane & 31;
     int row_tile, z;
     attn_block(row_tile, z);
-    const int q0 = row_tile * AT_QROWS + wave * 32;               // this wave's first query row
+    const int q0 = SPLIT ? row_tile * 32 : row_tile * AT_QROWS + wave * 32;               // this wave's first query row
     const uint16_t* Q = (const uint16_t*)g.Q + (long long)z * g.q_bs;
     const uint16_t* K = (const uint16_t*)g.K + (long long)z * g.k_bs;
     const uint16_t* V = (const uint16_t*)g.V + (long long)z * g.v_bs;
@@ -88,8 +152,8 @@ __global__ void __launch_bounds__(256, D <= 64 ? 3 : 1) attention_fwd16_kernel(A
         const __amdgpu_buffer_rsrc_t rsrc = buffer_rsrc(mp, kb < g.sk ? (long long)(end - mp) : 0);
 #pragma unroll
         for (int i = 0; i < VPIECES; i++) {
-            const int id = threadIdx.x + 256 * i, key = id / (D / 8), d8 = (id % (D / 8)) * 8;
-            const bool live = AT_KEYS * D / 8 >= 256 || id < AT_KEYS * D / 8;
+            const int id = tid + LANES * i, key = id / (D / 8), d8 = (id % (D / 8)) * 8;
+            const bool live = KEYS * D / 8 >= LANES || id < KEYS * D / 8;
             r[i] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, live ? (int)(((long long)key * rs + d8) * 2) : (int)BUFFER_OOB, 0, 0);
         }
     };
@@ -99,16 +163,16 @@ __global__ void __launch_bounds__(256, D <= 64 ? 3 : 1) attention_fwd16_kernel(A
     auto store_k = [&](const u32x4_t (&kr)[VPIECES], uint16_t* stage) {
 #pragma unroll
         for (int i = 0; i < VPIECES; i++) {
-            const int id = threadIdx.x + 256 * i, key = id / (D / 8), d8 = (id % (D / 8)) * 8;
-            if (AT_KEYS * D / 8 >= 256 || id < AT_KEYS * D / 8) *(u32x4_t*)(stage + key * RP + d8) = kr[i];
+            const int id = tid + LANES * i, key = id / (D / 8), d8 = (id % (D / 8)) * 8;
+            if (KEYS * D / 8 >= LANES || id < KEYS * D / 8) *(u32x4_t*)(stage + key * RP + d8) = kr[i];
         }
     };
     const int k_fr0 = c * RP + 8 * h;
     auto store_v = [&](const u32x4_t (&vr)[VPIECES], uint16_t* stage) {
 #pragma unroll
         for (int i = 0; i < VPIECES; i++) {
-            const int id = threadIdx.x + 256 * i, key = id / (D / 8), d8 = (id % (D / 8)) * 8;
-            if (AT_KEYS * D / 8 >= 256 || id < AT_KEYS * D / 8) *(u32x4_t*)(stage + key * VP + d8) = vr[i];
+            const int id = tid + LANES * i, key = id / (D / 8), d8 = (id % (D / 8)) * 8;
+            if (KEYS * D / 8 >= LANES || id < KEYS * D / 8) *(u32x4_t*)(stage + key * VP + d8) = vr[i];
         }
     };
     // V^T as an A operand of the second product: lane row d = 32*dt + c, k slot e of MFMA t <-> key 16t + 8*(e/4) + 4h + e%4.
@@ -131,92 +195,142 @@ __global__ void __launch_bounds__(256, D <= 64 ? 3 : 1) attention_fwd16_kernel(A
     for (int dt = 0; dt < DT; dt++)
 #pragma unroll
         for (int v = 0; v < 16; v++) ot[dt][v] = 0.f;
-    float m_run = -INFINITY, l_run = 0.f;            // running maximum (of the raw, sign-adjusted scores) and this lane's share of the running sum
+    float m_run = -INFINITY, msc = 0.f, l_run = 0.f;         // running maximum (of the raw, sign-adjusted scores), the same times sc, and this lane's share of the running sum
 
-    const int nblocks = (g.sk + AT_KEYS - 1) / AT_KEYS;
+    const int nblocks = (g.sk + KEYS - 1) / KEYS;
+    const int blk0 = SPLIT ? wave : 0;
+    constexpr int stride = SPLIT ? 4 : 1;            // blocks from one step to the next
     u32x4_t kr[VPIECES], vr[VPIECES];
-    load_k(kr, 0);
-    load_v(vr, 0);
-    store_k(kr, klds[0]);
-    store_v(vr, vlds[0]);
-    load_k(kr, AT_KEYS);
-    load_v(vr, AT_KEYS);
-    __syncthreads();
+    load_k(kr, blk0 * KEYS);
+    load_v(vr, blk0 * KEYS);
+    store_k(kr, klds[blk0]);
+    store_v(vr, vlds[blk0]);
+    load_k(kr, (blk0 + stride) * KEYS);
+    load_v(vr, (blk0 + stride) * KEYS);
+    if constexpr (SPLIT) attn_wave_order();
+    else __syncthreads();
 
     auto step = [&](int blk) {
-        const int kb = blk * AT_KEYS;
-        const uint16_t* stage = vlds[blk & 1];
-        const uint16_t* kstage = klds[blk & 1];
-        // scores of 32 keys x 32 queries
-        f32x16_t st;
+        const int kb = blk * KEYS;
+        const int cur = SPLIT ? wave : blk & 1, next = SPLIT ? wave : cur ^ 1;
+        const uint16_t* stage = vlds[cur];
+        const uint16_t* kstage = klds[cur];
+        // scores of KEYS keys x 32 queries
+        f32x16_t st[NB];
 #pragma unroll
-        for (int v = 0; v < 16; v++) st[v] = 0.f;
+        for (int b = 0; b < NB; b++) {
 #pragma unroll
-        for (int ks = 0; ks < KS; ks++) st = mfma16_ops<T>::mma(*(const s16x8_t*)(kstage + k_fr0 + 16 * ks), qf[ks], st);
-        // the next block goes to the other stage (everyone left it at the previous barrier); then request the one after
-        store_k(kr, klds[(blk & 1) ^ 1]);
-        store_v(vr, vlds[(blk & 1) ^ 1]);
-        load_k(kr, kb + 2 * AT_KEYS);
-        load_v(vr, kb + 2 * AT_KEYS);
-
-        // this step's V^T fragments, requested before the softmax arithmetic that hides their latency
+            for (int v = 0; v < 16; v++) st[b][v] = 0.f;
+#pragma unroll
+            for (int ks = 0; ks < KS; ks++) st[b] = mfma16_ops<T>::mma(*(const s16x8_t*)(kstage + 32 * b * RP + k_fr0 + 16 * ks), qf[ks], st[b]);
+        }
+        // the V^T fragments of the first 32 keys, requested before the softmax arithmetic that hides their latency
         s16x8_t vfr[2][DT];
+        auto read_vs = [&](int b) {
 #pragma unroll
-        for (int t = 0; t < 2; t++)
+            for (int t = 0; t < 2; t++)
 #pragma unroll
-            for (int dt = 0; dt < DT; dt++) vfr[t][dt] = read_v(stage, dt, t);
+                for (int dt = 0; dt < DT; dt++) vfr[t][dt] = read_v(stage + 32 * b * VP, dt, t);
+        };
+        if constexpr (SPLIT) {
+            read_vs(0);
+            attn_wave_order();
+        }
+        // the next block goes to the other stage (everyone left it at the previous barrier); then request the one after
+        store_k(kr, klds[next]);
+        store_v(vr, vlds[next]);
+        load_k(kr, kb + 2 * stride * KEYS);
+        load_v(vr, kb + 2 * stride * KEYS);
+        if constexpr (SPLIT) attn_wave_order();
+        else read_vs(0);
 
         if (flip) {
 #pragma unroll
-            for (int v = 0; v < 16; v++) st[v] = -st[v];
+            for (int b = 0; b < NB; b++)
+#pragma unroll
+                for (int v = 0; v < 16; v++) st[b][v] = -st[b][v];
         }
-        const bool ragged = kb + AT_KEYS > g.sk;            // the last block of a ragged sk
+        const bool ragged = kb + KEYS > g.sk;               // the last block of a ragged sk
         if (ragged) {
 #pragma unroll
-            for (int v = 0; v < 16; v++)
-                if (kb + 8 * (v / 4) + 4 * h + (v % 4) >= g.sk) st[v] = -INFINITY;
+            for (int b = 0; b < NB; b++)
+#pragma unroll
+                for (int v = 0; v < 16; v++)
+                    if (kb + 32 * b + 8 * (v / 4) + 4 * h + (v % 4) >= g.sk) st[b][v] = -INFINITY;
         }
         float mx = m_run;
 #pragma unroll
-        for (int v = 0; v < 16; v++) mx = fmaxf(st[v], mx);
-        const float other = __shfl_xor(mx, 32, 64);         // the lane that holds this query's other 16 keys
-        mx = fmaxf(other, mx);
+        for (int b = 0; b < NB; b++)
+#pragma unroll
+            for (int v = 0; v < 16; v++) mx = fmaxf(st[b][v], mx);
+        mx = attn_pair_max(mx);                // the lane 32 away holds this query's other keys
         // a query row beyond sq (or a block of masked keys met first) keeps mx = -inf: exp2(-inf - -inf) must not produce NaN
-        const float m_use = mx == -INFINITY ? 0.f : mx;
-        const float msc = m_use * sc;
-        const float alpha = __builtin_amdgcn_exp2f(m_run == -INFINITY ? -INFINITY : m_run * sc - msc);
-        float psum = 0.f;
-        float e[16];
-#pragma unroll
-        for (int v = 0; v < 16; v++) e[v] = __builtin_amdgcn_exp2f(fmaf(st[v], sc, -msc));
-        if (ragged) {                                       // a masked score times a zero scale would be NaN, not 0
-#pragma unroll
-            for (int v = 0; v < 16; v++)
-                if (kb + 8 * (v / 4) + 4 * h + (v % 4) >= g.sk) e[v] = 0.f;
-        }
-#pragma unroll
-        for (int v = 0; v < 16; v++) psum += e[v];
-        l_run = l_run * alpha + psum;
+        const float before = m_run == -INFINITY ? -INFINITY : msc;
+        msc = (mx == -INFINITY ? 0.f : mx) * sc;
+        const float alpha = __builtin_amdgcn_exp2f(before - msc);
         m_run = mx;
+        l_run *= alpha;
         if (__builtin_amdgcn_ballot_w64(alpha != 1.f)) {   // once the running maxima have settled there is nothing to rescale
 #pragma unroll
             for (int dt = 0; dt < DT; dt++)
 #pragma unroll
                 for (int v = 0; v < 16; v++) ot[dt][v] *= alpha;
         }
-        // O^T += V^T * P^T, 16 keys per MFMA
 #pragma unroll
-        for (int t = 0; t < 2; t++) {
-            const s16x8_t pb = pack8<T>(e + 8 * t);
+        for (int b = 0; b < NB; b++) {
+            float e[16], psum = 0.f;
 #pragma unroll
-            for (int dt = 0; dt < DT; dt++) ot[dt] = mfma16_ops<T>::mma(vfr[t][dt], pb, ot[dt]);
+            for (int v = 0; v < 16; v++) e[v] = __builtin_amdgcn_exp2f(fmaf(st[b][v], sc, -msc));
+            if (ragged) {                                   // a masked score times a zero scale would be NaN, not 0
+#pragma unroll
+                for (int v = 0; v < 16; v++)
+                    if (kb + 32 * b + 8 * (v / 4) + 4 * h + (v % 4) >= g.sk) e[v] = 0.f;
+            }
+#pragma unroll
+            for (int v = 0; v < 16; v++) psum += e[v];
+            l_run += psum;
+            // O^T += V^T * P^T, 16 keys per MFMA
+            if (b > 0) read_vs(b);
+#pragma unroll
+            for (int t = 0; t < 2; t++) {
+                const s16x8_t pb = pack8<T>(e + 8 * t);
+#pragma unroll
+                for (int dt = 0; dt < DT; dt++) ot[dt] = mfma16_ops<T>::mma(vfr[t][dt], pb, ot[dt]);
+            }
         }
-        __syncthreads();                                    // next stage is written, this one is free
+        if constexpr (!SPLIT) __syncthreads();              // next stage is written, this one is free
     };
-    for (int blk = 0; blk < nblocks; blk++) step(blk);
+    for (int blk = blk0; blk < nblocks; blk += stride) step(blk);
 
     // finish: the two lanes of a query add their sums; O[q][d] = O^T[d][q] / l
     const float l_all = l_run + __shfl_xor(l_run, 32, 64);
+    if constexpr (SPLIT) {
+        float* parts = (float*)fwd_lds;
+        float (*ms)[32] = (float (*)[32])(fwd_lds + attn_parts_bytes<D>() / 2);       // [wave][query]: reference points, then sums
+        float (*ls)[32] = ms + 4;
+        __syncthreads();                                    // everyone is done with the blocks that this overwrites
+        attn_put_part<D>(parts, wave, h, c, ot);
+        if (h == 0) {
+            ms[wave][c] = m_run == -INFINITY ? -INFINITY : msc;
+            ls[wave][c] = l_all;
+        }
+        __syncthreads();
+        const int r = threadIdx.x / 8, q = q0 + r;
+        if (q >= g.sq) return;
+        float top = fmaxf(fmaxf(ms[0][r], ms[1][r]), fmaxf(ms[2][r], ms[3][r])), l = 0.f, weight[4];
+        if (top == -INFINITY) top = 0.f;
+#pragma unroll
+        for (int w = 0; w < 4; w++) {
+            weight[w] = __builtin_amdgcn_exp2f(ms[w][r] - top);
+            l = fmaf(ls[w][r], weight[w], l);
+        }
+        const float inv = l > 0.f ? 1.f / l : 0.f;
+#pragma unroll
+        for (int w = 0; w < 4; w++) weight[w] *= inv;
+        attn_add_parts<T, D>((T*)g.O + (long long)z * g.o_bs + (long long)q * g.o_rs, parts, weight);
+        if (g.L && threadIdx.x % 8 == 0) g.L[(long long)z * g.sq + q] = (top + __builtin_amdgcn_logf(l)) * 0.693147180559945309f;
+        return;
+    }
     const float inv = l_all > 0.f ? 1.f / l_all : 0.f;
     const int q = q0 + c;
     if (q < g.sq) {
@@ -233,7 +347,7 @@ __global__ void __launch_bounds__(256, D <= 64 ? 3 : 1) attention_fwd16_kernel(A
                 memcpy(&w, out, 8);
                 *(uint2*)(orow + 32 * dt + 8 * v4 + 4 * h) = w;
             }
-        if (g.L && h == 0) g.L[(long long)z * g.sq + q] = (m_run * sc + __builtin_amdgcn_logf(l_all)) * 0.693147180559945309f;   // natural log of the row sum of exp(scale * s)
+        if (g.L && h == 0) g.L[(long long)z * g.sq + q] = (msc + __builtin_amdgcn_logf(l_all)) * 0.693147180559945309f;   // natural log of the row sum of exp(scale * s)
     }
 }
 
@@ -249,26 +363,28 @@ __global__ void __launch_bounds__(256, D <= 64 ? 3 : 1) attention_fwd16_kernel(A
 // ds_read_tr16_b64.
 // ============================================================================
 // A [32 rows][D] block of a d-contiguous matrix, staged in LDS for transposed MFMA operand reads.
-template <int D>
+// LANES threads stage it: the workgroup, or each wave blocks of its own.
+template <int D, int LANES = 256>
 struct AttnBlock {
     static constexpr int VP = m16_mc_pitch(D);
     static constexpr int ELEMS = AT_KEYS * VP;
-    static constexpr int PIECES = AT_KEYS * D / 8 / 256 > 0 ? AT_KEYS * D / 8 / 256 : 1;
+    static __device__ __forceinline__ int tid() { return LANES == 256 ? threadIdx.x : threadIdx.x & 63; }
+    static constexpr int PIECES = AT_KEYS * D / 8 / LANES > 0 ? AT_KEYS * D / 8 / LANES : 1;
     static __device__ __forceinline__ void load(u32x4_t (&r)[PIECES], const uint16_t* M, long long rs, int row0, int rows, const char* end) {
         const char* p = (const char*)(M + (long long)row0 * rs);
         const __amdgpu_buffer_rsrc_t rsrc = buffer_rsrc(p, row0 < rows ? (long long)(end - p) : 0);
 #pragma unroll
         for (int i = 0; i < PIECES; i++) {
-            const int id = threadIdx.x + 256 * i, row = id / (D / 8), d8 = (id % (D / 8)) * 8;
-            const bool live = AT_KEYS * D / 8 >= 256 || id < AT_KEYS * D / 8;
+            const int id = tid() + LANES * i, row = id / (D / 8), d8 = (id % (D / 8)) * 8;
+            const bool live = AT_KEYS * D / 8 >= LANES || id < AT_KEYS * D / 8;
             r[i] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, live ? (int)(((long long)row * rs + d8) * 2) : (int)BUFFER_OOB, 0, 0);
         }
     }
     static __device__ __forceinline__ void store(const u32x4_t (&r)[PIECES], uint16_t* stage) {
 #pragma unroll
         for (int i = 0; i < PIECES; i++) {
-            const int id = threadIdx.x + 256 * i, row = id / (D / 8), d8 = (id % (D / 8)) * 8;
-            if (AT_KEYS * D / 8 >= 256 || id < AT_KEYS * D / 8) *(u32x4_t*)(stage + row * VP + d8) = r[i];
+            const int id = tid() + LANES * i, row = id / (D / 8), d8 = (id % (D / 8)) * 8;
+            if (AT_KEYS * D / 8 >= LANES || id < AT_KEYS * D / 8) *(u32x4_t*)(stage + row * VP + d8) = r[i];
         }
     }
     // the same block kept a second way, for operands whose fragments are 8 consecutive d of one row (ds_read_b128):
@@ -278,8 +394,8 @@ struct AttnBlock {
     static __device__ __forceinline__ void store_rows(const u32x4_t (&r)[PIECES], uint16_t* stage) {
 #pragma unroll
         for (int i = 0; i < PIECES; i++) {
-            const int id = threadIdx.x + 256 * i, row = id / (D / 8), d8 = (id % (D / 8)) * 8;
-            if (AT_KEYS * D / 8 >= 256 || id < AT_KEYS * D / 8) *(u32x4_t*)(stage + row * RP + d8) = r[i];
+            const int id = tid() + LANES * i, row = id / (D / 8), d8 = (id % (D / 8)) * 8;
+            if (AT_KEYS * D / 8 >= LANES || id < AT_KEYS * D / 8) *(u32x4_t*)(stage + row * RP + d8) = r[i];
         }
     }
     // fragment ks of block row c: d = 16*ks + 8h .. +7 (an A operand with row = lane % 32)
@@ -313,19 +429,28 @@ __device__ __forceinline__ void attn_load_rows(s16x8_t (&f)[KS], const uint16_t*
 }
 
 // dQ: a wave owns 32 queries and walks the keys.
-template <typename T, int D>
-__global__ void __launch_bounds__(256, D <= 64 ? 3 : 1) attention_bwd_dq16_kernel(AttnBwdArgs g) {
+template <int D>
+constexpr int attn_dq_split_lds_bytes() {
+    return attn_max(4 * (AttnBlock<D>::ELEMS + 2 * AttnBlock<D>::ROW_ELEMS) * 2, attn_parts_bytes<D>());
+}
+
+template <typename T, int D, bool SPLIT, int PER_CU>
+__global__ void __launch_bounds__(256, PER_CU) attention_bwd_dq16_kernel(AttnBwdArgs g) {
     constexpr int KS = D / 16, DT = D / 32;
-    using Blk = AttnBlock<D>;
-    __shared__ __attribute__((aligned(16))) uint16_t klds[2][Blk::ELEMS];           // K for transposed reads (K^T of the dQ product)
-    __shared__ __attribute__((aligned(16))) uint16_t krows[2][Blk::ROW_ELEMS];       // K and V for row fragments (S^T and dP^T)
-    __shared__ __attribute__((aligned(16))) uint16_t vrows[2][Blk::ROW_ELEMS];
+    constexpr int STAGES = SPLIT ? 4 : 2;                                            // [stage, or wave]
+    using Blk = AttnBlock<D, SPLIT ? 64 : 256>;
+    // arrays of their own where 64 KB are enough: the compiler may then move reads of one past writes to another
+    extern __shared__ __attribute__((aligned(16))) uint16_t dq_lds[];                                       // SPLIT only
+    __shared__ __attribute__((aligned(16))) uint16_t ks[SPLIT ? 1 : STAGES][Blk::ELEMS], kr_s[SPLIT ? 1 : STAGES][Blk::ROW_ELEMS], vr_s[SPLIT ? 1 : STAGES][Blk::ROW_ELEMS];
+    uint16_t (*const klds)[Blk::ELEMS] = SPLIT ? (uint16_t (*)[Blk::ELEMS])dq_lds : ks;                     // K for transposed reads (K^T of the dQ product)
+    uint16_t (*const krows)[Blk::ROW_ELEMS] = SPLIT ? (uint16_t (*)[Blk::ROW_ELEMS])(dq_lds + STAGES * Blk::ELEMS) : kr_s;      // K and V for row fragments (S^T and dP^T)
+    uint16_t (*const vrows)[Blk::ROW_ELEMS] = SPLIT ? krows + STAGES : vr_s;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int h = lane >> 5, c = lane & 31;
     int row_tile, z;
     attn_block(row_tile, z);
-    const int q0 = row_tile * AT_QROWS + wave * 32;
+    const int q0 = SPLIT ? row_tile * 32 : row_tile * AT_QROWS + wave * 32;
     const uint16_t* Q = (const uint16_t*)g.Q + (long long)z * g.q_bs;
     const uint16_t* K = (const uint16_t*)g.K + (long long)z * g.k_bs;
     const uint16_t* V = (const uint16_t*)g.V + (long long)z * g.v_bs;
@@ -356,7 +481,7 @@ __global__ void __launch_bounds__(256, D <= 64 ? 3 : 1) attention_bwd_dq16_kerne
                 dq_dot += widen(a) * widen(b);
             }
         dq_dot += __shfl_xor(dq_dot, 32, 64);
-        if (q < g.sq && h == 0) g.Dq[(long long)z * g.sq + q] = dq_dot;
+        if (q < g.sq && h == 0 && (!SPLIT || wave == 0)) g.Dq[(long long)z * g.sq + q] = dq_dot;
     }
     const float dq_dot_scaled = dq_dot * g.scale;
 
@@ -371,20 +496,23 @@ __global__ void __launch_bounds__(256, D <= 64 ? 3 : 1) attention_bwd_dq16_kerne
     // K and V blocks are staged by the whole workgroup with row-contiguous loads (fragment loads straight from
     // global memory touch 32 cache lines per instruction and wave, more than the vector cache's tag pipeline sustains)
     u32x4_t kr[Blk::PIECES], vr[Blk::PIECES];
-    Blk::load(kr, K, g.k_rs, 0, g.sk, k_end);
-    Blk::load(vr, V, g.v_rs, 0, g.sk, v_end);
-    Blk::store(kr, klds[0]); Blk::store_rows(kr, krows[0]); Blk::store_rows(vr, vrows[0]);
-    Blk::load(kr, K, g.k_rs, AT_KEYS, g.sk, k_end);
-    Blk::load(vr, V, g.v_rs, AT_KEYS, g.sk, v_end);
-    __syncthreads();
+    const int blk0 = SPLIT ? wave : 0;
+    constexpr int stride = SPLIT ? 4 : 1;            // blocks from one step to the next
+    Blk::load(kr, K, g.k_rs, blk0 * AT_KEYS, g.sk, k_end);
+    Blk::load(vr, V, g.v_rs, blk0 * AT_KEYS, g.sk, v_end);
+    Blk::store(kr, klds[blk0]); Blk::store_rows(kr, krows[blk0]); Blk::store_rows(vr, vrows[blk0]);
+    Blk::load(kr, K, g.k_rs, (blk0 + stride) * AT_KEYS, g.sk, k_end);
+    Blk::load(vr, V, g.v_rs, (blk0 + stride) * AT_KEYS, g.sk, v_end);
+    if constexpr (SPLIT) attn_wave_order();
+    else __syncthreads();
 
     auto step = [&](int blk) {
         const int kb = blk * AT_KEYS;
-        const uint16_t* stage = klds[blk & 1];
+        const int cur = SPLIT ? wave : blk & 1, next = SPLIT ? wave : cur ^ 1;
+        const uint16_t* stage = klds[cur];
         f32x16_t st, dp;
 #pragma unroll
         for (int v = 0; v < 16; v++) { st[v] = 0.f; dp[v] = 0.f; }
-        const int cur = blk & 1;
 #pragma unroll
         for (int ks = 0; ks < KS; ks++) st = mfma16_ops<T>::mma(Blk::frag(krows[cur], c, h, ks), qf[ks], st);        // S^T: keys x queries
 #pragma unroll
@@ -395,9 +523,11 @@ __global__ void __launch_bounds__(256, D <= 64 ? 3 : 1) attention_bwd_dq16_kerne
         for (int t = 0; t < 2; t++)
 #pragma unroll
             for (int dt = 0; dt < DT; dt++) ktf[t][dt] = Blk::read_tr(stage, tr0, dt, t);
-        Blk::store(kr, klds[cur ^ 1]); Blk::store_rows(kr, krows[cur ^ 1]); Blk::store_rows(vr, vrows[cur ^ 1]);
-        Blk::load(kr, K, g.k_rs, kb + 2 * AT_KEYS, g.sk, k_end);
-        Blk::load(vr, V, g.v_rs, kb + 2 * AT_KEYS, g.sk, v_end);
+        if constexpr (SPLIT) attn_wave_order();
+        Blk::store(kr, klds[next]); Blk::store_rows(kr, krows[next]); Blk::store_rows(vr, vrows[next]);
+        Blk::load(kr, K, g.k_rs, kb + 2 * stride * AT_KEYS, g.sk, k_end);
+        Blk::load(vr, V, g.v_rs, kb + 2 * stride * AT_KEYS, g.sk, v_end);
+        if constexpr (SPLIT) attn_wave_order();
         float ds[16];
 #pragma unroll
         for (int v = 0; v < 16; v++) {
@@ -415,9 +545,17 @@ __global__ void __launch_bounds__(256, D <= 64 ? 3 : 1) attention_bwd_dq16_kerne
 #pragma unroll
             for (int dt = 0; dt < DT; dt++) acc[dt] = mfma16_ops<T>::mma(ktf[t][dt], dsb, acc[dt]);      // dQ^T += K^T dS^T
         }
-        __syncthreads();
+        if constexpr (!SPLIT) __syncthreads();
     };
-    for (int blk = 0; blk < nblocks; blk++) step(blk);
+    for (int blk = blk0; blk < nblocks; blk += stride) step(blk);
+    if constexpr (SPLIT) {
+        __syncthreads();                                    // everyone is done with the blocks that this overwrites
+        attn_put_part<D>((float*)dq_lds, wave, h, c, acc);
+        __syncthreads();
+        const int r = threadIdx.x / 8;
+        if (q0 + r < g.sq) attn_add_parts<T, D>((T*)g.dQ + ((long long)z * g.sq + q0 + r) * D, (const float*)dq_lds, {1.f, 1.f, 1.f, 1.f});
+        return;
+    }
     if (q < g.sq) {
         T* row = (T*)g.dQ + ((long long)z * g.sq + q) * D;
 #pragma unroll
@@ -435,24 +573,25 @@ __global__ void __launch_bounds__(256, D <= 64 ? 3 : 1) attention_bwd_dq16_kerne
 }
 
 // dK and dV: a wave owns 32 keys and walks the queries.
-template <typename T, int D>
-__global__ void __launch_bounds__(256, D <= 64 ? 2 : 1) attention_bwd_dkv16_kernel(AttnBwdArgs g) {
+template <typename T, int D, bool SPLIT, int PER_CU>
+__global__ void __launch_bounds__(256, PER_CU) attention_bwd_dkv16_kernel(AttnBwdArgs g) {
     constexpr int KS = D / 16, DT = D / 32;
-    using Blk = AttnBlock<D>;
+    constexpr int STAGES = SPLIT ? 4 : 2;                                            // [stage, or wave]
+    using Blk = AttnBlock<D, SPLIT ? 64 : 256>;
     // dynamic LDS (above 64 KB for d = 128): Q and dO blocks, each kept for transposed reads (Q^T, dO^T of the dK and
-    // dV products) and for row fragments (S and dP), two stages; then L and Dq of the block's queries
+    // dV products) and for row fragments (S and dP); then L and Dq of the block's queries
     extern __shared__ __attribute__((aligned(16))) uint16_t dkv_lds[];
     uint16_t (*qlds)[Blk::ELEMS] = (uint16_t (*)[Blk::ELEMS])dkv_lds;
-    uint16_t (*dolds)[Blk::ELEMS] = (uint16_t (*)[Blk::ELEMS])(dkv_lds + 2 * Blk::ELEMS);
-    uint16_t (*qrows)[Blk::ROW_ELEMS] = (uint16_t (*)[Blk::ROW_ELEMS])(dkv_lds + 4 * Blk::ELEMS);
-    uint16_t (*dorows)[Blk::ROW_ELEMS] = (uint16_t (*)[Blk::ROW_ELEMS])(dkv_lds + 4 * Blk::ELEMS + 2 * Blk::ROW_ELEMS);
-    float (*rowlds)[2][AT_KEYS] = (float (*)[2][AT_KEYS])(dkv_lds + 4 * Blk::ELEMS + 4 * Blk::ROW_ELEMS);        // [stage][L, Dq][query of the block]
+    uint16_t (*dolds)[Blk::ELEMS] = qlds + STAGES;
+    uint16_t (*qrows)[Blk::ROW_ELEMS] = (uint16_t (*)[Blk::ROW_ELEMS])(dkv_lds + 2 * STAGES * Blk::ELEMS);
+    uint16_t (*dorows)[Blk::ROW_ELEMS] = qrows + STAGES;
+    float (*rowlds)[2][AT_KEYS] = (float (*)[2][AT_KEYS])(dkv_lds + 2 * STAGES * (Blk::ELEMS + Blk::ROW_ELEMS));        // [stage][L, Dq][query of the block]
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int h = lane >> 5, c = lane & 31;
     int row_tile, z;
     attn_block(row_tile, z);
-    const int k0 = row_tile * AT_QROWS + wave * 32;               // this wave's first key
+    const int k0 = SPLIT ? row_tile * 32 : row_tile * AT_QROWS + wave * 32;               // this wave's first key
     const uint16_t* Q = (const uint16_t*)g.Q + (long long)z * g.q_bs;
     const uint16_t* K = (const uint16_t*)g.K + (long long)z * g.k_bs;
     const uint16_t* V = (const uint16_t*)g.V + (long long)z * g.v_bs;
@@ -479,7 +618,7 @@ __global__ void __launch_bounds__(256, D <= 64 ? 2 : 1) attention_bwd_dkv16_kern
     const int nblocks = (g.sq + AT_KEYS - 1) / AT_KEYS;
     u32x4_t qr[Blk::PIECES], dor[Blk::PIECES];
     // L and Dq of the block's 32 queries: every lane requests query qb + lane % 32 (buffer loads, zero past sq, so
-    // that no branch surrounds them and the wait for them can be counted); wave 0 puts them in LDS: its lower half
+    // that no branch surrounds them and the wait for them can be counted); wave 0 (SPLIT: each wave its own) puts them in LDS: its lower half
     // the L (in log2 units, +inf past sq, which makes those rows' probabilities exactly 0), its upper half Dq * scale
     const __amdgpu_buffer_rsrc_t l_rsrc = buffer_rsrc(Lz, (long long)g.sq * 4), d_rsrc = buffer_rsrc(Dz, (long long)g.sq * 4);
     float row_l = 0.f, row_d = 0.f;
@@ -488,22 +627,25 @@ __global__ void __launch_bounds__(256, D <= 64 ? 2 : 1) attention_bwd_dkv16_kern
         row_d = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(d_rsrc, (qb + c) * 4, 0, 0));
     };
     auto store_rowv = [&](int stage, int qb) {
-        if (wave == 0) rowlds[stage][h][c] = h ? row_d * g.scale : (qb + c < g.sq ? row_l * 1.44269504088896341f : INFINITY);
+        if (SPLIT || wave == 0) rowlds[stage][h][c] = h ? row_d * g.scale : (qb + c < g.sq ? row_l * 1.44269504088896341f : INFINITY);
     };
-    Blk::load(qr, Q, g.q_rs, 0, g.sq, q_end);
-    Blk::load(dor, dO, g.do_rs, 0, g.sq, do_end);
-    load_rowv(0);
-    Blk::store(qr, qlds[0]); Blk::store_rows(qr, qrows[0]);
-    Blk::store(dor, dolds[0]); Blk::store_rows(dor, dorows[0]);
-    store_rowv(0, 0);
-    Blk::load(qr, Q, g.q_rs, AT_KEYS, g.sq, q_end);
-    Blk::load(dor, dO, g.do_rs, AT_KEYS, g.sq, do_end);
-    load_rowv(AT_KEYS);
-    __syncthreads();
+    const int blk0 = SPLIT ? wave : 0;
+    constexpr int stride = SPLIT ? 4 : 1;            // blocks from one step to the next
+    Blk::load(qr, Q, g.q_rs, blk0 * AT_KEYS, g.sq, q_end);
+    Blk::load(dor, dO, g.do_rs, blk0 * AT_KEYS, g.sq, do_end);
+    load_rowv(blk0 * AT_KEYS);
+    Blk::store(qr, qlds[blk0]); Blk::store_rows(qr, qrows[blk0]);
+    Blk::store(dor, dolds[blk0]); Blk::store_rows(dor, dorows[blk0]);
+    store_rowv(blk0, blk0 * AT_KEYS);
+    Blk::load(qr, Q, g.q_rs, (blk0 + stride) * AT_KEYS, g.sq, q_end);
+    Blk::load(dor, dO, g.do_rs, (blk0 + stride) * AT_KEYS, g.sq, do_end);
+    load_rowv((blk0 + stride) * AT_KEYS);
+    if constexpr (SPLIT) attn_wave_order();
+    else __syncthreads();
 
     auto step = [&](int blk) {
         const int qb = blk * AT_KEYS;
-        const int cur = blk & 1;
+        const int cur = SPLIT ? wave : blk & 1, next = SPLIT ? wave : cur ^ 1;
         f32x16_t st, dp;
 #pragma unroll
         for (int v = 0; v < 16; v++) { st[v] = 0.f; dp[v] = 0.f; }
@@ -511,12 +653,15 @@ __global__ void __launch_bounds__(256, D <= 64 ? 2 : 1) attention_bwd_dkv16_kern
         for (int ks = 0; ks < KS; ks++) st = mfma16_ops<T>::mma(Blk::frag(qrows[cur], c, h, ks), kf[ks], st);        // S: queries x keys
 #pragma unroll
         for (int ks = 0; ks < KS; ks++) dp = mfma16_ops<T>::mma(Blk::frag(dorows[cur], c, h, ks), vf[ks], dp);       // dP
-        Blk::store(qr, qlds[cur ^ 1]); Blk::store_rows(qr, qrows[cur ^ 1]);
-        Blk::store(dor, dolds[cur ^ 1]); Blk::store_rows(dor, dorows[cur ^ 1]);
-        store_rowv(cur ^ 1, qb + AT_KEYS);
-        Blk::load(qr, Q, g.q_rs, qb + 2 * AT_KEYS, g.sq, q_end);
-        Blk::load(dor, dO, g.do_rs, qb + 2 * AT_KEYS, g.sq, do_end);
-        load_rowv(qb + 2 * AT_KEYS);
+        auto next_block = [&] {
+            Blk::store(qr, qlds[next]); Blk::store_rows(qr, qrows[next]);
+            Blk::store(dor, dolds[next]); Blk::store_rows(dor, dorows[next]);
+            store_rowv(next, qb + stride * AT_KEYS);
+            Blk::load(qr, Q, g.q_rs, qb + 2 * stride * AT_KEYS, g.sq, q_end);
+            Blk::load(dor, dO, g.do_rs, qb + 2 * stride * AT_KEYS, g.sq, do_end);
+            load_rowv(qb + 2 * stride * AT_KEYS);
+        };
+        if constexpr (!SPLIT) next_block();
         float p[16], ds[16];
 #pragma unroll
         for (int v4 = 0; v4 < 4; v4++) {
@@ -539,9 +684,28 @@ __global__ void __launch_bounds__(256, D <= 64 ? 2 : 1) attention_bwd_dkv16_kern
                 dkt[dt] = mfma16_ops<T>::mma(Blk::read_tr(qlds[cur], tr0, dt, t), dsb, dkt[dt]);      // dK^T += Q^T dS
             }
         }
-        __syncthreads();
+        if constexpr (SPLIT) {
+            attn_wave_order();
+            next_block();
+            attn_wave_order();
+        } else __syncthreads();
     };
-    for (int blk = 0; blk < nblocks; blk++) step(blk);
+    for (int blk = blk0; blk < nblocks; blk += stride) step(blk);
+    if constexpr (SPLIT) {
+        float* parts_k = (float*)dkv_lds;
+        float* parts_v = parts_k + attn_parts_bytes<D>() / 4;
+        __syncthreads();                                    // everyone is done with the blocks that this overwrites
+        attn_put_part<D>(parts_k, wave, h, c, dkt);
+        attn_put_part<D>(parts_v, wave, h, c, dvt);
+        __syncthreads();
+        const int r = threadIdx.x / 8;
+        if (k0 + r < g.sk) {
+            const long long row = ((long long)z * g.sk + k0 + r) * D;
+            attn_add_parts<T, D>((T*)g.dK + row, parts_k, {1.f, 1.f, 1.f, 1.f});
+            attn_add_parts<T, D>((T*)g.dV + row, parts_v, {1.f, 1.f, 1.f, 1.f});
+        }
+        return;
+    }
     const int key = k0 + c;
     if (key < g.sk) {
         T* krow = (T*)g.dK + ((long long)z * g.sk + key) * D;
@@ -561,18 +725,54 @@ __global__ void __launch_bounds__(256, D <= 64 ? 2 : 1) attention_bwd_dkv16_kern
     }
 }
 
-template <int D>
-constexpr size_t attn_dkv_lds_bytes() { return (size_t)(4 * AttnBlock<D>::ELEMS + 4 * AttnBlock<D>::ROW_ELEMS) * 2 + 2 * 2 * AT_KEYS * sizeof(float); }
+template <int D, bool SPLIT>
+constexpr int attn_dkv_lds_bytes() {
+    constexpr int stages = SPLIT ? 4 : 2;
+    constexpr int blocks = stages * (2 * (AttnBlock<D>::ELEMS + AttnBlock<D>::ROW_ELEMS) * 2 + 2 * AT_KEYS * 4);
+    return SPLIT ? attn_max(blocks, 2 * attn_parts_bytes<D>()) : blocks;
+}
+
+static long long attn_groups(int rows, int batch) { return (long long)((rows + AT_QROWS - 1) / AT_QROWS) * batch; }
+
+// Whether a wave's 32 rows become a workgroup of their own that splits the walked axis (SPLIT): where the workgroups of 128 rows
+// leave CUs idle, or are mostly empty, and the walk is long enough to be shared.  bf16, forward / backward in us, unsplit and split:
+//   [12, 512, 512, 64] 11.2 / 29.4 and 6.3 / 15.5      [24, 512, 512, 64] 11.3 / 29.6 and 8.7 / 25.4     [40, 512, 512, 64] 10.9 / 30.0 and 11.0 / 37
+//   [32, 512, 512, 32] 10.2 / 24.2 and 6.5 / 14.9      [100, 37, 777, 64] 14.9 / 33.6 and 8.3 / 25.6     [1, 1, 4096, 64] 60 / 72 and 21 / 27
+//   [300, 37, 777, 64] 21.9 / 59.4 and 16.5 / 56.3     [192, 40, 140, 64] 6.5 / 16.6 and 6.5 / 17.9      [192, 1, 40, 64] 4.5 / 9.0 and 4.4 / 13.7
+// The limit of two 32-row tiles per CU is where they cross; at d = 128 a workgroup takes most of a CU's LDS, and two per CU pay
+// only over long walks: [192, 33, 300, 128] 13.0 / 43.1 and 16.4 / 47.3, [4, 4096, 4096, 128] 108 / 282 and 63 / 214.
+static bool attn_split(int d, int rows, int walked, int batch) {
+    const long long tiles = (long long)((rows + 31) / 32) * batch, cus = device_cu_count();
+    if (walked <= 4 * AT_KEYS) return false;
+    if (tiles <= cus) return true;
+    if (walked < (d > 64 ? 1024 : 256)) return false;
+    return tiles <= 2 * cus || (d <= 64 && tiles <= 2 * attn_groups(rows, batch));
+}
+
+template <typename Kernel, typename Args>
+static int launch_attn(Kernel kernel, int rows, bool split, int smem, const Args& g) {
+    if (smem > 64 * 1024 && !check_hip(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, smem), "hipFuncSetAttribute")) return -1;
+    const int per = split ? 32 : AT_QROWS;
+    hipLaunchKernelGGL(kernel, dim3((rows + per - 1) / per, g.batch), dim3(256), smem, current_stream(), g);
+    return 0;
+}
 
 template <typename T, int D>
 static int launch_attention_bwd_d(const AttnBwdArgs& g) {
-    dim3 gq((g.sq + AT_QROWS - 1) / AT_QROWS, g.batch), gk((g.sk + AT_QROWS - 1) / AT_QROWS, g.batch);
-    constexpr size_t smem = attn_dkv_lds_bytes<D>();
-    auto dkv = attention_bwd_dkv16_kernel<T, D>;
-    if (smem > 64 * 1024 && !check_hip(hipFuncSetAttribute((const void*)dkv, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem), "hipFuncSetAttribute")) return -1;
-    hipLaunchKernelGGL((attention_bwd_dq16_kernel<T, D>), gq, dim3(256), 0, current_stream(), g);
-    hipLaunchKernelGGL(dkv, gk, dim3(256), smem, current_stream(), g);
-    return check_launch("attention backward kernels") ? 0 : -1;
+    // Workgroups per CU that the unsplit kernels are compiled for.  Each more costs registers (spills at the last one), which pays
+    // once there are enough workgroups to fill it: dK / dV at d = 64 with two and three, [192, 512, 512] 72.4 and 68.6 us the whole
+    // backward, [24, 512, 512] 29.4 and 31.1; at d = 128 one and two, [128, 512, 512] 110 and 97, [32, 512, 512] 50.6 and 53.9.
+    constexpr int split = D <= 64 ? 2 : 1;
+    constexpr int dq_few = D <= 64 ? 3 : 1, dq_many = D <= 64 ? 3 : 2, dkv_few = D <= 64 ? 2 : 1, dkv_many = D <= 64 ? 3 : 2;
+    int rq, rk;
+    if (attn_split(D, g.sq, g.sk, g.batch)) rq = launch_attn(attention_bwd_dq16_kernel<T, D, true, split>, g.sq, true, attn_dq_split_lds_bytes<D>(), g);
+    else if (dq_few == dq_many || attn_groups(g.sq, g.batch) <= dq_few * device_cu_count()) rq = launch_attn(attention_bwd_dq16_kernel<T, D, false, dq_few>, g.sq, false, 0, g);
+    else rq = launch_attn(attention_bwd_dq16_kernel<T, D, false, dq_many>, g.sq, false, 0, g);
+    if (rq != 0) return -1;
+    if (attn_split(D, g.sk, g.sq, g.batch)) rk = launch_attn(attention_bwd_dkv16_kernel<T, D, true, split>, g.sk, true, attn_dkv_lds_bytes<D, true>(), g);
+    else if (attn_groups(g.sk, g.batch) <= dkv_few * device_cu_count()) rk = launch_attn(attention_bwd_dkv16_kernel<T, D, false, dkv_few>, g.sk, false, attn_dkv_lds_bytes<D, false>(), g);
+    else rk = launch_attn(attention_bwd_dkv16_kernel<T, D, false, dkv_many>, g.sk, false, attn_dkv_lds_bytes<D, false>(), g);
+    return rk == 0 && check_launch("attention backward kernels") ? 0 : -1;
 }
 
 template <typename T>
@@ -585,16 +785,24 @@ static int launch_attention_bwd_t(const AttnBwdArgs& g, int d) {
     }
 }
 
+template <typename T, int D>
+static int launch_attention_d(const AttnArgs& g) {
+    int rc;
+    if (attn_split(D, g.sq, g.sk, g.batch)) rc = launch_attn(attention_fwd16_kernel<T, D, true, 1>, g.sq, true, attn_fwd_lds_bytes<D, true, 1>(), g);
+    // where half of a first or second block of 64 keys would be past the end (192 x 500 queries, one key: 9.8 us against 9.1)
+    else if (g.sk <= 32 || (g.sk > 64 && g.sk <= 96)) rc = launch_attn(attention_fwd16_kernel<T, D, false, 1>, g.sq, false, attn_fwd_lds_bytes<D, false, 1>(), g);
+    else rc = launch_attn(attention_fwd16_kernel<T, D, false, 2>, g.sq, false, attn_fwd_lds_bytes<D, false, 2>(), g);
+    return rc == 0 && check_launch("attention_fwd16_kernel") ? 0 : -1;
+}
+
 template <typename T>
 static int launch_attention_t(const AttnArgs& g, int d) {
-    dim3 grid((g.sq + AT_QROWS - 1) / AT_QROWS, g.batch);
     switch (d) {
-        case 32:  hipLaunchKernelGGL((attention_fwd16_kernel<T, 32>), grid, dim3(256), 0, current_stream(), g); break;
-        case 64:  hipLaunchKernelGGL((attention_fwd16_kernel<T, 64>), grid, dim3(256), 0, current_stream(), g); break;
-        case 128: hipLaunchKernelGGL((attention_fwd16_kernel<T, 128>), grid, dim3(256), 0, current_stream(), g); break;
+        case 32: return launch_attention_d<T, 32>(g);
+        case 64: return launch_attention_d<T, 64>(g);
+        case 128: return launch_attention_d<T, 128>(g);
         default: set_error("rp_hip_attention_forward: head dimension %d (supported: 32, 64, 128)", d); return -1;
     }
-    return check_launch("attention_fwd16_kernel") ? 0 : -1;
 }
 
 }  // namespace rp

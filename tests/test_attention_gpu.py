@@ -71,6 +71,23 @@ def test_fused_attention_large_scores_and_config4_size():
     assert oracle.rel_err(oracle.to_f64(got[sel], BF16), want) <= 1e-2
 
 
+@pytest.mark.parametrize("dt", [BF16, F16], ids=lambda d: NAMES[d])
+@pytest.mark.parametrize("Z", [3, 300])
+@pytest.mark.parametrize("first,last", [(-40.0, 40.0), (-2.0, 6.0), (0.0, 5.6), (30.0, -30.0)])
+def test_fused_attention_scores_that_rise_along_the_keys(dt, Z, first, last):
+    """The running maximum moves in every block of keys, now and then, and never again.  Few heads and many: the two ways the
+    rows are dealt to workgroups."""
+    rng = np.random.default_rng(65)
+    sq, sk, d = 40, 200, 32
+    q = oracle.to_storage(1 + rng.normal(0, 0.1, (Z, sq, d)), dt)
+    k = oracle.to_storage(np.linspace(first, last, sk)[None, :, None] / d + rng.normal(0, 0.02, (Z, sk, d)), dt)
+    v = rand_storage(rng, (Z, sk, d), dt)
+    got, lse = _fused(q, k, v, dt, 1.0, want_lse=True)
+    want, want_lse = _f64(q, k, v, dt, 1.0)
+    assert oracle.rel_err(oracle.to_f64(got, dt), want) <= FWD_TOL[dt]
+    assert np.max(np.abs(lse - want_lse)) <= 1e-3 * max(1.0, np.max(np.abs(want_lse)))
+
+
 def test_fused_attention_rejects_bad_arguments():
     d = capi.DeviceBuffer(4096)
     L = capi.lib()
@@ -80,6 +97,29 @@ def test_fused_attention_rejects_bad_arguments():
     assert L.rp_hip_attention_forward(d.ptr, d.ptr, d.ptr, d.ptr, None, 1, 4, 4, 96, 384, 96, 384, 96, 384, 96, 384, 96, 1.0, capi.F32) == -1
     assert L.rp_hip_attention_forward(d.ptr, d.ptr, d.ptr, d.ptr, None, 1, 4, 4, 64, 256, 66, 256, 64, 256, 64, 256, 64, 1.0, capi.F32) == -1      # row stride not a multiple of 16 bytes
     assert L.rp_hip_attention_forward(d.ptr, d.ptr, d.ptr, d.ptr, None, 1, 4, 4, 64, 256, 60, 256, 64, 256, 64, 256, 64, 1.0, BF16) == -1
+
+
+@pytest.mark.parametrize("dt", [BF16, F16], ids=lambda d: NAMES[d])
+@pytest.mark.parametrize("shape", [
+    (130, 140, 300, 64), (200, 260, 200, 64), (90, 300, 270, 128), (300, 130, 140, 32),         # 128 rows a workgroup: few and many of them
+    (256, 32, 129, 64), (257, 32, 255, 64), (257, 32, 256, 64), (600, 33, 257, 32),              # either side of the rules that split the walk
+    (40, 1, 130, 128), (1, 1, 1000, 64), (3, 257, 1024, 128), (300, 40, 1024, 128),
+    (2, 129, 32, 64), (2, 40, 64, 64), (2, 40, 65, 64), (2, 70, 96, 128), (2, 70, 97, 32),       # either side of the step of 32 or 64 keys
+], ids=lambda s: "x".join(map(str, s)))
+def test_fused_attention_ways_of_dealing_the_rows(dt, shape):
+    Z, sq, sk, d = shape
+    rng = np.random.default_rng(66)
+    q, k, v, g = rand_storage(rng, (Z, sq, d), dt), rand_storage(rng, (Z, sk, d), dt), rand_storage(rng, (Z, sk, d), dt), rand_storage(rng, (Z, sq, d), dt)
+    scale = -1.0 / np.sqrt(d) if sq % 2 else 1.0 / np.sqrt(d)
+    got, lse = _fused(q, k, v, dt, scale, want_lse=True)
+    grads = _fused_backward(q, k, v, g, dt, scale)
+    sel = sorted({0, Z // 2, Z - 1})
+    want, want_lse = _f64(q[sel], k[sel], v[sel], dt, scale)
+    assert oracle.rel_err(oracle.to_f64(got[sel], dt), want) <= FWD_TOL[dt]
+    assert np.max(np.abs(lse[sel] - want_lse)) <= 1e-3 * max(1.0, np.max(np.abs(want_lse)))
+    for name, a, b in zip(("dQ", "dK", "dV"), grads, _f64_backward(q[sel], k[sel], v[sel], g[sel], dt, scale)):
+        assert oracle.rel_err(oracle.to_f64(a[sel], dt), b) <= BWD_TOL[dt], name
+    assert np.all(np.isfinite(lse)) and all(np.all(np.isfinite(oracle.to_f64(x, dt))) for x in (got, *grads))
 
 
 def _f64_backward(q, k, v, g, dt, scale):
