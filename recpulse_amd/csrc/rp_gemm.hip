@@ -334,6 +334,28 @@ int* noalloc_arrival_counters() {
     return (int*)g_noalloc_base;
 }
 
+// First byte and one past the last of an operand of a product
+struct Span { const char* lo; const char* hi; };
+static Span span_of(const void* p, int rows, int cols, long long rs, long long cs, int esz) {
+    return {(const char*)p, (const char*)p + ((rows - 1) * rs + (cols - 1) * cs + 1) * esz};
+}
+static bool overlap(const Span& a, const Span& b) { return a.lo < b.hi && b.lo < a.hi; }
+
+// Whether dX and dW of a 16-bit Linear layer go out as one launch: both on the 64 x 64 tile (an output of under half a CU count
+// of 128 x 128 tiles) in the layouts of dense X and W, and neither gradient written over anything that the other product reads
+// (one launch after the other, dW over W was fine).  Larger tiles fill a CU by themselves and gain nothing from company.
+static bool linear_backward_pairs(const GemmArgs& gx, const GemmArgs& gw, int dtype, bool& edge) {
+    if (path_disabled("pair16") || !(aligned16(gx.A) && aligned16(gx.B) && aligned16(gw.A))) return false;
+    const Plan px = make_plan(1, gx.m, gx.k, gx.n, gx.a_rs, gx.a_cs, gx.b_rs, gx.b_cs, gx.c_rs, gx.c_cs, 0, 0, dtype);
+    const Plan pw = make_plan(1, gw.m, gw.k, gw.n, gw.a_rs, gw.a_cs, gw.b_rs, gw.b_cs, gw.c_rs, gw.c_cs, 0, 0, dtype);
+    if (px.fam != FAM_MFMA16 || px.bm != 64 || px.bn != 64 || px.ragged || px.a_mc || px.b_mc) return false;
+    if (pw.fam != FAM_MFMA16 || pw.bm != 64 || pw.bn != 64 || pw.ragged || !pw.a_mc || !pw.b_mc) return false;
+    edge = px.edge || pw.edge;
+    const Span dx = span_of(gx.C, gx.m, gx.n, gx.c_rs, gx.c_cs, 2), dw = span_of(gw.C, gw.m, gw.n, gw.c_rs, gw.c_cs, 2);
+    const Span dy = span_of(gx.A, gx.m, gx.k, gx.a_rs, gx.a_cs, 2), w = span_of(gx.B, gx.k, gx.n, gx.b_rs, gx.b_cs, 2), x = span_of(gw.A, gw.m, gw.k, gw.a_rs, gw.a_cs, 2);
+    return !(overlap(dx, dw) || overlap(dx, dy) || overlap(dx, x) || overlap(dw, dy) || overlap(dw, w));
+}
+
 }  // namespace rp
 
 using namespace rp;
@@ -412,8 +434,14 @@ int rp_hip_linear_backward(void* dx, void* dw, void* db, const void* dy, const v
         if (!dw) gw.m = 0;
         return launch_linear_backward_tiny(gx, gw, db, dy, m, n, accumulate_db);
     }
-    if (dx && run_gemm(gx, dtype) != 0) return -1;
-    if (dw && run_gemm(gw, dtype) != 0) return -1;
+    bool edge = false;
+    if ((dtype == RP_DTYPE_BFLOAT16 || dtype == RP_DTYPE_FLOAT16) && dx && dw && linear_backward_pairs(gx, gw, dtype, edge)) {
+        g_last_kernel = "mfma16_64x64";
+        if (launch_linear_backward16(gx, gw, edge, dtype) != 0) return -1;
+    } else {
+        if (dx && run_gemm(gx, dtype) != 0) return -1;
+        if (dw && run_gemm(gw, dtype) != 0) return -1;
+    }
     if (db && rp_hip_reduce_rows(db, dy, m, n, accumulate_db, dtype) != 0) return -1;
     return 0;
 }

@@ -156,8 +156,9 @@ __device__ __forceinline__ u32x4_t m16_pull_shift(u32x4_t v, int pull) {
 }
 typedef unsigned int u32x4_any_t __attribute__((ext_vector_type(4), aligned(2)));       // a 16-byte vector at any element
 
+// What one workgroup does: slots first_slot, first_slot + stride, ... of the schedule of matrix z
 template <typename T, int BM, int BN, int WGM, bool A_MC, bool B_MC, int EDGE, bool SPLITK>
-__global__ void __launch_bounds__(256) gemm_mfma16_kernel(GemmArgs g, int tiles_m, int tiles_n, float* partials, int k_per_split, int sched_total) {
+__device__ __forceinline__ void gemm_mfma16_block(const GemmArgs& g, int tiles_m, int tiles_n, float* partials, int k_per_split, int sched_total, int first_slot, int z, int stride) {
     constexpr int WGN = 4 / WGM;
     constexpr int WM = BM / WGM, WN = BN / WGN;       // wave patch
     constexpr int MT = SPLITK ? 32 : m16_mfma_tile(BM, BN);      // MFMA tile edge; k-steps of 16 (MT 32) or 32 (MT 16)
@@ -176,14 +177,12 @@ __global__ void __launch_bounds__(256) gemm_mfma16_kernel(GemmArgs g, int tiles_
     constexpr int NMFMA = TMI * TNI;
     extern __shared__ __attribute__((aligned(16))) uint16_t smem[];
 
-    int first_slot, z;
-    batched_block(tiles_m, tiles_n, first_slot, z);
     // A workgroup walks the schedule with the grid's stride.  The launcher starts one workgroup per slot of the schedule,
     // except for the 256 x 256 tile, which fills a CU by itself: there one workgroup per CU stays resident and takes its
     // tiles one after the other, so that a tile's output stores drain, and the next tile's first loads fly, while MFMAs
     // run; a workgroup per tile would hold the CU idle until its last store was acknowledged.  A stride that is a
     // multiple of 8 keeps a workgroup's tiles on the XCD the schedule assigned them to.
-    for (int tile_id = first_slot; tile_id < sched_total; tile_id += gridDim.x) {
+    for (int tile_id = first_slot; tile_id < sched_total; tile_id += stride) {
     TileCoord tc = schedule_tile(tile_id, tiles_m, tiles_n);
     if (!tc.valid) continue;
     const int m0 = tc.tm * BM, n0 = tc.tn * BN;
@@ -634,6 +633,13 @@ __global__ void __launch_bounds__(256) gemm_mfma16_kernel(GemmArgs g, int tiles_
         }
     }
     }   // tiles of this workgroup
+}
+
+template <typename T, int BM, int BN, int WGM, bool A_MC, bool B_MC, int EDGE, bool SPLITK>
+__global__ void __launch_bounds__(256) gemm_mfma16_kernel(GemmArgs g, int tiles_m, int tiles_n, float* partials, int k_per_split, int sched_total) {
+    int first_slot, z;
+    batched_block(tiles_m, tiles_n, first_slot, z);
+    gemm_mfma16_block<T, BM, BN, WGM, A_MC, B_MC, EDGE, SPLITK>(g, tiles_m, tiles_n, partials, k_per_split, sched_total, first_slot, z, (int)gridDim.x);
 }
 
 // Launch one instantiation.  nsplit > 1 selects the split-k variant: partials must hold batch * nsplit * m * n floats.

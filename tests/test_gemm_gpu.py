@@ -629,6 +629,33 @@ def test_linear_backward_in_one_call(dt):
     assert L.rp_hip_linear_backward(None, None, None, None, None, None, 4, 4, 4, 4, 1, 4, 1, 4, 1, 4, 1, 0, 0, 0, dt) == -1
 
 
+@pytest.mark.parametrize("dt", [BF16, F16], ids=lambda d: NAMES[d])
+@pytest.mark.parametrize("shape", [(64, 64, 64), (72, 136, 264), (8, 512, 520), (200, 1032, 72), (448, 704, 1024), (1024, 1024, 1024)], ids=lambda s: "x".join(map(str, s)))
+def test_linear_backward_pair_16bit(dt, shape):
+    """dX and dW of a 16-bit layer in one launch: the bits of the two products, also accumulated and in padded rows; dW written
+    over W (which dX reads) is the two products one after the other."""
+    m, k, n = shape
+    rng = np.random.default_rng(43)
+    L = capi.lib()
+    x, w, dy = rand_storage(rng, (m, k), dt), rand_storage(rng, (k, n), dt), rand_storage(rng, (m, n), dt)
+    pad = 3                                             # rows of the gradients that start anywhere
+    dx0, dw0 = rand_storage(rng, (m, k + pad), dt), rand_storage(rng, (k, n + pad), dt)
+    d_x, d_w, d_dy = Dev(x, dt), Dev(w, dt), Dev(dy, dt)
+    for acc in (0, 1):
+        want_dx, want_dw, got_dx, got_dw = Dev(dx0, dt), Dev(dw0, dt), Dev(dx0, dt), Dev(dw0, dt)
+        capi.gemm(want_dx.ptr, d_dy.ptr, d_w.ptr, None, 1, m, n, k, (0, n, 1), (0, 1, n), (0, k + pad, 1), bool(acc), dt)
+        capi.gemm(want_dw.ptr, d_x.ptr, d_dy.ptr, None, 1, k, m, n, (0, 1, k), (0, n, 1), (0, n + pad, 1), bool(acc), dt)
+        capi.check(L.rp_hip_linear_backward(got_dx.ptr, got_dw.ptr, None, d_dy.ptr, d_x.ptr, d_w.ptr, m, k, n,
+                                            k, 1, n, 1, k + pad, 1, n + pad, 1, acc, acc, 0, dt), "linear_backward")
+        assert np.array_equal(got_dx.numpy(), want_dx.numpy()) and np.array_equal(got_dw.numpy(), want_dw.numpy())
+    want_dx, want_dw, got_dx = Dev.empty((m, k), dt), Dev.empty((k, n), dt), Dev.empty((m, k), dt)
+    capi.gemm(want_dx.ptr, d_dy.ptr, d_w.ptr, None, 1, m, n, k, (0, n, 1), (0, 1, n), (0, k, 1), False, dt)
+    capi.gemm(want_dw.ptr, d_x.ptr, d_dy.ptr, None, 1, k, m, n, (0, 1, k), (0, n, 1), (0, n, 1), False, dt)
+    capi.check(L.rp_hip_linear_backward(got_dx.ptr, d_w.ptr, None, d_dy.ptr, d_x.ptr, d_w.ptr, m, k, n,
+                                        k, 1, n, 1, k, 1, n, 1, 0, 0, 0, dt), "dW over W")
+    assert np.array_equal(got_dx.numpy(), want_dx.numpy()) and np.array_equal(d_w.numpy(), want_dw.numpy())
+
+
 def test_batch_longer_than_a_grid_axis():
     """70 000 tiny matrices in one call (the batch index rides on a grid axis of at most 65 535 blocks), A shared by
     all of them through a zero batch stride."""
