@@ -24,7 +24,7 @@
 // instead: 4096^3 788 us against 745, 2048^3 162 against 129).
 //
 // What bounds it: 52 % of the cycles are MFMA-busy, at a clock of 1.9 GHz and less that the power limit leaves.  4096^3: 750 -
-// 800 us where the fp32 MFMAs take 1 050 - 1 170; 2048^3 128 against 160; 3001 x 1027 x 2049 101 against 225.
+// 800 us (890 back to back for long) where the fp32 MFMAs take 1 050 - 1 240; 2048^3 128 against 160; 3001 x 1027 x 2049 101 against 225.
 #include "rp_gemm.h"
 
 namespace rp {
