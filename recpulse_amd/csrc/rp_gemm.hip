@@ -215,6 +215,10 @@ static int run_gemm(const GemmArgs& g, int dtype) {
     }
     if (p.fam != FAM_GENERIC && p.fam != FAM_TINY && !p.ragged && !(aligned16(g.A) && aligned16(g.B)))
         p = make_plan(g.batch, g.m, g.k, g.n, g.a_rs, g.a_cs, g.b_rs, g.b_cs, g.c_rs, g.c_cs, g.a_bs, g.b_bs, dtype, false, false);
+    // Ragged few-row products whose partial sums do not fit the fixed array of the entry point that allocates nothing: unsplit
+    // tiles, which need none (that entry point takes ragged products of any size)
+    if (p.ragged && p.fam == FAM_MFMA16_SKINNY && noalloc_active() && skinny16_workspace(g) > (size_t)RP_HIP_NOALLOC_WORKSPACE_BYTES)
+        choose_tile16(p, g.batch, g.m, g.k, g.n);
     g_last_kernel = p.name;
     switch (p.fam) {
         case FAM_MFMA16:

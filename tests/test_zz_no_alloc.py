@@ -8,6 +8,7 @@ sums, counters) is in place when the second runs.
 import numpy as np
 import pytest
 
+import oracle
 from recpulse_amd import capi
 from devhelp import BF16, F16, F32, rand_storage
 
@@ -96,6 +97,23 @@ def test_noalloc_rejects_a_workspace_beyond_the_fixed_array():
     capi.synchronize()
     want, got = _both(rng, 8, 2048, 1024, BF16)
     assert np.array_equal(want, got)
+
+
+@pytest.mark.parametrize("m,k,n", [(96, 4096, 16257), (32, 1025, 131075)])
+def test_noalloc_takes_ragged_products_of_any_size(m, k, n):
+    """Ragged few-row products whose split-k partial sums would exceed the array run on kernels that need none."""
+    rng = np.random.default_rng(74)
+    a, b = rand_storage(rng, (m, k), BF16), rand_storage(rng, (k, n), BF16)
+    da, db, dc = capi.DeviceBuffer.from_numpy(a), capi.DeviceBuffer.from_numpy(b), capi.DeviceBuffer(m * n * 2)
+    before = _alloc_counters()
+    capi.check(capi.lib().rp_hip_gemm_strided_batched_noalloc(dc.ptr, da.ptr, db.ptr, None, 1, m, k, n, 0, k, 1, 0, n, 1, 0, n, 1, 0, BF16), "noalloc")
+    assert _alloc_counters() == before
+    capi.synchronize()
+    got = dc.to_numpy(np.uint16, (m, n))
+    cols = np.r_[0:160, n - 160:n]
+    want = oracle.to_f64(a, BF16) @ oracle.to_f64(np.ascontiguousarray(b[:, cols]), BF16)
+    # one rounding to bf16: at most 2^-8 of a value
+    assert np.linalg.norm(oracle.to_f64(np.ascontiguousarray(got[:, cols]), BF16) - want) <= 2.0 ** -8 * np.linalg.norm(want)
 
 
 @pytest.mark.parametrize("m,k,n", [(4, 4096, 4096), (8, 4096, 4096), (40, 4096, 4096)])
