@@ -69,12 +69,22 @@ static void choose_tile_wide(Plan& p, int batch, int m, int k, int n, int dtype)
     p.edge = (m % p.bm) || (n % p.bn) || (k % (dtype == RP_DTYPE_FLOAT32 ? 32 : 16));
 }
 
+// With k = 1 nothing is ever read along the k axis and its strides may hold anything: a contiguous [m, 1] has (1, 1), an
+// expanded one 0.  The 16-bit kernels mask k rows past the end of a free-axis-contiguous operand by the end of its
+// buffer descriptor alone, which holds only if such rows start behind the operand: give the axis the stride of dense rows.
+static void plain_k_strides(int m, int k, int n, long long a_rs, long long& a_cs, long long& b_rs, long long b_cs) {
+    if (k != 1) return;
+    if (a_rs == 1) a_cs = m;
+    if (b_cs == 1) b_rs = n;
+}
+
 // Decide the kernel family and tile from shapes and strides alone (pointer
 // alignment is checked by the caller, which may still fall back to generic).
 static Plan make_plan(int batch, int m, int k, int n, long long a_rs, long long a_cs, long long b_rs, long long b_cs,
                       long long c_rs, long long c_cs, long long a_bs, long long b_bs, int dtype, bool allow_direct = true, bool bases_aligned = true) {
     Plan p{FAM_GENERIC, 64, 64, false, false, true, "generic"};
     if (path_disabled("mfma")) return p;
+    plain_k_strides(m, k, n, a_rs, a_cs, b_rs, b_cs);
     const int vec = 16 / (int)dtype_size(dtype);                // elements per 16-byte vector
     // operand layouts: KC = unit stride along k, MC = unit stride along the free axis.
     // Extent-1 axes make the other stride irrelevant, but vector loads still need alignment of the non-unit stride.
@@ -87,8 +97,11 @@ static Plan make_plan(int batch, int m, int k, int n, long long a_rs, long long 
     // the MFMA kernels address a tile with 32-bit byte offsets from a 64-bit tile pointer
     const long long max_stride = 1ll << 22;
     const bool strides_ok = a_rs < max_stride && a_cs < max_stride && b_rs < max_stride && b_cs < max_stride;
-    const bool mfma_ok = (a_kc || a_mc) && (b_kc || b_mc) && batch_ok && strides_ok;
     const bool is16 = dtype == RP_DTYPE_FLOAT16 || dtype == RP_DTYPE_BFLOAT16;
+    // k rows that overlap (an operand expanded along k): rows past the end of k lie inside the buffer (see plain_k_strides),
+    // which is harmless only if no slab hangs over
+    const bool overlapping_k = is16 && k % M16_BK != 0 && ((a_mc && !a_kc && a_cs < m) || (b_mc && b_rs < n));
+    const bool mfma_ok = (a_kc || a_mc) && (b_kc || b_mc) && batch_ok && strides_ok && !overlapping_k;
 
     // 16-bit, few rows, deep k: split k over many blocks so that B streams at HBM speed (output columns in whole 8s).
     // Up to 32 rows always; up to SKINNY_MAX_ROWS when the 128 x 128 tiles of the output would occupy under half the
@@ -160,8 +173,8 @@ static Plan make_plan(int batch, int m, int k, int n, long long a_rs, long long 
         // vector's worth of elements along the unit-stride axis and rows that do not overlap.  Outputs of less than two
         // 64 x 64 tiles between small operands stay on the generic kernel, which splits their k over the chip (a handful of
         // MFMA workgroups would walk it slab by slab).
-        const bool ak = a_cs == 1 && k >= vec && (a_rs >= k || m == 1), am = a_rs == 1 && m >= vec && (a_cs >= m || k == 1);
-        const bool bn = b_cs == 1 && n >= vec && (b_rs >= n || k == 1), bk = b_rs == 1 && k >= vec && (b_cs >= k || n == 1);
+        const bool ak = a_cs == 1 && k >= vec && (a_rs >= k || m == 1), am = a_rs == 1 && m >= vec && a_cs >= m;
+        const bool bn = b_cs == 1 && n >= vec && b_rs >= n, bk = b_rs == 1 && k >= vec && (b_cs >= k || n == 1);
         const bool worth = (long long)m * n * batch >= 8192 || (long long)k * n >= (1 << 18) || (long long)m * k >= (1 << 18);
         if ((ak || am) && (bn || bk) && worth) {
             p.ragged = true;
@@ -191,7 +204,8 @@ static Plan make_plan(int batch, int m, int k, int n, long long a_rs, long long 
 
 static thread_local const char* g_last_kernel = "none";      // what rp_hip_last_gemm_kernel reports
 
-static int run_gemm(const GemmArgs& g, int dtype) {
+static int run_gemm(GemmArgs g, int dtype) {
+    plain_k_strides(g.m, g.k, g.n, g.a_rs, g.a_cs, g.b_rs, g.b_cs);
     Plan p = make_plan(g.batch, g.m, g.k, g.n, g.a_rs, g.a_cs, g.b_rs, g.b_cs, g.c_rs, g.c_cs, g.a_bs, g.b_bs, dtype);
     if (p.fam == FAM_PIPE32) {
         if (pipe32_takes(g)) { g_last_kernel = p.name; return launch_pipe32(g); }
@@ -429,6 +443,8 @@ int rp_hip_linear_backward(void* dx, void* dw, void* db, const void* dy, const v
     // dx[m, k] = dy[m, n] . w^T (w [k, n] read with its strides swapped); dw[k, n] = x^T . dy (x [m, k] likewise)
     GemmArgs gx{dx, dy, w, nullptr, 1, m, n, k, 0, n, 1, 0, w_cs, w_rs, 0, dx_rs, dx_cs, accumulate_dx};
     GemmArgs gw{dw, x, dy, nullptr, 1, k, m, n, 0, x_cs, x_rs, 0, n, 1, 0, dw_rs, dw_cs, accumulate_dw};
+    plain_k_strides(gx.m, gx.k, gx.n, gx.a_rs, gx.a_cs, gx.b_rs, gx.b_cs);
+    plain_k_strides(gw.m, gw.k, gw.n, gw.a_rs, gw.a_cs, gw.b_rs, gw.b_cs);
     bool fused = dtype == RP_DTYPE_FLOAT32 && (dx || dw);
     if (fused && dx) fused = make_plan(1, gx.m, gx.k, gx.n, gx.a_rs, gx.a_cs, gx.b_rs, gx.b_cs, gx.c_rs, gx.c_cs, 0, 0, dtype).fam == FAM_TINY;
     if (fused && dw) fused = make_plan(1, gw.m, gw.k, gw.n, gw.a_rs, gw.a_cs, gw.b_rs, gw.b_cs, gw.c_rs, gw.c_cs, 0, 0, dtype).fam == FAM_TINY;

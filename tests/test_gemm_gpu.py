@@ -593,6 +593,51 @@ def test_ragged_rows(dt, batch, m, k, n, kernel, layout):
 
 
 @pytest.mark.parametrize("dt", ALL, ids=lambda d: NAMES[d])
+@pytest.mark.parametrize("m,n", [(256, 784), (251, 785), (4096, 9), (9, 4096), (128, 96)])
+def test_outer_products(dt, m, n):
+    """k = 1, where the strides of k may hold anything: those of a contiguous [m, 1] and of an expanded row are 1 and 0.  An
+    infinity and a NaN spoil their own row and column and nothing beside them."""
+    rng = np.random.default_rng(52)
+    a64, b64 = rng.integers(-2, 3, (m, 1)).astype(np.float64), rng.integers(-2, 3, (1, n)).astype(np.float64)
+    a64[m // 2], b64[0, n - 1] = np.inf, np.nan
+    a, b = oracle.to_storage(a64, dt), oracle.to_storage(b64, dt)
+    da, db, dc = Dev(a, dt), Dev(b, dt), Dev.empty((m, n), dt)
+    with np.errstate(invalid="ignore"):
+        want = oracle.to_f64(oracle.to_storage(a64 * b64, dt), dt)
+    for a_k in (0, 1, m, m + 3):
+        for b_k in (0, 1, n, n + 5):
+            capi.gemm(dc.ptr, da.ptr, db.ptr, None, 1, m, 1, n, (0, 1, a_k), (0, b_k, 1), (0, n, 1), False, dt)
+            assert np.array_equal(oracle.to_f64(dc.numpy(), dt), want, equal_nan=True), (a_k, b_k, capi.last_gemm_kernel())
+    # the gradients of a layer with one output: dx = dy . w^T is such a product, dw = x^T . dy has one column
+    x = rand_storage(rng, (m, n), dt)
+    dy = oracle.to_storage(rng.integers(-2, 3, (m, 1)).astype(np.float64), dt)
+    w = oracle.to_storage(rng.integers(-2, 3, (n, 1)).astype(np.float64), dt)
+    d_x, d_w, d_dy, d_dx, d_dw, d_db = Dev(x, dt), Dev(w, dt), Dev(dy, dt), Dev.empty((m, n), dt), Dev.empty((n, 1), dt), Dev.empty((1,), dt)
+    capi.check(capi.lib().rp_hip_linear_backward(d_dx.ptr, d_dw.ptr, d_db.ptr, d_dy.ptr, d_x.ptr, d_w.ptr, m, n, 1, n, 1, 1, 1, n, 1, 1, 1, 0, 0, 0, dt), "linear_backward")
+    assert np.array_equal(oracle.to_f64(d_dx.numpy(), dt), oracle.to_f64(dy, dt) @ oracle.to_f64(w, dt).T)
+    want_dw = oracle.to_f64(x, dt).T @ oracle.to_f64(dy, dt)
+    assert oracle.rel_err(oracle.to_f64(d_dw.numpy(), dt), want_dw) <= tol(dt, m)
+    assert d_db.numpy()[0] == oracle.to_storage(oracle.to_f64(dy, dt).sum(0), dt)[0]
+
+
+@pytest.mark.parametrize("dt", HALF, ids=lambda d: NAMES[d])
+@pytest.mark.parametrize("k", [8, 72, 128, 1032])
+def test_operands_expanded_along_k(dt, k):
+    """Both operands with k stride 0 or rows of k that overlap: what lies behind the last k row is inside the buffer."""
+    rng = np.random.default_rng(53)
+    m, n = 128, 256
+    for a_k, b_k in ((0, 0), (8, 8), (0, n), (m, 8)):
+        a, b = rng.integers(-2, 3, m + max(a_k, 8) * k).astype(np.float64), rng.integers(-2, 3, n + max(b_k, 8) * k).astype(np.float64)
+        b[n + b_k * (k - 1):] = np.nan
+        es = a.itemsize
+        av = np.lib.stride_tricks.as_strided(a, (m, k), (es, a_k * es))
+        bv = np.lib.stride_tricks.as_strided(b, (k, n), (b_k * es, es))
+        da, db, dc = Dev(oracle.to_storage(a, dt), dt), Dev(oracle.to_storage(b, dt), dt), Dev.empty((m, n), dt)
+        capi.gemm(dc.ptr, da.ptr, db.ptr, None, 1, m, k, n, (0, 1, a_k), (0, b_k, 1), (0, n, 1), False, dt)
+        assert np.array_equal(dc.numpy(), oracle.to_storage(np.matmul(av, bv), dt)), (a_k, b_k, capi.last_gemm_kernel())
+
+
+@pytest.mark.parametrize("dt", ALL, ids=lambda d: NAMES[d])
 def test_linear_backward_in_one_call(dt):
     """rp_hip_linear_backward against two GEMM calls with swapped strides and rp_hip_reduce_rows: the same bits,
     whether the three run as one launch (small float32 layers) or one after the other; outputs that are absent,
