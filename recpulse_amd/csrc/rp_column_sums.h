@@ -7,8 +7,8 @@
 // of one of rows terms, and four waves add at a time).
 //
 // What bounds it is not the arithmetic but how many loads are in flight: a thread that walks its column with
-// sixteen loads at a time spends a memory round trip per sixteen rows (1024 x 1024 in bf16 took 23 us).  256 threads
-// therefore fetch a tile of WIDTH bytes times ROWS rows at once, 16 bytes per load and all of them in flight together,
+// sixteen loads at a time spends a memory round trip per sixteen rows (1024 x 1024 in bf16 took 23 us).  The threads
+// of a workgroup therefore fetch a tile of WIDTH bytes times ROWS rows at once, 16 bytes per load and all of them in flight together,
 // park it in LDS, and the rows are added out of LDS, a column per lane.
 #pragma once
 #include "rp_common.h"
@@ -19,11 +19,13 @@ namespace rp {
 
 constexpr int COLSUM_CHUNK = 256, COLSUM_RUN = 64;
 
-template <typename T, int WIDTH, int ROWS>
+// PADDED: a row's gap after every run, so that lanes of different runs read different LDS banks.
+template <typename T, int WIDTH, int ROWS, int THREADS = 256, bool PADDED = false>
 struct ColumnTile {
     static constexpr int COLS = WIDTH / (int)sizeof(T), VEC = 16 / (int)sizeof(T);
-    static constexpr int VPR = WIDTH / 16, RPP = 256 / VPR, NV = ROWS / RPP;         // vectors per row, rows per pass of 256 threads, passes
-    static constexpr size_t BYTES = (size_t)WIDTH * ROWS;
+    static constexpr int VPR = WIDTH / 16, RPP = THREADS / VPR, NV = ROWS / RPP;     // vectors per row, rows per pass of the threads, passes
+    static constexpr size_t BYTES = (size_t)WIDTH * (ROWS + (PADDED ? ROWS / COLSUM_RUN : 0));
+    static __device__ __forceinline__ int row_offset(int row) { return (row + (PADDED ? row / COLSUM_RUN : 0)) * COLS; }
     typedef __attribute__((ext_vector_type(4))) unsigned int vec_t;
     vec_t v[NV];
     // rows from r0 on (zeros from r1 on), columns from c0 on
@@ -47,9 +49,9 @@ struct ColumnTile {
     }
     __device__ __forceinline__ void store(T* lds, int t) const {
 #pragma unroll
-        for (int i = 0; i < NV; i++) *(vec_t*)(lds + (size_t)(t / VPR + RPP * i) * COLS + (t % VPR) * VEC) = v[i];
+        for (int i = 0; i < NV; i++) *(vec_t*)(lds + row_offset(t / VPR + RPP * i) + (t % VPR) * VEC) = v[i];
     }
-    // s + the first n rows from lds on, top to bottom, sixteen rows read ahead of the ones being added (adding the zeros
+    // s + the first n rows from lds on (of one run, if padded), top to bottom, sixteen rows read ahead of the ones being added (adding the zeros
     // past the last row changes nothing: s is never -0)
     static __device__ __forceinline__ typename traits<T>::acc add(typename traits<T>::acc s, const T* lds, int col, int n) {
         constexpr int U = 16;

@@ -524,100 +524,122 @@ __global__ void sum_dim_kernel(T* out, const T* x, size_t outer, size_t dim, siz
     }
 }
 
-// Linear's bias gradient: out[j] = sum_i grad[i, j] in the order of rp_column_sums.h.  A block is 1 to 4 groups of 256 threads, a group owns one chunk of WIDTH bytes' worth
-// of columns.  Up to 1024 rows the groups meet in LDS and the block finishes; beyond that every group is a block of its
-// own that leaves its chunk's sums in `partials` [chunk][cols], and column_sums_finish_kernel adds them (one block walking
-// more rows has one tile of loads in flight at a time; 8192 x 8192 then keeps 128 of the 256 CUs busy).
-// WIDTH: 64 in the first case, where blocks are few and a CU's own bandwidth counts, whole cache lines in the second.
-template <typename T, int WIDTH>
-__global__ void __launch_bounds__(1024) column_sums_kernel(T* out, typename traits<T>::acc* partials, const T* grad, int rows, int cols, int accumulate) {
+// Linear's bias gradient: out[j] = sum_i grad[i, j] in the order of rp_column_sums.h.  No workspace: the sums of all rows meet
+// inside one workgroup, so calls on several streams share nothing and a first call can be recorded.  (Partial sums of all
+// chunks in a workspace, added by a second launch, put more CUs to work on tall narrow matrices: 8192 x 1024 bf16 6.6 us
+// against 9.5, 65536 x 64 8.9 against 91.  But a block of the pool is not safe across streams, and tying it to its stream with
+// an event or a stream-ordered allocation costs 5 or 11 us a call.)
+//
+// Up to COLSUM_CHUNK rows: a thread per column, the loads of 64 rows in flight together.  64 x 4096 bf16 2.7 us, 256 x 4096
+// 4.5 us a call (staged in LDS, where one wave adds them: 3.2 and 5.3).
+template <typename T>
+__global__ void __launch_bounds__(64) column_sums_short_kernel(T* out, const T* grad, int rows, int cols, int accumulate) {
     using A = typename traits<T>::acc;
-    using Tile = ColumnTile<T, WIDTH, COLSUM_CHUNK>;
-    constexpr int COLS = Tile::COLS;
-    extern __shared__ __attribute__((aligned(16))) unsigned char colsum_lds[];
-    const int t = threadIdx.x & 255, group = threadIdx.x >> 8, groups = blockDim.x >> 8;
-    const int chunk = blockIdx.y * groups + group, r0 = chunk * COLSUM_CHUNK;
-    const int r1 = r0 + COLSUM_CHUNK < rows ? r0 + COLSUM_CHUNK : rows;
-    const int c0 = blockIdx.x * COLS;
-    T* tile = (T*)(colsum_lds + group * Tile::BYTES);
-    {
-        Tile regs;
-        regs.load(grad, r0, r1, c0, cols, t);
-        regs.store(tile, t);
-    }
-    __syncthreads();
-    // rows <= COLSUM_CHUNK: the group's first wave adds all of them; otherwise each of its four waves adds a run
-    const int lane = t & 63, wave = t >> 6, runs = rows <= COLSUM_CHUNK ? 1 : COLSUM_CHUNK / COLSUM_RUN;
-    const int first = wave * COLSUM_RUN, mine = runs == 1 ? r1 - r0 : (r1 - r0 - first < COLSUM_RUN ? r1 - r0 - first : COLSUM_RUN);
-    A s = 0;
-    if (wave < runs && lane < COLS && mine > 0) s = Tile::add(s, tile + first * COLS, lane, mine);
-    __syncthreads();                                    // the tiles have been read: their LDS carries the runs' sums now
-    A* parts = (A*)colsum_lds + (size_t)group * (COLSUM_CHUNK / COLSUM_RUN) * COLS;
-    if (wave < runs && lane < COLS) parts[wave * COLS + lane] = s;
-    __syncthreads();
-    if (t >= COLS) return;                              // (no barrier after this point)
-    const int j = c0 + t;
+    const int j = blockIdx.x * 64 + threadIdx.x;
     if (j >= cols) return;
-    if (partials) {
-        for (int q = 1; q < runs; q++) s += parts[q * COLS + t];
-        partials[(size_t)chunk * cols + j] = s;
-        return;
-    }
-    if (group > 0) return;
-    s = 0;
-    for (int g = 0; g < groups; g++) {
-        const A* p = (const A*)colsum_lds + (size_t)g * (COLSUM_CHUNK / COLSUM_RUN) * COLS + t;
-        A c = p[0];
-        for (int q = 1; q < runs; q++) c += p[q * COLS];
-        s += c;
+    const T* p = grad + j;
+    A s = 0;
+    int i = 0;
+    auto whole = [&](auto uc) {
+        constexpr int U = decltype(uc)::value;
+        T v[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) v[u] = p[(size_t)(i + u) * cols];
+#pragma unroll
+        for (int u = 0; u < U; u++) s += widen(v[u]);
+        i += U;
+    };
+    while (i + 64 <= rows) whole(std::integral_constant<int, 64>{});
+    while (i + 16 <= rows) whole(std::integral_constant<int, 16>{});
+    if (i < rows) {                                     // the rest of a group of 16 in one go (rows past the end: the last one again, not added)
+        T v[16];
+#pragma unroll
+        for (int u = 0; u < 16; u++) v[u] = p[(size_t)(i + u < rows ? i + u : rows - 1) * cols];
+#pragma unroll
+        for (int u = 0; u < 16; u++) if (i + u < rows) s += widen(v[u]);
     }
     T r = narrow<T>(s);
     if (accumulate) r = narrow<T>(widen(out[j]) + widen(r));
     out[j] = r;
 }
 
-template <typename T>
-__global__ void __launch_bounds__(64) column_sums_finish_kernel(T* out, const typename traits<T>::acc* partials, int chunks, int cols, int accumulate) {
+// More rows: a workgroup of 1024 threads walks a strip of WIDTH bytes' worth of columns, 64 KB of it at a time: the next 64 KB are on
+// their way to registers while the threads add the present ones out of LDS, a lane per run and column.
+// WIDTH: 64 where such strips occupy at least half the CUs, else 16 (four times the workgroups, a quarter of the passes; a cache
+// line is then touched by eight workgroups instead of two, which all run on one XCD).  What bounds it: memory with strips of 64
+// (8192 x 8192 bf16 27 us, 4096 x 4096 fp32 15), the lines that the CU's vector cache takes in for 16 bytes of each with strips of
+// 16 (a pass of 4096 rows 3 - 6 us; 1024 x 1024 bf16 4.1 us a call, 2048 x 512 4.4, where a thread per column took 15 and 28).
+template <typename T, int WIDTH>
+struct ColumnWalk {
+    static constexpr int ROWS = 65536 / WIDTH, RUNS = ROWS / COLSUM_RUN, COLS = WIDTH / (int)sizeof(T);
+    using Tile = ColumnTile<T, WIDTH, ROWS, 1024, true>;
+    static constexpr size_t LDS = Tile::BYTES + (size_t)RUNS * COLS * sizeof(typename traits<T>::acc);
+};
+
+template <typename T, int WIDTH>
+__global__ void __launch_bounds__(1024) column_sums_kernel(T* out, const T* grad, int rows, int cols, int accumulate) {
     using A = typename traits<T>::acc;
-    const int j = blockIdx.x * 64 + threadIdx.x;
-    if (j >= cols) return;
+    using Walk = ColumnWalk<T, WIDTH>;
+    using Tile = typename Walk::Tile;
+    constexpr int COLS = Walk::COLS, ROWS = Walk::ROWS, RUNS = Walk::RUNS, RPC = COLSUM_CHUNK / COLSUM_RUN;
+    static_assert(RUNS * COLS <= 1024, "a lane per run and column");
+    extern __shared__ __attribute__((aligned(16))) unsigned char colsum_lds[];
+    T* tile = (T*)colsum_lds;
+    A* parts = (A*)(colsum_lds + Tile::BYTES);          // [run][column]
+    const int t = threadIdx.x, run = t / COLS, col = t % COLS;
+    // workgroup ids go to the XCDs in turn: the 128 / WIDTH strips of a cache line go to ids of one residue modulo 8
+    constexpr unsigned PER_LINE = 128 / WIDTH, GROUP = 8 * PER_LINE;
+    unsigned strip = blockIdx.x;
+    const unsigned first = strip / GROUP * GROUP, in = strip - first;
+    if (first + GROUP <= gridDim.x) strip = first + (in % 8) * PER_LINE + in / 8;
+    const int c0 = (int)(strip * COLS);
+    Tile regs;
+    regs.load(grad, 0, rows, c0, cols, t);
     A s = 0;
-    int i = 0;
-    constexpr int U = 32;                               // independent loads in flight; the adds stay in chunk order
-    for (; i + U <= chunks; i += U) {
-        A v[U];
+    for (long long base = 0; base < rows; base += ROWS) {
+        regs.store(tile, t);
+        __syncthreads();                                // (the previous pass's partial sums have been read, too)
+        const int left = (int)(rows - base), ahead = left - ROWS;
+        if (ahead > 0) regs.load(grad + (size_t)(base + ROWS) * cols, 0, ahead, c0, cols, t);
+        if (t < RUNS * COLS) {
+            const int n = left - run * COLSUM_RUN;
+            parts[t] = n > 0 ? Tile::add(0, tile + Tile::row_offset(run * COLSUM_RUN), col, n < COLSUM_RUN ? n : COLSUM_RUN) : (A)0;
+        }
+        __syncthreads();
+        if (t < COLS) {
 #pragma unroll
-        for (int u = 0; u < U; u++) v[u] = partials[(size_t)(i + u) * cols + j];
+            for (int q = 0; q < RUNS; q += RPC) {       // (runs past the last row add nothing)
+                A c = parts[q * COLS + t];
 #pragma unroll
-        for (int u = 0; u < U; u++) s += v[u];
+                for (int e = 1; e < RPC; e++) c += parts[(q + e) * COLS + t];
+                s += c;
+            }
+        }
     }
-    for (; i < chunks; i++) s += partials[(size_t)i * cols + j];
+    const int j = c0 + t;
+    if (t >= COLS || j >= cols) return;
     T r = narrow<T>(s);
     if (accumulate) r = narrow<T>(widen(out[j]) + widen(r));
     out[j] = r;
+}
+
+template <typename T, int WIDTH>
+static int launch_column_walk(T* out, const T* grad, int rows, int cols, int accumulate) {
+    using Walk = ColumnWalk<T, WIDTH>;
+    auto kern = column_sums_kernel<T, WIDTH>;
+    if (!check_hip(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)Walk::LDS), "hipFuncSetAttribute")) return -1;
+    hipLaunchKernelGGL(kern, dim3((cols - 1) / Walk::COLS + 1), dim3(1024), Walk::LDS, current_stream(), out, grad, rows, cols, accumulate);
+    return check_launch("column_sums_kernel") ? 0 : -1;
 }
 
 template <typename T>
 static int launch_column_sums(T* out, const T* grad, int rows, int cols, int accumulate) {
-    using A = typename traits<T>::acc;
-    const int chunks = (rows + COLSUM_CHUNK - 1) / COLSUM_CHUNK;
-    if (chunks <= 4) {
-        using Tile = ColumnTile<T, 64, COLSUM_CHUNK>;
-        hipLaunchKernelGGL((column_sums_kernel<T, 64>), dim3((cols + Tile::COLS - 1) / Tile::COLS), dim3(256 * chunks), chunks * Tile::BYTES, current_stream(),
-                           out, (A*)nullptr, grad, rows, cols, accumulate);
-        return check_launch("column_sums_kernel") ? 0 : -1;
+    if (rows <= COLSUM_CHUNK) {
+        hipLaunchKernelGGL(column_sums_short_kernel<T>, dim3((cols - 1) / 64 + 1), dim3(64), 0, current_stream(), out, grad, rows, cols, accumulate);
+        return check_launch("column_sums_short_kernel") ? 0 : -1;
     }
-    void* ws = nullptr;
-    if (rp_hip_malloc(&ws, (size_t)chunks * cols * sizeof(A)) != 0) return -1;
-    using Tile = ColumnTile<T, 128, COLSUM_CHUNK>;
-    constexpr int MOST = 65535;                         // chunks one launch can hold
-    for (int c = 0; c < chunks; c += MOST)
-        hipLaunchKernelGGL((column_sums_kernel<T, 128>), dim3((cols + Tile::COLS - 1) / Tile::COLS, chunks - c < MOST ? chunks - c : MOST), dim3(256), Tile::BYTES, current_stream(),
-                           out, (A*)ws + (size_t)c * cols, grad + (size_t)c * COLSUM_CHUNK * cols, rows - c * COLSUM_CHUNK, cols, accumulate);
-    hipLaunchKernelGGL(column_sums_finish_kernel<T>, dim3((cols + 63) / 64), dim3(64), 0, current_stream(), out, (const A*)ws, chunks, cols, accumulate);
-    const bool ok = check_launch("column_sums_kernel");
-    rp_hip_free(ws);                                    // back to the pool while the kernels are still queued: safe for later work on this stream
-    return ok ? 0 : -1;
+    if ((cols - 1) / ColumnWalk<T, 64>::COLS + 1 >= device_cu_count() / 2) return launch_column_walk<T, 64>(out, grad, rows, cols, accumulate);
+    return launch_column_walk<T, 16>(out, grad, rows, cols, accumulate);
 }
 
 // ---- cross-entropy ----------------------------------------------------------------------

@@ -121,31 +121,94 @@ def test_reduce_rows_matches_reference_order_bit_exact(dt):
         capi.check(L().rp_hip_reduce_rows(do.ptr, dg.ptr, rows, cols, 1, dt), "reduce_rows")
         assert np.array_equal(do.numpy(), oracle.add(want, want, dt))
 
+
+def _column_sums(g, dt):
+    """The documented order: up to 256 rows top to bottom, more as runs of 64 rows, four of them to a chunk."""
+    acc = np.float64 if dt == F64 else np.float32
+    rows, cols = g.shape
+    wide = oracle.to_f64(g, dt).astype(acc)                     # exact: every storage value is a float32
+    total = np.zeros(cols, acc)
+    for r0 in range(0, rows, 256):
+        chunk = np.zeros(cols, acc)
+        for q0 in range(r0, min(r0 + 256, rows), 64 if rows > 256 else 256):
+            run = np.zeros(cols, acc)
+            for row in wide[q0:min(q0 + (64 if rows > 256 else 256), r0 + 256)]:
+                run += row
+            chunk += run
+        total += chunk
+    return oracle.to_storage(total.astype(np.float64), dt)
+
+
 @pytest.mark.parametrize("dt", ALL, ids=lambda d: NAMES[d])
 @pytest.mark.parametrize("rows", [255, 257, 1024, 1025, 2600])
 def test_reduce_rows_beyond_one_chunk_bit_exact(dt, rows):
-    """Runs of 64 rows, four of them to a chunk of 256, every level added top to bottom: one block up to 1024 rows, a
-    finishing launch beyond.  Columns on both sides of a 128-byte tile, and a width that leaves the rows unaligned."""
+    """Runs of 64 rows, four of them to a chunk of 256, every level added top to bottom.  Columns on both sides of a 128-byte
+    tile, and a width that leaves the rows unaligned."""
     rng = np.random.default_rng(46)
     for cols in (1, 63, 128, 261):
         g = rand_storage(rng, (rows, cols), dt)
         dg, do = Dev(g, dt), Dev.empty((cols,), dt)
         capi.check(L().rp_hip_reduce_rows(do.ptr, dg.ptr, rows, cols, 0, dt), "reduce_rows")
-        acc = np.float64 if dt == F64 else np.float32
-        wide = oracle.to_f64(g, dt).astype(acc)                 # exact: every storage value is a float32
-        total = np.zeros(cols, acc)
-        for r0 in range(0, rows, 256):
-            chunk = np.zeros(cols, acc)
-            for q0 in range(r0, min(r0 + 256, rows), 64 if rows > 256 else 256):
-                run = np.zeros(cols, acc)
-                for row in wide[q0:min(q0 + (64 if rows > 256 else 256), r0 + 256)]:
-                    run += row
-                chunk += run
-            total += chunk
-        want = oracle.to_storage(total.astype(np.float64), dt)
+        want = _column_sums(g, dt)
         assert np.array_equal(do.numpy(), want)
         capi.check(L().rp_hip_reduce_rows(do.ptr, dg.ptr, rows, cols, 1, dt), "reduce_rows")
         assert np.array_equal(do.numpy(), oracle.add(want, want, dt))
+
+
+@pytest.mark.parametrize("dt", ALL, ids=lambda d: NAMES[d])
+@pytest.mark.parametrize("rows,cols", [(16, 70), (17, 70), (79, 70), (255, 4099), (257, 8200), (1030, 8200), (2600, 4099), (4096, 9), (4097, 9), (8261, 33)])
+def test_reduce_rows_strips_wide_and_narrow_bit_exact(dt, rows, cols):
+    """Few rows (groups of 64 and 16 and a rest), strips of 64 bytes (enough of them for half the CUs) and of 16, one pass and more."""
+    rng = np.random.default_rng(47)
+    g = rand_storage(rng, (rows, cols), dt)
+    dg, do = Dev(g, dt), Dev.empty((cols,), dt)
+    capi.check(L().rp_hip_reduce_rows(do.ptr, dg.ptr, rows, cols, 0, dt), "reduce_rows")
+    assert np.array_equal(do.numpy(), _column_sums(g, dt))
+
+
+def _memory_stats():
+    v = [ctypes.c_longlong(0) for _ in range(4)]
+    capi.check(L().rp_hip_memory_stats(*[ctypes.byref(x) for x in v]), "rp_hip_memory_stats")
+    return tuple(x.value for x in v)
+
+
+@pytest.mark.parametrize("dt", [F32, BF16], ids=lambda d: NAMES[d])
+@pytest.mark.parametrize("rows,cols", [(200, 300), (5000, 72), (3000, 4200)])
+def test_bias_gradients_share_nothing(dt, rows, cols):
+    """Column sums take no block of the pool, whatever the number of rows: two streams of one device sum different matrices of
+    one shape at the same time, and a first call can be recorded."""
+    rng = np.random.default_rng(48)
+    gs = [rand_storage(rng, (rows, cols), dt) for _ in range(2)]
+    want = [_column_sums(g, dt) for g in gs]
+    dg, do = [Dev(g, dt) for g in gs], [Dev.empty((cols,), dt) for _ in gs]
+    capi.synchronize()
+    before = _memory_stats()
+    streams = [capi.Stream() for _ in gs]
+    for _ in range(20):
+        for st, g, o in zip(streams, dg, do):
+            with st:
+                capi.check(L().rp_hip_reduce_rows(o.ptr, g.ptr, rows, cols, 0, dt), "reduce_rows")
+    capi.synchronize()
+    assert _memory_stats() == before
+    for o, w in zip(do, want):
+        assert np.array_equal(o.numpy(), w)
+    dr = Dev.empty((cols,), dt)
+    with streams[0]:
+        with capi.Graph.capture() as graph:
+            capi.check(L().rp_hip_reduce_rows(dr.ptr, dg[0].ptr, rows, cols, 0, dt), "reduce_rows")
+        for _ in range(3):
+            capi.check(L().rp_hip_memset(dr.ptr, 0xff, dr.size * capi.DTYPE_SIZE[dt]), "memset")
+            graph.launch()
+            capi.check(L().rp_hip_stream_synchronize(), "sync")
+            assert np.array_equal(dr.numpy(), want[0])
+    # the bias gradient that comes with the two products of a layer
+    k = 64
+    x, w = Dev(rand_storage(rng, (rows, k), dt), dt), Dev(rand_storage(rng, (k, cols), dt), dt)
+    capi.synchronize()
+    before = _memory_stats()
+    capi.check(L().rp_hip_linear_backward(None, None, do[0].ptr, dg[1].ptr, x.ptr, w.ptr, rows, k, cols, k, 1, cols, 1, k, 1, cols, 1, 0, 0, 0, dt), "db only")
+    assert _memory_stats() == before
+    assert np.array_equal(do[0].numpy(), want[1])
 
 
 @pytest.mark.parametrize("dt", ALL, ids=lambda d: NAMES[d])
