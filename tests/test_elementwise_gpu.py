@@ -166,6 +166,22 @@ def test_reduce_rows_strips_wide_and_narrow_bit_exact(dt, rows, cols):
     assert np.array_equal(do.numpy(), _column_sums(g, dt))
 
 
+def test_reduce_rows_of_nearly_two_to_the_31_rows():
+    """One column whose number of rows cannot be rounded up to whole chunks in 32 bits (every value is the bf16 0x3c3c)."""
+    rows = 2 ** 31 - 100
+    dg, do = capi.DeviceBuffer(rows * 2), Dev.empty((1,), BF16)
+    capi.check(L().rp_hip_memset(dg.ptr, 0x3c, rows * 2), "memset")
+    capi.check(L().rp_hip_reduce_rows(do.ptr, dg.ptr, rows, 1, 0, BF16), "reduce_rows")
+    got = do.numpy()
+    dg.free()
+    capi.check(L().rp_hip_empty_cache(), "empty_cache")
+    value = oracle.to_f64(np.array([0x3c3c], np.uint16), BF16)[0]
+    # whole chunks of 256 and what is left, one after the other in fp32 (a chunk's own sum is exact)
+    chunks = np.full(rows // 256 + 1, 256 * value, np.float32)
+    chunks[-1] = rows % 256 * value
+    assert got[0] == oracle.to_storage(np.cumsum(chunks, dtype=np.float32)[-1:].astype(np.float64), BF16)[0]
+
+
 def _memory_stats():
     v = [ctypes.c_longlong(0) for _ in range(4)]
     capi.check(L().rp_hip_memory_stats(*[ctypes.byref(x) for x in v]), "rp_hip_memory_stats")
