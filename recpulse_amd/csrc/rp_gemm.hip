@@ -182,7 +182,11 @@ static Plan make_plan(int batch, int m, int k, int n, long long a_rs, long long 
             p.b_mc = bn;
             if (!is16) {
                 choose_tile_wide(p, batch, m, k, n, dtype);
-            } else if (few_rows && n >= 256 && k >= 1024 && (long long)k * n >= (1ll << 22)) {
+            } else if (few_rows && n >= 256 && k >= 1024 && (long long)k * n >= (1ll << 22) &&
+                       skinny16_workspace(batch, m, k, n) <= (size_t)RP_HIP_NOALLOC_WORKSPACE_BYTES) {
+                // (partial sums beyond the fixed array of the entry point that allocates nothing: unsplit tiles, which need none.  That
+                // entry point takes ragged products of any size, with the bits of the one that allocates: one rule for both.  At that size
+                // the split pays no more: bf16 96 x 2049 x 16201 47.8 us split and 39.4 unsplit, 32 x 8193 x 140001 523 and 495)
                 p.fam = FAM_MFMA16_SKINNY; p.bm = 32; p.bn = 128; p.edge = true; p.name = "mfma16_skinny_32x128";
             } else {
                 choose_tile16(p, batch, m, k, n);
@@ -229,10 +233,6 @@ static int run_gemm(GemmArgs g, int dtype) {
     }
     if (p.fam != FAM_GENERIC && p.fam != FAM_TINY && !p.ragged && !(aligned16(g.A) && aligned16(g.B)))
         p = make_plan(g.batch, g.m, g.k, g.n, g.a_rs, g.a_cs, g.b_rs, g.b_cs, g.c_rs, g.c_cs, g.a_bs, g.b_bs, dtype, false, false);
-    // Ragged few-row products whose partial sums do not fit the fixed array of the entry point that allocates nothing: unsplit
-    // tiles, which need none (that entry point takes ragged products of any size)
-    if (p.ragged && p.fam == FAM_MFMA16_SKINNY && noalloc_active() && skinny16_workspace(g) > (size_t)RP_HIP_NOALLOC_WORKSPACE_BYTES)
-        choose_tile16(p, g.batch, g.m, g.k, g.n);
     g_last_kernel = p.name;
     switch (p.fam) {
         case FAM_MFMA16:

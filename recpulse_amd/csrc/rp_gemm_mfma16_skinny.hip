@@ -19,29 +19,29 @@ static int launch_skinny16_t(const GemmArgs& g, const Plan& p, float* partials, 
     return m16_launch<T, BM, BN, WGM, true, false, EDGE, true>(g, partials, nsplit, k_per_split);
 }
 
-static int skinny16_splits(const GemmArgs& g, int& k_per_split) {
+static int skinny16_splits(int batch, int m, int k, int n, int& k_per_split) {
     constexpr int BN = 128;
-    const int tiles = ((g.n + BN - 1) / BN) * ((g.m + 31) / 32) * g.batch;
+    const int tiles = ((n + BN - 1) / BN) * ((m + 31) / 32) * batch;
     // about three blocks per CU in flight, each split at least four slabs deep
     int nsplit = (768 + tiles - 1) / tiles;
-    int max_split = g.k / (4 * M16_BK) > 0 ? g.k / (4 * M16_BK) : 1;
+    int max_split = k / (4 * M16_BK) > 0 ? k / (4 * M16_BK) : 1;
     if (nsplit > max_split) nsplit = max_split;
-    k_per_split = ((g.k + nsplit - 1) / nsplit + M16_BK - 1) / M16_BK * M16_BK;
-    return (g.k + k_per_split - 1) / k_per_split;
+    k_per_split = ((k + nsplit - 1) / nsplit + M16_BK - 1) / M16_BK * M16_BK;
+    return (k + k_per_split - 1) / k_per_split;
 }
 
-size_t skinny16_workspace(const GemmArgs& g) {
+size_t skinny16_workspace(int batch, int m, int k, int n) {
     int k_per_split;
-    return (size_t)g.batch * skinny16_splits(g, k_per_split) * g.m * g.n * sizeof(float);
+    return (size_t)batch * skinny16_splits(batch, m, k, n, k_per_split) * m * n * sizeof(float);
 }
 
 int launch_mfma16_skinny(const GemmArgs& g, const Plan& p, int dtype) {
     if (dtype != RP_DTYPE_BFLOAT16 && dtype != RP_DTYPE_FLOAT16) { set_error("mfma16 skinny GEMM: unsupported dtype %d", dtype); return -1; }
     if (!p.ragged && !p.a_mc && p.b_mc && stream128_takes(g)) return launch_stream128(g, dtype);
     int k_per_split;
-    const int nsplit = skinny16_splits(g, k_per_split);
+    const int nsplit = skinny16_splits(g.batch, g.m, g.k, g.n, k_per_split);
     void* ws = nullptr;
-    if (gemm_workspace(&ws, skinny16_workspace(g)) != 0) return -1;
+    if (gemm_workspace(&ws, (size_t)g.batch * nsplit * g.m * g.n * sizeof(float)) != 0) return -1;
     int rc;
     const bool bf = dtype == RP_DTYPE_BFLOAT16;
     if (p.ragged) rc = bf ? launch_skinny16_t<bf16_t, M16_RAGGED>(g, p, (float*)ws, nsplit, k_per_split) : launch_skinny16_t<f16_t, M16_RAGGED>(g, p, (float*)ws, nsplit, k_per_split);

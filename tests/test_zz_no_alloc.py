@@ -99,9 +99,10 @@ def test_noalloc_rejects_a_workspace_beyond_the_fixed_array():
     assert np.array_equal(want, got)
 
 
-@pytest.mark.parametrize("m,k,n", [(96, 4096, 16257), (32, 1025, 131075)])
+@pytest.mark.parametrize("m,k,n", [(96, 4096, 16257), (96, 2049, 16201), (128, 4096, 16249), (32, 1025, 131071), (32, 1025, 131075)])
 def test_noalloc_takes_ragged_products_of_any_size(m, k, n):
-    """Ragged few-row products whose split-k partial sums would exceed the array run on kernels that need none."""
+    """Ragged few-row products whose split-k partial sums would exceed the array run on kernels that need none, in both entry
+    points: the same bits, on either side of the limit."""
     rng = np.random.default_rng(74)
     a, b = rand_storage(rng, (m, k), BF16), rand_storage(rng, (k, n), BF16)
     da, db, dc = capi.DeviceBuffer.from_numpy(a), capi.DeviceBuffer.from_numpy(b), capi.DeviceBuffer(m * n * 2)
@@ -114,6 +115,11 @@ def test_noalloc_takes_ragged_products_of_any_size(m, k, n):
     want = oracle.to_f64(a, BF16) @ oracle.to_f64(np.ascontiguousarray(b[:, cols]), BF16)
     # one rounding to bf16: at most 2^-8 of a value
     assert np.linalg.norm(oracle.to_f64(np.ascontiguousarray(got[:, cols]), BF16) - want) <= 2.0 ** -8 * np.linalg.norm(want)
+    kernel = capi.last_gemm_kernel()
+    capi.gemm(dc.ptr, da.ptr, db.ptr, None, 1, m, k, n, (0, k, 1), (0, n, 1), (0, n, 1), False, BF16)
+    assert capi.last_gemm_kernel() == kernel
+    capi.synchronize()
+    assert np.array_equal(dc.to_numpy(np.uint16, (m, n)), got)
 
 
 @pytest.mark.parametrize("m,k,n", [(4, 4096, 4096), (8, 4096, 4096), (40, 4096, 4096)])
