@@ -36,15 +36,13 @@ constexpr int S32_PITCH = 3 * S32_BK + 8;           // 16-bit elements per LDS r
 
 typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2_t;
 
-// The smallest non-zero magnitude met so far, in the terms of a pair of bf16 values: 2 |h| - 1 as a 16-bit integer orders
-// magnitudes, with zero above all others; the two halves run separately.
-typedef __attribute__((ext_vector_type(2))) unsigned short u16x2_t;
-__device__ __forceinline__ uint32_t s32_least(uint32_t so_far, uint32_t h) {
-    uint32_t key;
-    asm("v_pk_mad_u16 %0, %1, %2, %3" : "=v"(key) : "v"(h), "s"(0x00020002u), "v"(0xFFFFFFFFu));
-    return __builtin_bit_cast(uint32_t, __builtin_elementwise_min(__builtin_bit_cast(u16x2_t, so_far), __builtin_bit_cast(u16x2_t, key)));
+// The smallest non-zero magnitude met so far: twice the bits of a value, less one, orders magnitudes with zero above all others.
+// (Of the value itself: below 2^-134 its bf16 is zero.)
+__device__ __forceinline__ uint32_t s32_least(uint32_t so_far, float x0, float x1) {
+    const uint32_t k0 = 2u * __float_as_uint(x0) - 1u, k1 = 2u * __float_as_uint(x1) - 1u;
+    return min(so_far, min(k0, k1));
 }
-constexpr uint32_t S32_LEAST = ((127u - 110u) << 8) - 1u;           // the key of 2^-110
+constexpr uint32_t S32_LEAST = 2u * ((127u - 110u) << 23) - 1u;           // the key of 2^-110
 
 __device__ __forceinline__ uint32_t s32_pack(float a, float b) {
     const bf16x2_t v = {(__bf16)a, (__bf16)b};                        // one packed conversion, round to nearest even
@@ -131,7 +129,7 @@ struct S32Slab {
         const float x0 = MC ? at(2 * p, j) : at(j, 2 * p), x1 = MC ? at(2 * p + 1, j) : at(j, 2 * p + 1);
         uint32_t h, m, l;
         s32_split2(x0, x1, h, m, l);
-        least = s32_least(least, h);
+        least = s32_least(least, x0, x1);
         planes[j][0][p] = h; planes[j][1][p] = m; planes[j][2][p] = l;
     }
     __device__ __forceinline__ void split_all(uint32_t& least) {
@@ -252,7 +250,7 @@ __global__ void __launch_bounds__(256, 2) gemm_split32_kernel(GemmArgs g, int ti
         for (; kleft > S32_BK; kleft -= S32_BK) step(kleft, std::true_type{});
         step(kleft, std::false_type{});
     }
-    bool redo = (least & 0xFFFFu) < S32_LEAST || (least >> 16) < S32_LEAST;
+    bool redo = least < S32_LEAST;
 #pragma unroll
     for (int i = 0; i < TM; i++)
 #pragma unroll

@@ -1082,8 +1082,7 @@ def test_split32_is_as_close_as_fp32_sums(batch, m, k, n, layout):
 def test_split32_values_that_do_not_split(m, k, n, value):
     """Infinities, NaN, magnitudes that round to bf16 infinity and magnitudes whose last bits bf16 cannot hold: a tile that meets
     one is computed with fp32 MFMAs.  One row of A is `value` times N(0, 1) where that is tiny (fp32 sums of k products then
-    bound the row's error by itself; the smallest stays a normal number, the fp32 MFMA takes subnormals as zero), otherwise
-    `value` stands in two places."""
+    bound the row's error by itself), otherwise `value` stands in two places."""
     rng = np.random.default_rng(48)
     a, b = rng.normal(0, 1, (m, k)).astype(np.float32), rng.normal(0, 1, (k, n)).astype(np.float32)
     tiny = abs(value) < 1
@@ -1110,3 +1109,26 @@ def test_split32_values_that_do_not_split(m, k, n, value):
         if not tiny and rows.start == 5:
             continue
         assert np.linalg.norm((g - w)[keep]) <= 2.0 ** -24 * (np.sqrt(k) + 4) * np.linalg.norm(w[keep])
+
+
+def _split32_error(a, b, rows):
+    """2-norm error of these rows of A.B against float64, in units of 2^-24 of the result, and the largest relative one of a value."""
+    m, k = a.shape
+    n = b.shape[1]
+    dc, da, db = capi.DeviceBuffer(m * n * 4), capi.DeviceBuffer.from_numpy(a), capi.DeviceBuffer.from_numpy(b)
+    capi.gemm(dc.ptr, da.ptr, db.ptr, None, 1, m, k, n, (0, k, 1), (0, n, 1), (0, n, 1), False, F32)
+    assert capi.last_gemm_kernel() == "mfma32_128x128"
+    got = dc.to_numpy(np.float32, (m, n))[rows].astype(np.float64)
+    want = a[rows].astype(np.float64) @ b.astype(np.float64)
+    return np.linalg.norm(got - want) / np.linalg.norm(want) * 2 ** 24, np.max(np.abs(got - want)[want != 0] / np.abs(want[want != 0])) * 2 ** 24
+
+
+@pytest.mark.parametrize("exponent", [-115, -127, -130, -136, -140])
+def test_split32_subnormal_operands(exponent):
+    """A row of A around 2^exponent (subnormal below 2^-126, a bf16 zero below 2^-134) against values around 2^100."""
+    rng = np.random.default_rng(49)
+    m, k, n = 1408, 96, 1536
+    a, b = rng.normal(0, 1, (m, k)).astype(np.float32), (rng.normal(0, 1, (k, n)) * 2.0 ** 100).astype(np.float32)
+    a[5] = (rng.normal(0, 1, k) * 2.0 ** exponent).astype(np.float32)
+    for rows in (slice(5, 6), slice(0, 5), slice(128, m)):
+        assert _split32_error(a, b, rows)[0] <= np.sqrt(k) + 4
