@@ -12,8 +12,9 @@
 //
 // What the split cannot hold: infinities, NaN and values that round to bf16 infinity (their m and l become NaN, so every
 // output they touch is NaN, here or in a finite dot product that overflowed), and values below 2^-110, whose last bits fall
-// below the smallest bf16 subnormal.  The tile looks for both - non-finite accumulators at the end, the smallest non-zero
-// magnitude while it splits - and, if it met one, is computed again with fp32 MFMAs (the whole workgroup together).  So
+// below the smallest bf16 subnormal.  Nor are the small products of results below 2^-110 held: they are subnormal, and each of the
+// 6 k / 16 sums rounds to 2^-149 (up to k = 2^16 less than half an ulp of 2^-110).  The tile looks for all of them - non-finite
+// and tiny accumulators at the end, the smallest non-zero magnitude while it splits - and, if it met one, is computed again with fp32 MFMAs (the whole workgroup together).  So
 // the results for such inputs are the ones the fp32 kernel gives; they cost the sum of both.
 //
 // Shape: 128 x 128 tile, 4 waves of 64 x 64, k slab 32.  A slab is fetched to registers as fp32 (16 values of either operand
@@ -43,6 +44,7 @@ __device__ __forceinline__ uint32_t s32_least(uint32_t so_far, float x0, float x
     return min(so_far, min(k0, k1));
 }
 constexpr uint32_t S32_LEAST = 2u * ((127u - 110u) << 23) - 1u;           // the key of 2^-110
+constexpr float S32_SMALL = 7.703719777548943e-34f;                        // 2^-110
 
 __device__ __forceinline__ uint32_t s32_pack(float a, float b) {
     const bf16x2_t v = {(__bf16)a, (__bf16)b};                        // one packed conversion, round to nearest even
@@ -258,7 +260,8 @@ __global__ void __launch_bounds__(256, 2) gemm_split32_kernel(GemmArgs g, int ti
 #pragma unroll
             for (int v = 0; v < 16; v++) {
                 big[i][j][v] += small[i][j][v];
-                redo |= !(fabsf(big[i][j][v]) <= 3.402823466e38f);
+                const float x = fabsf(big[i][j][v]);
+                redo |= !(x <= 3.402823466e38f) || (x < S32_SMALL && x != 0.f);
             }
 
     const int lf = lane & 31, lk = lane >> 5;

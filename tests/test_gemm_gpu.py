@@ -1132,3 +1132,22 @@ def test_split32_subnormal_operands(exponent):
     a[5] = (rng.normal(0, 1, k) * 2.0 ** exponent).astype(np.float32)
     for rows in (slice(5, 6), slice(0, 5), slice(128, m)):
         assert _split32_error(a, b, rows)[0] <= np.sqrt(k) + 4
+
+
+@pytest.mark.parametrize("k", [96, 2048])
+def test_split32_at_the_ends_of_its_range(k):
+    """Operands just above the limit of what splits (their last planes are bf16 subnormals) stay on the split path.  Results near
+    the smallest normal number, whose small products would be subnormal, are fp32 sums; a single product is then rounded once."""
+    rng = np.random.default_rng(50)
+    m, n = 1408, 1536
+    sign = rng.choice([-1.0, 1.0], (m, k))
+    a, b = (sign * 2.0 ** rng.uniform(-110, -104, (m, k))).astype(np.float32), (rng.normal(0, 1, (k, n)) * 2.0 ** 60).astype(np.float32)
+    assert np.min(np.abs(a)) >= 2.0 ** -110
+    assert _split32_error(a, b, slice(0, m))[0] <= np.sqrt(k / 16) + 4
+    for e in (-58, -60, -61):
+        a, b = (rng.normal(0, 1, (m, k)) * 2.0 ** e).astype(np.float32), (rng.normal(0, 1, (k, n)) * 2.0 ** e).astype(np.float32)
+        assert _split32_error(a, b, slice(0, m))[0] <= np.sqrt(k) + 4
+    a = np.zeros((m, k), np.float32)
+    a[np.arange(m), np.arange(m) % k] = rng.uniform(1, 2, m) * 2.0 ** -62.5
+    b = (rng.uniform(1, 2, (k, n)) * 2.0 ** -62.5).astype(np.float32)
+    assert _split32_error(a, b, slice(0, m))[1] <= 1 + 1e-6
