@@ -13,9 +13,12 @@
 // What the split cannot hold: infinities, NaN and values that round to bf16 infinity (their m and l become NaN, so every
 // output they touch is NaN, here or in a finite dot product that overflowed), and values below 2^-110, whose last bits fall
 // below the smallest bf16 subnormal.  Nor are the small products of results below 2^-110 held: they are subnormal, and each of the
-// 6 k / 16 sums rounds to 2^-149 (up to k = 2^16 less than half an ulp of 2^-110).  The tile looks for all of them - non-finite
-// and tiny accumulators at the end, the smallest non-zero magnitude while it splits - and, if it met one, is computed again with fp32 MFMAs (the whole workgroup together).  So
-// the results for such inputs are the ones the fp32 kernel gives; they cost the sum of both.
+// 6 k / 16 sums rounds to 2^-149 (up to k = 2^16 less than half an ulp of 2^-110).  A wave that meets a tiny operand while it splits
+// says so in LDS; from that slab on the workgroup multiplies with fp32 MFMAs.  A tile whose result holds an infinity, a NaN or a
+// tiny value is computed again that way from the first slab on.  So such inputs get the fp32 kernel's precision.  4096^3, one value of
+// 2^-115 per 128 rows, at the first, the middle and the last k: 1 190, 930 and 743 us, a sixteenth of all values 1 195 (733 without,
+// 1 075 on the fp32 kernel; finding out at the end and computing such tiles again took 1 880); one infinity per 128 rows 1 835.
+// Finding out slab by slab costs every product: 4096^3 723 -> 733 us, 2048^3 127.5 -> 130.5, 1536 x 512 x 1536 38.5 -> 40.2.
 //
 // Shape: 128 x 128 tile, 4 waves of 64 x 64, k slab 32.  A slab is fetched to registers as fp32 (16 values of either operand
 // per thread), split there and written to LDS as rows of [32 h | 32 m | 32 l]; all four operand layouts leave the same
@@ -24,8 +27,8 @@
 // 48 MFMAs and split between those of the second half, two values after one or two MFMAs (splitting between the two barriers
 // instead: 4096^3 788 us against 745, 2048^3 162 against 129).
 //
-// What bounds it: 52 % of the cycles are MFMA-busy, at a clock of 1.9 GHz and less that the power limit leaves.  4096^3: 750 -
-// 800 us (890 back to back for long) where the fp32 MFMAs take 1 050 - 1 240; 2048^3 128 against 160; 3001 x 1027 x 2049 101 against 225.
+// What bounds it: 52 % of the cycles are MFMA-busy, at a clock of 1.9 GHz and less that the power limit leaves.  4096^3: 730 -
+// 800 us (890 back to back for long) where the fp32 MFMAs take 1 075 - 1 240; 2048^3 131 against 153; 3001 x 1027 x 2049 100 against 222.
 #include "rp_gemm.h"
 
 namespace rp {
@@ -35,13 +38,19 @@ namespace {
 constexpr int S32_BK = 32;
 constexpr int S32_PITCH = 3 * S32_BK + 8;           // 16-bit elements per LDS row: 16 rows of ds_read_b128 cover all banks once
 
+// the products that are kept, as planes of A and B (0: h, 1: m, 2: l), the large one first
+constexpr int S32_PA[6] = {0, 0, 1, 1, 0, 2}, S32_PB[6] = {0, 1, 0, 1, 2, 0};
+constexpr int S32_MFMAS = 6 * 4;        // of a k-step of 16: four tiles of 32 x 32
+
 typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2_t;
 
 // The smallest non-zero magnitude met so far: twice the bits of a value, less one, orders magnitudes with zero above all others.
 // (Of the value itself: below 2^-134 its bf16 is zero.)
 __device__ __forceinline__ uint32_t s32_least(uint32_t so_far, float x0, float x1) {
     const uint32_t k0 = 2u * __float_as_uint(x0) - 1u, k1 = 2u * __float_as_uint(x1) - 1u;
-    return min(so_far, min(k0, k1));
+    uint32_t least;
+    asm("v_min3_u32 %0, %1, %2, %3" : "=v"(least) : "v"(so_far), "v"(k0), "v"(k1));      // (the compiler pairs the values first: an instruction more)
+    return least;
 }
 constexpr uint32_t S32_LEAST = 2u * ((127u - 110u) << 23) - 1u;           // the key of 2^-110
 constexpr float S32_SMALL = 7.703719777548943e-34f;                        // 2^-110
@@ -77,10 +86,10 @@ struct S32Slab {
     const char* slab;
     const char* end;
     long long slab_step;
-    __device__ __forceinline__ void init(const float* base, long long free_stride, long long k_stride, int row0, int free_extent, int k, int t) {
+    __device__ __forceinline__ void init(const float* base, long long free_stride, long long k_stride, int row0, int free_extent, int k0, int k, int t) {
         r0 = MC ? 4 * (t / 8) : t / 8;
         kk0 = 4 * (t % 8);
-        slab = (const char*)(base + (long long)row0 * free_stride);
+        slab = (const char*)(base + (long long)row0 * free_stride + (long long)k0 * k_stride);
         end = (const char*)(base + (long long)(free_extent - 1) * free_stride + (long long)(k - 1) * k_stride + 1);
         slab_step = (long long)S32_BK * k_stride * 4;
         step = (int)((MC ? k_stride : 32 * free_stride) * 4);
@@ -163,6 +172,8 @@ template <bool A_MC, bool B_MC, bool EDGE>
 __global__ void __launch_bounds__(256, 2) gemm_split32_kernel(GemmArgs g, int tiles_m, int tiles_n) {
     constexpr int BM = 128, BN = 128, TM = 2, TN = 2;
     __shared__ __attribute__((aligned(16))) uint16_t lds[(BM + BN) * S32_PITCH];
+    __shared__ int spare[64];
+    __shared__ int odd_slab;             // the last slab that met a value which does not split
     static_assert(sizeof(lds) >= (size_t)S32_BK * (BM + 4 + BN + 4) * 4, "room for the fp32 slab");
     const TileCoord tc = schedule_tile(blockIdx.x, tiles_m, tiles_n);
     if (!tc.valid) return;
@@ -170,11 +181,13 @@ __global__ void __launch_bounds__(256, 2) gemm_split32_kernel(GemmArgs g, int ti
     const int t = threadIdx.x, lane = t & 63;
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const int wm0 = (wave >> 1) * 64, wn0 = (wave & 1) * 64;
+    const int lf = lane & 31, lk = lane >> 5;
     const float* A = (const float*)g.A + (long long)z * g.a_bs;
     const float* B = (const float*)g.B + (long long)z * g.b_bs;
     uint16_t* const a_lds = lds;
     uint16_t* const b_lds = lds + BM * S32_PITCH;
-    const int nslabs = (g.k + S32_BK - 1) / S32_BK;
+    float* const a_plain = (float*)lds;
+    float* const b_plain = a_plain + S32_BK * (BM + 4);
 
     f32x16_t big[TM][TN], small[TM][TN];
     auto clear = [&](f32x16_t (&acc)[TM][TN]) {
@@ -187,113 +200,138 @@ __global__ void __launch_bounds__(256, 2) gemm_split32_kernel(GemmArgs g, int ti
     };
     clear(big);
     clear(small);
+    S32Slab<BM, A_MC, EDGE> sa;
+    S32Slab<BN, B_MC, EDGE> sb;
+    auto init = [&](int k0) {
+        sa.init(A, g.a_rs, g.a_cs, m0, g.m, k0, g.k, t);
+        sb.init(B, g.b_cs, g.b_rs, n0, g.n, k0, g.k, t);
+    };
+    auto request = [&](int kleft) { sa.load(kleft); sb.load(kleft); };
+    auto settle = [&](int kleft) { sa.settle(kleft); sb.settle(kleft); };
+    auto store = [&] { sa.store(a_lds); sb.store(b_lds); };
+    // the slab in LDS as fp32 on the fp32 MFMAs
+    auto multiply_plain = [&] {
+        for (int kk = lk; kk < S32_BK; kk += 2) {
+            float af[TM], bf[TN];
+#pragma unroll
+            for (int i = 0; i < TM; i++) af[i] = a_plain[kk * (BM + 4) + wm0 + 32 * i + lf];
+#pragma unroll
+            for (int j = 0; j < TN; j++) bf[j] = b_plain[kk * (BN + 4) + wn0 + 32 * j + lf];
+#pragma unroll
+            for (int i = 0; i < TM; i++)
+#pragma unroll
+                for (int j = 0; j < TN; j++) big[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(af[i], bf[j], big[i][j], 0, 0, 0);
+        }
+    };
+
+    // A slab is split, its waves say whether they met a value that does not split (`mark`), a barrier lets go of the slab
+    // before it, its planes are stored, and after the next barrier all waves know (`odd`) how it is to be multiplied.
     uint32_t least = 0xFFFFFFFFu;
-    {
-        S32Slab<BM, A_MC, EDGE> sa;
-        S32Slab<BN, B_MC, EDGE> sb;
-        sa.init(A, g.a_rs, g.a_cs, m0, g.m, g.k, t);
-        sb.init(B, g.b_cs, g.b_rs, n0, g.n, g.k, t);
-        sa.load(g.k);
-        sb.load(g.k);
-        // lane's fragment of MFMA tile i: row 32 i + lane % 32, k 8 (lane / 32) .. + 7 of a step of 16
-        const uint16_t* const a_fr = a_lds + (wm0 + (lane & 31)) * S32_PITCH + 8 * (lane >> 5);
-        const uint16_t* const b_fr = b_lds + (wn0 + (lane & 31)) * S32_PITCH + 8 * (lane >> 5);
-        sa.settle(g.k);
-        sb.settle(g.k);
-        sa.split_all(least);
-        sb.split_all(least);
-        sa.store(a_lds);
-        sb.store(b_lds);
+    auto mark = [&](int slab) {
+        (least < S32_LEAST ? &odd_slab : spare + lane)[0] = slab;         // (no branch here: with one, 2048^3 took 143 us instead of 130.5)
+        least = 0xFFFFFFFFu;
+    };
+    int odd;
+    auto publish = [&] {
         __syncthreads();
-        // one slab: 48 MFMAs; the next one is requested at its start and split between the MFMAs of its second half
-        auto step = [&](int kleft, auto next_tag) {
-            constexpr bool NEXT = decltype(next_tag)::value;
-            if constexpr (NEXT) {
-                sa.load(kleft - S32_BK);
-                sb.load(kleft - S32_BK);
+        odd = odd_slab;
+        store();
+        __syncthreads();
+        odd = __builtin_amdgcn_readfirstlane(odd);
+    };
+    // lane's fragment of MFMA tile i: row 32 i + lane % 32, k 8 (lane / 32) .. + 7 of a step of 16
+    const uint16_t* const a_fr = a_lds + (wm0 + lf) * S32_PITCH + 8 * lk;
+    const uint16_t* const b_fr = b_lds + (wn0 + lf) * S32_PITCH + 8 * lk;
+    // one slab out of its planes; the next one is requested at its start and split between the MFMAs of its second half
+    auto step = [&](int kleft, auto next_tag) {
+        constexpr bool NEXT = decltype(next_tag)::value;
+        if constexpr (NEXT) request(kleft - S32_BK);
+        static_for<0, 2>([&](auto ksc) {
+            constexpr int ks = decltype(ksc)::value;
+            bf16x8_t af[TM][3], bf[TN][3];
+#pragma unroll
+            for (int p = 0; p < 3; p++) {
+#pragma unroll
+                for (int i = 0; i < TM; i++) af[i][p] = *(const bf16x8_t*)(a_fr + 32 * i * S32_PITCH + p * S32_BK + 16 * ks);
+#pragma unroll
+                for (int j = 0; j < TN; j++) bf[j][p] = *(const bf16x8_t*)(b_fr + 32 * j * S32_PITCH + p * S32_BK + 16 * ks);
             }
-            static_for<0, 2>([&](auto ksc) {
-                constexpr int ks = decltype(ksc)::value;
-                bf16x8_t af[TM][3], bf[TN][3];
-#pragma unroll
-                for (int p = 0; p < 3; p++) {
-#pragma unroll
-                    for (int i = 0; i < TM; i++) af[i][p] = *(const bf16x8_t*)(a_fr + 32 * i * S32_PITCH + p * S32_BK + 16 * ks);
-#pragma unroll
-                    for (int j = 0; j < TN; j++) bf[j][p] = *(const bf16x8_t*)(b_fr + 32 * j * S32_PITCH + p * S32_BK + 16 * ks);
-                }
+            if constexpr (NEXT && ks == 1) settle(kleft - S32_BK);
+            static_for<0, S32_MFMAS>([&](auto qc) {
+                constexpr int q = decltype(qc)::value, i = (q / TN) % TM, j = q % TN, prod = q / (TM * TN);
+                f32x16_t& acc = prod == 0 ? big[i][j] : small[i][j];
+                acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[i][S32_PA[prod]], bf[j][S32_PB[prod]], acc, 0, 0, 0);
                 if constexpr (NEXT && ks == 1) {
-                    sa.settle(kleft - S32_BK);
-                    sb.settle(kleft - S32_BK);
+                    static_for<16 * q / S32_MFMAS, 16 * (q + 1) / S32_MFMAS>([&](auto uc) {
+                        constexpr int u = decltype(uc)::value;
+                        if constexpr (u < 8) sa.template split<u>(least);
+                        else sb.template split<u - 8>(least);
+                    });
+                    __builtin_amdgcn_sched_barrier(0);
                 }
-                static_for<0, 24>([&](auto qc) {
-                    constexpr int q = decltype(qc)::value, i = (q / TN) % TM, j = q % TN, prod = q / (TM * TN);
-                    constexpr int PA[6] = {0, 0, 1, 1, 0, 2}, PB[6] = {0, 1, 0, 1, 2, 0};
-                    f32x16_t& acc = prod == 0 ? big[i][j] : small[i][j];
-                    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[i][PA[prod]], bf[j][PB[prod]], acc, 0, 0, 0);
-                    if constexpr (NEXT && ks == 1) {
-                        static_for<16 * q / 24, 16 * (q + 1) / 24>([&](auto uc) {
-                            constexpr int u = decltype(uc)::value;
-                            if constexpr (u < 8) sa.template split<u>(least);
-                            else sb.template split<u - 8>(least);
-                        });
-                        __builtin_amdgcn_sched_barrier(0);
-                    }
-                });
             });
-            if constexpr (NEXT) {
-                __syncthreads();
-                sa.store(a_lds);
-                sb.store(b_lds);
-            }
-            __syncthreads();
-        };
-        int kleft = g.k;
-        for (; kleft > S32_BK; kleft -= S32_BK) step(kleft, std::true_type{});
-        step(kleft, std::false_type{});
+        });
+    };
+
+    init(0);
+    request(g.k);
+    if (t == 0) odd_slab = -1;
+    settle(g.k);
+    sa.split_all(least);
+    sb.split_all(least);
+    __syncthreads();
+    mark(0);
+    publish();
+    int kleft = g.k, slab = 0;
+    for (; kleft > S32_BK && odd != slab; kleft -= S32_BK) {
+        step(kleft, std::true_type{});
+        mark(++slab);
+        publish();
     }
-    bool redo = least < S32_LEAST;
+    if (odd != slab) {
+        step(kleft, std::false_type{});
+        kleft = 0;
+    }
+    // whether a result is one that the split cannot hold
+    auto unsplittable = [&] {
+        bool any = false;
+#pragma unroll
+        for (int i = 0; i < TM; i++)
+#pragma unroll
+            for (int j = 0; j < TN; j++)
+#pragma unroll
+                for (int v = 0; v < 16; v++) {
+                    const float x = fabsf(big[i][j][v]);
+                    any |= !(x <= 3.402823466e38f) || (x < S32_SMALL && x != 0.f);
+                }
+        return __syncthreads_or(any) != 0;
+    };
 #pragma unroll
     for (int i = 0; i < TM; i++)
 #pragma unroll
         for (int j = 0; j < TN; j++)
 #pragma unroll
-            for (int v = 0; v < 16; v++) {
-                big[i][j][v] += small[i][j][v];
-                const float x = fabsf(big[i][j][v]);
-                redo |= !(x <= 3.402823466e38f) || (x < S32_SMALL && x != 0.f);
-            }
-
-    const int lf = lane & 31, lk = lane >> 5;
-    if (__syncthreads_or(redo)) {
-        float* const ap = (float*)lds;
-        float* const bp = ap + S32_BK * (BM + 4);
+            for (int v = 0; v < 16; v++) big[i][j][v] += small[i][j][v];
+    if (unsplittable()) {                  // all of the tile again
         clear(big);
-        S32Slab<BM, A_MC, EDGE> sa;
-        S32Slab<BN, B_MC, EDGE> sb;
-        sa.init(A, g.a_rs, g.a_cs, m0, g.m, g.k, t);
-        sb.init(B, g.b_cs, g.b_rs, n0, g.n, g.k, t);
-        for (int s = 0; s < nslabs; s++) {
-            const int kleft = g.k - s * S32_BK;
-            sa.load(kleft);
-            sb.load(kleft);
-            sa.settle(kleft);
-            sb.settle(kleft);
-            sa.store_plain(ap);
-            sb.store_plain(bp);
+        kleft = g.k;
+    }
+    while (kleft > 0) {                    // what is left from the first odd slab on, or everything
+        const bool whole = kleft == g.k;
+        init(g.k - kleft);
+        request(kleft);
+        for (; kleft > 0; kleft -= S32_BK) {
+            settle(kleft);
+            sa.store_plain(a_plain);
+            sb.store_plain(b_plain);
             __syncthreads();
-            for (int kk = lk; kk < S32_BK; kk += 2) {
-                float af[TM], bf[TN];
-#pragma unroll
-                for (int i = 0; i < TM; i++) af[i] = ap[kk * (BM + 4) + wm0 + 32 * i + lf];
-#pragma unroll
-                for (int j = 0; j < TN; j++) bf[j] = bp[kk * (BN + 4) + wn0 + 32 * j + lf];
-#pragma unroll
-                for (int i = 0; i < TM; i++)
-#pragma unroll
-                    for (int j = 0; j < TN; j++) big[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(af[i], bf[j], big[i][j], 0, 0, 0);
-            }
+            if (kleft > S32_BK) request(kleft - S32_BK);
+            multiply_plain();
             __syncthreads();
+        }
+        if (!whole && unsplittable()) {
+            clear(big);
+            kleft = g.k;
         }
     }
 

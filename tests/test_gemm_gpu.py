@@ -1151,3 +1151,39 @@ def test_split32_at_the_ends_of_its_range(k):
     a[np.arange(m), np.arange(m) % k] = rng.uniform(1, 2, m) * 2.0 ** -62.5
     b = (rng.uniform(1, 2, (k, n)) * 2.0 ** -62.5).astype(np.float32)
     assert _split32_error(a, b, slice(0, m))[1] <= 1 + 1e-6
+
+
+@pytest.mark.parametrize("layout", LAYOUTS)
+@pytest.mark.parametrize("m,k,n", [(1408, 160, 1536), (1411, 170, 1405), (1501, 21, 1499)])
+def test_split32_tiles_that_change_over(m, k, n, layout):
+    """From the first slab of k that holds a value below 2^-110 on, a tile is multiplied with fp32 MFMAs: at the first, an inner and the
+    last k, from either operand.  Integers otherwise, so every sum that is not zero has known bits; then an infinity as well."""
+    rng = np.random.default_rng(54)
+    a0, b0 = rng.integers(-4, 5, (m, k)).astype(np.float32), rng.integers(-4, 5, (k, n)).astype(np.float32)
+    whole = a0.astype(np.float64) @ b0.astype(np.float64)
+    dc = capi.DeviceBuffer(m * n * 4)
+
+    def product(a, b):
+        a_st, b_st = ((0, k, 1) if layout[0] == "n" else (0, 1, m)), ((0, n, 1) if layout[1] == "n" else (0, 1, k))
+        da, db = capi.DeviceBuffer.from_numpy(np.ascontiguousarray(a if layout[0] == "n" else a.T)), capi.DeviceBuffer.from_numpy(np.ascontiguousarray(b if layout[1] == "n" else b.T))
+        capi.gemm(dc.ptr, da.ptr, db.ptr, None, 1, m, k, n, a_st, b_st, (0, n, 1), False, F32)
+        assert capi.last_gemm_kernel() == "mfma32_128x128"
+        out = dc.to_numpy(np.float32, (m, n))
+        da.free(); db.free()
+        return out
+
+    for at in sorted({0, min(33, k - 1), k // 2, k - 1}):
+        a, b = a0.copy(), b0.copy()
+        a[7, at], a[m - 1, at], b[at, 9], b[at, n - 1] = 2.0 ** -115, 2.0 ** -140, -2.0 ** -120, 2.0 ** -130
+        want = a.astype(np.float64) @ b.astype(np.float64)
+        sure = np.abs(want) >= 1                               # (a tiny term beside an integer sum is rounded away)
+        got = product(a, b)
+        assert np.array_equal(got[sure], np.rint(want)[sure].astype(np.float32)) and np.all(np.abs(got[~sure]) < 1e-30)
+        a[200, k - 1 - at // 2] = np.inf
+        got = product(a, b)
+        with np.errstate(invalid="ignore"):
+            row = (a[200].astype(np.float64)[:, None] * b.astype(np.float64)).sum(0)
+        assert np.array_equal(got[200], row.astype(np.float32), equal_nan=True)
+        sure[200] = False
+        assert np.array_equal(got[sure], np.rint(want)[sure].astype(np.float32))
+    assert np.array_equal(product(a0, b0), whole.astype(np.float32))
