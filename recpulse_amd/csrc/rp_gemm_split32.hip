@@ -3,12 +3,15 @@
 // The fp32 MFMA runs 128 multiply-adds per cycle and CU, the bf16 MFMA sixteen times as many.  x = h + m + l with h = bf16(x),
 // m = bf16(x - h), l = x - h - m is exact (8 + 8 + 8 significant bits, each with its own sign, cover 24), so
 //   a b = ah bh + (ah bm + am bh) + (am bm + ah bl + al bh) + [am bl + al bm + al bl]
-// where the bracket is at most 2^-25 |a b|, under the rounding of a single fp32 product, and is left out: six bf16 MFMAs (whose
-// products are exact in fp32) of 32 cycles per k-step of 16 stand in for eight fp32 MFMAs of 64.  The five small products
-// go to an accumulator of their own, and the two meet once, in the epilogue: the large one then rounds once per 16 k instead
-// of once per product or two.  2-norm error against 64 bits, N(0,1) values, this kernel / the fp32 MFMA kernel: k = 67
-// 5.1e-8 / 1.5e-7, 256 8.9e-8 / 2.9e-7, 1024 1.9e-7 / 5.7e-7, 4096 4.0e-7 / 1.15e-6, the same in every layout; uniform values
-// in [0, 1) 0.35 - 0.45 of it; values spread over 2^+-30 equal it within 10 % either way at k <= 128 and are 0.85 of it at 4096.
+// where the bracket is at most 2^-24 |a b| (|m| <= 2^-8 |h| and |l| <= 2^-17 |h|, so am bl and al bm reach 2^-25 each), as much as the
+// rounding of a single fp32 product, and is left out: six bf16 MFMAs (whose products are exact in fp32) of 32 cycles per
+// k-step of 16 stand in for eight fp32 MFMAs of 64.  The five small products go to an accumulator of their own, and the two
+// meet once, in the epilogue: the large one then rounds once per 16 k instead of once per product or two.  2-norm error against
+// 64 bits, this kernel / the fp32 MFMA kernel: N(0,1) values, k = 67 5.1e-8 / 1.5e-7, 256 9.0e-8 / 2.9e-7, 1024 1.9e-7 / 5.7e-7, 4096
+// 4.0e-7 / 1.15e-6, the same in every layout; uniform values in [0, 1), k = 256 8.4e-8 / 2.2e-7, 4096 3.0e-7 / 8.4e-7; values spread over
+// 2^+-30, k = 128 6.48e-8 / 6.46e-8, 4096 2.9e-7 / 3.3e-7.  Where a row has one significant term there is nothing to gain and the bracket
+// shows: a diagonal matrix of N(0,1) times N(0,1) 2.60e-8 / 2.53e-8, the largest error of a value 1.67 x 2^-24 instead of 1.00.  (With
+// am bl and al bm kept it is 1.00 again and no other figure moves by more than 1 %; 4096^3 then takes 870 us, 2048^3 150.)
 //
 // What the split cannot hold: infinities, NaN and values that round to bf16 infinity (their m and l become NaN, so every
 // output they touch is NaN, here or in a finite dot product that overflowed), and values below 2^-110, whose last bits fall

@@ -1187,3 +1187,19 @@ def test_split32_tiles_that_change_over(m, k, n, layout):
         sure[200] = False
         assert np.array_equal(got[sure], np.rint(want)[sure].astype(np.float32))
     assert np.array_equal(product(a0, b0), whole.astype(np.float32))
+
+
+def test_split32_single_products_and_repeated_values():
+    """The three smallest of the nine partial products are left out: at most 2^-24 of a product (8 significant bits leave
+    |m| <= 2^-8 |h|, |l| <= 2^-17 |h|), beside the sum's own rounding of 2^-24.  That shows where a row of A has one significant term,
+    and, always to the same side, where the values repeat (1.0038986 is close to the worst one)."""
+    rng = np.random.default_rng(51)
+    m, k, n = 1408, 512, 1536
+    a = np.zeros((m, k), np.float32)
+    a[np.arange(m), np.arange(m) % k] = rng.normal(0, 1, m)
+    b = rng.normal(0, 1, (k, n)).astype(np.float32)
+    assert _split32_error(a, b, slice(0, m))[1] <= 2 + 1e-3
+    a[a != 0], b[:] = 1.0038986, 1.0038986
+    assert _split32_error(a, b, slice(0, m))[1] <= 2 + 1e-3
+    a[:] = 1.0038986
+    assert _split32_error(a, b, slice(0, m))[1] <= 2 + k / 16      # a rounding per 16 k, which may all go one way too
