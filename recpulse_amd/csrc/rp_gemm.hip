@@ -456,7 +456,7 @@ int rp_hip_linear_backward(void* dx, void* dw, void* db, const void* dy, const v
     }
     bool edge = false;
     if ((dtype == RP_DTYPE_BFLOAT16 || dtype == RP_DTYPE_FLOAT16) && dx && dw && linear_backward_pairs(gx, gw, dtype, edge)) {
-        g_last_kernel = "mfma16_64x64";
+        g_last_kernel = "linear_backward16_64x64";
         if (launch_linear_backward16(gx, gw, edge, dtype) != 0) return -1;
     } else {
         if (dx && run_gemm(gx, dtype) != 0) return -1;

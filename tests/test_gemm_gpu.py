@@ -692,12 +692,14 @@ def test_linear_backward_pair_16bit(dt, shape):
         capi.gemm(want_dw.ptr, d_x.ptr, d_dy.ptr, None, 1, k, m, n, (0, 1, k), (0, n, 1), (0, n + pad, 1), bool(acc), dt)
         capi.check(L.rp_hip_linear_backward(got_dx.ptr, got_dw.ptr, None, d_dy.ptr, d_x.ptr, d_w.ptr, m, k, n,
                                             k, 1, n, 1, k + pad, 1, n + pad, 1, acc, acc, 0, dt), "linear_backward")
+        assert capi.last_gemm_kernel() == "linear_backward16_64x64"
         assert np.array_equal(got_dx.numpy(), want_dx.numpy()) and np.array_equal(got_dw.numpy(), want_dw.numpy())
     want_dx, want_dw, got_dx = Dev.empty((m, k), dt), Dev.empty((k, n), dt), Dev.empty((m, k), dt)
     capi.gemm(want_dx.ptr, d_dy.ptr, d_w.ptr, None, 1, m, n, k, (0, n, 1), (0, 1, n), (0, k, 1), False, dt)
     capi.gemm(want_dw.ptr, d_x.ptr, d_dy.ptr, None, 1, k, m, n, (0, 1, k), (0, n, 1), (0, n, 1), False, dt)
     capi.check(L.rp_hip_linear_backward(got_dx.ptr, d_w.ptr, None, d_dy.ptr, d_x.ptr, d_w.ptr, m, k, n,
                                         k, 1, n, 1, k, 1, n, 1, 0, 0, 0, dt), "dW over W")
+    assert capi.last_gemm_kernel() != "linear_backward16_64x64"
     assert np.array_equal(got_dx.numpy(), want_dx.numpy()) and np.array_equal(d_w.numpy(), want_dw.numpy())
 
 
