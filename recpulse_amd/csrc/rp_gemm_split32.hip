@@ -14,14 +14,15 @@
 // am bl and al bm kept it is 1.00 again and no other figure moves by more than 1 %; 4096^3 then takes 870 us, 2048^3 150.)
 //
 // What the split cannot hold: infinities, NaN and values that round to bf16 infinity (their m and l become NaN, so every
-// output they touch is NaN, here or in a finite dot product that overflowed), and values below 2^-110, whose last bits fall
-// below the smallest bf16 subnormal.  Nor are the small products of results below 2^-110 held: they are subnormal, and each of the
-// 6 k / 16 sums rounds to 2^-149 (up to k = 2^16 less than half an ulp of 2^-110).  A wave that meets a tiny operand while it splits
-// says so in LDS; from that slab on the workgroup multiplies with fp32 MFMAs.  A tile whose result holds an infinity, a NaN or a
-// tiny value is computed again that way from the first slab on.  So such inputs get the fp32 kernel's precision.  4096^3, one value of
-// 2^-115 per 128 rows, at the first, the middle and the last k: 1 190, 930 and 743 us, a sixteenth of all values 1 195 (733 without,
-// 1 075 on the fp32 kernel; finding out at the end and computing such tiles again took 1 880); one infinity per 128 rows 1 835.
-// Finding out slab by slab costs every product: 4096^3 723 -> 733 us, 2048^3 127.5 -> 130.5, 1536 x 512 x 1536 38.5 -> 40.2.
+// output they touch is NaN, here or in a finite dot product that overflowed), and values below 2^-110 whose last bits fall
+// below the smallest bf16 subnormal (then what is left for l is no bf16 value).  Nor are the small products of results below
+// 2^-110 held: they are subnormal, and each of the 6 k / 16 sums rounds to 2^-149 (up to k = 2^16 less than half an ulp of 2^-110).
+// A wave that splits a value with such a rest says so in LDS; from that slab on the workgroup multiplies with fp32 MFMAs.  A tile
+// whose result holds an infinity, a NaN or a tiny value is computed again that way from the first slab on.  So such inputs get the
+// fp32 kernel's precision.  4096^3, one value of 1.2345 x 2^-115 per 128 rows, at the first, the middle and the last k: 1 200, 925 and
+// 727 us, a sixteenth of all values 1 200 (725 without, 1 075 on the fp32 kernel; finding out at the end and computing such
+// tiles again took 1 880); one infinity per 128 rows 1 820.  Looking for the smallest magnitude instead of a rest: 733 without.
+// The check of the results costs 0.5 us: 1536 x 96 x 1536 16.3 -> 16.8 us, 2048^3 128 -> 131.
 //
 // Shape: 128 x 128 tile, 4 waves of 64 x 64, k slab 32.  A slab is fetched to registers as fp32 (16 values of either operand
 // per thread), split there and written to LDS as rows of [32 h | 32 m | 32 l]; all four operand layouts leave the same
@@ -30,7 +31,7 @@
 // 48 MFMAs and split between those of the second half, two values after one or two MFMAs (splitting between the two barriers
 // instead: 4096^3 788 us against 745, 2048^3 162 against 129).
 //
-// What bounds it: 52 % of the cycles are MFMA-busy, at a clock of 1.9 GHz and less that the power limit leaves.  4096^3: 730 -
+// What bounds it: 52 % of the cycles are MFMA-busy, at a clock of 1.9 GHz and less that the power limit leaves.  4096^3: 725 -
 // 800 us (890 back to back for long) where the fp32 MFMAs take 1 075 - 1 240; 2048^3 131 against 153; 3001 x 1027 x 2049 100 against 222.
 #include "rp_gemm.h"
 
@@ -43,32 +44,25 @@ constexpr int S32_PITCH = 3 * S32_BK + 8;           // 16-bit elements per LDS r
 
 // the products that are kept, as planes of A and B (0: h, 1: m, 2: l), the large one first
 constexpr int S32_PA[6] = {0, 0, 1, 1, 0, 2}, S32_PB[6] = {0, 1, 0, 1, 2, 0};
+constexpr int FP_NAN_INF_SUBNORMAL = 0x297;         // of v_cmp_class: both NaNs, both infinities, both signs of subnormal
 constexpr int S32_MFMAS = 6 * 4;        // of a k-step of 16: four tiles of 32 x 32
 
 typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2_t;
-
-// The smallest non-zero magnitude met so far: twice the bits of a value, less one, orders magnitudes with zero above all others.
-// (Of the value itself: below 2^-134 its bf16 is zero.)
-__device__ __forceinline__ uint32_t s32_least(uint32_t so_far, float x0, float x1) {
-    const uint32_t k0 = 2u * __float_as_uint(x0) - 1u, k1 = 2u * __float_as_uint(x1) - 1u;
-    uint32_t least;
-    asm("v_min3_u32 %0, %1, %2, %3" : "=v"(least) : "v"(so_far), "v"(k0), "v"(k1));      // (the compiler pairs the values first: an instruction more)
-    return least;
-}
-constexpr uint32_t S32_LEAST = 2u * ((127u - 110u) << 23) - 1u;           // the key of 2^-110
-constexpr float S32_SMALL = 7.703719777548943e-34f;                        // 2^-110
 
 __device__ __forceinline__ uint32_t s32_pack(float a, float b) {
     const bf16x2_t v = {(__bf16)a, (__bf16)b};                        // one packed conversion, round to nearest even
     return __builtin_bit_cast(uint32_t, v);
 }
 
-// two values -> their h, m and l pairs
-__device__ __forceinline__ void s32_split2(float x0, float x1, uint32_t& h, uint32_t& m, uint32_t& l) {
+// two values -> their h, m and l pairs.  lost collects the bits of what is left for l: it is a bf16 value, as it always is unless it
+// falls below the bf16 subnormals, if its low half is zero.
+__device__ __forceinline__ void s32_split2(float x0, float x1, uint32_t& h, uint32_t& m, uint32_t& l, uint32_t& lost) {
     h = s32_pack(x0, x1);
     const float r0 = x0 - __uint_as_float(h << 16), r1 = x1 - __uint_as_float(h & 0xFFFF0000u);
     m = s32_pack(r0, r1);
-    l = s32_pack(r0 - __uint_as_float(m << 16), r1 - __uint_as_float(m & 0xFFFF0000u));
+    const float l0 = r0 - __uint_as_float(m << 16), l1 = r1 - __uint_as_float(m & 0xFFFF0000u);
+    l = s32_pack(l0, l1);
+    lost |= __float_as_uint(l0) | __float_as_uint(l1);
 }
 
 // One operand's slab traffic.  A thread holds four vectors of four values along the unit-stride axis.
@@ -138,16 +132,15 @@ struct S32Slab {
     __device__ __forceinline__ float at(int i, int e) const { return __uint_as_float(v[i][e]); }
     // unit u = 0 .. 7 of the split: two values of row u / 2 of the thread's four
     template <int U>
-    __device__ __forceinline__ void split(uint32_t& least) {
+    __device__ __forceinline__ void split(uint32_t& lost) {
         constexpr int j = U / 2, p = U % 2;
         const float x0 = MC ? at(2 * p, j) : at(j, 2 * p), x1 = MC ? at(2 * p + 1, j) : at(j, 2 * p + 1);
         uint32_t h, m, l;
-        s32_split2(x0, x1, h, m, l);
-        least = s32_least(least, x0, x1);
+        s32_split2(x0, x1, h, m, l, lost);
         planes[j][0][p] = h; planes[j][1][p] = m; planes[j][2][p] = l;
     }
-    __device__ __forceinline__ void split_all(uint32_t& least) {
-        static_for<0, 8>([&](auto u) { split<decltype(u)::value>(least); });
+    __device__ __forceinline__ void split_all(uint32_t& lost) {
+        static_for<0, 8>([&](auto u) { split<decltype(u)::value>(lost); });
     }
     __device__ __forceinline__ void store(uint16_t* lds) const {
 #pragma unroll
@@ -229,10 +222,10 @@ __global__ void __launch_bounds__(256, 2) gemm_split32_kernel(GemmArgs g, int ti
 
     // A slab is split, its waves say whether they met a value that does not split (`mark`), a barrier lets go of the slab
     // before it, its planes are stored, and after the next barrier all waves know (`odd`) how it is to be multiplied.
-    uint32_t least = 0xFFFFFFFFu;
+    uint32_t lost = 0;
     auto mark = [&](int slab) {
-        (least < S32_LEAST ? &odd_slab : spare + lane)[0] = slab;         // (no branch here: with one, 2048^3 took 143 us instead of 130.5)
-        least = 0xFFFFFFFFu;
+        ((lost & 0xFFFFu) != 0 ? &odd_slab : spare + lane)[0] = slab;         // (no branch here: with one, 2048^3 took 143 us instead of 130.5)
+        lost = 0;
     };
     int odd;
     auto publish = [&] {
@@ -267,8 +260,8 @@ __global__ void __launch_bounds__(256, 2) gemm_split32_kernel(GemmArgs g, int ti
                 if constexpr (NEXT && ks == 1) {
                     static_for<16 * q / S32_MFMAS, 16 * (q + 1) / S32_MFMAS>([&](auto uc) {
                         constexpr int u = decltype(uc)::value;
-                        if constexpr (u < 8) sa.template split<u>(least);
-                        else sb.template split<u - 8>(least);
+                        if constexpr (u < 8) sa.template split<u>(lost);
+                        else sb.template split<u - 8>(lost);
                     });
                     __builtin_amdgcn_sched_barrier(0);
                 }
@@ -280,8 +273,8 @@ __global__ void __launch_bounds__(256, 2) gemm_split32_kernel(GemmArgs g, int ti
     request(g.k);
     if (t == 0) odd_slab = -1;
     settle(g.k);
-    sa.split_all(least);
-    sb.split_all(least);
+    sa.split_all(lost);
+    sb.split_all(lost);
     __syncthreads();
     mark(0);
     publish();
@@ -304,8 +297,8 @@ __global__ void __launch_bounds__(256, 2) gemm_split32_kernel(GemmArgs g, int ti
             for (int j = 0; j < TN; j++)
 #pragma unroll
                 for (int v = 0; v < 16; v++) {
-                    const float x = fabsf(big[i][j][v]);
-                    any |= !(x <= 3.402823466e38f) || (x < S32_SMALL && x != 0.f);
+                    // (subnormal after 2^-16: below 2^-110)
+                    any |= __builtin_amdgcn_classf(big[i][j][v] * 1.52587890625e-05f, FP_NAN_INF_SUBNORMAL);
                 }
         return __syncthreads_or(any) != 0;
     };

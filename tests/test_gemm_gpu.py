@@ -1158,8 +1158,8 @@ def test_split32_at_the_ends_of_its_range(k):
 @pytest.mark.parametrize("layout", LAYOUTS)
 @pytest.mark.parametrize("m,k,n", [(1408, 160, 1536), (1411, 170, 1405), (1501, 21, 1499)])
 def test_split32_tiles_that_change_over(m, k, n, layout):
-    """From the first slab of k that holds a value below 2^-110 on, a tile is multiplied with fp32 MFMAs: at the first, an inner and the
-    last k, from either operand.  Integers otherwise, so every sum that is not zero has known bits; then an infinity as well."""
+    """From the first slab of k on that holds a value whose last bits bf16 cannot hold, a tile is multiplied with fp32 MFMAs: at the
+    first, an inner and the last k, from either operand.  Integers otherwise, so every sum that is not zero has known bits; then an infinity as well."""
     rng = np.random.default_rng(54)
     a0, b0 = rng.integers(-4, 5, (m, k)).astype(np.float32), rng.integers(-4, 5, (k, n)).astype(np.float32)
     whole = a0.astype(np.float64) @ b0.astype(np.float64)
@@ -1176,7 +1176,7 @@ def test_split32_tiles_that_change_over(m, k, n, layout):
 
     for at in sorted({0, min(33, k - 1), k // 2, k - 1}):
         a, b = a0.copy(), b0.copy()
-        a[7, at], a[m - 1, at], b[at, 9], b[at, n - 1] = 2.0 ** -115, 2.0 ** -140, -2.0 ** -120, 2.0 ** -130
+        a[7, at], a[m - 1, at], b[at, 9], b[at, n - 1] = 1.2345 * 2.0 ** -115, 2.0 ** -140, -1.2345 * 2.0 ** -120, 1.2345 * 2.0 ** -130
         want = a.astype(np.float64) @ b.astype(np.float64)
         sure = np.abs(want) >= 1                               # (a tiny term beside an integer sum is rounded away)
         got = product(a, b)
