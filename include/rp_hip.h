@@ -223,8 +223,8 @@ int rp_hip_linear_backward(void* dx, void* dw, void* db, const void* dy, const v
 
 /* Bias gradient of Linear on the device: grad [rows, cols] dense -> out [cols],
  * each column summed in fp32 (fp64 for float64): up to 256 rows top to bottom, more
- * rows as runs of 64, four runs to a chunk, each level top to bottom.  Takes no workspace:
- * calls on several streams share nothing, and a first call can be recorded.  Stands in for
+ * rows as runs of 64, four runs to a chunk, each level top to bottom.  Takes no block of the
+ * pool: calls on several streams share nothing, and a first call can be recorded.  Stands in for
  * the device->host->device round trip of reduce_grad_to_shape
  * (ops/ops.c:6970-7101) in the [rows, cols] -> [cols] case. */
 int rp_hip_reduce_rows(void* out, const void* grad, int rows, int cols, int accumulate, int dtype);

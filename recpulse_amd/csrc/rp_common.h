@@ -15,6 +15,18 @@ hipStream_t current_stream();
 bool check_hip(hipError_t e, const char* what);          // false (and error text) on failure
 bool check_launch(const char* what);                     // hipGetLastError after a launch
 bool stream_is_capturing();                              // the calling thread's stream is recording a graph
+// 16 MiB of device memory for work on the null stream, or null: on any other stream, for more bytes, or without memory.  Kernels
+// on the null stream run one after the other, whichever threads launched them, so what one sequence of launches leaves there is
+// not touched before the sequence is over if the lease is held until its last launch.  (Another stream's work could overlap, and
+// its handle could come back as that of a new stream.)
+class NullStreamScratch {
+public:
+    explicit NullStreamScratch(size_t bytes);
+    ~NullStreamScratch();
+    NullStreamScratch(const NullStreamScratch&) = delete;
+    NullStreamScratch& operator=(const NullStreamScratch&) = delete;
+    void* ptr = nullptr;
+};
 int device_cu_count();                                   // compute units of the current device (0 when it cannot be read)
 // Kernel families can be switched off for cross-checks and same-machine comparisons: RP_HIP_DISABLE holds a comma-separated
 // list of names (read once per process).  The dispatcher then takes what it would take if that kernel did not exist.

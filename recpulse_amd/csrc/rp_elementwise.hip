@@ -524,11 +524,9 @@ __global__ void sum_dim_kernel(T* out, const T* x, size_t outer, size_t dim, siz
     }
 }
 
-// Linear's bias gradient: out[j] = sum_i grad[i, j] in the order of rp_column_sums.h.  No workspace: the sums of all rows meet
-// inside one workgroup, so calls on several streams share nothing and a first call can be recorded.  (Partial sums of all
-// chunks in a workspace, added by a second launch, put more CUs to work on tall narrow matrices: 8192 x 1024 bf16 6.6 us
-// against 9.5, 65536 x 64 8.9 against 91.  But a block of the pool is not safe across streams, and tying it to its stream with
-// an event or a stream-ordered allocation costs 5 or 11 us a call.)
+// Linear's bias gradient: out[j] = sum_i grad[i, j] in the order of rp_column_sums.h.  No block of the pool: it is not safe across
+// streams, so the sums of all rows meet inside one workgroup; calls on several streams share nothing and a first call can be
+// recorded.  (Tall matrices on the null stream, whose scratch memory is safe, go chunk by chunk, see below.)
 //
 // Up to COLSUM_CHUNK rows: a thread per column, the loads of 64 rows in flight together.  64 x 4096 bf16 2.7 us, 256 x 4096
 // 4.5 us a call (staged in LDS, where one wave adds them: 3.2 and 5.3).
@@ -565,9 +563,9 @@ __global__ void __launch_bounds__(64) column_sums_short_kernel(T* out, const T* 
 
 // More rows: a workgroup of 1024 threads walks a strip of WIDTH bytes' worth of columns, 64 KB of it at a time: the next 64 KB are on
 // their way to registers while the threads add the present ones out of LDS, a lane per run and column.
-// WIDTH: 64 where such strips occupy at least half the CUs, else 16 (four times the workgroups, a quarter of the passes; a cache
+// WIDTH: 64 where such strips occupy at least half the CUs (a quarter if one pass does), else 16 (four times the workgroups, a quarter of the passes; a cache
 // line is then touched by eight workgroups instead of two, which all run on one XCD).  What bounds it: memory with strips of 64
-// (8192 x 8192 bf16 27 us, 4096 x 4096 fp32 15), the lines that the CU's vector cache takes in for 16 bytes of each with strips of
+// (4096 x 4096 fp32 14.6 us), the lines that the CU's vector cache takes in for 16 bytes of each with strips of
 // 16 (a pass of 4096 rows 3 - 6 us; 1024 x 1024 bf16 4.1 us a call, 2048 x 512 4.4, where a thread per column took 15 and 28).
 template <typename T, int WIDTH>
 struct ColumnWalk {
@@ -623,6 +621,60 @@ __global__ void __launch_bounds__(1024) column_sums_kernel(T* out, const T* grad
     out[j] = r;
 }
 
+// Tall matrices on the null stream: a workgroup per chunk and strip of 128 bytes leaves the chunk's sums in `partials`
+// [chunk][cols], and a second launch adds them.
+template <typename T>
+__global__ void __launch_bounds__(256) column_chunks_kernel(typename traits<T>::acc* partials, const T* grad, int rows, int cols) {
+    using A = typename traits<T>::acc;
+    using Tile = ColumnTile<T, 128, COLSUM_CHUNK>;
+    constexpr int COLS = Tile::COLS, RPC = COLSUM_CHUNK / COLSUM_RUN;
+    __shared__ __attribute__((aligned(16))) T tile[COLSUM_CHUNK * COLS];
+    __shared__ A parts[RPC][COLS];
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const long long r0 = (long long)blockIdx.y * COLSUM_CHUNK;
+    const int left = (int)(rows - r0 < COLSUM_CHUNK ? rows - r0 : COLSUM_CHUNK), c0 = blockIdx.x * COLS;
+    {
+        Tile regs;
+        regs.load(grad + (size_t)r0 * cols, 0, left, c0, cols, t);
+        regs.store(tile, t);
+    }
+    __syncthreads();
+    const int n = left - wave * COLSUM_RUN;             // rows of this wave's run
+    if (lane < COLS) parts[wave][lane] = n > 0 ? Tile::add(0, tile + wave * COLSUM_RUN * COLS, lane, n < COLSUM_RUN ? n : COLSUM_RUN) : (A)0;
+    __syncthreads();
+    if (t >= COLS || c0 + t >= cols) return;
+    A c = parts[0][t];
+#pragma unroll
+    for (int q = 1; q < RPC; q++) c += parts[q][t];
+    partials[(size_t)blockIdx.y * cols + c0 + t] = c;
+}
+
+template <typename T>
+__global__ void __launch_bounds__(64) column_sums_finish_kernel(T* out, const typename traits<T>::acc* partials, int chunks, int cols, int accumulate) {
+    using A = typename traits<T>::acc;
+    const int j = blockIdx.x * 64 + threadIdx.x;
+    if (j >= cols) return;
+    A s = 0;
+    constexpr int U = 32;                               // independent loads in flight; the adds stay in chunk order
+    int i = 0;
+    A v[U];
+    for (; i + U <= chunks; i += U) {
+#pragma unroll
+        for (int u = 0; u < U; u++) v[u] = partials[(size_t)(i + u) * cols + j];
+#pragma unroll
+        for (int u = 0; u < U; u++) s += v[u];
+    }
+    if (i < chunks) {                                   // the rest in one go (past the end: the last chunk again, not added)
+#pragma unroll
+        for (int u = 0; u < U; u++) v[u] = partials[(size_t)(i + u < chunks ? i + u : chunks - 1) * cols + j];
+#pragma unroll
+        for (int u = 0; u < U; u++) if (i + u < chunks) s += v[u];
+    }
+    T r = narrow<T>(s);
+    if (accumulate) r = narrow<T>(widen(out[j]) + widen(r));
+    out[j] = r;
+}
+
 template <typename T, int WIDTH>
 static int launch_column_walk(T* out, const T* grad, int rows, int cols, int accumulate) {
     using Walk = ColumnWalk<T, WIDTH>;
@@ -638,7 +690,19 @@ static int launch_column_sums(T* out, const T* grad, int rows, int cols, int acc
         hipLaunchKernelGGL(column_sums_short_kernel<T>, dim3((cols - 1) / 64 + 1), dim3(64), 0, current_stream(), out, grad, rows, cols, accumulate);
         return check_launch("column_sums_short_kernel") ? 0 : -1;
     }
-    if ((cols - 1) / ColumnWalk<T, 64>::COLS + 1 >= device_cu_count() / 2) return launch_column_walk<T, 64>(out, grad, rows, cols, accumulate);
+    // Tall: chunk by chunk where that is safe (chunks / walk, us: bf16 4096 x 1024 6.2 / 5.7, 5000 x 64 6.3 / 6.7, 5000 x 8192 19.5 / 18.5, 8192 x 1024
+    // 6.4 / 9.5, 8192 x 4096 16.0 / 26.9, 65536 x 64 8.7 / 91; fp32 4096 x 4096 16.0 / 14.6, 8192 x 8192 46 / 53)
+    if (rows > 4096) {
+        const int chunks = (rows - 1) / COLSUM_CHUNK + 1;
+        using A = typename traits<T>::acc;
+        NullStreamScratch scratch((size_t)chunks * cols * sizeof(A));
+        if (scratch.ptr && chunks <= 65535) {
+            hipLaunchKernelGGL(column_chunks_kernel<T>, dim3((cols - 1) / ColumnTile<T, 128, COLSUM_CHUNK>::COLS + 1, chunks), dim3(256), 0, nullptr, (A*)scratch.ptr, grad, rows, cols);
+            hipLaunchKernelGGL(column_sums_finish_kernel<T>, dim3((cols - 1) / 64 + 1), dim3(64), 0, nullptr, out, (const A*)scratch.ptr, chunks, cols, accumulate);
+            return check_launch("column_chunks_kernel") ? 0 : -1;
+        }
+    }
+    if ((cols - 1) / ColumnWalk<T, 64>::COLS + 1 >= device_cu_count() / (rows <= ColumnWalk<T, 64>::ROWS ? 4 : 2)) return launch_column_walk<T, 64>(out, grad, rows, cols, accumulate);
     return launch_column_walk<T, 16>(out, grad, rows, cols, accumulate);
 }
 

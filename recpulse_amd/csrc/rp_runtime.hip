@@ -155,6 +155,24 @@ static size_t round_size(size_t bytes) {
     return (bytes + ((1u << 21) - 1)) & ~(size_t)((1u << 21) - 1);         // 2 MiB steps above
 }
 
+// One block per device, kept until rp_hip_empty_cache.
+constexpr size_t NULL_STREAM_SCRATCH = (size_t)16 << 20;
+constexpr int NULL_STREAM_DEVICES = 64;
+static std::mutex g_null_stream_mu;
+static void* g_null_stream_scratch[NULL_STREAM_DEVICES] = {};
+
+NullStreamScratch::NullStreamScratch(size_t bytes) {
+    int dev = 0;
+    if (current_stream() || bytes > NULL_STREAM_SCRATCH) return;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= NULL_STREAM_DEVICES) { (void)hipGetLastError(); return; }
+    g_null_stream_mu.lock();
+    void*& block = g_null_stream_scratch[dev];
+    if (!block && hipMalloc(&block, NULL_STREAM_SCRATCH) != hipSuccess) { (void)hipGetLastError(); block = nullptr; }
+    ptr = block;
+    if (!ptr) g_null_stream_mu.unlock();
+}
+NullStreamScratch::~NullStreamScratch() { if (ptr) g_null_stream_mu.unlock(); }
+
 struct SmallPayload { uint32_t w[512]; };            // 2 KiB, passed by value in the kernel arguments
 __global__ void upload_small_kernel(uint32_t* dst, SmallPayload payload, int nwords) {
     int i = blockIdx.x * 256 + threadIdx.x;
@@ -292,6 +310,9 @@ int rp_hip_empty_cache(void) {
     }
     bool ok = true;
     for (void* b : blocks) ok = check_hip(hipFree(b), "hipFree") && ok;
+    std::lock_guard<std::mutex> lk(g_null_stream_mu);
+    for (void*& b : g_null_stream_scratch)              // (hipFree waits for the work that uses a block)
+        if (b) { ok = check_hip(hipFree(b), "hipFree") && ok; b = nullptr; }
     return ok ? 0 : -1;
 }
 

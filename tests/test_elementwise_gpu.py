@@ -1,5 +1,6 @@
 """GPU parity of the non-GEMM entry points against the CPU oracle."""
 import ctypes
+import threading
 
 import numpy as np
 import pytest
@@ -156,7 +157,7 @@ def test_reduce_rows_beyond_one_chunk_bit_exact(dt, rows):
 
 
 @pytest.mark.parametrize("dt", ALL, ids=lambda d: NAMES[d])
-@pytest.mark.parametrize("rows,cols", [(16, 70), (17, 70), (79, 70), (255, 4099), (257, 8200), (1030, 8200), (2600, 4099), (4096, 9), (4097, 9), (8261, 33)])
+@pytest.mark.parametrize("rows,cols", [(16, 70), (17, 70), (79, 70), (255, 4099), (257, 8200), (1030, 8200), (2600, 4099), (4096, 9), (4096, 4099), (4097, 9), (8261, 33)])
 def test_reduce_rows_strips_wide_and_narrow_bit_exact(dt, rows, cols):
     """Few rows (groups of 64 and 16 and a rest), strips of 64 bytes (enough of them for half the CUs) and of 16, one pass and more."""
     rng = np.random.default_rng(47)
@@ -164,6 +165,42 @@ def test_reduce_rows_strips_wide_and_narrow_bit_exact(dt, rows, cols):
     dg, do = Dev(g, dt), Dev.empty((cols,), dt)
     capi.check(L().rp_hip_reduce_rows(do.ptr, dg.ptr, rows, cols, 0, dt), "reduce_rows")
     assert np.array_equal(do.numpy(), _column_sums(g, dt))
+
+
+@pytest.mark.parametrize("dt", ALL, ids=lambda d: NAMES[d])
+@pytest.mark.parametrize("rows,cols", [(4097, 33), (8192, 9), (9000, 4200), (17000, 261)])
+def test_tall_column_sums_of_several_threads(dt, rows, cols):
+    """Tall matrices go chunk by chunk through memory that belongs to the null stream, and are walked on any other: the same
+    bits.  Three threads on the null stream and one on a stream of its own, each with a matrix of its own."""
+    rng = np.random.default_rng(49)
+    gs = [rand_storage(rng, (rows, cols), dt) for _ in range(4)]
+    want = [_column_sums(g, dt) for g in gs]
+    dg, do = [Dev(g, dt) for g in gs], [Dev.empty((cols,), dt) for _ in gs]
+    got = [None] * 4
+    capi.synchronize()
+
+    def work(i):
+        stream = capi.Stream() if i == 3 else None
+        if stream:
+            stream.__enter__()
+        ok = True
+        for _ in range(30):
+            ok = ok and L().rp_hip_reduce_rows(do[i].ptr, dg[i].ptr, rows, cols, 0, dt) == 0
+        ok = ok and L().rp_hip_stream_synchronize() == 0
+        got[i] = (ok, do[i].buf.to_numpy(capi.NP_STORAGE[dt], (cols,)))
+        if stream:
+            stream.__exit__()
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+    for th in threads:
+        th.start()
+    for th in threads:
+        th.join()
+    for (ok, out), w in zip(got, want):
+        assert ok and np.array_equal(out, w)
+    capi.check(L().rp_hip_empty_cache(), "empty_cache")          # gives the memory back; the next call takes it again
+    capi.check(L().rp_hip_reduce_rows(do[0].ptr, dg[0].ptr, rows, cols, 0, dt), "reduce_rows")
+    assert np.array_equal(do[0].numpy(), want[0])
 
 
 def test_reduce_rows_of_nearly_two_to_the_31_rows():
@@ -189,7 +226,7 @@ def _memory_stats():
 
 
 @pytest.mark.parametrize("dt", [F32, BF16], ids=lambda d: NAMES[d])
-@pytest.mark.parametrize("rows,cols", [(200, 300), (5000, 72), (3000, 4200)])
+@pytest.mark.parametrize("rows,cols", [(200, 300), (9000, 72), (3000, 4200)])
 def test_bias_gradients_share_nothing(dt, rows, cols):
     """Column sums take no block of the pool, whatever the number of rows: two streams of one device sum different matrices of
     one shape at the same time, and a first call can be recorded."""
