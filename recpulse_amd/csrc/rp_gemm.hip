@@ -63,8 +63,12 @@ static void choose_tile16(Plan& p, int batch, int m, int k, int n) {
 static void choose_tile_wide(Plan& p, int batch, int m, int k, int n, int dtype) {
     p.fam = FAM_MFMAW;
     const long long tiles128 = (long long)((m + 127) / 128) * ((n + 127) / 128) * batch;
-    // a 128 x 128 tile over a 64-wide output would compute and fetch half of it for nothing
-    if (m > 64 && n > 64 && tiles128 >= cu_tiles() / 2) { p.bm = 128; p.bn = 128; p.name = (dtype == RP_DTYPE_FLOAT32) ? "mfma32_128x128" : "mfma64_128x128"; }
+    // a 128 x 128 tile over a 64-wide output would compute and fetch half of it for nothing.  Ragged rows take it only in fp32 on the
+    // bf16 matrix cores, and only for k that is worth that kernel's prologue: the 128 x 128 tile of the fp32 / fp64 MFMA kernel holds
+    // a CU by itself and cannot cover its unaligned loads (us, 128 x 128 and 64 x 64: fp64 501 x 1025 x 4001 376 / 164, 1411 x 129 x 1500 60 / 31,
+    // 4999 x 513 x 4999 921 / 689; fp32 in bf16 501 x 33 x 4001 16.4 / 9.4, 3001 x 49 x 2999 31.7 / 28.3, 4999 x 49 x 4999 62.3 / 63.8, 2001 x 97 x 2003 20.5 / 22.4).
+    const bool tile128 = !p.ragged || (dtype == RP_DTYPE_FLOAT32 && k > 48 && !path_disabled("split32"));
+    if (tile128 && m > 64 && n > 64 && tiles128 >= cu_tiles() / 2) { p.bm = 128; p.bn = 128; p.name = (dtype == RP_DTYPE_FLOAT32) ? "mfma32_128x128" : "mfma64_128x128"; }
     else { p.bm = 64; p.bn = 64; p.name = (dtype == RP_DTYPE_FLOAT32) ? "mfma32_64x64" : "mfma64_64x64"; }
     p.edge = (m % p.bm) || (n % p.bn) || (k % (dtype == RP_DTYPE_FLOAT32 ? 32 : 16));
 }

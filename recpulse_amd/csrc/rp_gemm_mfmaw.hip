@@ -473,18 +473,21 @@ static int mw_launch(const GemmArgs& g, dim3 grid, int tiles_m, int tiles_n, flo
 
 template <typename T, int BM, int BN, bool A_MC, bool B_MC>
 static int launch_mfmaw_edge(const GemmArgs& g, const Plan& p, float* partials, int nsplit, int k_per_split) {
+    if (BM != 64 && p.ragged) { set_error("mfmaw GEMM: ragged rows on a %d x %d tile", BM, BN); return -1; }
     int tiles_m = (g.m + BM - 1) / BM, tiles_n = (g.n + BN - 1) / BN;
     if (nsplit > 1) {
         if constexpr (sizeof(T) == 4) {           // split-k partials are fp32; always a predicated variant
             dim3 grid(scheduled_grid(tiles_m, tiles_n), g.batch, nsplit);
-            if (p.ragged) return mw_launch<T, BM, BN, A_MC, B_MC, MW_RAGGED, true>(g, grid, tiles_m, tiles_n, partials, k_per_split);
+            if constexpr (BM == 64)
+                if (p.ragged) return mw_launch<T, BM, BN, A_MC, B_MC, MW_RAGGED, true>(g, grid, tiles_m, tiles_n, partials, k_per_split);
             return mw_launch<T, BM, BN, A_MC, B_MC, MW_EDGE, true>(g, grid, tiles_m, tiles_n, partials, k_per_split);
         }
         set_error("mfmaw GEMM: split-k is fp32 only");
         return -1;
     }
     dim3 grid(scheduled_grid(tiles_m, tiles_n), g.batch);
-    if (p.ragged) return mw_launch<T, BM, BN, A_MC, B_MC, MW_RAGGED, false>(g, grid, tiles_m, tiles_n, nullptr, 0);
+    if constexpr (BM == 64)                   // (the dispatcher's only tile for ragged rows here)
+        if (p.ragged) return mw_launch<T, BM, BN, A_MC, B_MC, MW_RAGGED, false>(g, grid, tiles_m, tiles_n, nullptr, 0);
     if (p.edge) return mw_launch<T, BM, BN, A_MC, B_MC, MW_EDGE, false>(g, grid, tiles_m, tiles_n, nullptr, 0);
     return mw_launch<T, BM, BN, A_MC, B_MC, MW_WHOLE, false>(g, grid, tiles_m, tiles_n, nullptr, 0);
 }
