@@ -1156,7 +1156,7 @@ def test_split32_at_the_ends_of_its_range(k):
 
 
 @pytest.mark.parametrize("layout", LAYOUTS)
-@pytest.mark.parametrize("m,k,n", [(1408, 160, 1536), (1411, 170, 1405), (1501, 69, 1499)])
+@pytest.mark.parametrize("m,k,n", [(1408, 288, 1536), (1411, 170, 1405), (1501, 69, 1499)])
 def test_split32_tiles_that_change_over(m, k, n, layout):
     """From the first slab of k on that holds a value whose last bits bf16 cannot hold, a tile is multiplied with fp32 MFMAs: at the
     first, an inner and the last k, from either operand.  Integers otherwise, so every sum that is not zero has known bits; then an infinity as well."""
