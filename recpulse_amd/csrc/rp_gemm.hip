@@ -180,7 +180,11 @@ static Plan make_plan(int batch, int m, int k, int n, long long a_rs, long long 
         const bool ak = a_cs == 1 && k >= vec && (a_rs >= k || m == 1), am = a_rs == 1 && m >= vec && a_cs >= m;
         const bool bn = b_cs == 1 && n >= vec && b_rs >= n, bk = b_rs == 1 && k >= vec && (b_cs >= k || n == 1);
         const bool worth = (long long)m * n * batch >= 8192 || (long long)k * n >= (1 << 18) || (long long)m * k >= (1 << 18);
-        if ((ak || am) && (bn || bk) && worth) {
+        // The same for 16-bit outputs of up to four tiles whose k is deeper than ten slabs a tile (bf16, us, MFMA and generic: 156 x 4097 x 59
+        // 26.7 / 20.5, 33 x 8001 x 129 47.4 / 29.8, 65 x 2049 x 127 16.0 / 17.5; nine tiles, 130 x 8001 x 130 47.7 / 78)
+        const int tiles64 = ((m + 63) / 64) * ((n + 63) / 64);
+        const bool too_deep = is16 && batch == 1 && tiles64 <= 4 && k > 10 * M16_BK * tiles64;
+        if ((ak || am) && (bn || bk) && worth && !too_deep) {
             p.ragged = true;
             p.a_mc = !ak;
             p.b_mc = bn;

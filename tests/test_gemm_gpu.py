@@ -543,7 +543,7 @@ def test_wide_tiles_for_outputs_of_at_most_64_rows():
 RAGGED_SHAPES = [  # (batch, m, k, n, kernel): every 16-bit tile, k of one slab and its tails, free axes that end 1 .. 7 past a vector
     (1, 1000, 9, 9, "mfma16_64x64"), (1, 131, 8, 65, "mfma16_64x64"), (1, 203, 63, 129, "mfma16_64x64"), (3, 121, 65, 71, "mfma16_64x64"),
     (1, 199, 391, 137, "mfma16_64x64"), (1, 1450, 127, 1403, "mfma16_128x128"), (130, 33, 77, 261, "mfma16_64x128"), (66, 35, 1025, 305, "mfma16_64x256"),
-    (1, 3000, 259, 2821, "mfma16_256x256"), (1, 5, 4099, 1027, "mfma16_skinny_32x128"), (1, 33, 4102, 1035, "mfma16_skinny_32x128")]
+    (1, 3000, 259, 2821, "mfma16_256x256"), (1, 65, 2561, 127, "generic"), (1, 65, 2557, 127, "mfma16_64x64"), (1, 5, 4099, 1027, "mfma16_skinny_32x128"), (1, 33, 4102, 1035, "mfma16_skinny_32x128")]
 
 
 RAGGED_WIDE_SHAPES = [  # the same for fp32 (with and without a k split) and fp64
