@@ -7,14 +7,16 @@
 // two fast layouts, chosen from its strides:
 //   KC  the reduction (k) axis is the unit-stride one      (A row-major, or Bᵀ stored)
 //   MC  the free (m or n) axis is the unit-stride one       (B row-major, or Aᵀ stored)
-// Anything else (both strides > 1, misaligned bases, odd extents) takes the
-// generic strided kernel.
+// Rows that are no whole number of 16-byte vectors, or start at any element, have
+// "ragged" variants of the MFMA kernels.  Anything else (both strides > 1, rows that
+// overlap, small outputs between small ragged operands) takes the generic strided kernel.
 //
 // Kernel families:
 //   mfma16   bf16 / fp16 inputs, fp32 accumulate, v_mfma_f32_32x32x16_{bf16,f16};
 //            KC tiles are read from LDS with ds_read_b128, MC tiles with the
 //            transposing ds_read_b64_tr_b16, so no layout needs a copy.
 //   mfmaw    fp32 (v_mfma_f32_32x32x2_f32) and fp64 (v_mfma_f64_16x16x4_f64).
+//   split32  fp32 outputs of 128 x 128 tiles on the bf16 matrix cores, every value split in three (a kernel of family mfmaw).
 //   skinny   m <= 8 against a row-major B: a split-k streaming kernel bound by HBM.
 //   tiny     fp32 outputs of a few hundred 16 x 16 tiles: one launch, k split over the waves of a workgroup.
 //   generic  any strides, any shape; LDS-tiled scalar FMA.
