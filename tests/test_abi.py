@@ -74,3 +74,22 @@ def test_kernel_selection_names():
     assert name(Z, S, D, S, (D, 1), (1, D), (1, S), capi.BF16) == "mfma16_128x128"        # 16-bit C not row-major
     assert name(1, 5, 7, 3, (7, 1), (3, 1), (3, 1), capi.BF16) == "generic"                                # odd extents
     assert name(1, 64, 64, 64, (128, 2), (64, 1), (64, 1), capi.F64) == "generic"                          # no unit stride
+
+
+def test_kernel_selection_of_ragged_rows_and_overlapping_k():
+    name = capi.gemm_kernel_name
+    for dt in (capi.BF16, capi.F16):
+        # k rows that overlap are not masked past the end of k by the buffer's end: only where no slab hangs over
+        assert name(1, 128, 72, 256, (1, 0), (256, 1), (256, 1), dt) == "generic"
+        assert name(1, 128, 72, 256, (1, 128), (8, 1), (256, 1), dt) == "generic"
+        assert name(1, 128, 128, 256, (1, 0), (0, 1), (256, 1), dt) == "mfma16_64x64"
+        # with k = 1 the k strides say nothing
+        for a_k, b_k in ((0, 0), (1, 1), (256, 784)):
+            assert name(1, 256, 1, 784, (1, a_k), (b_k, 1), (784, 1), dt) == name(1, 256, 1, 784, (1, 256), (784, 1), (784, 1), dt)
+        # partial sums on either side of 16 MiB, and a small output of a deep k
+        assert name(1, 32, 1025, 131071, (1025, 1), (131071, 1), (131071, 1), dt) == "mfma16_skinny_32x128"
+        assert name(1, 32, 1025, 131075, (1025, 1), (131075, 1), (131075, 1), dt) == "mfma16_64x256"
+        assert name(1, 33, 8001, 129, (8001, 1), (129, 1), (129, 1), dt) == "generic"
+    assert name(1, 1411, 129, 1500, (1, 1411), (1500, 1), (1500, 1), capi.F64) == "mfma64_64x64"
+    assert name(1, 3001, 31, 2999, (31, 1), (2999, 1), (2999, 1), capi.F32) == "mfma32_64x64"
+    assert name(1, 3001, 129, 2999, (129, 1), (2999, 1), (2999, 1), capi.F32) == "mfma32_128x128"
