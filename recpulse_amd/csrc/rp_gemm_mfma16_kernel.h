@@ -16,13 +16,13 @@ namespace rp {
 // writes its fp32 partial tile to a workspace [matrix][split][m][n] and a
 // combine kernel finishes.
 //
-// Software pipeline, per slab s (4 k-steps of 16):
+// Software pipeline, per slab s (4 k-steps of 16), with PF register sets:
 //   k-steps 0-2  MFMAs on fragments(ks) | read fragments(ks+1) | a third of: registers of slab s+1 -> other
-//                LDS buffer, then the global load of slab s+2 into the register just freed
+//                LDS buffer, then the global load of slab s+1+PF into the register just freed
 //   barrier      (slab s+1 is now complete in LDS, and nobody reads this slab's buffer any more)
 //   k-step 3     MFMAs on fragments(3) | read fragments(0) of slab s+1
 // so LDS reads run one k-step ahead of the MFMAs that use them, global loads
-// have a full slab of MFMA time to land, and the single barrier per slab sits
+// have PF slabs of MFMA time to land, and the single barrier per slab sits
 // where only one MFMA group is left to issue.  Every MFMA is followed by its
 // share of DS / VMEM work and a scheduling barrier, which pins the interleaving.
 // The 256 x 256 tile multiplies with 16x16x32 MFMAs instead (m16_mfma_tile): two
@@ -85,6 +85,11 @@ __host__ __device__ constexpr size_t m16_smem_bytes(int bm, int bn, int wgm, boo
     return loop > epi ? loop : epi;
 }
 
+// Workgroups of 256 threads whose registers have to fit a CU together (their LDS allows two of the 128 x 128 tile, three of the
+// 64 x 64 one).  The ragged 128 x 128 kernels took a few registers more than that when left alone, and an output of 288
+// tiles then went in two full rounds (fp16 1500 x 2049 x 3003 54.5 us, 48.6 now; bf16 1900 x 777 x 2500 27.7, 22.4 now).
+__host__ __device__ constexpr int m16_blocks_per_cu(int bm, int bn, int edge, int sets) { return sets > 1 ? 3 : bm == 128 && bn == 128 && edge == 2 ? 2 : 1; }
+
 typedef uint16_t __attribute__((address_space(3))) lds_u16;
 
 
@@ -140,6 +145,15 @@ struct FragMap {
     }
 };
 
+// PF: slabs of both operands that travel in registers at a time, each in a set of its own.  One set gives a load the time of one
+// slab to arrive.  For the 64 x 64 tile that is less than a load from another XCD's memory takes, and with the one or two workgroups
+// per CU of a small product nothing else covers it; three sets do (bf16, us, 1 set and 3: 1024^3 8.9 / 8.0, 256 x 4096 x 256 23.1 / 17.4,
+// 64 x 1024 x 4096 8.4 / 7.5).  The 128 x 128 tile gains nothing (2048^3 20.5 / 20.3: it is bound by what a CU can fetch from its L2,
+// 32 KB a slab at 39 B a cycle).  The loop runs whole rounds of PF slabs, up to two of them zeros, which a k of few slabs would feel
+// (600 x 264 x 600 6.4 / 6.9): from twelve slabs on.  Ragged rows stay at one set, their loads take twice the time to issue.
+constexpr int M16_DEEP_SETS = 3;
+static inline bool m16_deep(int k) { return k > 11 * M16_BK; }
+
 // EDGE: what of the tile may hang over the problem.
 enum { M16_WHOLE = 0, M16_EDGE = 1, M16_RAGGED = 2 };
 // M16_WHOLE: nothing.  M16_EDGE: m, n or k end inside a tile, in whole 16-byte vectors.  M16_RAGGED: anywhere, and rows may
@@ -157,7 +171,7 @@ __device__ __forceinline__ u32x4_t m16_pull_shift(u32x4_t v, int pull) {
 typedef unsigned int u32x4_any_t __attribute__((ext_vector_type(4), aligned(2)));       // a 16-byte vector at any element
 
 // What one workgroup does: slots first_slot, first_slot + stride, ... of the schedule of matrix z
-template <typename T, int BM, int BN, int WGM, bool A_MC, bool B_MC, int EDGE, bool SPLITK>
+template <typename T, int BM, int BN, int WGM, bool A_MC, bool B_MC, int EDGE, bool SPLITK, int PF>
 __device__ __forceinline__ void gemm_mfma16_block(const GemmArgs& g, int tiles_m, int tiles_n, float* partials, int k_per_split, int sched_total, int first_slot, int z, int stride) {
     constexpr int WGN = 4 / WGM;
     constexpr int WM = BM / WGM, WN = BN / WGN;       // wave patch
@@ -257,7 +271,7 @@ __device__ __forceinline__ void gemm_mfma16_block(const GemmArgs& g, int tiles_m
 #pragma unroll
             for (int v = 0; v < NV; v++) acc[i][j][v] = 0.f;
 
-    u32x4_t ra[NA], rb[NB];
+    u32x4_t ra[PF][NA], rb[PF][NB];                   // slab s travels in set s % PF
     const int nslabs = (kend - kbeg + M16_BK - 1) / M16_BK;
     // M16_RAGGED: how many elements of this thread's vectors stick out of their row in the last slab (0: none or all)
     int a_pull = 0, b_pull = 0;
@@ -270,46 +284,52 @@ __device__ __forceinline__ void gemm_mfma16_block(const GemmArgs& g, int tiles_m
     __amdgpu_buffer_rsrc_t a_rsrc, b_rsrc;
     int kleft = 0;        // k still in range counted from the slab the descriptors point at (EDGE, KC operands)
 
-    auto point_at_slab = [&](int k0) {
-        a_rsrc = buffer_rsrc(a_slab - BACK, EDGE ? (long long)(a_end - a_slab) + BACK : 0x7fffffffll);
-        b_rsrc = buffer_rsrc(b_slab - BACK, EDGE ? (long long)(b_end - b_slab) + BACK : 0x7fffffffll);
-        kleft = kend - kbeg - k0;
+    // (slabs past the last one are requested too and read as zeros)
+    auto point_at_slab = [&](int slab) {
+        const bool live = slab < nslabs;
+        a_rsrc = buffer_rsrc(a_slab - BACK, !live ? 0 : EDGE ? (long long)(a_end - a_slab) + BACK : 0x7fffffffll);
+        b_rsrc = buffer_rsrc(b_slab - BACK, !live ? 0 : EDGE ? (long long)(b_end - b_slab) + BACK : 0x7fffffffll);
+        kleft = kend - kbeg - slab * M16_BK;
     };
     // Without edges piece i sits a uniform number of bytes after piece 0: one lane offset per operand plus a scalar
     // offset per piece, instead of a register per piece.
     const int a_piece_step = (int)((long long)MapA::PIECE_ROWS * (A_MC ? a_ks : a_fs) * 2);
     const int b_piece_step = (int)((long long)MapB::PIECE_ROWS * (B_MC ? b_ks : b_fs) * 2);
-    auto load_piece_a = [&](auto ic) {
-        constexpr int i = decltype(ic)::value;
+    auto load_piece_a = [&](auto setc, auto ic) {
+        constexpr int i = decltype(ic)::value, S = decltype(setc)::value;
         if constexpr (!EDGE) {
-            ra[i] = __builtin_amdgcn_raw_buffer_load_b128(a_rsrc, (int)a_goff[0], i * a_piece_step, 0);
+            ra[S][i] = __builtin_amdgcn_raw_buffer_load_b128(a_rsrc, (int)a_goff[0], i * a_piece_step, 0);
         } else {
             uint32_t off = a_goff[i];
             if (!A_MC && a_kk0 >= kleft) off = BUFFER_OOB;
             if (EDGE == M16_RAGGED && kleft <= M16_BK) off -= 2 * a_pull;
-            ra[i] = __builtin_amdgcn_raw_buffer_load_b128(a_rsrc, (int)off, 0, 0);
+            ra[S][i] = __builtin_amdgcn_raw_buffer_load_b128(a_rsrc, (int)off, 0, 0);
         }
     };
-    auto load_piece_b = [&](auto ic) {
-        constexpr int i = decltype(ic)::value;
+    auto load_piece_b = [&](auto setc, auto ic) {
+        constexpr int i = decltype(ic)::value, S = decltype(setc)::value;
         if constexpr (!EDGE) {
-            rb[i] = __builtin_amdgcn_raw_buffer_load_b128(b_rsrc, n_segmented ? (int)b_goff[i] : (int)b_goff[0], n_segmented ? 0 : i * b_piece_step, 0);
+            rb[S][i] = __builtin_amdgcn_raw_buffer_load_b128(b_rsrc, n_segmented ? (int)b_goff[i] : (int)b_goff[0], n_segmented ? 0 : i * b_piece_step, 0);
         } else {
             uint32_t off = b_goff[i];
             if (!B_MC && b_kk0 >= kleft) off = BUFFER_OOB;
             if (EDGE == M16_RAGGED && kleft <= M16_BK) off -= 2 * b_pull;
-            rb[i] = __builtin_amdgcn_raw_buffer_load_b128(b_rsrc, (int)off, 0, 0);
+            rb[S][i] = __builtin_amdgcn_raw_buffer_load_b128(b_rsrc, (int)off, 0, 0);
         }
     };
-    auto store_piece_a = [&](uint16_t* stage, auto ic, auto last_tag) {
-        constexpr int i = decltype(ic)::value;
-        if constexpr (EDGE == M16_RAGGED && decltype(last_tag)::value) ra[i] = m16_pull_shift(ra[i], a_pull);
-        *(u32x4_t*)(stage + a_wr0 + i * MapA::LDS_STEP) = ra[i];
+    auto store_piece_a = [&](uint16_t* stage, auto setc, auto ic) {
+        constexpr int i = decltype(ic)::value, S = decltype(setc)::value;
+        *(u32x4_t*)(stage + a_wr0 + i * MapA::LDS_STEP) = ra[S][i];
     };
-    auto store_piece_b = [&](uint16_t* stage, auto ic, auto last_tag) {
-        constexpr int i = decltype(ic)::value;
-        if constexpr (EDGE == M16_RAGGED && decltype(last_tag)::value) rb[i] = m16_pull_shift(rb[i], b_pull);
-        *(u32x4_t*)(stage + b_wr0 + i * MapB::LDS_STEP) = rb[i];
+    auto store_piece_b = [&](uint16_t* stage, auto setc, auto ic) {
+        constexpr int i = decltype(ic)::value, S = decltype(setc)::value;
+        *(u32x4_t*)(stage + b_wr0 + i * MapB::LDS_STEP) = rb[S][i];
+    };
+    // M16_RAGGED, before the last slab goes to LDS: its straddling vectors were loaded `pull` elements early
+    auto pull_into_place = [&](auto setc) {
+        constexpr int S = decltype(setc)::value;
+        static_for<0, NA>([&](auto ic) { ra[S][decltype(ic)::value] = m16_pull_shift(ra[S][decltype(ic)::value], a_pull); });
+        static_for<0, NB>([&](auto ic) { rb[S][decltype(ic)::value] = m16_pull_shift(rb[S][decltype(ic)::value], b_pull); });
     };
 
     // B fragments have two slots (the next k-step's are read while this one's are multiplied).  With 32 x 32 tiles
@@ -335,50 +355,43 @@ __device__ __forceinline__ void gemm_mfma16_block(const GemmArgs& g, int tiles_m
     using I2 = std::integral_constant<int, 2>;
     using I3 = std::integral_constant<int, 3>;
 
-    // ---- prologue: slab 0 into LDS buffer 0, slab 1 into registers, fragments(0) of slab 0 ----
-    point_at_slab(0);
-    static_for<0, NA>([&](auto ic) { load_piece_a(ic); });
-    static_for<0, NB>([&](auto ic) { load_piece_b(ic); });
-    if (tile_id != first_slot) __syncthreads();            // the previous tile's epilogue has read its staged rows out of LDS
-    auto store_first = [&](auto last_tag) {
-        static_for<0, NA>([&](auto ic) { store_piece_a(smem, ic, last_tag); });
-        static_for<0, NB>([&](auto ic) { store_piece_b(smem, ic, last_tag); });
+    // ---- prologue: slabs 0 .. PF - 1 requested, slab 0 into LDS buffer 0, slab PF requested, fragments(0) of slab 0 ----
+    auto load_slab = [&](auto setc, int slab) {
+        point_at_slab(slab);
+        static_for<0, NA>([&](auto ic) { load_piece_a(setc, ic); });
+        static_for<0, NB>([&](auto ic) { load_piece_b(setc, ic); });
+        a_slab += a_step;
+        advance_b();
     };
-    if (EDGE == M16_RAGGED && nslabs == 1) store_first(std::true_type{});
-    else store_first(std::false_type{});
-    a_slab += a_step;
-    advance_b();
-    if (nslabs > 1) {
-        point_at_slab(M16_BK);
-        static_for<0, NA>([&](auto ic) { load_piece_a(ic); });
-        static_for<0, NB>([&](auto ic) { load_piece_b(ic); });
-    }
-    a_slab += a_step;
-    advance_b();
+    static_for<0, PF>([&](auto setc) { load_slab(setc, decltype(setc)::value); });
+    if (tile_id != first_slot) __syncthreads();            // the previous tile's epilogue has read its staged rows out of LDS
+    if (EDGE == M16_RAGGED && nslabs == 1) pull_into_place(I0{});
+    static_for<0, NA>([&](auto ic) { store_piece_a(smem, I0{}, ic); });
+    static_for<0, NB>([&](auto ic) { store_piece_b(smem, I0{}, ic); });
+    if (nslabs > 1) load_slab(I0{}, PF);
     __syncthreads();
     static_for<0, RD_A + RD_B>([&](auto rc) { read_item(smem, I0{}, I0{}, rc); });
 
     // Pieces of both operands in one list: 0 .. NA-1 are A's, NA .. NA+NB-1 are B's.
-    auto store_piece = [&](uint16_t* stage, auto pc, auto last_tag) {
+    auto store_piece = [&](uint16_t* stage, auto setc, auto pc) {
         constexpr int p = decltype(pc)::value;
-        if constexpr (p < NA) store_piece_a(stage, std::integral_constant<int, p>{}, last_tag);
-        else store_piece_b(stage, std::integral_constant<int, p - NA>{}, last_tag);
+        if constexpr (p < NA) store_piece_a(stage, setc, std::integral_constant<int, p>{});
+        else store_piece_b(stage, setc, std::integral_constant<int, p - NA>{});
     };
-    auto load_piece = [&](auto pc) {
+    auto load_piece = [&](auto setc, auto pc) {
         constexpr int p = decltype(pc)::value;
-        if constexpr (p < NA) load_piece_a(std::integral_constant<int, p>{});
-        else load_piece_b(std::integral_constant<int, p - NA>{});
+        if constexpr (p < NA) load_piece_a(setc, std::integral_constant<int, p>{});
+        else load_piece_b(setc, std::integral_constant<int, p - NA>{});
     };
 
     // One k-step: NMFMA micro-steps, each one MFMA on fragment slot MSLOT followed by its share of the side
     // work: fragment reads for k-step RKS into the other slot, and pieces [P0, P1) of slab traffic (LDS store of
-    // the registers holding slab s+1 when WR, then the global load of slab s+2 into the same registers when LD).
+    // register set `setc`, which holds slab s+1, when WR, then the global load of slab s+1+PF into the same registers when LD).
     // A scheduling barrier closes every micro-step so the interleaving is the one written.
-    auto kstep = [&](auto mslotc, auto rksc, auto readc, auto p0c, auto p1c, auto wrc, auto ldc,
+    auto kstep = [&](auto setc, auto mslotc, auto rksc, auto readc, auto p0c, auto p1c, auto wrc, auto ldc,
                      const uint16_t* rd_stage, uint16_t* wr_stage) {
         constexpr int MSLOT = decltype(mslotc)::value;
         constexpr bool DO_READ = decltype(readc)::value, WR = decltype(wrc)::value, LD = decltype(ldc)::value;
-        constexpr std::integral_constant<bool, WR && !LD> last{};            // what is written to LDS is the last slab: no further one is requested
         constexpr int P0 = decltype(p0c)::value, NP = decltype(p1c)::value - P0;
         constexpr int NR = DO_READ ? RD_A + RD_B : 0;
         static_for<0, NMFMA>([&](auto qc) {
@@ -408,11 +421,11 @@ __device__ __forceinline__ void gemm_mfma16_block(const GemmArgs& g, int tiles_m
                 }
                 if constexpr (j == 1 || j == 3) {
                     constexpr int p = P0 + i * PPR + (j == 3 ? 1 : 0);
-                    if constexpr (WR && (j == 1 || PPR == 2) && p < P0 + NP) store_piece(wr_stage, std::integral_constant<int, p>{}, last);
+                    if constexpr (WR && (j == 1 || PPR == 2) && p < P0 + NP) store_piece(wr_stage, setc, std::integral_constant<int, p>{});
                 }
                 if constexpr (j == 4 || j == 5) {
                     constexpr int p = P0 + i * PPR + (j == 5 ? 1 : 0);
-                    if constexpr (LD && (j == 4 || PPR == 2) && p < P0 + NP) load_piece(std::integral_constant<int, p>{});
+                    if constexpr (LD && (j == 4 || PPR == 2) && p < P0 + NP) load_piece(setc, std::integral_constant<int, p>{});
                 }
             }
             if constexpr (A_SLOTS == 1) {
@@ -423,18 +436,18 @@ __device__ __forceinline__ void gemm_mfma16_block(const GemmArgs& g, int tiles_m
                 constexpr int D = NMFMA - 1;
                 if constexpr (q < D) {
                     static_for<P0 + (NP * q) / D, P0 + (NP * (q + 1)) / D>([&](auto pc) {
-                        if constexpr (WR) store_piece(wr_stage, pc, last);
+                        if constexpr (WR) store_piece(wr_stage, setc, pc);
                     });
                 }
                 if constexpr (q > 0) {
                     static_for<P0 + (NP * (q - 1)) / D, P0 + (NP * q) / D>([&](auto pc) {
-                        if constexpr (LD) load_piece(pc);
+                        if constexpr (LD) load_piece(setc, pc);
                     });
                 }
             } else {
                 static_for<P0 + (NP * q) / NMFMA, P0 + (NP * (q + 1)) / NMFMA>([&](auto pc) {
-                    if constexpr (WR) store_piece(wr_stage, pc, last);
-                    if constexpr (LD) load_piece(pc);
+                    if constexpr (WR) store_piece(wr_stage, setc, pc);
+                    if constexpr (LD) load_piece(setc, pc);
                 });
             }
             __builtin_amdgcn_sched_barrier(0);
@@ -444,27 +457,29 @@ __device__ __forceinline__ void gemm_mfma16_block(const GemmArgs& g, int tiles_m
     int cur = 0;
     // Slab traffic is spread over the three k-steps that precede the barrier.
     constexpr int NP_ALL = NA + NB, CUT1 = (NP_ALL + 2) / 3, CUT2 = (2 * NP_ALL + 2) / 3;
-    // One slab of the pipeline.  NEXT: slab s+1 exists (its registers are written to LDS here and the barrier runs);
-    // NEXT2: slab s+2 exists (its global loads are issued here).
-    auto slab_step = [&](int s, auto next_tag, auto next2_tag) {
-        constexpr bool NEXT = decltype(next_tag)::value;
+    // One slab of the pipeline.  NEXT: register set `setc`, which holds slab s+1, is written to LDS and the barrier runs.
+    // FETCH: the global loads of slab s+1+PF into that set are issued.
+    auto slab_step = [&](auto setc, int s, auto next_tag, auto fetch_tag) {
+        constexpr bool NEXT = decltype(next_tag)::value, FETCH = decltype(fetch_tag)::value;
+        using no = std::false_type;
         using C0 = std::integral_constant<int, 0>;
         using C1 = std::integral_constant<int, CUT1>;
         using C2 = std::integral_constant<int, CUT2>;
         using C3 = std::integral_constant<int, NP_ALL>;
         const uint16_t* stage = smem + cur * STAGE;
         uint16_t* other = smem + (cur ^ 1) * STAGE;
-        if constexpr (decltype(next2_tag)::value) point_at_slab((s + 2) * M16_BK);
+        if constexpr (FETCH) point_at_slab(s + 1 + PF);
+        if constexpr (EDGE == M16_RAGGED && NEXT && !FETCH) pull_into_place(setc);        // nothing more to request: slab s+1 is the last one
         if constexpr (NKS == 4) {
-            kstep(I0{}, I1{}, std::true_type{}, C0{}, C1{}, next_tag, next2_tag, stage, other);
-            kstep(I1{}, I2{}, std::true_type{}, C1{}, C2{}, next_tag, next2_tag, stage, other);
-            kstep(I0{}, I3{}, std::true_type{}, C2{}, C3{}, next_tag, next2_tag, stage, other);
+            kstep(setc, I0{}, I1{}, std::true_type{}, C0{}, C1{}, next_tag, fetch_tag, stage, other);
+            kstep(setc, I1{}, I2{}, std::true_type{}, C1{}, C2{}, next_tag, fetch_tag, stage, other);
+            kstep(setc, I0{}, I3{}, std::true_type{}, C2{}, C3{}, next_tag, fetch_tag, stage, other);
         } else {
             // two k-steps of 32: the first carries all of the slab traffic (it is as long as two of the others)
-            kstep(I0{}, I1{}, std::true_type{}, C0{}, C3{}, next_tag, next2_tag, stage, other);
+            kstep(setc, I0{}, I1{}, std::true_type{}, C0{}, C3{}, next_tag, fetch_tag, stage, other);
         }
         if constexpr (NEXT) __syncthreads();
-        kstep(I1{}, I0{}, next_tag, C0{}, C0{}, std::false_type{}, std::false_type{}, other, other);
+        kstep(setc, I1{}, I0{}, next_tag, C0{}, C0{}, no{}, no{}, other, other);
         a_slab += a_step;
         advance_b();
         cur ^= 1;
@@ -472,10 +487,19 @@ __device__ __forceinline__ void gemm_mfma16_block(const GemmArgs& g, int tiles_m
 
     using yes = std::true_type;
     using no = std::false_type;
-    int s = 0;
-    for (; s + 2 < nslabs; s++) slab_step(s, yes{}, yes{});
-    if (s + 1 < nslabs) { slab_step(s, yes{}, no{}); s++; }
-    slab_step(s, no{}, no{});
+    if constexpr (PF == 1) {
+        int s = 0;
+        for (; s + 2 < nslabs; s++) slab_step(I0{}, s, yes{}, yes{});
+        if (s + 1 < nslabs) { slab_step(I0{}, s, yes{}, no{}); s++; }
+        slab_step(I0{}, s, no{}, no{});
+    } else {
+        static_assert(MT == 32 && EDGE != M16_RAGGED, "the in-place MFMAs need the loop above, the last slab of ragged rows a step of its own");
+        // Whole rounds of PF steps, in which the register sets take turns.  Where nslabs is not 1 more than a multiple of PF the
+        // last steps multiply slabs of zeros: leaving the round early would make the compiler wait for all loads at every step.
+        for (int s = 0; s + 1 < nslabs; s += PF)
+            static_for<0, PF>([&](auto uc) { slab_step(std::integral_constant<int, (decltype(uc)::value + 1) % PF>{}, s + decltype(uc)::value, yes{}, yes{}); });
+        slab_step(I0{}, nslabs, no{}, no{});
+    }
 
     if constexpr (MT == 16) asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");      // the in-place MFMAs above are opaque to the compiler: let the last ones drain before their results are read
     // ---- epilogue ----
@@ -635,15 +659,15 @@ __device__ __forceinline__ void gemm_mfma16_block(const GemmArgs& g, int tiles_m
     }   // tiles of this workgroup
 }
 
-template <typename T, int BM, int BN, int WGM, bool A_MC, bool B_MC, int EDGE, bool SPLITK>
-__global__ void __launch_bounds__(256) gemm_mfma16_kernel(GemmArgs g, int tiles_m, int tiles_n, float* partials, int k_per_split, int sched_total) {
+template <typename T, int BM, int BN, int WGM, bool A_MC, bool B_MC, int EDGE, bool SPLITK, int PF>
+__global__ void __launch_bounds__(256, m16_blocks_per_cu(BM, BN, EDGE, PF)) gemm_mfma16_kernel(GemmArgs g, int tiles_m, int tiles_n, float* partials, int k_per_split, int sched_total) {
     int first_slot, z;
     batched_block(tiles_m, tiles_n, first_slot, z);
-    gemm_mfma16_block<T, BM, BN, WGM, A_MC, B_MC, EDGE, SPLITK>(g, tiles_m, tiles_n, partials, k_per_split, sched_total, first_slot, z, (int)gridDim.x);
+    gemm_mfma16_block<T, BM, BN, WGM, A_MC, B_MC, EDGE, SPLITK, PF>(g, tiles_m, tiles_n, partials, k_per_split, sched_total, first_slot, z, (int)gridDim.x);
 }
 
 // Launch one instantiation.  nsplit > 1 selects the split-k variant: partials must hold batch * nsplit * m * n floats.
-template <typename T, int BM, int BN, int WGM, bool A_MC, bool B_MC, int EDGE, bool SPLITK>
+template <typename T, int BM, int BN, int WGM, bool A_MC, bool B_MC, int EDGE, bool SPLITK, int PF = 1>
 static int m16_launch(const GemmArgs& g, float* partials, int nsplit, int k_per_split) {
     int tiles_m = (g.m + BM - 1) / BM, tiles_n = (g.n + BN - 1) / BN;
     const int sched_total = scheduled_grid(tiles_m, tiles_n);
@@ -655,24 +679,27 @@ static int m16_launch(const GemmArgs& g, float* partials, int nsplit, int k_per_
     }
     dim3 grid(blocks, g.batch, SPLITK ? nsplit : 1);
     size_t smem = m16_smem_bytes(BM, BN, WGM, A_MC, B_MC, (!SPLITK && g.k <= M16_BK) ? 1 : 2, SPLITK ? 32 : m16_mfma_tile(BM, BN));
-    auto kern = gemm_mfma16_kernel<T, BM, BN, WGM, A_MC, B_MC, EDGE, SPLITK>;
+    auto kern = gemm_mfma16_kernel<T, BM, BN, WGM, A_MC, B_MC, EDGE, SPLITK, PF>;
     if (smem > 64 * 1024 && !check_hip(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem), "hipFuncSetAttribute")) return -1;
     hipLaunchKernelGGL(kern, grid, dim3(256), smem, current_stream(), g, tiles_m, tiles_n, partials, k_per_split, sched_total);
     return check_launch("gemm_mfma16_kernel") ? 0 : -1;
 }
 
 // Layout and edge dispatch for one tile shape (no split-k).
-template <typename T, int BM, int BN, int WGM, int EDGE>
+template <typename T, int BM, int BN, int WGM, int EDGE, int PF = 1>
 static int m16_launch_layout(const GemmArgs& g, const Plan& p) {
-    if (!p.a_mc && p.b_mc) return m16_launch<T, BM, BN, WGM, false, true, EDGE, false>(g, nullptr, 1, 0);
-    if (!p.a_mc && !p.b_mc) return m16_launch<T, BM, BN, WGM, false, false, EDGE, false>(g, nullptr, 1, 0);
-    if (p.a_mc && p.b_mc) return m16_launch<T, BM, BN, WGM, true, true, EDGE, false>(g, nullptr, 1, 0);
-    return m16_launch<T, BM, BN, WGM, true, false, EDGE, false>(g, nullptr, 1, 0);
+    if (!p.a_mc && p.b_mc) return m16_launch<T, BM, BN, WGM, false, true, EDGE, false, PF>(g, nullptr, 1, 0);
+    if (!p.a_mc && !p.b_mc) return m16_launch<T, BM, BN, WGM, false, false, EDGE, false, PF>(g, nullptr, 1, 0);
+    if (p.a_mc && p.b_mc) return m16_launch<T, BM, BN, WGM, true, true, EDGE, false, PF>(g, nullptr, 1, 0);
+    return m16_launch<T, BM, BN, WGM, true, false, EDGE, false, PF>(g, nullptr, 1, 0);
 }
 
 template <typename T, int BM, int BN, int WGM>
 static int m16_launch_tile(const GemmArgs& g, const Plan& p) {
     if (p.ragged) return m16_launch_layout<T, BM, BN, WGM, M16_RAGGED>(g, p);
+    if constexpr (BM == 64 && BN == 64) {
+        if (m16_deep(g.k)) return p.edge ? m16_launch_layout<T, BM, BN, WGM, M16_EDGE, M16_DEEP_SETS>(g, p) : m16_launch_layout<T, BM, BN, WGM, M16_WHOLE, M16_DEEP_SETS>(g, p);
+    }
     if (p.edge) return m16_launch_layout<T, BM, BN, WGM, M16_EDGE>(g, p);
     return m16_launch_layout<T, BM, BN, WGM, M16_WHOLE>(g, p);
 }

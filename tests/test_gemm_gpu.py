@@ -592,6 +592,22 @@ def test_ragged_rows(dt, batch, m, k, n, kernel, layout):
         dc.free()
 
 
+@pytest.mark.parametrize("layout", LAYOUTS)
+@pytest.mark.parametrize("dt", HALF, ids=lambda d: NAMES[d])
+@pytest.mark.parametrize("m,k,n", [(64, 704, 128), (64, 768, 128), (128, 832, 64), (64, 896, 192), (72, 712, 136), (136, 776, 200), (200, 840, 72), (8, 904, 72), (64, 961, 129), (130, 1535, 66)])
+def test_deep_prefetch_small_tiles(m, k, n, dt, layout):
+    """64 x 64 tiles around the number of k slabs from which three of them travel at a time, for every remainder of the slabs by
+    three, whole and hanging over; sums of small integers, so every slab must be added exactly once."""
+    rng = np.random.default_rng(m * 7 + k + n)
+    a = oracle.to_storage(rng.integers(-2, 3, (m, k) if layout[0] == "n" else (k, m)).astype(np.float64), dt)
+    b = oracle.to_storage(rng.integers(-2, 3, (k, n) if layout[1] == "n" else (n, k)).astype(np.float64), dt)
+    av, bv = (a if layout[0] == "n" else a.T), (b if layout[1] == "n" else b.T)
+    bias = oracle.to_storage(rng.integers(-3, 4, n).astype(np.float64), dt)
+    got = device_gemm(av, bv, dt, bias=bias)
+    # sums of at most 1535 products of at most 4 in magnitude whose spread is about 80: rounded to 16 bits once, then the bias once
+    assert np.array_equal(got, oracle_gemm(av, bv, dt, bias=bias))
+
+
 @pytest.mark.parametrize("dt", ALL, ids=lambda d: NAMES[d])
 @pytest.mark.parametrize("m,n", [(256, 784), (251, 785), (4096, 9), (9, 4096), (128, 96)])
 def test_outer_products(dt, m, n):
