@@ -326,6 +326,8 @@ __global__ void channel_sums_finish_kernel(T* out, const typename traits<T>::acc
 }
 
 // ---- convolution without a lowered matrix (stride 1, "same" padding) ----
+// 16-bit images go to the kernels that read them in place (rp_conv_direct.hip) where those take the shape; what follows is for
+// fp32 and fp64, wide rows, taps other than k x 3 and k x 5, and outputs that overlap their input.
 // With the image copied once into planes of pitch Wp >= W + 2 * pad with a zero border, output position f = oh * Wp + ow
 // of tap (kh, kw) reads padded element f + kh * Wp + kw: every tap is the same matrix [C, H * Wp] at a different
 // offset, which the GEMM reads in place as a segment of its k axis (GemmArgs::seg_*).  The product comes out in the
@@ -636,6 +638,13 @@ static int same_conv_backward(void* dx, void* dw, const void* dy, const void* x,
     return ok ? 0 : -1;
 }
 
+// Whether the kernels that read the image in place may write `out` while `in` is being read (the padded-plane path copies it first)
+static bool images_apart(const void* out, int out_channels, const void* in, int in_channels, int batch, int H, int W, int dtype) {
+    const size_t plane = (size_t)batch * H * W * dtype_size(dtype);
+    const char *o = (const char*)out, *i = (const char*)in;
+    return o + plane * out_channels <= i || i + plane * in_channels <= o;
+}
+
 static bool geom_ok(const ConvGeom& g) {
     if (g.N <= 0 || g.C <= 0 || g.H <= 0 || g.W <= 0 || g.kH <= 0 || g.kW <= 0 || g.sh <= 0 || g.sw <= 0 || g.ph < 0 || g.pw < 0 ||
         g.dh <= 0 || g.dw <= 0 || g.oH <= 0 || g.oW <= 0) return false;
@@ -772,6 +781,8 @@ int rp_hip_conv2d_same_forward(void* y, const void* x, const void* w, const void
     }
     const size_t esz = dtype_size(dtype);
     if (((uintptr_t)x | (uintptr_t)y) & (esz - 1)) { set_error("rp_hip_conv2d_same_forward: misaligned operand"); return -1; }
+    if (conv_taps16_takes(batch, C_in, C_out, H, W, kH, kW, dtype) && images_apart(y, C_out, x, C_in, batch, H, W, dtype))
+        return launch_conv_taps16(y, x, w, bias, batch, C_in, C_out, H, W, kH, kW, false, dtype);
     RP_DISPATCH_DTYPE(dtype, return same_conv<T>(y, x, w, bias, batch, C_in, C_out, H, W, kH, kW, false, dtype));
     return -1;
 }
@@ -782,6 +793,8 @@ int rp_hip_conv2d_same_backward_input(void* dx, const void* dy, const void* w, i
         set_error("rp_hip_conv2d_same_backward_input: null operand or a shape outside rp_hip_conv2d_same_supported");
         return -1;
     }
+    if (conv_taps16_takes(batch, C_out, C_in, H, W, kH, kW, dtype) && images_apart(dx, C_in, dy, C_out, batch, H, W, dtype))
+        return launch_conv_taps16(dx, dy, w, nullptr, batch, C_out, C_in, H, W, kH, kW, true, dtype);
     RP_DISPATCH_DTYPE(dtype, return same_conv_backward<T>(dx, nullptr, dy, nullptr, w, batch, C_in, H, W, C_out, kH, kW, dtype));
     return -1;
 }
@@ -793,6 +806,15 @@ int rp_hip_conv2d_same_backward(void* dx, void* dw, const void* dy, const void* 
         set_error("rp_hip_conv2d_same_backward: null operand or a shape outside rp_hip_conv2d_same_supported");
         return -1;
     }
+    // each gradient on its own kernel, dX first; whatever neither takes goes through the padded planes together
+    const bool direct_dx = dx && conv_taps16_takes(batch, C_out, C_in, H, W, kH, kW, dtype) && images_apart(dx, C_in, dy, C_out, batch, H, W, dtype);
+    const bool direct_dw = dw && conv_dw16_takes(batch, C_in, C_out, H, W, kH, kW, dtype) && (!dx || direct_dx);
+    if (direct_dx) {
+        if (launch_conv_taps16(dx, dy, w, nullptr, batch, C_out, C_in, H, W, kH, kW, true, dtype) != 0) return -1;
+        dx = nullptr;
+    }
+    if (direct_dw) return launch_conv_dw16(dw, dy, x, batch, C_in, C_out, H, W, kH, kW, dtype);
+    if (!dx && !dw) return 0;
     RP_DISPATCH_DTYPE(dtype, return same_conv_backward<T>(dx, dw, dy, x, w, batch, C_in, H, W, C_out, kH, kW, dtype));
     return -1;
 }

@@ -232,6 +232,11 @@ int launch_pipe16k(const GemmArgs& g, int dtype);
 bool pipe32k_takes(const GemmArgs& g);         // and its fp32 twin
 int launch_pipe32k(const GemmArgs& g);
 int launch_gemm_segmented_b(const GemmArgs& g, int dtype);
+// 16-bit same-padding convolutions straight from the image (rp_conv_direct.hip); outputs must not overlap the images they are read from
+bool conv_taps16_takes(int batch, int C_from, int C_to, int H, int W, int kH, int kW, int dtype);
+int launch_conv_taps16(void* out, const void* in, const void* w, const void* bias, int batch, int C_from, int C_to, int H, int W, int kH, int kW, bool for_input_grad, int dtype);
+bool conv_dw16_takes(int batch, int C_in, int C_out, int H, int W, int kH, int kW, int dtype);
+int launch_conv_dw16(void* dw, const void* dy, const void* x, int batch, int C_in, int C_out, int H, int W, int kH, int kW, int dtype);
 int launch_linear_backward_tiny(const GemmArgs& gx, const GemmArgs& gw, void* db, const void* dy, int rows, int cols, int accumulate_db);
 // adds k-split partials [g.batch][nsplit][part_rows][n] (fp32, rows beyond g.m unused) in split order and runs the epilogue into C
 int launch_splitk_combine(const GemmArgs& g, const float* partials, int nsplit, int part_rows, int dtype);

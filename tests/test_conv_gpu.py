@@ -169,6 +169,54 @@ def test_same_convolution_without_lowered_matrix(dt, case):
         assert np.array_equal(both_x.numpy(), dgx_.numpy()) and np.array_equal(both_w.numpy(), dgw_.numpy())
 
 
+DIRECT_CASES = [  # (batch, C_in, H, W, C_out, kH, kW): rows of any width (whole fours, twos, odd), many small samples in a strip, strips
+                  # that begin inside a row, 64 and 256 positions a workgroup, channels and strips that end inside a tile
+    (11, 64, 7, 7, 64, 3, 3), (3, 128, 10, 6, 64, 5, 3), (2, 64, 3, 50, 128, 3, 5), (1, 64, 5, 127, 64, 3, 3), (2, 64, 2, 130, 64, 1, 3),
+    (64, 64, 32, 32, 64, 3, 3), (70, 64, 31, 31, 64, 3, 3), (66, 64, 30, 34, 64, 1, 5), (24, 64, 12, 300, 64, 3, 3), (1, 64, 1, 1, 64, 3, 3)]
+
+
+@pytest.mark.parametrize("dt", [F16, BF16], ids=lambda d: NAMES[d])
+@pytest.mark.parametrize("case", DIRECT_CASES, ids=lambda c: "x".join(map(str, c)))
+def test_same_convolution_from_the_image_is_exact_on_integers(dt, case):
+    """Small integers: every sum is an integer below 2^24, exact in fp32, so the results are that sum rounded once (the
+    forward's bias: rounded again), bit for bit."""
+    import torch
+    N, Ci, H, W, Co, kH, kW = case
+    L = capi.lib()
+    rng = np.random.default_rng(N + W)
+    ints = lambda *shape: rng.integers(-1, 2, shape).astype(np.float64)          # noqa: E731
+    x, w, b, g = ints(N, Ci, H, W), ints(Co, Ci, kH, kW), ints(Co), ints(N, Co, H, W)
+    dx_, dw_, db_, dg_ = (Dev(oracle.to_storage(v, dt), dt) for v in (x, w, b, g))
+    y, gx, gw = Dev.empty((N, Co, H, W), dt), Dev.empty((N, Ci, H, W), dt), Dev.empty((Co, Ci, kH, kW), dt)
+    capi.check(L.rp_hip_conv2d_same_forward(y.ptr, dx_.ptr, dw_.ptr, db_.ptr, N, Ci, H, W, Co, kH, kW, dt), "same forward")
+    capi.check(L.rp_hip_conv2d_same_backward(gx.ptr, gw.ptr, dg_.ptr, dx_.ptr, dw_.ptr, N, Ci, H, W, Co, kH, kW, dt), "same backward")
+    xt, wt, gt = (torch.tensor(v, dtype=torch.float32) for v in (x, w, g))       # sums of integers below 2^24: exact in any order
+    pad = (kH // 2, kW // 2)
+    want = oracle.to_storage(torch.nn.functional.conv2d(xt, wt, None, padding=pad).numpy(), dt)
+    want = oracle.to_storage(oracle.to_f64(want, dt) + b[None, :, None, None], dt)
+    assert np.array_equal(oracle.to_f64(y.numpy(), dt), oracle.to_f64(want, dt))
+    want = oracle.to_storage(torch.nn.grad.conv2d_input((N, Ci, H, W), wt, gt, padding=pad).numpy(), dt)
+    assert np.array_equal(oracle.to_f64(gx.numpy(), dt), oracle.to_f64(want, dt))
+    want = oracle.to_storage(torch.nn.grad.conv2d_weight(xt, (Co, Ci, kH, kW), gt, padding=pad).numpy(), dt)
+    assert np.array_equal(oracle.to_f64(gw.numpy(), dt), oracle.to_f64(want, dt))
+
+
+@pytest.mark.parametrize("dt", [F16, BF16], ids=lambda d: NAMES[d])
+def test_same_convolution_over_its_own_input(dt):
+    """An output that overlaps the image it is computed from: the image is copied first, as for any other convolution."""
+    N, C, H, W = 2, 64, 9, 12
+    L = capi.lib()
+    rng = np.random.default_rng(86)
+    x, w = rand_storage(rng, (N, C, H, W), dt), oracle.to_storage(rng.standard_normal((C, C, 3, 3)) * 0.2, dt)
+    dw_ = Dev(w, dt)
+    for call in (lambda out, img: L.rp_hip_conv2d_same_forward(out, img, dw_.ptr, None, N, C, H, W, C, 3, 3, dt),
+                 lambda out, img: L.rp_hip_conv2d_same_backward_input(out, img, dw_.ptr, N, C, H, W, C, 3, 3, dt)):
+        src, out = Dev(x, dt), Dev.empty((N, C, H, W), dt)
+        capi.check(call(out.ptr, src.ptr), "apart")
+        capi.check(call(src.ptr, src.ptr), "in place")
+        assert oracle.rel_err(oracle.to_f64(src.numpy(), dt), oracle.to_f64(out.numpy(), dt)) <= {BF16: 2.0 ** -8, F16: 2.0 ** -11}[dt]
+
+
 def test_same_convolution_in_chunks_of_the_batch(monkeypatch):
     """With room for two samples at a time a batch of five goes in three chunks: same bits as in one piece (the weight
     gradient adds its chunks in fp32 and rounds after each, so it is compared to tolerance)."""
