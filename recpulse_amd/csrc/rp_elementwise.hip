@@ -707,118 +707,121 @@ static int launch_column_sums(T* out, const T* grad, int rows, int cols, int acc
 }
 
 // ---- cross-entropy ----------------------------------------------------------------------
-// One block.  Threads stride the batch in chunks of blockDim rows; each computes its row's
-// log-softmax and softmax serially (class counts are small), writes the scaled gradient and
-// leaves -logp[target] in LDS; thread 0 adds every chunk's losses in batch order in fp64, as
-// the reference's host loop does (ops/ops.c:5342-5352).
-template <typename T>
-__global__ void cross_entropy_kernel(T* loss, T* grad, const T* logits, const int* targets,
-                                     int batch, int classes, T upstream, const T* upstream_dev) {
-    __shared__ double nll[kThreads];
+// Every reduction (0 none, 1 mean, 2 sum: reference ops/ops.h:109-111), on logits and on probabilities (reference
+// ops/ops.c:5545-5643, 5412-5543), value (loss: batch elements for 'none', one otherwise) and / or gradient.
+// `group` neighbouring lanes share a row (a power of two, about four classes a lane; VAL: classes a lane keeps in registers,
+// 0: it reads them again): one round trip to memory per row where a thread per row made one per class and pass.
+// upstream_dev: the gradient of the loss where it lives, batch elements for 'none', one otherwise.
+// The losses are added in double, as the reference's host loop does (ops/ops.c:5342-5352): a row's in its group's first
+// lane, lanes and waves pairwise; several workgroups leave their sums in `partial` for cross_entropy_finish_kernel.
+// What bounds it is that chain: 256 x 10 fp32 7.4 us with a thread per row in one workgroup, 4.0 now;
+// a training step whose loss has 280 x 571 logits 744 us and 52, one with 94 x 804 458 and 54.
+template <typename T, int VAL>
+__global__ void __launch_bounds__(1024) cross_entropy_kernel(T* loss, double* partial, T* grad, const T* x, const int* targets, int batch, int classes,
+                                                             int group, int reduction, int from_logits, T upstream, const T* upstream_dev) {
+    __shared__ double waves[16];
+    const int lane = threadIdx.x % group, rows = blockDim.x / group;
+    if (upstream_dev && reduction != 0) upstream *= upstream_dev[0];      // no host round trip
     double total = 0.0;
-    if (upstream_dev) upstream *= upstream_dev[0];           // the upstream gradient where it lives: no host round trip
-    for (int b0 = 0; b0 < batch; b0 += blockDim.x) {
-        int b = b0 + threadIdx.x;
-        if (b < batch) {
-            const T* row = logits + (size_t)b * classes;
-            T mx = lowest<T>();
-            for (int c = 0; c < classes; c++) mx = row[c] > mx ? row[c] : mx;
-            T sum = 0;
-            for (int c = 0; c < classes; c++) sum += rp_exp(row[c] - mx);
-            T lse = rp_log(sum);
-            int t = targets[b];
-            bool valid = (t >= 0 && t < classes);      // callers validate; a bad index poisons the loss instead of reading out of bounds
-            nll[threadIdx.x] = valid ? -(double)(row[t] - mx - lse) : (double)NAN;
-            if (grad) {
-                T sc = (T)1 / (T)batch;
-                for (int c = 0; c < classes; c++) {
-                    T p = rp_exp(row[c] - mx) / sum;
-                    if (c == t) p -= (T)1;
-                    p *= sc;
-                    grad[(size_t)b * classes + c] = p * upstream;
-                }
+    for (long long b0 = (long long)blockIdx.x * rows; b0 < batch; b0 += (long long)gridDim.x * rows) {
+        const int b = (int)(b0 + threadIdx.x / group);
+        if (b >= batch) continue;                            // (whole groups: the exchanges below stay inside one)
+        const T* row = x + (size_t)b * classes;
+        const int t = targets[b];
+        const bool valid = t >= 0 && t < classes;            // callers validate; a bad index poisons the loss instead of reading out of bounds
+        T v[VAL > 0 ? VAL : 1];
+        if constexpr (VAL > 0) {
+#pragma unroll
+            for (int i = 0; i < VAL; i++) {
+                const int c = lane + i * group;
+                v[i] = c < classes ? row[c] : lowest<T>();
             }
         }
-        if (!loss) continue;                           // gradient only: nobody needs the sum (uniform: no thread reaches the barriers)
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            const int lim = batch - b0 < (int)blockDim.x ? batch - b0 : (int)blockDim.x;
-            int i = 0;
-            for (; i + 16 <= lim; i += 16) {             // sixteen LDS reads in flight, the adds still one by one in batch order
-                double v[16];
+        const T xt = valid ? row[t] : (T)0;
+        auto each = [&](auto f) {                            // f(class, value) over this lane's classes
+            if constexpr (VAL > 0) {
 #pragma unroll
-                for (int u = 0; u < 16; u++) v[u] = nll[i + u];
-#pragma unroll
-                for (int u = 0; u < 16; u++) total += v[u];
+                for (int i = 0; i < VAL; i++) if (lane + i * group < classes) f(lane + i * group, v[i]);
+            } else {
+                for (int c = lane; c < classes; c += group) f(c, row[c]);
             }
-            for (; i < lim; i++) total += nll[i];
+        };
+        T mx = 0, sum = 1, logp = 0;
+        if (from_logits) {
+            mx = lowest<T>();
+            each([&](int, T y) { mx = y > mx ? y : mx; });
+            for (int o = 1; o < group; o *= 2) { const T y = __shfl_xor(mx, o); mx = y > mx ? y : mx; }
+            sum = 0;
+            each([&](int, T y) { sum += rp_exp(y - mx); });
+            for (int o = 1; o < group; o *= 2) sum += __shfl_xor(sum, o);
+            if (valid) logp = xt - mx - rp_log(sum);
+        } else if (valid) {
+            logp = rp_log(xt);
         }
-        __syncthreads();
+        if (lane == 0) {
+            total += valid ? -(double)logp : (double)NAN;
+            if (loss && reduction == 0) loss[b] = valid ? -logp : (T)NAN;
+        }
+        if (grad) {
+            const T up = reduction == 0 && upstream_dev ? upstream_dev[b] : upstream;
+            const T sc = (T)1 / (T)batch;
+            T* out = grad + (size_t)b * classes;
+            each([&](int c, T y) {
+                T g;
+                if (from_logits) { g = rp_exp(y - mx) / sum; if (c == t) g -= (T)1; }
+                else g = (c == t) ? (T)-1 / y : (T)0;
+                if (reduction == 1) g *= sc;
+                out[c] = g * up;
+            });
+        }
     }
-    if (threadIdx.x == 0 && loss) {
-        if (sizeof(T) == 8) loss[0] = (T)(total / (double)batch);
-        else { float f = (float)total; f /= (float)batch; loss[0] = (T)f; }
-    }
+    if (!loss || reduction == 0) return;                     // (uniform: no thread reaches the barrier)
+    for (int o = 1; o < 64; o *= 2) total += __shfl_xor(total, o);
+    if ((threadIdx.x & 63) == 0) waves[threadIdx.x >> 6] = total;
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    total = 0.0;
+    for (int w = 0; w < (int)(blockDim.x >> 6); w++) total += waves[w];
+    if (partial) { partial[blockIdx.x] = total; return; }
+    if (sizeof(T) == 8) loss[0] = (T)(reduction == 1 ? total / (double)batch : total);
+    else { float f = (float)total; if (reduction == 1) f /= (float)batch; loss[0] = (T)f; }
 }
 
-// The same with every reduction (0 none, 1 mean, 2 sum: reference ops/ops.h:109-111) and on probabilities as well as on
-// logits (reference ops/ops.c:5545-5643, 5412-5543).  loss: batch elements for 'none', one otherwise.  upstream_dev: the
-// gradient of the loss on the device, batch elements for 'none', one otherwise (grad only).
 template <typename T>
-__global__ void cross_entropy_any_kernel(T* loss, T* grad, const T* x, const int* targets, int batch, int classes,
-                                         int reduction, int from_logits, const T* upstream_dev) {
-    __shared__ double nll[kThreads];
+__global__ void __launch_bounds__(64) cross_entropy_finish_kernel(T* loss, const double* partial, int n, int batch, int reduction) {
     double total = 0.0;
-    for (int b0 = 0; b0 < batch; b0 += blockDim.x) {
-        int b = b0 + threadIdx.x;
-        if (b < batch) {
-            const T* row = x + (size_t)b * classes;
-            int t = targets[b];
-            bool valid = (t >= 0 && t < classes);      // callers validate; a bad index poisons the loss instead of reading out of bounds
-            T mx = 0, sum = 1, logp = 0;
-            if (from_logits) {
-                mx = lowest<T>();
-                for (int c = 0; c < classes; c++) mx = row[c] > mx ? row[c] : mx;
-                sum = 0;
-                for (int c = 0; c < classes; c++) sum += rp_exp(row[c] - mx);
-                if (valid) logp = row[t] - mx - rp_log(sum);
-            } else if (valid) {
-                logp = rp_log(row[t]);
-            }
-            nll[threadIdx.x] = valid ? -(double)logp : (double)NAN;
-            if (loss && reduction == 0) loss[b] = valid ? -logp : (T)NAN;
-            if (grad) {
-                const T up = upstream_dev[reduction == 0 ? b : 0];
-                const T sc = (T)1 / (T)batch;
-                for (int c = 0; c < classes; c++) {
-                    T g;
-                    if (from_logits) { g = rp_exp(row[c] - mx) / sum; if (c == t) g -= (T)1; }
-                    else g = (c == t) ? (T)-1 / row[c] : (T)0;
-                    if (reduction == 1) g *= sc;
-                    grad[(size_t)b * classes + c] = g * up;
-                }
-            }
+    for (int i = threadIdx.x; i < n; i += 64) total += partial[i];
+    for (int o = 1; o < 64; o *= 2) total += __shfl_xor(total, o);
+    if (threadIdx.x != 0) return;
+    if (sizeof(T) == 8) loss[0] = (T)(reduction == 1 ? total / (double)batch : total);
+    else { float f = (float)total; if (reduction == 1) f /= (float)batch; loss[0] = (T)f; }
+}
+
+template <typename T>
+static int launch_cross_entropy(T* loss, T* grad, const T* x, const int* targets, int batch, int classes, int reduction, int from_logits, T upstream, const T* upstream_dev) {
+    int group = 1;
+    while (group < 64 && group * 4 < classes) group *= 2;
+    auto run = [&](dim3 blocks, int threads, double* partial) {
+        hipStream_t s = current_stream();
+        if (classes <= 4 * group) hipLaunchKernelGGL((cross_entropy_kernel<T, 4>), blocks, dim3(threads), 0, s, loss, partial, grad, x, targets, batch, classes, group, reduction, from_logits, upstream, upstream_dev);
+        else if (classes <= 16 * group) hipLaunchKernelGGL((cross_entropy_kernel<T, 16>), blocks, dim3(threads), 0, s, loss, partial, grad, x, targets, batch, classes, group, reduction, from_logits, upstream, upstream_dev);
+        else hipLaunchKernelGGL((cross_entropy_kernel<T, 0>), blocks, dim3(threads), 0, s, loss, partial, grad, x, targets, batch, classes, group, reduction, from_logits, upstream, upstream_dev);
+        return check_launch("cross_entropy_kernel") ? 0 : -1;
+    };
+    const long long lanes = (long long)batch * group;
+    const int blocks = (int)((lanes + 255) / 256 < 1024 ? (lanes + 255) / 256 : 1024);
+    if (!loss || reduction == 0) return run(dim3(blocks), 256, nullptr);
+    // One sum over all rows: one workgroup while it takes that few passes over its lanes (a second launch costs as much as four of
+    // them), and where there is no memory for partial sums that no other stream could be using.
+    if (lanes > 4 * 1024) {
+        NullStreamScratch scratch((size_t)blocks * sizeof(double));
+        if (scratch.ptr) {
+            if (run(dim3(blocks), 256, (double*)scratch.ptr) != 0) return -1;
+            hipLaunchKernelGGL(cross_entropy_finish_kernel<T>, dim3(1), dim3(64), 0, nullptr, loss, (const double*)scratch.ptr, blocks, batch, reduction);
+            return check_launch("cross_entropy_finish_kernel") ? 0 : -1;
         }
-        if (!loss || reduction == 0) continue;         // uniform: no thread reaches the barriers
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            const int lim = batch - b0 < (int)blockDim.x ? batch - b0 : (int)blockDim.x;
-            int i = 0;
-            for (; i + 16 <= lim; i += 16) {             // sixteen LDS reads in flight, the adds one by one in batch order, in double (reference ops/ops.c:5342-5352)
-                double v[16];
-#pragma unroll
-                for (int u = 0; u < 16; u++) v[u] = nll[i + u];
-#pragma unroll
-                for (int u = 0; u < 16; u++) total += v[u];
-            }
-            for (; i < lim; i++) total += nll[i];
-        }
-        __syncthreads();
     }
-    if (threadIdx.x == 0 && loss && reduction != 0) {
-        if (sizeof(T) == 8) loss[0] = (T)(reduction == 1 ? total / (double)batch : total);
-        else { float f = (float)total; if (reduction == 1) f /= (float)batch; loss[0] = (T)f; }
-    }
+    return run(dim3(1), 1024, nullptr);
 }
 
 }  // namespace rp
@@ -1111,13 +1114,8 @@ int rp_hip_cross_entropy_mean(void* loss_out, void* grad_logits, const void* log
         set_error("rp_hip_cross_entropy_mean: float32 and float64 only");
         return -1;
     }
-    if (dtype == RP_DTYPE_FLOAT32)
-        hipLaunchKernelGGL(cross_entropy_kernel<float>, dim3(1), dim3(kThreads), 0, current_stream(), (float*)loss_out, (float*)grad_logits,
-                           (const float*)logits, targets, batch, classes, (float)upstream, (const float*)nullptr);
-    else
-        hipLaunchKernelGGL(cross_entropy_kernel<double>, dim3(1), dim3(kThreads), 0, current_stream(), (double*)loss_out, (double*)grad_logits,
-                           (const double*)logits, targets, batch, classes, upstream, (const double*)nullptr);
-    return check_launch("cross_entropy_kernel") ? 0 : -1;
+    if (dtype == RP_DTYPE_FLOAT32) return launch_cross_entropy((float*)loss_out, (float*)grad_logits, (const float*)logits, targets, batch, classes, 1, 1, (float)upstream, (const float*)nullptr);
+    return launch_cross_entropy((double*)loss_out, (double*)grad_logits, (const double*)logits, targets, batch, classes, 1, 1, upstream, (const double*)nullptr);
 }
 
 int rp_hip_cross_entropy_backward(void* grad_logits, const void* logits, const int* targets, int batch, int classes,
@@ -1127,39 +1125,24 @@ int rp_hip_cross_entropy_backward(void* grad_logits, const void* logits, const i
         set_error("rp_hip_cross_entropy_backward: float32 and float64 only");
         return -1;
     }
-    if (dtype == RP_DTYPE_FLOAT32)
-        hipLaunchKernelGGL(cross_entropy_kernel<float>, dim3(1), dim3(kThreads), 0, current_stream(), (float*)nullptr, (float*)grad_logits,
-                           (const float*)logits, targets, batch, classes, 1.0f, (const float*)upstream_dev);
-    else
-        hipLaunchKernelGGL(cross_entropy_kernel<double>, dim3(1), dim3(kThreads), 0, current_stream(), (double*)nullptr, (double*)grad_logits,
-                           (const double*)logits, targets, batch, classes, 1.0, (const double*)upstream_dev);
-    return check_launch("cross_entropy_kernel") ? 0 : -1;
+    if (dtype == RP_DTYPE_FLOAT32) return launch_cross_entropy((float*)nullptr, (float*)grad_logits, (const float*)logits, targets, batch, classes, 1, 1, 1.0f, (const float*)upstream_dev);
+    return launch_cross_entropy((double*)nullptr, (double*)grad_logits, (const double*)logits, targets, batch, classes, 1, 1, 1.0, (const double*)upstream_dev);
 }
 
 int rp_hip_cross_entropy_forward(void* loss_out, const void* x, const int* targets, int batch, int classes,
                                  int reduction, int from_logits, int dtype) {
     RP_REQUIRE(loss_out && x && targets && batch > 0 && classes > 0 && reduction >= 0 && reduction <= 2, "rp_hip_cross_entropy_forward");
     if (dtype != RP_DTYPE_FLOAT32 && dtype != RP_DTYPE_FLOAT64) { set_error("rp_hip_cross_entropy_forward: float32 and float64 only"); return -1; }
-    if (dtype == RP_DTYPE_FLOAT32)
-        hipLaunchKernelGGL(cross_entropy_any_kernel<float>, dim3(1), dim3(kThreads), 0, current_stream(), (float*)loss_out, (float*)nullptr,
-                           (const float*)x, targets, batch, classes, reduction, from_logits ? 1 : 0, (const float*)nullptr);
-    else
-        hipLaunchKernelGGL(cross_entropy_any_kernel<double>, dim3(1), dim3(kThreads), 0, current_stream(), (double*)loss_out, (double*)nullptr,
-                           (const double*)x, targets, batch, classes, reduction, from_logits ? 1 : 0, (const double*)nullptr);
-    return check_launch("cross_entropy_any_kernel") ? 0 : -1;
+    if (dtype == RP_DTYPE_FLOAT32) return launch_cross_entropy((float*)loss_out, (float*)nullptr, (const float*)x, targets, batch, classes, reduction, from_logits ? 1 : 0, 1.0f, (const float*)nullptr);
+    return launch_cross_entropy((double*)loss_out, (double*)nullptr, (const double*)x, targets, batch, classes, reduction, from_logits ? 1 : 0, 1.0, (const double*)nullptr);
 }
 
 int rp_hip_cross_entropy_grad(void* grad_x, const void* x, const int* targets, int batch, int classes,
                               int reduction, int from_logits, const void* upstream_dev, int dtype) {
     RP_REQUIRE(grad_x && x && targets && upstream_dev && batch > 0 && classes > 0 && reduction >= 0 && reduction <= 2, "rp_hip_cross_entropy_grad");
     if (dtype != RP_DTYPE_FLOAT32 && dtype != RP_DTYPE_FLOAT64) { set_error("rp_hip_cross_entropy_grad: float32 and float64 only"); return -1; }
-    if (dtype == RP_DTYPE_FLOAT32)
-        hipLaunchKernelGGL(cross_entropy_any_kernel<float>, dim3(1), dim3(kThreads), 0, current_stream(), (float*)nullptr, (float*)grad_x,
-                           (const float*)x, targets, batch, classes, reduction, from_logits ? 1 : 0, (const float*)upstream_dev);
-    else
-        hipLaunchKernelGGL(cross_entropy_any_kernel<double>, dim3(1), dim3(kThreads), 0, current_stream(), (double*)nullptr, (double*)grad_x,
-                           (const double*)x, targets, batch, classes, reduction, from_logits ? 1 : 0, (const double*)upstream_dev);
-    return check_launch("cross_entropy_any_kernel") ? 0 : -1;
+    if (dtype == RP_DTYPE_FLOAT32) return launch_cross_entropy((float*)nullptr, (float*)grad_x, (const float*)x, targets, batch, classes, reduction, from_logits ? 1 : 0, 1.0f, (const float*)upstream_dev);
+    return launch_cross_entropy((double*)nullptr, (double*)grad_x, (const double*)x, targets, batch, classes, reduction, from_logits ? 1 : 0, 1.0, (const double*)upstream_dev);
 }
 
 int rp_hip_fill_scaled(void* ptr, const void* scalar_dev, double scale, size_t size, int dtype) {

@@ -320,6 +320,40 @@ def test_cross_entropy(dt):
 
 
 @pytest.mark.parametrize("dt", [F32, F64], ids=lambda d: NAMES[d])
+@pytest.mark.parametrize("stream", [False, True], ids=["null-stream", "own-stream"])
+@pytest.mark.parametrize("batch,classes", [(1, 1), (3, 4), (65, 5), (1025, 3), (300, 65), (130, 256), (129, 257), (7, 1024), (9, 1025), (5, 3000), (1024, 1000), (70000, 2)])
+def test_cross_entropy_rows_shared_by_lanes(dt, batch, classes, stream):
+    """Around the changes of lanes per row, of classes a lane keeps and of one workgroup to many, values and gradients of the mean.
+    Bound: the oracle's sums run one class after the other (n roundings, error at most n eps in the worst case, sqrt(n) eps in
+    the usual one), exp and log are within two units in the last place each: (8 + 2 sqrt(n)) eps of the row's probabilities."""
+    rng = np.random.default_rng(batch + classes)
+    logits = oracle.to_storage(rng.normal(0, 3, (batch, classes)), dt)
+    t = rng.integers(0, classes, batch).astype(np.int32)
+    dl, dtg = Dev(logits, dt), capi.DeviceBuffer.from_numpy(t)
+    loss, grad = Dev.empty((1,), dt), Dev.empty((batch, classes), dt)
+    handle = ctypes.c_void_p()
+    if stream:
+        capi.check(L().rp_hip_stream_create(ctypes.byref(handle)), "stream")
+        capi.check(L().rp_hip_set_stream(handle), "set stream")
+    try:
+        capi.check(L().rp_hip_cross_entropy_mean(loss.ptr, grad.ptr, dl.ptr, dtg.ptr, batch, classes, 1.0, dt), "ce")
+        capi.synchronize()
+    finally:
+        if stream:
+            L().rp_hip_set_stream(None)
+    x = logits.astype(np.float64)
+    e = np.exp(x - x.max(1, keepdims=True))
+    p = e / e.sum(1, keepdims=True)
+    nll = -(x - x.max(1, keepdims=True) - np.log(e.sum(1, keepdims=True)))[np.arange(batch), t]
+    eps = np.finfo(np.float32 if dt == F32 else np.float64).eps
+    bound = (8 + 2 * np.sqrt(classes)) * eps
+    want = p.copy()
+    want[np.arange(batch), t] -= 1
+    assert abs(float(loss.numpy()[0]) - nll.mean()) <= bound * max(1.0, np.abs(x).max())
+    assert np.abs(grad.numpy() - want / batch).max() <= bound * 8 / batch
+
+
+@pytest.mark.parametrize("dt", [F32, F64], ids=lambda d: NAMES[d])
 def test_cross_entropy_backward_reads_the_upstream_gradient_on_the_device(dt):
     """Same gradient, bit for bit, as the entry that takes the upstream factor from the host."""
     rng = np.random.default_rng(49)
