@@ -369,6 +369,9 @@ static Span span_of(const void* p, int rows, int cols, long long rs, long long c
 }
 static bool overlap(const Span& a, const Span& b) { return a.lo < b.hi && b.lo < a.hi; }
 
+// Rows up to which the column sums of dY join the other gradients of a 16-bit layer: eight chunks of 256, some 6 us
+constexpr int LINEAR_DB_ROWS = 2048;
+
 // Whether dX and dW of a 16-bit Linear layer go out as one launch: both on the 64 x 64 tile (an output of under half a CU count
 // of 128 x 128 tiles) in the layouts of dense X and W, and neither gradient written over anything that the other product reads
 // (one launch after the other, dW over W was fine).  Larger tiles fill a CU by themselves and gain nothing from company.
@@ -467,7 +470,13 @@ int rp_hip_linear_backward(void* dx, void* dw, void* db, const void* dy, const v
     bool edge = false;
     if ((dtype == RP_DTYPE_BFLOAT16 || dtype == RP_DTYPE_FLOAT16) && dx && dw && linear_backward_pairs(gx, gw, dtype, edge)) {
         g_last_kernel = "linear_backward16_64x64";
-        if (launch_linear_backward16(gx, gw, edge, dtype) != 0) return -1;
+        // The bias gradient rides along unless it would be written over something that is still read (one launch after the other
+        // was fine), or its chain of chunks outlasts the products.
+        const Span b = span_of(db, 1, n, 0, 1, 2), dys = span_of(dy, m, n, n, 1, 2), ws = span_of(w, k, n, w_rs, w_cs, 2), xs = span_of(x, m, k, x_rs, x_cs, 2);
+        const Span dxs = span_of(dx, m, k, dx_rs, dx_cs, 2), dws = span_of(dw, k, n, dw_rs, dw_cs, 2);
+        const bool rides = db && m <= LINEAR_DB_ROWS && !(overlap(b, dys) || overlap(b, ws) || overlap(b, xs) || overlap(b, dxs) || overlap(b, dws));
+        if (launch_linear_backward16(gx, gw, rides ? db : nullptr, accumulate_db, edge, dtype) != 0) return -1;
+        if (rides) return 0;
     } else {
         if (dx && run_gemm(gx, dtype) != 0) return -1;
         if (dw && run_gemm(gw, dtype) != 0) return -1;

@@ -1,41 +1,103 @@
 // bf16 / fp16 MFMA GEMM, 64 x 64 block tile (2 x 2 waves).
+#include "rp_column_sums.h"
 #include "rp_gemm_mfma16_kernel.h"
 
 namespace rp {
 
 int launch_mfma16_64(const GemmArgs& g, const Plan& p, int dtype) { return m16_launch_tile_dtype<64, 64, 2>(g, p, dtype); }
 
-// Both matrix gradients of a Linear layer in one launch: the first workgroups compute dX = dY . W^T (k-contiguous operands), the
-// others dW = X^T . dY (free-index-contiguous ones), tile for tile what the two launches would do, so the same bits.
+// Column sums of one strip of 64 bytes' worth of columns by a workgroup of 256 threads, in the order of rp_column_sums.h: a chunk
+// of 256 rows at a time in LDS, its four runs added side by side, the next chunk on its way to registers meanwhile.
+struct BiasGradient {
+    void* out;
+    int cols, accumulate;
+    int blocks;              // workgroups it takes (0: no bias gradient)
+};
+template <typename T>
+struct StripSums {
+    using A = typename traits<T>::acc;
+    using Tile = ColumnTile<T, 64, COLSUM_CHUNK, 256, true>;
+    static constexpr int COLS = Tile::COLS, RUNS = COLSUM_CHUNK / COLSUM_RUN;
+    static constexpr size_t LDS = Tile::BYTES + RUNS * COLS * sizeof(A);
+    static __device__ void run(T* out, const T* grad, int rows, int cols, int accumulate, int strip, unsigned char* lds) {
+        T* tile = (T*)lds;
+        A* parts = (A*)(lds + Tile::BYTES);              // [run][column]
+        const int t = threadIdx.x, run = t / COLS, col = t % COLS, c0 = strip * COLS;
+        Tile regs;
+        regs.load(grad, 0, rows, c0, cols, t);
+        A s = 0;
+        for (int r = 0; r < rows; r += COLSUM_CHUNK) {
+            regs.store(tile, t);
+            __syncthreads();
+            if (r + COLSUM_CHUNK < rows) regs.load(grad, r + COLSUM_CHUNK, rows, c0, cols, t);
+            if (rows <= COLSUM_CHUNK) {                  // one chunk: all of its rows top to bottom
+                if (t < COLS)
+                    for (int q = 0; q * COLSUM_RUN < rows; q++)
+                        s = Tile::add(s, tile + Tile::row_offset(q * COLSUM_RUN), col, rows - q * COLSUM_RUN < COLSUM_RUN ? rows - q * COLSUM_RUN : COLSUM_RUN);
+            } else {
+                if (t < RUNS * COLS) {
+                    const int n = rows - r - run * COLSUM_RUN;
+                    parts[t] = n > 0 ? Tile::add(0, tile + Tile::row_offset(run * COLSUM_RUN), col, n < COLSUM_RUN ? n : COLSUM_RUN) : (A)0;
+                }
+                __syncthreads();
+                if (t < COLS) {
+                    A c = parts[t];
+#pragma unroll
+                    for (int q = 1; q < RUNS; q++) c += parts[q * COLS + t];
+                    s += c;
+                }
+            }
+            __syncthreads();
+        }
+        const int j = c0 + t;
+        if (t >= COLS || j >= cols) return;
+        T y = narrow<T>(s);
+        if (accumulate) y = narrow<T>(widen(out[j]) + widen(y));
+        out[j] = y;
+    }
+};
+
+// All gradients of a Linear layer in one launch: the first workgroups add up the columns of dY (their chain of chunks is the longest of
+// any), the next ones compute dX = dY . W^T (k-contiguous operands), the others dW = X^T . dY (free-index-contiguous ones), tile for
+// tile and chunk for chunk what separate launches would do, so the same bits.
 // A 64 x 64 tile is bound by the latency of its slab chain with one workgroup per CU (1024^3: 19.1 K cycles for 2.05 K of MFMA);
 // two or three of them share a CU's LDS, and the two products' chains run side by side.
-// bf16 layer of 1024 x 1024 x 1024 (bias too), forward and backward: 31.3 us with two launches, 24.6 with this one.
+// bf16 layer of 1024 x 1024 x 1024 (bias too), forward and backward: 31.3 us with a launch per gradient, 24.6 with the matrices in one,
+// 22.3 with three slabs in flight, 20.3 with the column sums in it too.
 template <typename T, int EDGE, int PF>
-__global__ void __launch_bounds__(256, m16_blocks_per_cu(64, 64, EDGE, PF)) linear_backward16_kernel(GemmArgs gx, GemmArgs gw, int x_tiles_m, int x_tiles_n, int w_tiles_m, int w_tiles_n, int x_slots, int w_slots) {
-    const int b = blockIdx.x;
-    if (b < x_slots) gemm_mfma16_block<T, 64, 64, 2, false, false, EDGE, false, PF>(gx, x_tiles_m, x_tiles_n, nullptr, 0, x_slots, b, 0, x_slots);
+__global__ void __launch_bounds__(256, m16_blocks_per_cu(64, 64, EDGE, PF)) linear_backward16_kernel(GemmArgs gx, GemmArgs gw, BiasGradient db, int x_tiles_m, int x_tiles_n, int w_tiles_m, int w_tiles_n, int x_slots, int w_slots) {
+    const int b = (int)blockIdx.x - db.blocks;
+    if (b < 0) {
+        extern __shared__ __attribute__((aligned(16))) uint16_t smem[];
+        if ((int)blockIdx.x * StripSums<T>::COLS < db.cols) StripSums<T>::run((T*)db.out, (const T*)gx.A, gx.m, db.cols, db.accumulate, blockIdx.x, (unsigned char*)smem);
+    } else if (b < x_slots) gemm_mfma16_block<T, 64, 64, 2, false, false, EDGE, false, PF>(gx, x_tiles_m, x_tiles_n, nullptr, 0, x_slots, b, 0, x_slots);
     else gemm_mfma16_block<T, 64, 64, 2, true, true, EDGE, false, PF>(gw, w_tiles_m, w_tiles_n, nullptr, 0, w_slots, b - x_slots, 0, w_slots);
 }
 
 template <typename T, int EDGE, int PF>
-static int launch_linear_backward16_t(const GemmArgs& gx, const GemmArgs& gw) {
+static int launch_linear_backward16_t(const GemmArgs& gx, const GemmArgs& gw, void* db, int accumulate_db) {
     const int xm = (gx.m + 63) / 64, xn = (gx.n + 63) / 64, wm = (gw.m + 63) / 64, wn = (gw.n + 63) / 64;
     const int x_slots = scheduled_grid(xm, xn), w_slots = scheduled_grid(wm, wn);
     constexpr size_t x_smem = m16_smem_bytes(64, 64, 2, false, false, 2, 32), w_smem = m16_smem_bytes(64, 64, 2, true, true, 2, 32);
     constexpr size_t smem = x_smem > w_smem ? x_smem : w_smem;
+    static_assert(StripSums<T>::LDS <= smem, "the column sums use the tiles' LDS");
+    // whole rounds of the XCDs, so that the tiles' workgroups stay where the schedule wants them
+    const BiasGradient sums{db, gx.k, accumulate_db, db ? ((gx.k - 1) / StripSums<T>::COLS + 8) / 8 * 8 : 0};
     static_assert(smem <= 64 * 1024, "no attribute needed");
-    hipLaunchKernelGGL((linear_backward16_kernel<T, EDGE, PF>), dim3(x_slots + w_slots), dim3(256), smem, current_stream(), gx, gw, xm, xn, wm, wn, x_slots, w_slots);
+    hipLaunchKernelGGL((linear_backward16_kernel<T, EDGE, PF>), dim3(sums.blocks + x_slots + w_slots), dim3(256), smem, current_stream(), gx, gw, sums, xm, xn, wm, wn, x_slots, w_slots);
     return check_launch("linear_backward16_kernel") ? 0 : -1;
 }
 
 template <typename T>
-static int launch_linear_backward16_d(const GemmArgs& gx, const GemmArgs& gw, bool edge) {
-    if (m16_deep(gx.k) && m16_deep(gw.k)) return edge ? launch_linear_backward16_t<T, M16_EDGE, M16_DEEP_SETS>(gx, gw) : launch_linear_backward16_t<T, M16_WHOLE, M16_DEEP_SETS>(gx, gw);
-    return edge ? launch_linear_backward16_t<T, M16_EDGE, 1>(gx, gw) : launch_linear_backward16_t<T, M16_WHOLE, 1>(gx, gw);
+static int launch_linear_backward16_d(const GemmArgs& gx, const GemmArgs& gw, void* db, int accumulate_db, bool edge) {
+    if (m16_deep(gx.k) && m16_deep(gw.k))
+        return edge ? launch_linear_backward16_t<T, M16_EDGE, M16_DEEP_SETS>(gx, gw, db, accumulate_db) : launch_linear_backward16_t<T, M16_WHOLE, M16_DEEP_SETS>(gx, gw, db, accumulate_db);
+    return edge ? launch_linear_backward16_t<T, M16_EDGE, 1>(gx, gw, db, accumulate_db) : launch_linear_backward16_t<T, M16_WHOLE, 1>(gx, gw, db, accumulate_db);
 }
 
-int launch_linear_backward16(const GemmArgs& gx, const GemmArgs& gw, bool edge, int dtype) {
-    return dtype == RP_DTYPE_BFLOAT16 ? launch_linear_backward16_d<bf16_t>(gx, gw, edge) : launch_linear_backward16_d<f16_t>(gx, gw, edge);
+// gx.A is dY [gx.m, gx.k], dense; db: gx.k column sums of it, or null
+int launch_linear_backward16(const GemmArgs& gx, const GemmArgs& gw, void* db, int accumulate_db, bool edge, int dtype) {
+    return dtype == RP_DTYPE_BFLOAT16 ? launch_linear_backward16_d<bf16_t>(gx, gw, db, accumulate_db, edge) : launch_linear_backward16_d<f16_t>(gx, gw, db, accumulate_db, edge);
 }
 
 }  // namespace rp

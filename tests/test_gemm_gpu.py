@@ -719,6 +719,27 @@ def test_linear_backward_pair_16bit(dt, shape):
     assert np.array_equal(got_dx.numpy(), want_dx.numpy()) and np.array_equal(d_w.numpy(), want_dw.numpy())
 
 
+@pytest.mark.parametrize("dt", HALF, ids=lambda d: NAMES[d])
+@pytest.mark.parametrize("m,n", [(8, 8), (64, 72), (248, 40), (256, 264), (264, 32), (520, 1032), (2048, 136), (2056, 64)])
+def test_bias_gradient_beside_the_paired_gradients(dt, m, n):
+    """db in the launch of dX and dW (up to 2048 rows), around its chunks of rows and strips of columns: the bits of
+    rp_hip_reduce_rows, written and added; over W, which the launch still reads, it comes in a launch of its own."""
+    rng = np.random.default_rng(m + n)
+    L, k = capi.lib(), 64
+    x, w, dy, db0 = rand_storage(rng, (m, k), dt), rand_storage(rng, (k, n), dt), rand_storage(rng, (m, n), dt), rand_storage(rng, (n,), dt)
+    d_x, d_w, d_dy, d_dx, d_dw = Dev(x, dt), Dev(w, dt), Dev(dy, dt), Dev.empty((m, k), dt), Dev.empty((k, n), dt)
+    for acc in (0, 1):
+        want, got = Dev(db0, dt), Dev(db0, dt)
+        capi.check(L.rp_hip_reduce_rows(want.ptr, d_dy.ptr, m, n, acc, dt), "reduce_rows")
+        capi.check(L.rp_hip_linear_backward(d_dx.ptr, d_dw.ptr, got.ptr, d_dy.ptr, d_x.ptr, d_w.ptr, m, k, n, k, 1, n, 1, k, 1, n, 1, 0, 0, acc, dt), "backward")
+        assert L.rp_hip_last_gemm_kernel() == b"linear_backward16_64x64"
+        assert np.array_equal(got.numpy(), want.numpy())
+    want_dx = d_dx.numpy()
+    capi.check(L.rp_hip_linear_backward(d_dx.ptr, d_dw.ptr, d_w.ptr, d_dy.ptr, d_x.ptr, d_w.ptr, m, k, n, k, 1, n, 1, k, 1, n, 1, 0, 0, 0, dt), "db over W")
+    capi.check(L.rp_hip_reduce_rows(want.ptr, d_dy.ptr, m, n, 0, dt), "reduce_rows")
+    assert np.array_equal(d_dx.numpy(), want_dx) and np.array_equal(d_w.numpy().reshape(-1)[:n], want.numpy())
+
+
 def test_batch_longer_than_a_grid_axis():
     """70 000 tiny matrices in one call (the batch index rides on a grid axis of at most 65 535 blocks), A shared by
     all of them through a zero batch stride."""
