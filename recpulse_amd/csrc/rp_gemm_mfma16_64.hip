@@ -63,18 +63,19 @@ struct StripSums {
 // A 64 x 64 tile is bound by the latency of its slab chain with one workgroup per CU (1024^3: 19.1 K cycles for 2.05 K of MFMA);
 // two or three of them share a CU's LDS, and the two products' chains run side by side.
 // bf16 layer of 1024 x 1024 x 1024 (bias too), forward and backward: 31.3 us with a launch per gradient, 24.6 with the matrices in one,
-// 22.3 with three slabs in flight, 20.3 with the column sums in it too.
-template <typename T, int EDGE, int PF>
-__global__ void __launch_bounds__(256, m16_blocks_per_cu(64, 64, EDGE, PF)) linear_backward16_kernel(GemmArgs gx, GemmArgs gw, BiasGradient db, int x_tiles_m, int x_tiles_n, int w_tiles_m, int w_tiles_n, int x_slots, int w_slots) {
+// 21 with the column sums in it too.  (Three slabs in flight, as for a product with one workgroup per CU, give nothing here:
+// 768 x 768 x 768 8.6 us either way, 1280 x 768 x 1280 15.7 and 16.6.)
+template <typename T, int EDGE>
+__global__ void __launch_bounds__(256) linear_backward16_kernel(GemmArgs gx, GemmArgs gw, BiasGradient db, int x_tiles_m, int x_tiles_n, int w_tiles_m, int w_tiles_n, int x_slots, int w_slots) {
     const int b = (int)blockIdx.x - db.blocks;
     if (b < 0) {
         extern __shared__ __attribute__((aligned(16))) uint16_t smem[];
         if ((int)blockIdx.x * StripSums<T>::COLS < db.cols) StripSums<T>::run((T*)db.out, (const T*)gx.A, gx.m, db.cols, db.accumulate, blockIdx.x, (unsigned char*)smem);
-    } else if (b < x_slots) gemm_mfma16_block<T, 64, 64, 2, false, false, EDGE, false, PF>(gx, x_tiles_m, x_tiles_n, nullptr, 0, x_slots, b, 0, x_slots);
-    else gemm_mfma16_block<T, 64, 64, 2, true, true, EDGE, false, PF>(gw, w_tiles_m, w_tiles_n, nullptr, 0, w_slots, b - x_slots, 0, w_slots);
+    } else if (b < x_slots) gemm_mfma16_block<T, 64, 64, 2, false, false, EDGE, false, 1>(gx, x_tiles_m, x_tiles_n, nullptr, 0, x_slots, b, 0, x_slots);
+    else gemm_mfma16_block<T, 64, 64, 2, true, true, EDGE, false, 1>(gw, w_tiles_m, w_tiles_n, nullptr, 0, w_slots, b - x_slots, 0, w_slots);
 }
 
-template <typename T, int EDGE, int PF>
+template <typename T, int EDGE>
 static int launch_linear_backward16_t(const GemmArgs& gx, const GemmArgs& gw, void* db, int accumulate_db) {
     const int xm = (gx.m + 63) / 64, xn = (gx.n + 63) / 64, wm = (gw.m + 63) / 64, wn = (gw.n + 63) / 64;
     const int x_slots = scheduled_grid(xm, xn), w_slots = scheduled_grid(wm, wn);
@@ -84,20 +85,14 @@ static int launch_linear_backward16_t(const GemmArgs& gx, const GemmArgs& gw, vo
     // whole rounds of the XCDs, so that the tiles' workgroups stay where the schedule wants them
     const BiasGradient sums{db, gx.k, accumulate_db, db ? ((gx.k - 1) / StripSums<T>::COLS + 8) / 8 * 8 : 0};
     static_assert(smem <= 64 * 1024, "no attribute needed");
-    hipLaunchKernelGGL((linear_backward16_kernel<T, EDGE, PF>), dim3(sums.blocks + x_slots + w_slots), dim3(256), smem, current_stream(), gx, gw, sums, xm, xn, wm, wn, x_slots, w_slots);
+    hipLaunchKernelGGL((linear_backward16_kernel<T, EDGE>), dim3(sums.blocks + x_slots + w_slots), dim3(256), smem, current_stream(), gx, gw, sums, xm, xn, wm, wn, x_slots, w_slots);
     return check_launch("linear_backward16_kernel") ? 0 : -1;
-}
-
-template <typename T>
-static int launch_linear_backward16_d(const GemmArgs& gx, const GemmArgs& gw, void* db, int accumulate_db, bool edge) {
-    if (m16_deep(gx.k) && m16_deep(gw.k))
-        return edge ? launch_linear_backward16_t<T, M16_EDGE, M16_DEEP_SETS>(gx, gw, db, accumulate_db) : launch_linear_backward16_t<T, M16_WHOLE, M16_DEEP_SETS>(gx, gw, db, accumulate_db);
-    return edge ? launch_linear_backward16_t<T, M16_EDGE, 1>(gx, gw, db, accumulate_db) : launch_linear_backward16_t<T, M16_WHOLE, 1>(gx, gw, db, accumulate_db);
 }
 
 // gx.A is dY [gx.m, gx.k], dense; db: gx.k column sums of it, or null
 int launch_linear_backward16(const GemmArgs& gx, const GemmArgs& gw, void* db, int accumulate_db, bool edge, int dtype) {
-    return dtype == RP_DTYPE_BFLOAT16 ? launch_linear_backward16_d<bf16_t>(gx, gw, db, accumulate_db, edge) : launch_linear_backward16_d<f16_t>(gx, gw, db, accumulate_db, edge);
+    if (dtype == RP_DTYPE_BFLOAT16) return edge ? launch_linear_backward16_t<bf16_t, M16_EDGE>(gx, gw, db, accumulate_db) : launch_linear_backward16_t<bf16_t, M16_WHOLE>(gx, gw, db, accumulate_db);
+    return edge ? launch_linear_backward16_t<f16_t, M16_EDGE>(gx, gw, db, accumulate_db) : launch_linear_backward16_t<f16_t, M16_WHOLE>(gx, gw, db, accumulate_db);
 }
 
 }  // namespace rp

@@ -150,9 +150,11 @@ struct FragMap {
 // per CU of a small product nothing else covers it; three sets do (bf16, us, 1 set and 3: 1024^3 8.9 / 8.0, 256 x 4096 x 256 23.1 / 17.4,
 // 64 x 1024 x 4096 8.4 / 7.5).  The 128 x 128 tile gains nothing (2048^3 20.5 / 20.3: it is bound by what a CU can fetch from its L2,
 // 32 KB a slab at 39 B a cycle).  The loop runs whole rounds of PF slabs, up to two of them zeros, which a k of few slabs would feel
-// (600 x 264 x 600 6.4 / 6.9): from twelve slabs on.  Ragged rows stay at one set, their loads take twice the time to issue.
+// (600 x 264 x 600 6.4 / 6.9): from twelve slabs on.  Two workgroups on a CU cover each other's loads, and the registers of the sets get in
+// their way (fp16, us: 396 tiles of 2304 x 2880 x 704 25.0 / 30.0, 336 of 3584 x 5696 x 384 53.8 / 57.7; 256 of 2048 x 8192 x 512 63.1 / 38.6): up to one
+// tile per CU.  Ragged rows stay at one set, their loads take twice the time to issue.
 constexpr int M16_DEEP_SETS = 3;
-static inline bool m16_deep(int k) { return k > 11 * M16_BK; }
+static inline bool m16_deep(int k, long long tiles) { return k > 11 * M16_BK && tiles <= device_cu_count(); }
 
 // EDGE: what of the tile may hang over the problem.
 enum { M16_WHOLE = 0, M16_EDGE = 1, M16_RAGGED = 2 };
@@ -698,7 +700,7 @@ template <typename T, int BM, int BN, int WGM>
 static int m16_launch_tile(const GemmArgs& g, const Plan& p) {
     if (p.ragged) return m16_launch_layout<T, BM, BN, WGM, M16_RAGGED>(g, p);
     if constexpr (BM == 64 && BN == 64) {
-        if (m16_deep(g.k)) return p.edge ? m16_launch_layout<T, BM, BN, WGM, M16_EDGE, M16_DEEP_SETS>(g, p) : m16_launch_layout<T, BM, BN, WGM, M16_WHOLE, M16_DEEP_SETS>(g, p);
+        if (m16_deep(g.k, (long long)((g.m + BM - 1) / BM) * ((g.n + BN - 1) / BN) * g.batch)) return p.edge ? m16_launch_layout<T, BM, BN, WGM, M16_EDGE, M16_DEEP_SETS>(g, p) : m16_launch_layout<T, BM, BN, WGM, M16_WHOLE, M16_DEEP_SETS>(g, p);
     }
     if (p.edge) return m16_launch_layout<T, BM, BN, WGM, M16_EDGE>(g, p);
     return m16_launch_layout<T, BM, BN, WGM, M16_WHOLE>(g, p);
