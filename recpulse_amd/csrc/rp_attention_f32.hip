@@ -22,26 +22,34 @@ typedef __attribute__((ext_vector_type(4))) float f32x4v_t;
 
 __device__ __forceinline__ f32x16_t mma32(float a, float b, f32x16_t c) { return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0); }
 
-// A [32 rows][D] block of a d-contiguous float matrix in LDS.
-template <int D>
+// SPLIT (small grids): the workgroup owns 32 rows instead of 128, its four waves take every fourth block of 32 of the axis that is
+// walked, each in LDS of its own (a wave's LDS operations are executed in order: no barrier), and the four partial results
+// meet in LDS at the end.
+__device__ __forceinline__ void attn32_wave_order() {            // keeps the compiler from moving a wave's LDS accesses across
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// A [32 rows][D] block of a d-contiguous float matrix in LDS, staged by LANES threads: the workgroup, or a wave.
+template <int D, int LANES = 256>
 struct Blk32 {
     static constexpr int RP = D + 8;                                 // floats
     static constexpr int ELEMS = AT_KEYS * RP;
-    static constexpr int PIECES = AT_KEYS * D / 4 / 256;             // 16-byte pieces per thread
+    static constexpr int PIECES = AT_KEYS * D / 4 / LANES;           // 16-byte pieces per thread
     static_assert(PIECES >= 1, "a block is at least one piece per thread");
     static __device__ __forceinline__ void load(u32x4_t (&r)[PIECES], const float* M, long long rs, int row0, int rows, const char* end) {
         const char* p = (const char*)(M + (long long)row0 * rs);
         const __amdgpu_buffer_rsrc_t rsrc = buffer_rsrc(p, row0 < rows ? (long long)(end - p) : 0);      // rows past the end read zeros
 #pragma unroll
         for (int i = 0; i < PIECES; i++) {
-            const int id = threadIdx.x + 256 * i, row = id / (D / 4), d4 = (id % (D / 4)) * 4;
+            const int id = threadIdx.x % LANES + LANES * i, row = id / (D / 4), d4 = (id % (D / 4)) * 4;
             r[i] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)(((long long)row * rs + d4) * 4), 0, 0);
         }
     }
     static __device__ __forceinline__ void store(const u32x4_t (&r)[PIECES], float* stage) {
 #pragma unroll
         for (int i = 0; i < PIECES; i++) {
-            const int id = threadIdx.x + 256 * i, row = id / (D / 4), d4 = (id % (D / 4)) * 4;
+            const int id = threadIdx.x % LANES + LANES * i, row = id / (D / 4), d4 = (id % (D / 4)) * 4;
             *(u32x4_t*)(stage + row * RP + d4) = r[i];
         }
     }
@@ -85,6 +93,32 @@ __device__ __forceinline__ void product_over_rows(f32x16_t (&acc)[D / 32], const
     }
 }
 
+// SPLIT: a wave's 32 x D partial result (lane = row c, transposed accumulators) to its place in LDS, and thread t's share of the
+// sum of the four, weighted, in wave order: columns (t % 8) * D / 8 .. of row t / 8
+template <int D> constexpr int ATTN32_PART = D + 4;              // floats of a row of a partial result
+template <int D>
+__device__ __forceinline__ void put_part(float* parts, const f32x16_t (&acc)[D / 32], int wave, int c, int h) {
+    float* row = parts + (wave * 32 + c) * ATTN32_PART<D>;
+#pragma unroll
+    for (int dt = 0; dt < D / 32; dt++)
+#pragma unroll
+        for (int v4 = 0; v4 < 4; v4++) {
+            const f32x4v_t o = {acc[dt][4 * v4], acc[dt][4 * v4 + 1], acc[dt][4 * v4 + 2], acc[dt][4 * v4 + 3]};
+            *(f32x4v_t*)(row + 32 * dt + 8 * v4 + 4 * h) = o;
+        }
+}
+template <int D>
+__device__ __forceinline__ void write_sum_of_parts(float* out, const float* parts, const float (&weight)[4]) {
+    const int r = threadIdx.x / 8, d0 = (threadIdx.x % 8) * (D / 8);
+#pragma unroll
+    for (int i = 0; i < D / 32; i++) {
+        f32x4v_t sum = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int w = 0; w < 4; w++) sum += weight[w] * *(const f32x4v_t*)(parts + (w * 32 + r) * ATTN32_PART<D> + d0 + 4 * i);
+        *(f32x4v_t*)(out + d0 + 4 * i) = sum;
+    }
+}
+
 template <int D>
 __device__ __forceinline__ void write_rows_t(float* row, const f32x16_t (&acc)[D / 32], int h, float mul) {
     // the lane's column of the transposed accumulators is a row of the output: registers 4*v4 .. +3 are d = 32*dt + 8*v4 + 4h + (0..3)
@@ -97,18 +131,22 @@ __device__ __forceinline__ void write_rows_t(float* row, const f32x16_t (&acc)[D
         }
 }
 
-template <int D>
+template <int D, bool SPLIT>
 __global__ void __launch_bounds__(256, D <= 64 ? 2 : 1) attention_fwd32_kernel(AttnArgs g) {
     constexpr int KJ = D / 2, DT = D / 32;
-    using Blk = Blk32<D>;
-    __shared__ __attribute__((aligned(16))) float klds[2][Blk::ELEMS];
-    __shared__ __attribute__((aligned(16))) float vlds[2][Blk::ELEMS];
+    using Blk = Blk32<D, SPLIT ? 64 : 256>;
+    constexpr bool AHEAD = !SPLIT || D <= 64;        // the next block travels in registers meanwhile
+    extern __shared__ __attribute__((aligned(16))) float attn32_lds[];
+    // [stage of the workgroup, or wave][block]
+    float* const stages = attn32_lds + (SPLIT ? 2 * Blk::ELEMS * (threadIdx.x >> 6) : 0);
+    auto klds = [&](int stage) { return stages + stage * 2 * Blk::ELEMS; };
+    auto vlds = [&](int stage) { return stages + (stage * 2 + 1) * Blk::ELEMS; };
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int h = lane >> 5, c = lane & 31;
     int row_tile, z;
     attn_block(row_tile, z);
-    const int q0 = row_tile * AT_QROWS + wave * 32;
+    const int q0 = SPLIT ? row_tile * 32 : row_tile * AT_QROWS + wave * 32;
     const float* Q = (const float*)g.Q + (long long)z * g.q_bs;
     const float* K = (const float*)g.K + (long long)z * g.k_bs;
     const float* V = (const float*)g.V + (long long)z * g.v_bs;
@@ -130,23 +168,37 @@ __global__ void __launch_bounds__(256, D <= 64 ? 2 : 1) attention_fwd32_kernel(A
     float m_run = -INFINITY, l_run = 0.f;
 
     const int nblocks = (g.sk + AT_KEYS - 1) / AT_KEYS;
+    constexpr int STRIDE = SPLIT ? 4 : 1;            // blocks from one step to the next
+    const int first = SPLIT ? wave : 0;
     u32x4_t kr[Blk::PIECES], vr[Blk::PIECES];
-    Blk::load(kr, K, g.k_rs, 0, g.sk, k_end);
-    Blk::load(vr, V, g.v_rs, 0, g.sk, v_end);
-    Blk::store(kr, klds[0]); Blk::store(vr, vlds[0]);
-    Blk::load(kr, K, g.k_rs, AT_KEYS, g.sk, k_end);
-    Blk::load(vr, V, g.v_rs, AT_KEYS, g.sk, v_end);
-    __syncthreads();
+    auto request = [&](int blk) {                    // (blocks past the last one read zeros)
+        Blk::load(kr, K, g.k_rs, blk * AT_KEYS, g.sk, k_end);
+        Blk::load(vr, V, g.v_rs, blk * AT_KEYS, g.sk, v_end);
+    };
+    request(first);
+    if constexpr (!SPLIT) {
+        Blk::store(kr, klds(0)); Blk::store(vr, vlds(0));
+        request(1);
+        __syncthreads();
+    }
 
-    for (int blk = 0; blk < nblocks; blk++) {
-        const int kb = blk * AT_KEYS, cur = blk & 1;
+    for (int blk = first; blk < nblocks; blk += STRIDE) {
+        const int kb = blk * AT_KEYS, cur = SPLIT ? 0 : blk & 1;
+        if constexpr (SPLIT) {
+            attn32_wave_order();
+            if (!AHEAD && blk != first) request(blk);
+            Blk::store(kr, klds(0)); Blk::store(vr, vlds(0));
+            attn32_wave_order();
+            if (AHEAD) request(blk + STRIDE);
+        }
         f32x16_t st;
 #pragma unroll
         for (int v = 0; v < 16; v++) st[v] = 0.f;
-        st = product_over_d<D>(klds[cur], qf, c, h, st);                    // S^T: 32 keys x 32 queries
-        Blk::store(kr, klds[cur ^ 1]); Blk::store(vr, vlds[cur ^ 1]);       // everyone left that stage at the previous barrier
-        Blk::load(kr, K, g.k_rs, kb + 2 * AT_KEYS, g.sk, k_end);
-        Blk::load(vr, V, g.v_rs, kb + 2 * AT_KEYS, g.sk, v_end);
+        st = product_over_d<D>(klds(cur), qf, c, h, st);                    // S^T: 32 keys x 32 queries
+        if constexpr (!SPLIT) {
+            Blk::store(kr, klds(cur ^ 1)); Blk::store(vr, vlds(cur ^ 1));       // everyone left that stage at the previous barrier
+            request(blk + 2);
+        }
         if (flip) {
 #pragma unroll
             for (int v = 0; v < 16; v++) st[v] = -st[v];
@@ -183,11 +235,36 @@ __global__ void __launch_bounds__(256, D <= 64 ? 2 : 1) attention_fwd32_kernel(A
 #pragma unroll
                 for (int v = 0; v < 16; v++) ot[dt][v] *= alpha;
         }
-        product_over_rows<D>(ot, vlds[cur], e, c, h);       // O^T += V^T P^T
-        __syncthreads();
+        product_over_rows<D>(ot, vlds(cur), e, c, h);       // O^T += V^T P^T
+        if constexpr (!SPLIT) __syncthreads();
     }
 
     const float l_all = l_run + __shfl_xor(l_run, 32, 64);
+    if constexpr (SPLIT) {
+        // every wave has its own running maximum: weights exp2((m_w - m) sc) bring the parts together
+        __shared__ float m_of[4][32], l_of[4][32];
+        __syncthreads();                                    // every wave is done with its blocks
+        put_part<D>(attn32_lds, ot, wave, c, h);
+        if (h == 0) { m_of[wave][c] = m_run; l_of[wave][c] = l_all; }
+        __syncthreads();
+        const int r = threadIdx.x / 8, q = q0 + r;
+        if (q >= g.sq) return;
+        float m = m_of[0][r];
+#pragma unroll
+        for (int w = 1; w < 4; w++) m = fmaxf(m, m_of[w][r]);
+        float weight[4], l = 0.f;
+#pragma unroll
+        for (int w = 0; w < 4; w++) {
+            weight[w] = m_of[w][r] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((m_of[w][r] - m) * sc);       // (a wave without a block, or only masked keys)
+            l += weight[w] * l_of[w][r];
+        }
+        const float inv = l > 0.f ? 1.f / l : 0.f;
+#pragma unroll
+        for (int w = 0; w < 4; w++) weight[w] *= inv;
+        write_sum_of_parts<D>((float*)g.O + (long long)z * g.o_bs + (long long)q * g.o_rs, attn32_lds, weight);
+        if (g.L && threadIdx.x % 8 == 0) g.L[(long long)z * g.sq + q] = (m * sc + __builtin_amdgcn_logf(l)) * 0.693147180559945309f;
+        return;
+    }
     const float inv = l_all > 0.f ? 1.f / l_all : 0.f;
     const int q = q0 + c;
     if (q < g.sq) {
@@ -197,18 +274,22 @@ __global__ void __launch_bounds__(256, D <= 64 ? 2 : 1) attention_fwd32_kernel(A
 }
 
 // dQ: a wave owns 32 queries and walks the keys.
-template <int D>
+template <int D, bool SPLIT>
 __global__ void __launch_bounds__(256, D <= 64 ? 2 : 1) attention_bwd_dq32_kernel(AttnBwdArgs g) {
     constexpr int KJ = D / 2, DT = D / 32;
-    using Blk = Blk32<D>;
-    __shared__ __attribute__((aligned(16))) float klds[2][Blk::ELEMS];
-    __shared__ __attribute__((aligned(16))) float vlds[2][Blk::ELEMS];
+    using Blk = Blk32<D, SPLIT ? 64 : 256>;
+    constexpr bool AHEAD = !SPLIT || D <= 64;        // the next block travels in registers meanwhile
+    extern __shared__ __attribute__((aligned(16))) float attn32_lds[];
+    // [stage of the workgroup, or wave][block]
+    float* const stages = attn32_lds + (SPLIT ? 2 * Blk::ELEMS * (threadIdx.x >> 6) : 0);
+    auto klds = [&](int stage) { return stages + stage * 2 * Blk::ELEMS; };
+    auto vlds = [&](int stage) { return stages + (stage * 2 + 1) * Blk::ELEMS; };
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int h = lane >> 5, c = lane & 31;
     int row_tile, z;
     attn_block(row_tile, z);
-    const int q0 = row_tile * AT_QROWS + wave * 32;
+    const int q0 = SPLIT ? row_tile * 32 : row_tile * AT_QROWS + wave * 32;
     const float* Q = (const float*)g.Q + (long long)z * g.q_bs;
     const float* K = (const float*)g.K + (long long)z * g.k_bs;
     const float* V = (const float*)g.V + (long long)z * g.v_bs;
@@ -234,7 +315,7 @@ __global__ void __launch_bounds__(256, D <= 64 ? 2 : 1) attention_bwd_dq32_kerne
 #pragma unroll
         for (int j = 0; j < KJ; j++) dq_dot += dof[j] * of[j];
         dq_dot += __shfl_xor(dq_dot, 32, 64);
-        if (q < g.sq && h == 0) g.Dq[(long long)z * g.sq + q] = dq_dot;
+        if (q < g.sq && h == 0 && (!SPLIT || wave == 0)) g.Dq[(long long)z * g.sq + q] = dq_dot;
     }
     const float dq_dot_scaled = dq_dot * g.scale;
 
@@ -245,24 +326,38 @@ __global__ void __launch_bounds__(256, D <= 64 ? 2 : 1) attention_bwd_dq32_kerne
         for (int v = 0; v < 16; v++) acc[dt][v] = 0.f;
 
     const int nblocks = (g.sk + AT_KEYS - 1) / AT_KEYS;
+    constexpr int STRIDE = SPLIT ? 4 : 1;            // blocks from one step to the next
+    const int first = SPLIT ? wave : 0;
     u32x4_t kr[Blk::PIECES], vr[Blk::PIECES];
-    Blk::load(kr, K, g.k_rs, 0, g.sk, k_end);
-    Blk::load(vr, V, g.v_rs, 0, g.sk, v_end);
-    Blk::store(kr, klds[0]); Blk::store(vr, vlds[0]);
-    Blk::load(kr, K, g.k_rs, AT_KEYS, g.sk, k_end);
-    Blk::load(vr, V, g.v_rs, AT_KEYS, g.sk, v_end);
-    __syncthreads();
+    auto request = [&](int blk) {                    // (blocks past the last one read zeros)
+        Blk::load(kr, K, g.k_rs, blk * AT_KEYS, g.sk, k_end);
+        Blk::load(vr, V, g.v_rs, blk * AT_KEYS, g.sk, v_end);
+    };
+    request(first);
+    if constexpr (!SPLIT) {
+        Blk::store(kr, klds(0)); Blk::store(vr, vlds(0));
+        request(1);
+        __syncthreads();
+    }
 
-    for (int blk = 0; blk < nblocks; blk++) {
-        const int kb = blk * AT_KEYS, cur = blk & 1;
+    for (int blk = first; blk < nblocks; blk += STRIDE) {
+        const int kb = blk * AT_KEYS, cur = SPLIT ? 0 : blk & 1;
+        if constexpr (SPLIT) {
+            attn32_wave_order();
+            if (!AHEAD && blk != first) request(blk);
+            Blk::store(kr, klds(0)); Blk::store(vr, vlds(0));
+            attn32_wave_order();
+            if (AHEAD) request(blk + STRIDE);
+        }
         f32x16_t st, dp;
 #pragma unroll
         for (int v = 0; v < 16; v++) { st[v] = 0.f; dp[v] = 0.f; }
-        st = product_over_d<D>(klds[cur], qf, c, h, st);                    // S^T
-        dp = product_over_d<D>(vlds[cur], dof, c, h, dp);                   // dP^T
-        Blk::store(kr, klds[cur ^ 1]); Blk::store(vr, vlds[cur ^ 1]);
-        Blk::load(kr, K, g.k_rs, kb + 2 * AT_KEYS, g.sk, k_end);
-        Blk::load(vr, V, g.v_rs, kb + 2 * AT_KEYS, g.sk, v_end);
+        st = product_over_d<D>(klds(cur), qf, c, h, st);                    // S^T
+        dp = product_over_d<D>(vlds(cur), dof, c, h, dp);                   // dP^T
+        if constexpr (!SPLIT) {
+            Blk::store(kr, klds(cur ^ 1)); Blk::store(vr, vlds(cur ^ 1));
+            request(blk + 2);
+        }
         float ds[16];
 #pragma unroll
         for (int v = 0; v < 16; v++) {
@@ -274,26 +369,39 @@ __global__ void __launch_bounds__(256, D <= 64 ? 2 : 1) attention_bwd_dq32_kerne
             for (int v = 0; v < 16; v++)
                 if (kb + 8 * (v / 4) + 4 * h + (v % 4) >= g.sk) ds[v] = 0.f;
         }
-        product_over_rows<D>(acc, klds[cur], ds, c, h);                     // dQ^T += K^T dS^T
+        product_over_rows<D>(acc, klds(cur), ds, c, h);                     // dQ^T += K^T dS^T
+        if constexpr (!SPLIT) __syncthreads();
+    }
+    if constexpr (SPLIT) {
+        constexpr float ones[4] = {1.f, 1.f, 1.f, 1.f};
         __syncthreads();
+        put_part<D>(attn32_lds, acc, wave, c, h);
+        __syncthreads();
+        const int row = q0 + threadIdx.x / 8;
+        if (row < g.sq) write_sum_of_parts<D>((float*)g.dQ + ((long long)z * g.sq + row) * D, attn32_lds, ones);
+        return;
     }
     if (q < g.sq) write_rows_t<D>((float*)g.dQ + ((long long)z * g.sq + q) * D, acc, h, 1.f);
 }
 
 // dK and dV: a wave owns 32 keys and walks the queries.
-template <int D>
+template <int D, bool SPLIT>
 __global__ void __launch_bounds__(256, D <= 32 ? 2 : 1) attention_bwd_dkv32_kernel(AttnBwdArgs g) {
     constexpr int KJ = D / 2, DT = D / 32;
-    using Blk = Blk32<D>;
-    __shared__ __attribute__((aligned(16))) float qlds[2][Blk::ELEMS];
-    __shared__ __attribute__((aligned(16))) float dolds[2][Blk::ELEMS];
-    __shared__ __attribute__((aligned(16))) float rowlds[2][2][AT_KEYS];        // [stage][L, Dq * scale][query of the block]
+    using Blk = Blk32<D, SPLIT ? 64 : 256>;
+    constexpr bool AHEAD = !SPLIT || D <= 64;        // the next block travels in registers meanwhile
+    extern __shared__ __attribute__((aligned(16))) float attn32_lds[];
+    // [stage of the workgroup, or wave][block]
+    float* const stages = attn32_lds + (SPLIT ? 2 * Blk::ELEMS * (threadIdx.x >> 6) : 0);
+    auto qlds = [&](int stage) { return stages + stage * 2 * Blk::ELEMS; };
+    auto dolds = [&](int stage) { return stages + (stage * 2 + 1) * Blk::ELEMS; };
+    __shared__ __attribute__((aligned(16))) float rowlds[SPLIT ? 4 : 2][2][AT_KEYS];        // [stage, or wave][L, Dq * scale][query of the block]
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int h = lane >> 5, c = lane & 31;
     int row_tile, z;
     attn_block(row_tile, z);
-    const int k0 = row_tile * AT_QROWS + wave * 32;
+    const int k0 = SPLIT ? row_tile * 32 : row_tile * AT_QROWS + wave * 32;
     const float* Q = (const float*)g.Q + (long long)z * g.q_bs;
     const float* K = (const float*)g.K + (long long)z * g.k_bs;
     const float* V = (const float*)g.V + (long long)z * g.v_bs;
@@ -327,36 +435,49 @@ __global__ void __launch_bounds__(256, D <= 32 ? 2 : 1) attention_bwd_dkv32_kern
         row_d = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(d_rsrc, (qb + c) * 4, 0, 0));
     };
     auto store_rowv = [&](int stage, int qb) {
-        if (wave == 0) rowlds[stage][h][c] = h ? row_d * g.scale : (qb + c < g.sq ? row_l * 1.44269504088896341f : INFINITY);
+        if (SPLIT || wave == 0) rowlds[SPLIT ? wave : stage][h][c] = h ? row_d * g.scale : (qb + c < g.sq ? row_l * 1.44269504088896341f : INFINITY);
     };
-    Blk::load(qr, Q, g.q_rs, 0, g.sq, q_end);
-    Blk::load(dor, dO, g.do_rs, 0, g.sq, do_end);
-    load_rowv(0);
-    Blk::store(qr, qlds[0]); Blk::store(dor, dolds[0]);
-    store_rowv(0, 0);
-    Blk::load(qr, Q, g.q_rs, AT_KEYS, g.sq, q_end);
-    Blk::load(dor, dO, g.do_rs, AT_KEYS, g.sq, do_end);
-    load_rowv(AT_KEYS);
-    __syncthreads();
+    constexpr int STRIDE = SPLIT ? 4 : 1;            // blocks from one step to the next
+    const int first = SPLIT ? wave : 0;
+    auto request = [&](int blk) {                    // (blocks past the last one read zeros)
+        Blk::load(qr, Q, g.q_rs, blk * AT_KEYS, g.sq, q_end);
+        Blk::load(dor, dO, g.do_rs, blk * AT_KEYS, g.sq, do_end);
+        load_rowv(blk * AT_KEYS);
+    };
+    request(first);
+    if constexpr (!SPLIT) {
+        Blk::store(qr, qlds(0)); Blk::store(dor, dolds(0));
+        store_rowv(0, 0);
+        request(1);
+        __syncthreads();
+    }
 
-    for (int blk = 0; blk < nblocks; blk++) {
-        const int qb = blk * AT_KEYS, cur = blk & 1;
+    for (int blk = first; blk < nblocks; blk += STRIDE) {
+        const int qb = blk * AT_KEYS, cur = SPLIT ? 0 : blk & 1, row_stage = SPLIT ? wave : cur;
+        if constexpr (SPLIT) {
+            attn32_wave_order();
+            if (!AHEAD && blk != first) request(blk);
+            Blk::store(qr, qlds(0)); Blk::store(dor, dolds(0));
+            store_rowv(0, qb);
+            attn32_wave_order();
+            if (AHEAD) request(blk + STRIDE);
+        }
         f32x16_t st, dp;
 #pragma unroll
         for (int v = 0; v < 16; v++) { st[v] = 0.f; dp[v] = 0.f; }
-        st = product_over_d<D>(qlds[cur], kf, c, h, st);                    // S: queries x keys
-        dp = product_over_d<D>(dolds[cur], vf, c, h, dp);                   // dP
-        Blk::store(qr, qlds[cur ^ 1]); Blk::store(dor, dolds[cur ^ 1]);
-        store_rowv(cur ^ 1, qb + AT_KEYS);
-        Blk::load(qr, Q, g.q_rs, qb + 2 * AT_KEYS, g.sq, q_end);
-        Blk::load(dor, dO, g.do_rs, qb + 2 * AT_KEYS, g.sq, do_end);
-        load_rowv(qb + 2 * AT_KEYS);
+        st = product_over_d<D>(qlds(cur), kf, c, h, st);                    // S: queries x keys
+        dp = product_over_d<D>(dolds(cur), vf, c, h, dp);                   // dP
+        if constexpr (!SPLIT) {
+            Blk::store(qr, qlds(cur ^ 1)); Blk::store(dor, dolds(cur ^ 1));
+            store_rowv(cur ^ 1, qb + AT_KEYS);
+            request(blk + 2);
+        }
         float p[16], ds[16];
 #pragma unroll
         for (int v4 = 0; v4 < 4; v4++) {
             // registers 4*v4 .. +3 are queries qb + 8*v4 + 4h + (0..3)
-            const f32x4v_t l4 = *(const f32x4v_t*)&rowlds[cur][0][8 * v4 + 4 * h];
-            const f32x4v_t d4 = *(const f32x4v_t*)&rowlds[cur][1][8 * v4 + 4 * h];
+            const f32x4v_t l4 = *(const f32x4v_t*)&rowlds[row_stage][0][8 * v4 + 4 * h];
+            const f32x4v_t d4 = *(const f32x4v_t*)&rowlds[row_stage][1][8 * v4 + 4 * h];
 #pragma unroll
             for (int e = 0; e < 4; e++) {
                 const int v = 4 * v4 + e;
@@ -364,9 +485,22 @@ __global__ void __launch_bounds__(256, D <= 32 ? 2 : 1) attention_bwd_dkv32_kern
                 ds[v] = p[v] * fmaf(dp[v], g.scale, -d4[e]);
             }
         }
-        product_over_rows<D>(dvt, dolds[cur], p, c, h);                     // dV^T += dO^T P
-        product_over_rows<D>(dkt, qlds[cur], ds, c, h);                     // dK^T += Q^T dS
+        product_over_rows<D>(dvt, dolds(cur), p, c, h);                     // dV^T += dO^T P
+        product_over_rows<D>(dkt, qlds(cur), ds, c, h);                     // dK^T += Q^T dS
+        if constexpr (!SPLIT) __syncthreads();
+    }
+    if constexpr (SPLIT) {
+        constexpr float ones[4] = {1.f, 1.f, 1.f, 1.f};
+        const int row = k0 + threadIdx.x / 8;
         __syncthreads();
+        put_part<D>(attn32_lds, dkt, wave, c, h);
+        __syncthreads();
+        if (row < g.sk) write_sum_of_parts<D>((float*)g.dK + ((long long)z * g.sk + row) * D, attn32_lds, ones);
+        __syncthreads();
+        put_part<D>(attn32_lds, dvt, wave, c, h);
+        __syncthreads();
+        if (row < g.sk) write_sum_of_parts<D>((float*)g.dV + ((long long)z * g.sk + row) * D, attn32_lds, ones);
+        return;
     }
     const int key = k0 + c;
     if (key < g.sk) {
@@ -375,35 +509,52 @@ __global__ void __launch_bounds__(256, D <= 32 ? 2 : 1) attention_bwd_dkv32_kern
     }
 }
 
+// Whether a wave's 32 rows become a workgroup of their own that splits the walked axis: the kernels are bound by their MFMAs, so what
+// counts is the number of blocks that the CU with the most workgroups walks, and one more for bringing the parts together.
+static bool attn32_split(int rows, int walked, int batch) {
+    const long long cus = device_cu_count() > 0 ? device_cu_count() : 256, blocks = (walked + AT_KEYS - 1) / AT_KEYS;
+    const long long whole = ((long long)((rows + AT_QROWS - 1) / AT_QROWS) * batch + cus - 1) / cus, parts = ((long long)((rows + 31) / 32) * batch + cus - 1) / cus;
+    return !path_disabled("attnsplit32") && 10 * parts * ((blocks + 3) / 4 + 1) <= 9 * whole * blocks;
+}
+
+template <int D, typename Kernel, typename Args>
+static int launch_attn32(Kernel kernel, bool split, int rows, const Args& g) {
+    constexpr int block = Blk32<D>::ELEMS * 4, parts = 4 * 32 * ATTN32_PART<D> * 4;
+    const int smem = split ? (8 * block > parts ? 8 * block : parts) : 4 * block;
+    if (smem > 64 * 1024 && !check_hip(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, smem), "hipFuncSetAttribute")) return -1;
+    const int per = split ? 32 : AT_QROWS;
+    hipLaunchKernelGGL(kernel, dim3((rows + per - 1) / per, g.batch), dim3(256), smem, current_stream(), g);
+    return check_launch("attention kernel (float32)") ? 0 : -1;
+}
+
+template <int D>
+static int launch_attention_f32_d(const AttnArgs& g) {
+    if (attn32_split(g.sq, g.sk, g.batch)) return launch_attn32<D>(attention_fwd32_kernel<D, true>, true, g.sq, g);
+    return launch_attn32<D>(attention_fwd32_kernel<D, false>, false, g.sq, g);
+}
+
+template <int D>
+static int launch_attention_bwd_f32_d(const AttnBwdArgs& g) {
+    const int rc = attn32_split(g.sq, g.sk, g.batch) ? launch_attn32<D>(attention_bwd_dq32_kernel<D, true>, true, g.sq, g) : launch_attn32<D>(attention_bwd_dq32_kernel<D, false>, false, g.sq, g);
+    if (rc != 0) return rc;
+    if (attn32_split(g.sk, g.sq, g.batch)) return launch_attn32<D>(attention_bwd_dkv32_kernel<D, true>, true, g.sk, g);
+    return launch_attn32<D>(attention_bwd_dkv32_kernel<D, false>, false, g.sk, g);
+}
+
 int launch_attention_f32(const AttnArgs& g, int d) {
-    dim3 grid((g.sq + AT_QROWS - 1) / AT_QROWS, g.batch);
-    switch (d) {
-        case 32: hipLaunchKernelGGL((attention_fwd32_kernel<32>), grid, dim3(256), 0, current_stream(), g); break;
-        case 64: hipLaunchKernelGGL((attention_fwd32_kernel<64>), grid, dim3(256), 0, current_stream(), g); break;
-        case 128: hipLaunchKernelGGL((attention_fwd32_kernel<128>), grid, dim3(256), 0, current_stream(), g); break;      // (68 KB of static LDS: one workgroup per CU)
-        default: set_error("rp_hip_attention_forward: float32 head dimension %d (supported: 32, 64, 128)", d); return -1;
-    }
-    return check_launch("attention_fwd32_kernel") ? 0 : -1;
+    if (d == 32) return launch_attention_f32_d<32>(g);
+    if (d == 64) return launch_attention_f32_d<64>(g);
+    if (d == 128) return launch_attention_f32_d<128>(g);
+    set_error("rp_hip_attention_forward: float32 head dimension %d (supported: 32, 64, 128)", d);
+    return -1;
 }
 
 int launch_attention_bwd_f32(const AttnBwdArgs& g, int d) {
-    dim3 gq((g.sq + AT_QROWS - 1) / AT_QROWS, g.batch), gk((g.sk + AT_QROWS - 1) / AT_QROWS, g.batch);
-    switch (d) {
-        case 32:
-            hipLaunchKernelGGL((attention_bwd_dq32_kernel<32>), gq, dim3(256), 0, current_stream(), g);
-            hipLaunchKernelGGL((attention_bwd_dkv32_kernel<32>), gk, dim3(256), 0, current_stream(), g);
-            break;
-        case 64:
-            hipLaunchKernelGGL((attention_bwd_dq32_kernel<64>), gq, dim3(256), 0, current_stream(), g);
-            hipLaunchKernelGGL((attention_bwd_dkv32_kernel<64>), gk, dim3(256), 0, current_stream(), g);
-            break;
-        case 128:
-            hipLaunchKernelGGL((attention_bwd_dq32_kernel<128>), gq, dim3(256), 0, current_stream(), g);
-            hipLaunchKernelGGL((attention_bwd_dkv32_kernel<128>), gk, dim3(256), 0, current_stream(), g);
-            break;
-        default: set_error("rp_hip_attention_backward: float32 head dimension %d (supported: 32, 64, 128)", d); return -1;
-    }
-    return check_launch("attention backward kernels (float32)") ? 0 : -1;
+    if (d == 32) return launch_attention_bwd_f32_d<32>(g);
+    if (d == 64) return launch_attention_bwd_f32_d<64>(g);
+    if (d == 128) return launch_attention_bwd_f32_d<128>(g);
+    set_error("rp_hip_attention_backward: float32 head dimension %d (supported: 32, 64, 128)", d);
+    return -1;
 }
 
 }  // namespace rp

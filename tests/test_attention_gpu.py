@@ -149,6 +149,27 @@ def _fused_backward(q, k, v, g, dt, scale):
     return gq.numpy(), gk.numpy(), gv.numpy()
 
 
+@pytest.mark.parametrize("shape", [
+    (1, 1, 1000, 32), (2, 33, 129, 32), (3, 70, 300, 64), (1, 257, 97, 64), (2, 31, 161, 128), (1, 200, 513, 128), (5, 16, 84, 128),      # the walk is split
+    (300, 40, 33, 32), (280, 130, 40, 64), (270, 20, 60, 128), (120, 130, 300, 64),                                                      # rows fill the chip: it is not
+    (4, 64, 32, 64), (4, 64, 33, 64), (4, 64, 96, 32), (4, 64, 160, 128)], ids=lambda s: "x".join(map(str, s)))                          # fewer blocks than waves, and more
+def test_fused_attention_fp32_ways_of_dealing_the_rows(shape):
+    """Forward and backward of float32 with 128 rows a workgroup and with 32 whose waves share the walk, a negative scale among them."""
+    Z, sq, sk, d = shape
+    rng = np.random.default_rng(67)
+    q, k, v, g = (rand_storage(rng, s, F32) for s in ((Z, sq, d), (Z, sk, d), (Z, sk, d), (Z, sq, d)))
+    scale = -1.0 / np.sqrt(d) if sq % 2 else 1.0 / np.sqrt(d)
+    got, lse = _fused(q, k, v, F32, scale, want_lse=True)
+    grads = _fused_backward(q, k, v, g, F32, scale)
+    sel = sorted({0, Z // 2, Z - 1})
+    want, want_lse = _f64(q[sel], k[sel], v[sel], F32, scale)
+    assert oracle.rel_err(got[sel], want) <= FWD_TOL[F32]
+    assert np.max(np.abs(lse[sel] - want_lse)) <= 1e-5 * max(1.0, np.max(np.abs(want_lse)))
+    for name, a, b in zip(("dQ", "dK", "dV"), grads, _f64_backward(q[sel], k[sel], v[sel], g[sel], F32, scale)):
+        assert oracle.rel_err(a[sel], b) <= BWD_TOL[F32], name
+    assert np.all(np.isfinite(lse)) and all(np.all(np.isfinite(x)) for x in (got, *grads))
+
+
 @pytest.mark.parametrize("dt", [BF16, F16, F32], ids=lambda d: NAMES[d])
 @pytest.mark.parametrize("shape", [(6, 512, 512, 64), (3, 200, 333, 64), (2, 130, 65, 32), (2, 96, 160, 128), (1, 1, 1, 64), (5, 33, 31, 64)],
                          ids=lambda s: "x".join(map(str, s)))
