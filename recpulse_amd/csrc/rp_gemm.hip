@@ -235,6 +235,30 @@ static Plan make_plan(int batch, int m, int k, int n, long long a_rs, long long 
     return p;
 }
 
+// First byte and one past the last of an operand of a product
+struct Span { const char* lo; const char* hi; };
+static Span span_of(const void* p, int rows, int cols, long long rs, long long cs, int esz) {
+    return {(const char*)p, (const char*)p + ((rows - 1) * rs + (cols - 1) * cs + 1) * esz};
+}
+static bool overlap(const Span& a, const Span& b) { return a.lo < b.hi && b.lo < a.hi; }
+
+// Few 16-bit output tiles, deep k, both operands k-contiguous: the waves of a workgroup split k (rp_gemm_mfma16_wavek.hip).  Up to
+// one 32 x 32 tile per CU, against the k split in two launches two while a tile's rows are no longer than 4096 (us, before and here: 256 of them
+// 64 x 1024 x 4096 7.0 / 5.0, 128 x 8192 x 2048 18.8 / 14.7; 384 and 512 96 x 2048 x 4096 16.1 / 8.9, 64 x 4096 x 8192 19.6 / 15.1, 64 x 8192 x 8192
+// 40.7 / 42.5; against 64 x 64 tiles 256 x 2048 x 2048 10.6 / 9.0, 1024 x 4096 x 512 16.9 / 22).
+// (The k split with a launch of its own for the sums read all of its operands before it wrote C: outputs over an operand stay there.)
+static bool wavek16_takes(const GemmArgs& g, const Plan& p, int dtype) {
+    if ((dtype != RP_DTYPE_BFLOAT16 && dtype != RP_DTYPE_FLOAT16) || p.ragged || p.a_mc || p.b_mc || g.batch != 1 || path_disabled("wavek")) return false;
+    const bool split = p.fam == FAM_MFMA16_SKINNY;
+    if (!split && !(p.fam == FAM_MFMA16 && p.bm == 64 && p.bn == 64)) return false;
+    const long long tiles = (long long)((g.m + 31) / 32) * ((g.n + 31) / 32);
+    if (g.k < 512 || g.k >= (1 << 24) || !(tiles <= cu_tiles() || (split && g.k <= 4096 && tiles <= 2 * cu_tiles()))) return false;
+    if (g.seg_k || g.seg_n || g.bias_by_row || g.c_fold_from) return false;
+    const Span c = span_of(g.C, g.m, g.n, g.c_rs, g.c_cs, 2);
+    return !overlap(c, span_of(g.A, g.m, g.k, g.a_rs, g.a_cs, 2)) && !overlap(c, span_of(g.B, g.k, g.n, g.b_rs, g.b_cs, 2)) &&
+           !(g.bias && overlap(c, span_of(g.bias, 1, g.n, 0, 1, 2)));
+}
+
 static thread_local const char* g_last_kernel = "none";      // what rp_hip_last_gemm_kernel reports
 
 static int run_gemm(GemmArgs g, int dtype) {
@@ -262,6 +286,7 @@ static int run_gemm(GemmArgs g, int dtype) {
     }
     if (p.fam != FAM_GENERIC && p.fam != FAM_TINY && !p.ragged && !(aligned16(g.A) && aligned16(g.B)))
         p = make_plan(g.batch, g.m, g.k, g.n, g.a_rs, g.a_cs, g.b_rs, g.b_cs, g.c_rs, g.c_cs, g.a_bs, g.b_bs, dtype, false, false);
+    if (wavek16_takes(g, p, dtype)) { g_last_kernel = "mfma16_wavek"; return launch_mfma16_wavek(g, dtype); }
     g_last_kernel = p.name;
     switch (p.fam) {
         case FAM_MFMA16:
@@ -380,13 +405,6 @@ int* noalloc_arrival_counters() {
     }
     return (int*)g_noalloc_base;
 }
-
-// First byte and one past the last of an operand of a product
-struct Span { const char* lo; const char* hi; };
-static Span span_of(const void* p, int rows, int cols, long long rs, long long cs, int esz) {
-    return {(const char*)p, (const char*)p + ((rows - 1) * rs + (cols - 1) * cs + 1) * esz};
-}
-static bool overlap(const Span& a, const Span& b) { return a.lo < b.hi && b.lo < a.hi; }
 
 // Rows up to which the column sums of dY join the other gradients of a 16-bit layer: eight chunks of 256, some 6 us
 constexpr int LINEAR_DB_ROWS = 2048;
@@ -510,7 +528,7 @@ const char* rp_hip_gemm_kernel_name(int batch, int m, int k, int n, long long a_
                                     long long b_rs, long long b_cs, long long c_rs, long long c_cs, int dtype) {
     if (batch <= 0 || m <= 0 || k <= 0 || n <= 0 || !dtype_size(dtype)) return "invalid";
     Plan p = make_plan(batch, m, k, n, a_rs, a_cs, b_rs, b_cs, c_rs, c_cs, 0, 0, dtype);
-    return p.name;
+    return p.name;           // (mfma16_wavek, which stands in for two of the families where the pointers allow it, is reported by rp_hip_last_gemm_kernel)
 }
 
 }  // extern "C"
