@@ -242,17 +242,25 @@ static Span span_of(const void* p, int rows, int cols, long long rs, long long c
 }
 static bool overlap(const Span& a, const Span& b) { return a.lo < b.hi && b.lo < a.hi; }
 
-// Few 16-bit output tiles, deep k, both operands k-contiguous: the waves of a workgroup split k (rp_gemm_mfma16_wavek.hip).  Up to
+// Few 16-bit output tiles, deep k, A k-contiguous: the waves of a workgroup split k (rp_gemm_mfma16_wavek.hip).  B k-contiguous too: up to
 // one 32 x 32 tile per CU, against the k split in two launches two while a tile's rows are no longer than 4096 (us, before and here: 256 of them
 // 64 x 1024 x 4096 7.0 / 5.0, 128 x 8192 x 2048 18.8 / 14.7; 384 and 512 96 x 2048 x 4096 16.1 / 8.9, 64 x 4096 x 8192 19.6 / 15.1, 64 x 8192 x 8192
 // 40.7 / 42.5; against 64 x 64 tiles 256 x 2048 x 2048 10.6 / 9.0, 1024 x 4096 x 512 16.9 / 22).
+// B row-major: up to one 16 x 64 tile per CU, against the k split while k is up to 2048 (64 x 2048 x 2048 9.7 / 6.9, 64 x 4096 x 1024 10.0 / 11.7,
+// 96 x 4096 x 4096 with 384 tiles 16.4 / 19.2).
 // (The k split with a launch of its own for the sums read all of its operands before it wrote C: outputs over an operand stay there.)
 static bool wavek16_takes(const GemmArgs& g, const Plan& p, int dtype) {
-    if ((dtype != RP_DTYPE_BFLOAT16 && dtype != RP_DTYPE_FLOAT16) || p.ragged || p.a_mc || p.b_mc || g.batch != 1 || path_disabled("wavek")) return false;
+    if ((dtype != RP_DTYPE_BFLOAT16 && dtype != RP_DTYPE_FLOAT16) || p.ragged || p.a_mc || g.batch != 1 || path_disabled("wavek")) return false;
     const bool split = p.fam == FAM_MFMA16_SKINNY;
     if (!split && !(p.fam == FAM_MFMA16 && p.bm == 64 && p.bn == 64)) return false;
-    const long long tiles = (long long)((g.m + 31) / 32) * ((g.n + 31) / 32);
-    if (g.k < 512 || g.k >= (1 << 24) || !(tiles <= cu_tiles() || (split && g.k <= 4096 && tiles <= 2 * cu_tiles()))) return false;
+    if (g.k < 512 || g.k >= (1 << 24)) return false;
+    if (p.b_mc) {
+        if ((long long)((g.m + 15) / 16) * ((g.n + 63) / 64) > cu_tiles() || g.k * g.b_rs >= (1ll << 30)) return false;
+        if (split && (g.k > 2048 || stream128_shape(g.batch, g.m, g.k, g.n))) return false;
+    } else {
+        const long long tiles = (long long)((g.m + 31) / 32) * ((g.n + 31) / 32);
+        if (!(tiles <= cu_tiles() || (split && g.k <= 4096 && tiles <= 2 * cu_tiles()))) return false;
+    }
     if (g.seg_k || g.seg_n || g.bias_by_row || g.c_fold_from) return false;
     const Span c = span_of(g.C, g.m, g.n, g.c_rs, g.c_cs, 2);
     return !overlap(c, span_of(g.A, g.m, g.k, g.a_rs, g.a_cs, 2)) && !overlap(c, span_of(g.B, g.k, g.n, g.b_rs, g.b_cs, 2)) &&

@@ -1245,23 +1245,27 @@ def test_split32_single_products_and_repeated_values():
 
 
 @pytest.mark.parametrize("dt", [BF16, F16], ids=lambda d: NAMES[d])
-@pytest.mark.parametrize("m,k,n", [(1, 512, 1), (16, 520, 16), (17, 1024, 33), (65, 1032, 129), (31, 4096, 5), (40, 4104, 47), (300, 1536, 300),
-                                   (1024, 512, 250), (96, 2048, 2055), (100, 4096, 4088)])
-def test_waves_that_split_k(dt, m, k, n):
-    """Few tiles, deep k, both operands k-contiguous: every tile size, ragged ends of m, n and k, one and several rounds of loads.
+@pytest.mark.parametrize("layout,m,k,n",
+                         [("nt", *s) for s in [(1, 512, 1), (16, 520, 16), (17, 1024, 33), (65, 1032, 129), (31, 4096, 5), (40, 4104, 47), (300, 1536, 300),
+                                               (1024, 512, 250), (96, 2048, 2055), (100, 4096, 4088)]] +
+                         [("nn", *s) for s in [(1, 512, 8), (17, 1024, 40), (65, 1032, 136), (300, 1536, 304), (33, 5000, 72), (64, 2048, 2048), (10, 1016, 64)]])
+def test_waves_that_split_k(dt, layout, m, k, n):
+    """Few tiles, deep k, B either way round: every tile size, ragged ends of m, n and k, one and several rounds of loads.
     Operands are small integers (sums below 2^24: exact in any order) between NaNs that must not be read into a sum."""
     rng = np.random.default_rng(m + k + n)
     a64, b64 = rng.integers(-2, 3, (m, k)).astype(np.float64), rng.integers(-2, 3, (k, n)).astype(np.float64)
     pad = 8
-    arow, brow = np.full((m + 1, k + pad), np.nan), np.full((n + 1, k + pad), np.nan)
+    bt = b64.T if layout == "nt" else b64
+    arow, brow = np.full((m + 1, k + pad), np.nan), np.full((bt.shape[0] + 1, bt.shape[1] + pad), np.nan)
     arow[:m, :k] = a64
-    brow[:n, :k] = b64.T
+    brow[:bt.shape[0], :bt.shape[1]] = bt
+    b_st = (0, 1, k + pad) if layout == "nt" else (0, n + pad, 1)
     bias, old = oracle.to_storage(rng.integers(-4, 5, (n,)).astype(np.float64), dt), oracle.to_storage(rng.integers(-4, 5, (m, n)).astype(np.float64), dt)
     da, db, dbias = (capi.DeviceBuffer.from_numpy(v) for v in (oracle.to_storage(arow, dt), oracle.to_storage(brow, dt), bias))
     for with_bias, accumulate, transposed in ((False, False, False), (True, True, False), (True, False, True)):
         c0 = np.ascontiguousarray(old.T) if transposed else old
         dc = capi.DeviceBuffer.from_numpy(c0)
-        capi.gemm(dc.ptr, da.ptr, db.ptr, dbias.ptr if with_bias else None, 1, m, k, n, (0, k + pad, 1), (0, 1, k + pad), (0, 1, m) if transposed else (0, n, 1), accumulate, dt)
+        capi.gemm(dc.ptr, da.ptr, db.ptr, dbias.ptr if with_bias else None, 1, m, k, n, (0, k + pad, 1), b_st, (0, 1, m) if transposed else (0, n, 1), accumulate, dt)
         assert capi.last_gemm_kernel() == "mfma16_wavek"
         capi.synchronize()
         got = dc.to_numpy(capi.NP_STORAGE[dt], c0.shape)
