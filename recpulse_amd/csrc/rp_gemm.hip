@@ -248,12 +248,13 @@ static bool overlap(const Span& a, const Span& b) { return a.lo < b.hi && b.lo <
 // 40.7 / 42.5; against 64 x 64 tiles 256 x 2048 x 2048 10.6 / 9.0, 1024 x 4096 x 512 16.9 / 22).
 // B row-major: up to one 16 x 64 tile per CU, against the k split while k is up to 2048 (64 x 2048 x 2048 9.7 / 6.9, 64 x 4096 x 1024 10.0 / 11.7,
 // 96 x 4096 x 4096 with 384 tiles 16.4 / 19.2).
+// From ten slabs on: the eight of 128 x 512 x 512 take 5.3 and 4.8, and a small layer's dX keeps the bits it has in one launch with dW.
 // (The k split with a launch of its own for the sums read all of its operands before it wrote C: outputs over an operand stay there.)
 static bool wavek16_takes(const GemmArgs& g, const Plan& p, int dtype) {
     if ((dtype != RP_DTYPE_BFLOAT16 && dtype != RP_DTYPE_FLOAT16) || p.ragged || p.a_mc || g.batch != 1 || path_disabled("wavek")) return false;
     const bool split = p.fam == FAM_MFMA16_SKINNY;
     if (!split && !(p.fam == FAM_MFMA16 && p.bm == 64 && p.bn == 64)) return false;
-    if (g.k < 512 || g.k >= (1 << 24)) return false;
+    if (g.k < 10 * M16_BK || g.k >= (1 << 24)) return false;
     if (p.b_mc) {
         if ((long long)((g.m + 15) / 16) * ((g.n + 63) / 64) > cu_tiles() || g.k * g.b_rs >= (1ll << 30)) return false;
         if (split && (g.k > 2048 || stream128_shape(g.batch, g.m, g.k, g.n))) return false;

@@ -59,7 +59,7 @@ struct StripSums {
 
 // All gradients of a Linear layer in one launch: the first workgroups add up the columns of dY (their chain of chunks is the longest of
 // any), the next ones compute dX = dY . W^T (k-contiguous operands), the others dW = X^T . dY (free-index-contiguous ones), tile for
-// tile and chunk for chunk what separate launches would do, so the same bits.
+// tile and chunk for chunk what separate launches on 64 x 64 tiles would do, so the same bits.
 // A 64 x 64 tile is bound by the latency of its slab chain with one workgroup per CU (1024^3: 19.1 K cycles for 2.05 K of MFMA);
 // two or three of them share a CU's LDS, and the two products' chains run side by side.
 // bf16 layer of 1024 x 1024 x 1024 (bias too), forward and backward: 31.3 us with a launch per gradient, 24.6 with the matrices in one,

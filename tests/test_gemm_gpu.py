@@ -1246,9 +1246,9 @@ def test_split32_single_products_and_repeated_values():
 
 @pytest.mark.parametrize("dt", [BF16, F16], ids=lambda d: NAMES[d])
 @pytest.mark.parametrize("layout,m,k,n",
-                         [("nt", *s) for s in [(1, 512, 1), (16, 520, 16), (17, 1024, 33), (65, 1032, 129), (31, 4096, 5), (40, 4104, 47), (300, 1536, 300),
-                                               (1024, 512, 250), (96, 2048, 2055), (100, 4096, 4088)]] +
-                         [("nn", *s) for s in [(1, 512, 8), (17, 1024, 40), (65, 1032, 136), (300, 1536, 304), (33, 5000, 72), (64, 2048, 2048), (10, 1016, 64)]])
+                         [("nt", *s) for s in [(1, 640, 1), (16, 648, 16), (17, 1024, 33), (65, 1032, 129), (31, 4096, 5), (40, 4104, 47), (300, 1536, 300),
+                                               (1024, 640, 250), (96, 2048, 2055), (100, 4096, 4088)]] +
+                         [("nn", *s) for s in [(1, 640, 8), (17, 1024, 40), (65, 1032, 136), (300, 1536, 304), (33, 5000, 72), (64, 2048, 2048), (10, 1016, 64)]])
 def test_waves_that_split_k(dt, layout, m, k, n):
     """Few tiles, deep k, B either way round: every tile size, ragged ends of m, n and k, one and several rounds of loads.
     Operands are small integers (sums below 2^24: exact in any order) between NaNs that must not be read into a sum."""
