@@ -617,7 +617,10 @@ int launch_conv_taps16(void* out, const void* in, const void* w, const void* bia
     const int groups = (int)(((long long)batch * H * W + positions - 1) / positions), vw = group_width(W, in, out);
     // Workgroups that sort the weights themselves save a launch and take longer each (us, sorted by a launch and in the workgroups: 49
     // of them 11.4 / 8.9, 196 24 / 21, 784 26 / 30): as long as there is not more than one per CU.
-    const bool by_channel = kH == 3 && kW == 3 && !for_input_grad && ((uintptr_t)w & 15) == 0 && (long long)groups * ((C_to + CD_CO - 1) / CD_CO) <= 256;
+    // An output over the weights: a workgroup reads them for every 32 channels while others already store, so they are copied first.
+    const char *out0 = (const char*)out, *w0 = (const char*)w;
+    const bool apart = out0 + (size_t)batch * C_to * H * W * 2 <= w0 || w0 + (size_t)total * 2 <= out0;
+    const bool by_channel = kH == 3 && kW == 3 && !for_input_grad && apart && ((uintptr_t)w & 15) == 0 && (long long)groups * ((C_to + CD_CO - 1) / CD_CO) <= 256;
     void* wt = nullptr;
     if (!by_channel && rp_hip_malloc(&wt, (size_t)total * 2) != 0) return -1;
     if (!by_channel) hipLaunchKernelGGL(conv_weights_by_tap_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, current_stream(), (uint16_t*)wt, (const uint16_t*)w, C_from, C_to, taps, total,

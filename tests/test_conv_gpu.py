@@ -217,6 +217,31 @@ def test_same_convolution_over_its_own_input(dt):
         assert oracle.rel_err(oracle.to_f64(src.numpy(), dt), oracle.to_f64(out.numpy(), dt)) <= {BF16: 2.0 ** -8, F16: 2.0 ** -11}[dt]
 
 
+@pytest.mark.parametrize("dt", [F16, BF16], ids=lambda d: NAMES[d])
+@pytest.mark.parametrize("case", [(2, 128, 12, 16, 64), (3, 192, 14, 14, 128), (1, 64, 30, 30, 64)], ids=lambda c: "x".join(map(str, c)))
+@pytest.mark.parametrize("at", ["front", "back"])
+def test_same_convolution_over_its_own_weights(dt, case, at):
+    """An output that overlaps the weights it is computed from, at either end: the bits of one that does not (the weights are read before
+    anything is stored)."""
+    N, Ci, H, W, Co = case
+    L = capi.lib()
+    rng = np.random.default_rng(87)
+    x, w = rand_storage(rng, (N, Ci, H, W), dt), oracle.to_storage(rng.standard_normal((Co, Ci, 3, 3)) * 0.2, dt)
+    dx_, dw_, want = Dev(x, dt), Dev(w, dt), Dev.empty((N, Co, H, W), dt)
+    capi.check(L.rp_hip_conv2d_same_forward(want.ptr, dx_.ptr, dw_.ptr, None, N, Ci, H, W, Co, 3, 3, dt), "apart")
+    ny, nw = N * Co * H * W, w.size
+    shared = 1024                                   # elements that both hold: whole 16-byte vectors, fewer than either
+    both = np.zeros(ny + nw - shared, w.dtype)
+    w_at, y_at = (0, nw - shared) if at == "front" else (ny - shared, 0)
+    both[w_at:w_at + nw] = w.reshape(-1)
+    buf = capi.DeviceBuffer.from_numpy(both)
+    capi.check(L.rp_hip_conv2d_same_forward(buf.ptr + 2 * y_at, dx_.ptr, buf.ptr + 2 * w_at, None, N, Ci, H, W, Co, 3, 3, dt), "over the weights")
+    got = buf.to_numpy(both.dtype, both.shape)
+    assert np.array_equal(got[y_at:y_at + ny], want.numpy().reshape(-1))
+    keep = got[:y_at] if at == "front" else got[ny:]
+    assert np.array_equal(keep, w.reshape(-1)[:nw - shared] if at == "front" else w.reshape(-1)[shared:])
+
+
 def test_same_convolution_in_chunks_of_the_batch(monkeypatch):
     """With room for two samples at a time a batch of five goes in three chunks: same bits as in one piece (the weight
     gradient adds its chunks in fp32 and rounds after each, so it is compared to tolerance)."""
