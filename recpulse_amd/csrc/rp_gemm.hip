@@ -415,8 +415,11 @@ int* noalloc_arrival_counters() {
     return (int*)g_noalloc_base;
 }
 
-// Rows up to which the column sums of dY join the other gradients of a 16-bit layer: eight chunks of 256, some 6 us
-constexpr int LINEAR_DB_ROWS = 2048;
+// Rows up to which the column sums of dY join the other gradients of a 16-bit layer: four chunks of 256.  A strip's chunks are a chain
+// that narrow or uneven strips walk at up to 2.2 us a chunk, and a launch of their own costs 3 to 4 us (bf16, us, in the launch and
+// apart: 256 x 256 x 1024 7.0 / 11.4, 1024 x 512 x 512 8.9 / 12.0, 1024 x 8 x 16 11.7 / 11.5, 1280 x 768 x 264 16.4 / 15.1,
+// 1536 x 8 x 16 16.6 / 14.0, 2048 x 40 x 16 21.8 / 16.5, 2048 x 512 x 512 21.2 / 19.3).
+constexpr int LINEAR_DB_ROWS = 1024;
 
 // Whether dX and dW of a 16-bit Linear layer go out as one launch: both on the 64 x 64 tile (an output of under half a CU count
 // of 128 x 128 tiles) in the layouts of dense X and W, and neither gradient written over anything that the other product reads
