@@ -148,7 +148,9 @@ const char* rp_hip_gemm_kernel_name(int batch, int m, int k, int n,
                                     long long c_rs, long long c_cs, int dtype);
 /* Name of the kernel family and tile that the calling thread's most recent GEMM entry-point call dispatched ("none"
  * before the first): unlike rp_hip_gemm_kernel_name it reflects the bias, the accumulate flag and the pointers of that
- * call.  No counterpart in the reference (whose device GEMM is one cuBLAS call). */
+ * call.  The rp_hip_conv2d_same_* entries report theirs too: "conv_taps16_256x64" or "_64x64" (a workgroup's positions x channels)
+ * and "conv_dw16" for 16-bit images read in place, "conv_planes" for zero-bordered copies; a call with both gradients names the
+ * weight gradient's.  No counterpart in the reference (whose device GEMM is one cuBLAS call). */
 const char* rp_hip_last_gemm_kernel(void);
 
 /* ------------------------------------------------------------------------

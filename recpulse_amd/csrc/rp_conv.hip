@@ -531,6 +531,7 @@ template <typename T>
 static int same_conv(void* out, const void* in, const void* w, const void* bias, int batch, int C_from, int C_to,
                      int H, int W, int kH, int kW, bool for_input_grad, int dtype) {
     const int taps = kH * kW, total = C_from * C_to * taps;
+    report_kernel("conv_planes");
     void* wt = nullptr;
     if (rp_hip_malloc(&wt, (size_t)total * sizeof(T)) != 0) return -1;
     // w is [C_out, C_in, taps]: forward reduces over C_in (C_from = C_in, C_to = C_out), the input gradient over C_out
@@ -583,6 +584,7 @@ template <typename T>
 static int same_conv_backward(void* dx, void* dw, const void* dy, const void* x, const void* w, int batch, int C_in, int H, int W,
                               int C_out, int kH, int kW, int dtype) {
     constexpr int VEC = 16 / (int)sizeof(T);
+    report_kernel("conv_planes");
     const PadGeom pg = pad_geom(H, W, kH, kW, VEC);
     const int taps = kH * kW;
     const long long cols = (long long)H * pg.Wp, w_n = (long long)C_out * C_in * taps;

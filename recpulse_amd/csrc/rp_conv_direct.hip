@@ -634,6 +634,7 @@ int launch_conv_taps16(void* out, const void* in, const void* w, const void* bia
         else if (kW == 3) rc = bf ? launch_taps_k<bf16_t, 3, 1>(g, npos, vw) : launch_taps_k<f16_t, 3, 1>(g, npos, vw);
         else rc = bf ? launch_taps_k<bf16_t, 5, 1>(g, npos, vw) : launch_taps_k<f16_t, 5, 1>(g, npos, vw);
     }
+    report_kernel(npos == 256 ? "conv_taps16_256x64" : "conv_taps16_64x64");
     if (wt) rp_hip_free(wt);                     // back to the pool while the kernels are still queued: safe for later work on this stream
     return rc;
 }
@@ -682,6 +683,7 @@ int launch_conv_dw16(void* dw, const void* dy, const void* x, int batch, int C_i
     ConvDwArgs g{(float*)part, dy, x, batch, C_in, C_out, H, W, kH, rows, strips, per_split, (C_in + 63) / 64, splits};
     const int vw = group_width(W, dy, x);
     const int rc = dtype == RP_DTYPE_BFLOAT16 ? launch_dw<bf16_t>(g, kW, vw, dw) : launch_dw<f16_t>(g, kW, vw, dw);
+    report_kernel("conv_dw16");
     rp_hip_free(part);
     return rc;
 }

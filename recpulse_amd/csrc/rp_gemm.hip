@@ -269,6 +269,7 @@ static bool wavek16_takes(const GemmArgs& g, const Plan& p, int dtype) {
 }
 
 static thread_local const char* g_last_kernel = "none";      // what rp_hip_last_gemm_kernel reports
+void report_kernel(const char* name) { g_last_kernel = name; }
 
 static int run_gemm(GemmArgs g, int dtype) {
     plain_k_strides(g.m, g.k, g.n, g.a_rs, g.a_cs, g.b_rs, g.b_cs);

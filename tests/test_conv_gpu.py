@@ -169,17 +169,23 @@ def test_same_convolution_without_lowered_matrix(dt, case):
         assert np.array_equal(both_x.numpy(), dgx_.numpy()) and np.array_equal(both_w.numpy(), dgw_.numpy())
 
 
-DIRECT_CASES = [  # (batch, C_in, H, W, C_out, kH, kW): rows of any width (whole fours, twos, odd), many small samples in a strip, strips
-                  # that begin inside a row, 64 and 256 positions a workgroup, channels and strips that end inside a tile
-    (11, 64, 7, 7, 64, 3, 3), (3, 128, 10, 6, 64, 5, 3), (2, 64, 3, 50, 128, 3, 5), (1, 64, 5, 127, 64, 3, 3), (2, 64, 2, 130, 64, 1, 3),
-    (64, 64, 32, 32, 64, 3, 3), (70, 64, 31, 31, 64, 3, 3), (66, 64, 30, 34, 64, 1, 5), (24, 64, 12, 300, 64, 3, 3), (1, 64, 1, 1, 64, 3, 3)]
+T256, T64, DW, PLANES = "conv_taps16_256x64", "conv_taps16_64x64", "conv_dw16", "conv_planes"
+DIRECT_CASES = [  # (batch, C_in, H, W, C_out, kH, kW) and the kernels of forward, dX and dW on 256 CUs: rows of any width (whole eights, fours,
+                  # twos, odd), many small samples in a strip, strips that begin inside a row or are shortened to whole rows, 64 and 256
+                  # positions a workgroup with three and five taps a row, channels and strips that end inside a tile, shapes refused
+    ((11, 64, 7, 7, 64, 3, 3), T64, T64, DW), ((3, 128, 10, 6, 64, 5, 3), T64, T64, DW), ((2, 64, 3, 50, 128, 3, 5), T64, T64, PLANES),
+    ((1, 64, 5, 127, 64, 3, 3), PLANES, PLANES, DW), ((2, 64, 2, 130, 64, 1, 3), T64, T64, PLANES), ((64, 64, 32, 32, 64, 3, 3), T256, T256, DW),
+    ((70, 64, 31, 31, 64, 3, 3), T256, T256, DW), ((66, 64, 30, 34, 64, 1, 5), T256, T256, PLANES), ((24, 64, 12, 300, 64, 3, 3), PLANES, PLANES, PLANES),
+    ((1, 64, 1, 1, 64, 3, 3), PLANES, PLANES, PLANES), ((90, 64, 28, 28, 64, 3, 3), T256, T256, DW), ((64, 64, 56, 56, 64, 3, 3), T256, T256, DW),
+    ((90, 64, 28, 28, 64, 5, 5), T256, T256, DW), ((64, 64, 32, 32, 64, 5, 5), T256, T256, DW), ((70, 64, 31, 31, 64, 5, 5), T256, T256, PLANES),
+    ((23, 64, 56, 52, 64, 3, 3), PLANES, PLANES, DW), ((29, 64, 48, 48, 64, 5, 5), PLANES, PLANES, DW)]
 
 
 @pytest.mark.parametrize("dt", [F16, BF16], ids=lambda d: NAMES[d])
-@pytest.mark.parametrize("case", DIRECT_CASES, ids=lambda c: "x".join(map(str, c)))
-def test_same_convolution_from_the_image_is_exact_on_integers(dt, case):
-    """Small integers: every sum is an integer below 2^24, exact in fp32, so the results are that sum rounded once (the
-    forward's bias: rounded again), bit for bit."""
+@pytest.mark.parametrize("case,forward,input_grad,weight_grad", DIRECT_CASES, ids=["x".join(map(str, c[0])) for c in DIRECT_CASES])
+def test_same_convolution_from_the_image_is_exact_on_integers(dt, case, forward, input_grad, weight_grad):
+    """Small integers: every sum is an integer below 2^24, exact in fp32 (and a sample's share of a weight gradient below 2^8, exact in 16
+    bits), so the results are that sum rounded once (the forward's bias: rounded again), bit for bit; each on the kernel that is named."""
     import torch
     N, Ci, H, W, Co, kH, kW = case
     L = capi.lib()
@@ -189,7 +195,14 @@ def test_same_convolution_from_the_image_is_exact_on_integers(dt, case):
     dx_, dw_, db_, dg_ = (Dev(oracle.to_storage(v, dt), dt) for v in (x, w, b, g))
     y, gx, gw = Dev.empty((N, Co, H, W), dt), Dev.empty((N, Ci, H, W), dt), Dev.empty((Co, Ci, kH, kW), dt)
     capi.check(L.rp_hip_conv2d_same_forward(y.ptr, dx_.ptr, dw_.ptr, db_.ptr, N, Ci, H, W, Co, kH, kW, dt), "same forward")
+    assert capi.last_gemm_kernel() == forward
+    capi.check(L.rp_hip_conv2d_same_backward(gx.ptr, None, dg_.ptr, None, dw_.ptr, N, Ci, H, W, Co, kH, kW, dt), "same backward (input)")
+    assert capi.last_gemm_kernel() == input_grad
+    capi.check(L.rp_hip_conv2d_same_backward(None, gw.ptr, dg_.ptr, dx_.ptr, None, N, Ci, H, W, Co, kH, kW, dt), "same backward (weights)")
+    assert capi.last_gemm_kernel() == weight_grad
+    alone = gx.numpy(), gw.numpy()
     capi.check(L.rp_hip_conv2d_same_backward(gx.ptr, gw.ptr, dg_.ptr, dx_.ptr, dw_.ptr, N, Ci, H, W, Co, kH, kW, dt), "same backward")
+    assert np.array_equal(gx.numpy(), alone[0]) and np.array_equal(gw.numpy(), alone[1])
     xt, wt, gt = (torch.tensor(v, dtype=torch.float32) for v in (x, w, g))       # sums of integers below 2^24: exact in any order
     pad = (kH // 2, kW // 2)
     want = oracle.to_storage(torch.nn.functional.conv2d(xt, wt, None, padding=pad).numpy(), dt)
