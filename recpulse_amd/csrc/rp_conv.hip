@@ -808,17 +808,20 @@ int rp_hip_conv2d_same_backward(void* dx, void* dw, const void* dy, const void* 
         set_error("rp_hip_conv2d_same_backward: null operand or a shape outside rp_hip_conv2d_same_supported");
         return -1;
     }
-    // each gradient on its own kernel, dX first; whatever neither takes goes through the padded planes together
-    const bool direct_dx = dx && conv_taps16_takes(batch, C_out, C_in, H, W, kH, kW, dtype) && images_apart(dx, C_in, dy, C_out, batch, H, W, dtype);
-    const bool direct_dw = dw && conv_dw16_takes(batch, C_in, C_out, H, W, kH, kW, dtype) && (!dx || direct_dx);
-    if (direct_dx) {
-        if (launch_conv_taps16(dx, dy, w, nullptr, batch, C_out, C_in, H, W, kH, kW, true, dtype) != 0) return -1;
-        dx = nullptr;
+    // Each gradient on the kernel that takes it, whether or not the other is asked for, so that a gradient's bits do not depend on the
+    // call's other half; dX first (dW may be written over W).  The one exception: where dX overlaps dY, both come from the planes, which
+    // copy dY before dX is stored.
+    const bool apart = !dx || images_apart(dx, C_in, dy, C_out, batch, H, W, dtype);
+    const bool direct_dx = dx && apart && conv_taps16_takes(batch, C_out, C_in, H, W, kH, kW, dtype);
+    const bool direct_dw = dw && apart && conv_dw16_takes(batch, C_in, C_out, H, W, kH, kW, dtype);
+    void *const planes_dx = direct_dx ? nullptr : dx, *const planes_dw = direct_dw ? nullptr : dw;
+    if (direct_dx && launch_conv_taps16(dx, dy, w, nullptr, batch, C_out, C_in, H, W, kH, kW, true, dtype) != 0) return -1;
+    if (planes_dx || planes_dw) {
+        int rc = -1;
+        RP_DISPATCH_DTYPE(dtype, rc = same_conv_backward<T>(planes_dx, planes_dw, dy, x, w, batch, C_in, H, W, C_out, kH, kW, dtype));
+        if (rc != 0) return -1;
     }
-    if (direct_dw) return launch_conv_dw16(dw, dy, x, batch, C_in, C_out, H, W, kH, kW, dtype);
-    if (!dx && !dw) return 0;
-    RP_DISPATCH_DTYPE(dtype, return same_conv_backward<T>(dx, dw, dy, x, w, batch, C_in, H, W, C_out, kH, kW, dtype));
-    return -1;
+    return direct_dw ? launch_conv_dw16(dw, dy, x, batch, C_in, C_out, H, W, kH, kW, dtype) : 0;
 }
 
 int rp_hip_channel_bias_add(void* y, const void* bias, int batch, int channels, int hw, int dtype) {

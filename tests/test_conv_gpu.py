@@ -215,6 +215,33 @@ def test_same_convolution_from_the_image_is_exact_on_integers(dt, case, forward,
 
 
 @pytest.mark.parametrize("dt", [F16, BF16], ids=lambda d: NAMES[d])
+@pytest.mark.parametrize("case", [(23, 64, 56, 52, 64, 3), (29, 64, 48, 48, 64, 5), (2, 128, 12, 40, 64, 3), (1, 64, 53, 53, 128, 5)], ids=lambda c: "x".join(map(str, c)))
+def test_weight_gradient_does_not_depend_on_the_input_gradient(dt, case):
+    """dW alone and beside dX: the same kernel and the same bits, also where the in-place kernels take dW and refuse dX (the
+    first two shapes) and where they take dX and refuse dW (the last).  Beside a dX that is stored over dY, dW is that of the planes, to tolerance."""
+    N, Ci, H, W, Co, k = case
+    L = capi.lib()
+    rng = np.random.default_rng(88)
+    x, g, w = rand_storage(rng, (N, Ci, H, W), dt), rand_storage(rng, (N, Co, H, W), dt), oracle.to_storage(rng.standard_normal((Co, Ci, k, k)) * 0.2, dt)
+    dx_, dg_, dw_ = Dev(x, dt), Dev(g, dt), Dev(w, dt)
+    alone_x, alone_w, gx, gw = Dev.empty((N, Ci, H, W), dt), Dev.empty((Co, Ci, k, k), dt), Dev.empty((N, Ci, H, W), dt), Dev.empty((Co, Ci, k, k), dt)
+    capi.check(L.rp_hip_conv2d_same_backward(alone_x.ptr, None, dg_.ptr, None, dw_.ptr, N, Ci, H, W, Co, k, k, dt), "dX alone")
+    capi.check(L.rp_hip_conv2d_same_backward(None, alone_w.ptr, dg_.ptr, dx_.ptr, None, N, Ci, H, W, Co, k, k, dt), "dW alone")
+    kernel = capi.last_gemm_kernel()
+    capi.check(L.rp_hip_conv2d_same_backward(gx.ptr, gw.ptr, dg_.ptr, dx_.ptr, dw_.ptr, N, Ci, H, W, Co, k, k, dt), "both")
+    assert capi.last_gemm_kernel() == kernel
+    assert np.array_equal(gx.numpy(), alone_x.numpy()) and np.array_equal(gw.numpy(), alone_w.numpy())
+    capi.check(L.rp_hip_conv2d_same_backward(gx.ptr, dw_.ptr, dg_.ptr, dx_.ptr, dw_.ptr, N, Ci, H, W, Co, k, k, dt), "both, dW over W")
+    assert np.array_equal(gx.numpy(), alone_x.numpy()) and np.array_equal(dw_.numpy(), alone_w.numpy())
+    if Ci == Co:
+        dw2 = Dev(w, dt)
+        capi.check(L.rp_hip_conv2d_same_backward(dg_.ptr, gw.ptr, dg_.ptr, dx_.ptr, dw2.ptr, N, Ci, H, W, Co, k, k, dt), "both, dX over dY")
+        # the planes round every sample's share once more: half a unit of 16 bits of each, sqrt(N) of them against sqrt(N) of the sum
+        assert oracle.rel_err(oracle.to_f64(gw.numpy(), dt), oracle.to_f64(alone_w.numpy(), dt)) <= {BF16: 2.0 ** -7, F16: 2.0 ** -10}[dt]
+        assert oracle.rel_err(oracle.to_f64(dg_.numpy(), dt), oracle.to_f64(alone_x.numpy(), dt)) <= {BF16: 2.0 ** -8, F16: 2.0 ** -11}[dt]
+
+
+@pytest.mark.parametrize("dt", [F16, BF16], ids=lambda d: NAMES[d])
 def test_same_convolution_over_its_own_input(dt):
     """An output that overlaps the image it is computed from: the image is copied first, as for any other convolution."""
     N, C, H, W = 2, 64, 9, 12
