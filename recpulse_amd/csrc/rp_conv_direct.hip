@@ -546,9 +546,10 @@ static long long strip_cells(int positions, int batch, int H, int W, int kH, int
 }
 
 constexpr size_t CD_LDS = 160 * 1024;            // of a CU
+static int cus_of_device() { return device_cu_count() > 0 ? device_cu_count() : 256; }
 // Workgroups of the weight gradient in all, two per CU: more of them leave more partial sums to be written and added (us at 384,
 // 512 and 768: 64 x 64 x 56 x 56 3 x 3 38.8 / 36.2 / 44.6, 16 x 256 x 14 x 14 35.5 / 34.9 / 48.7, 20 x 64 x 50 x 50 38.2 / 36.9 / 48.1).
-constexpr int CD_DW_BLOCKS = 512;
+static int dw_blocks() { return 2 * cus_of_device(); }
 
 static size_t taps_smem(int npos, long long cells, int kH, int kW) {
     const int staged = kH == 3 && kW == 3 ? 9 : 2 * kW;                  // all taps once, or a tap row twice
@@ -580,8 +581,7 @@ static int group_width(int W, const void* a, const void* b) {
 
 static int taps_npos(int batch, int C_to, int H, int W) {
     const long long total = (long long)batch * H * W, at256 = (total + 255) / 256 * ((C_to + CD_CO - 1) / CD_CO);
-    const int cus = device_cu_count();
-    return at256 >= (cus > 0 ? cus : 256) ? 256 : 64;
+    return at256 >= cus_of_device() ? 256 : 64;
 }
 
 bool conv_taps16_takes(int batch, int C_from, int C_to, int H, int W, int kH, int kW, int dtype) {
@@ -589,10 +589,19 @@ bool conv_taps16_takes(int batch, int C_from, int C_to, int H, int W, int kH, in
     if ((kW != 3 && kW != 5) || kH % 2 == 0 || C_from % CD_CK || C_from <= 0 || C_to <= 0 || C_to > (1 << 20)) return false;
     if ((long long)batch * H * W >= (1ll << 30) || (long long)C_from * C_to * kH * kW >= (1ll << 30)) return false;
     if ((long long)H * W < 4) return false;
+    const long long total = (long long)batch * H * W;
     const int npos = taps_npos(batch, C_to, H, W), positions = positions_per_group(npos, batch, H, W, kH, kW);
     const long long cells = strip_cells(positions, batch, H, W, kH, kW), rows = cells / (W + kW - 1);
     const long long samples = W % 8 == 0 ? 0 : (positions + (long long)H * W - 2) / ((long long)H * W) + 1;       // that end inside a group
-    return rows * W + 7 * samples <= CD_STRIP && taps_smem(npos, cells, kH, kW) <= CD_LDS;
+    const size_t smem = taps_smem(npos, cells, kH, kW);
+    // 64 positions a workgroup, more than two rounds of the CUs: the planes are faster where the strip and the weights leave a CU one
+    // workgroup at a time (5 x 5, us, here and there: 12 x 192 x 39 x 39 -> 128 96 / 72, 5 x 256 x 45 x 38 -> 256 126 / 107, 22 x 192 x 39 x 39
+    // -> 64 94 / 83; two rounds 7 x 256 x 33 x 33 -> 192 83 / 95, one 4 x 256 x 38 x 38 -> 128 47 / 65), and where the strip is six and more
+    // times its positions (3 x 3: 2 x 192 x 96 x 96 -> 128 45 / 31, 5 x 192 x 96 x 96 -> 64 50 / 38, 11 x 192 x 75 x 75 -> 64 85 / 73;
+    // 13 x 64 x 42 x 67 -> 64 23 / 25).
+    const bool many = (total + positions - 1) / positions * ((C_to + CD_CO - 1) / CD_CO) > 2 * cus_of_device();
+    if (npos == 64 && many && (smem > CD_LDS / 2 || (W > 64 && C_from > 64))) return false;
+    return rows * W + 7 * samples <= CD_STRIP && smem <= CD_LDS;
 }
 
 template <typename T, int KW, int ROWS, int VW, int NPOS>
@@ -620,7 +629,7 @@ int launch_conv_taps16(void* out, const void* in, const void* w, const void* bia
     // An output over the weights: a workgroup reads them for every 32 channels while others already store, so they are copied first.
     const char *out0 = (const char*)out, *w0 = (const char*)w;
     const bool apart = out0 + (size_t)batch * C_to * H * W * 2 <= w0 || w0 + (size_t)total * 2 <= out0;
-    const bool by_channel = kH == 3 && kW == 3 && !for_input_grad && apart && ((uintptr_t)w & 15) == 0 && (long long)groups * ((C_to + CD_CO - 1) / CD_CO) <= 256;
+    const bool by_channel = kH == 3 && kW == 3 && !for_input_grad && apart && ((uintptr_t)w & 15) == 0 && (long long)groups * ((C_to + CD_CO - 1) / CD_CO) <= cus_of_device();
     void* wt = nullptr;
     if (!by_channel && rp_hip_malloc(&wt, (size_t)total * 2) != 0) return -1;
     if (!by_channel) hipLaunchKernelGGL(conv_weights_by_tap_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, current_stream(), (uint16_t*)wt, (const uint16_t*)w, C_from, C_to, taps, total,
@@ -646,6 +655,12 @@ bool conv_dw16_takes(int batch, int C_in, int C_out, int H, int W, int kH, int k
     // 5 x 5 taps on rows of arbitrary width: the words fetched for every tap row of every 64 x 64 channels cost more than the
     // padded planes, except for the narrowest images (us, here and there: 6 x 192 x 41 x 41 50 / 43, 21 x 64 x 18 x 18 29 / 25, 32 x 256 x 7 x 7 51 / 117)
     if (kW == 5 && W % 4 != 0 && W > 8) return false;
+    // The same words make three taps a row slower than the planes where every workgroup walks several strips of many channels (3 x 3, us,
+    // here and there, tiles of 64 x 64 channels times strips of the batch: 10 x 128 x 75 x 75 -> 256 6000 of them 232 / 124, 12 x 192 x 53 x 53
+    // -> 256 3816 156 / 121, 9 x 256 x 33 x 33 -> 256 1584 81 / 66, 4 x 192 x 41 x 41 -> 256 984 53 / 43; 27 x 64 x 35 x 23 -> 256 756 51 / 58,
+    // 31 x 192 x 15 x 15 -> 256 708 43 / 55; one tile, 64 strips and 2486, 18 / 34 and 110 / 133)
+    const long long tiles = (long long)((C_in + 63) / 64) * ((C_out + 63) / 64), strips = ((long long)batch * H + dw_rows(W) - 1) / dw_rows(W);
+    if (W % 4 != 0 && tiles > 1 && tiles * strips > 800) return false;
     return (long long)H * W >= 4 && dw_smem(W, kW) <= CD_LDS;
 }
 
@@ -674,7 +689,7 @@ int launch_conv_dw16(void* dw, const void* dy, const void* x, int batch, int C_i
     const int rows = dw_rows(W);
     const int strips = (int)(((long long)batch * H + rows - 1) / rows);
     const int tiles = ((C_in + 63) / 64) * ((C_out + 63) / 64);
-    int splits = CD_DW_BLOCKS / (tiles * kH);
+    int splits = dw_blocks() / (tiles * kH);
     splits = splits < 1 ? 1 : (splits > strips ? strips : splits);
     const int per_split = (strips + splits - 1) / splits;
     splits = (strips + per_split - 1) / per_split;

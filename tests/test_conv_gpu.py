@@ -178,7 +178,8 @@ DIRECT_CASES = [  # (batch, C_in, H, W, C_out, kH, kW) and the kernels of forwar
     ((70, 64, 31, 31, 64, 3, 3), T256, T256, DW), ((66, 64, 30, 34, 64, 1, 5), T256, T256, PLANES), ((24, 64, 12, 300, 64, 3, 3), PLANES, PLANES, PLANES),
     ((1, 64, 1, 1, 64, 3, 3), PLANES, PLANES, PLANES), ((90, 64, 28, 28, 64, 3, 3), T256, T256, DW), ((64, 64, 56, 56, 64, 3, 3), T256, T256, DW),
     ((90, 64, 28, 28, 64, 5, 5), T256, T256, DW), ((64, 64, 32, 32, 64, 5, 5), T256, T256, DW), ((70, 64, 31, 31, 64, 5, 5), T256, T256, PLANES),
-    ((23, 64, 56, 52, 64, 3, 3), PLANES, PLANES, DW), ((29, 64, 48, 48, 64, 5, 5), PLANES, PLANES, DW)]
+    ((23, 64, 56, 52, 64, 3, 3), PLANES, PLANES, DW), ((29, 64, 48, 48, 64, 5, 5), PLANES, PLANES, DW),
+    ((12, 128, 39, 39, 192, 5, 5), PLANES, PLANES, PLANES), ((40, 128, 31, 31, 192, 3, 3), T256, T256, PLANES)]
 
 
 @pytest.mark.parametrize("dt", [F16, BF16], ids=lambda d: NAMES[d])
