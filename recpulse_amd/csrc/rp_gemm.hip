@@ -248,7 +248,7 @@ static bool overlap(const Span& a, const Span& b) { return a.lo < b.hi && b.lo <
 // 40.7 / 42.5; against 64 x 64 tiles 256 x 2048 x 2048 10.6 / 9.0, 1024 x 4096 x 512 16.9 / 22).
 // B row-major: up to one 16 x 64 tile per CU, against the k split while k is up to 2048 (64 x 2048 x 2048 9.7 / 6.9, 64 x 4096 x 1024 10.0 / 11.7,
 // 96 x 4096 x 4096 with 384 tiles 16.4 / 19.2).
-// From ten slabs on: the eight of 128 x 512 x 512 take 5.3 and 4.8, and a small layer's dX keeps the bits it has in one launch with dW.
+// From ten slabs on: the eight of 128 x 512 x 512 take 5.3 and 4.8.  A small layer's dX in one launch with dW follows the same rule.
 // (The k split with a launch of its own for the sums read all of its operands before it wrote C: outputs over an operand stay there.)
 static bool wavek16_takes(const GemmArgs& g, const Plan& p, int dtype) {
     if ((dtype != RP_DTYPE_BFLOAT16 && dtype != RP_DTYPE_FLOAT16) || p.ragged || p.a_mc || g.batch != 1 || path_disabled("wavek")) return false;
@@ -425,13 +425,15 @@ constexpr int LINEAR_DB_ROWS = 1024;
 // Whether dX and dW of a 16-bit Linear layer go out as one launch: both on the 64 x 64 tile (an output of under half a CU count
 // of 128 x 128 tiles) in the layouts of dense X and W, and neither gradient written over anything that the other product reads
 // (one launch after the other, dW over W was fine).  Larger tiles fill a CU by themselves and gain nothing from company.
-static bool linear_backward_pairs(const GemmArgs& gx, const GemmArgs& gw, int dtype, bool& edge) {
+// dx_wavek: dX by itself would go to the kernel whose waves split k, and does so in the one launch too: the same bits either way.
+static bool linear_backward_pairs(const GemmArgs& gx, const GemmArgs& gw, int dtype, bool& edge, bool& dx_wavek) {
     if (path_disabled("pair16") || !(aligned16(gx.A) && aligned16(gx.B) && aligned16(gw.A))) return false;
     const Plan px = make_plan(1, gx.m, gx.k, gx.n, gx.a_rs, gx.a_cs, gx.b_rs, gx.b_cs, gx.c_rs, gx.c_cs, 0, 0, dtype);
     const Plan pw = make_plan(1, gw.m, gw.k, gw.n, gw.a_rs, gw.a_cs, gw.b_rs, gw.b_cs, gw.c_rs, gw.c_cs, 0, 0, dtype);
     if (px.fam != FAM_MFMA16 || px.bm != 64 || px.bn != 64 || px.ragged || px.a_mc || px.b_mc) return false;
     if (pw.fam != FAM_MFMA16 || pw.bm != 64 || pw.bn != 64 || pw.ragged || !pw.a_mc || !pw.b_mc) return false;
-    edge = px.edge || pw.edge;
+    dx_wavek = wavek16_takes(gx, px, dtype);
+    edge = pw.edge || (px.edge && !dx_wavek);
     const Span dx = span_of(gx.C, gx.m, gx.n, gx.c_rs, gx.c_cs, 2), dw = span_of(gw.C, gw.m, gw.n, gw.c_rs, gw.c_cs, 2);
     const Span dy = span_of(gx.A, gx.m, gx.k, gx.a_rs, gx.a_cs, 2), w = span_of(gx.B, gx.k, gx.n, gx.b_rs, gx.b_cs, 2), x = span_of(gw.A, gw.m, gw.k, gw.a_rs, gw.a_cs, 2);
     return !(overlap(dx, dw) || overlap(dx, dy) || overlap(dx, x) || overlap(dw, dy) || overlap(dw, w));
@@ -517,15 +519,15 @@ int rp_hip_linear_backward(void* dx, void* dw, void* db, const void* dy, const v
         if (!dw) gw.m = 0;
         return launch_linear_backward_tiny(gx, gw, db, dy, m, n, accumulate_db);
     }
-    bool edge = false;
-    if ((dtype == RP_DTYPE_BFLOAT16 || dtype == RP_DTYPE_FLOAT16) && dx && dw && linear_backward_pairs(gx, gw, dtype, edge)) {
+    bool edge = false, dx_wavek = false;
+    if ((dtype == RP_DTYPE_BFLOAT16 || dtype == RP_DTYPE_FLOAT16) && dx && dw && linear_backward_pairs(gx, gw, dtype, edge, dx_wavek)) {
         g_last_kernel = "linear_backward16_64x64";
         // The bias gradient rides along unless it would be written over something that is still read (one launch after the other
         // was fine), or its chain of chunks outlasts the products.
         const Span b = span_of(db, 1, n, 0, 1, 2), dys = span_of(dy, m, n, n, 1, 2), ws = span_of(w, k, n, w_rs, w_cs, 2), xs = span_of(x, m, k, x_rs, x_cs, 2);
         const Span dxs = span_of(dx, m, k, dx_rs, dx_cs, 2), dws = span_of(dw, k, n, dw_rs, dw_cs, 2);
         const bool rides = db && m <= LINEAR_DB_ROWS && !(overlap(b, dys) || overlap(b, ws) || overlap(b, xs) || overlap(b, dxs) || overlap(b, dws));
-        if (launch_linear_backward16(gx, gw, rides ? db : nullptr, accumulate_db, edge, dtype) != 0) return -1;
+        if (launch_linear_backward16(gx, gw, dx_wavek, rides ? db : nullptr, accumulate_db, edge, dtype) != 0) return -1;
         if (rides) return 0;
     } else {
         if (dx && run_gemm(gx, dtype) != 0) return -1;

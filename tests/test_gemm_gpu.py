@@ -720,6 +720,35 @@ def test_linear_backward_pair_16bit(dt, shape):
 
 
 @pytest.mark.parametrize("dt", HALF, ids=lambda d: NAMES[d])
+@pytest.mark.parametrize("shape", [(8, 8, 640), (72, 136, 648), (40, 24, 4104), (33, 72, 1032), (64, 256, 4096), (300, 304, 640), (264, 312, 1600),
+                                   (248, 1000, 1544), (512, 512, 640), (1024, 256, 704), (64, 1024, 1024)], ids=lambda s: "x".join(map(str, s)))
+def test_linear_backward_pair_whose_dx_splits_k(dt, shape):
+    """Layers whose dX has few tiles and a deep reduction: in one launch with dW and db, alone in its own call and as a separate product
+    the same bits (every tile size of the kernel whose waves split k, whole and ragged), accumulated and in padded rows too."""
+    m, k, n = shape
+    rng = np.random.default_rng(m + k + n)
+    L, pad = capi.lib(), 3
+    x, w, dy = rand_storage(rng, (m, k), dt), rand_storage(rng, (k, n), dt), rand_storage(rng, (m, n), dt)
+    dx0, dw0, db0 = rand_storage(rng, (m, k + pad), dt), rand_storage(rng, (k, n + pad), dt), rand_storage(rng, (n,), dt)
+    d_x, d_w, d_dy = Dev(x, dt), Dev(w, dt), Dev(dy, dt)
+    for acc in (0, 1):
+        want = Dev(dx0, dt), Dev(dw0, dt), Dev(db0, dt)
+        capi.gemm(want[0].ptr, d_dy.ptr, d_w.ptr, None, 1, m, n, k, (0, n, 1), (0, 1, n), (0, k + pad, 1), bool(acc), dt)
+        assert capi.last_gemm_kernel() == "mfma16_wavek"
+        capi.gemm(want[1].ptr, d_x.ptr, d_dy.ptr, None, 1, k, m, n, (0, 1, k), (0, n, 1), (0, n + pad, 1), bool(acc), dt)
+        capi.check(L.rp_hip_reduce_rows(want[2].ptr, d_dy.ptr, m, n, acc, dt), "reduce_rows")
+        got, alone = (Dev(dx0, dt), Dev(dw0, dt), Dev(db0, dt)), Dev(dx0, dt)
+        capi.check(L.rp_hip_linear_backward(got[0].ptr, got[1].ptr, got[2].ptr, d_dy.ptr, d_x.ptr, d_w.ptr, m, k, n,
+                                            k, 1, n, 1, k + pad, 1, n + pad, 1, acc, acc, acc, dt), "linear_backward")
+        assert capi.last_gemm_kernel() == "linear_backward16_64x64"
+        capi.check(L.rp_hip_linear_backward(alone.ptr, None, None, d_dy.ptr, None, d_w.ptr, m, k, n,
+                                            0, 0, n, 1, k + pad, 1, 0, 0, acc, 0, 0, dt), "linear_backward (dX alone)")
+        for name, a, b in zip(("dX", "dW", "db"), got, want):
+            assert np.array_equal(a.numpy(), b.numpy()), name
+        assert np.array_equal(alone.numpy(), want[0].numpy())
+
+
+@pytest.mark.parametrize("dt", HALF, ids=lambda d: NAMES[d])
 @pytest.mark.parametrize("m,n", [(8, 8), (64, 72), (248, 40), (256, 264), (264, 32), (520, 1032), (1024, 136), (1032, 64), (2048, 136), (2056, 64)])
 def test_bias_gradient_beside_the_paired_gradients(dt, m, n):
     """db in the launch of dX and dW (up to 1024 rows), around its chunks of rows and strips of columns: the bits of
