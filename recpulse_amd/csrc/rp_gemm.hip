@@ -44,19 +44,23 @@ static int cu_tiles() {
 // Whether 128 x 128 tiles are faster than 256 x 256 ones, by what the CU with the most tiles takes.  us on one CU, measured: a slab of
 // the large tile 1.32 while at most three quarters of the CUs have one, 1.55 (the power limit) when all do, and 7 a tile for its
 // prologue and epilogue, 16 where the tile hangs over the output (that kernel spills registers); a slab of the small tile 0.53 and
-// 1.2 a tile with two of them on a CU, 0.62 and 2 alone.  The large tile keeps what is within 5 % (and ragged rows, whose loads take
-// twice as long to issue: it issues half as many).  bf16, us, 256 and 128:
+// 1.2 a tile with two of them on a CU, 0.62 and 2 alone, a fifth more where small tiles hang over the output or k, a third with both
+// operands k-contiguous (3600 x 816 x 7904 that way 80 / 109, 3368 x 5960 x 3440 fp16, A^T and B^T, 175 / 212), and a tenth more from five tiles
+// a CU on (the power limit again: 7168 x 6144 x 2944 fp16 315 / 386).  The large tile keeps what is within 5 % (and ragged rows, whose
+// loads take twice as long to issue: it issues half as many).  Over 450 drawn outputs the choice costs 1.7 % against the better of the two
+// and saves 11 % against large tiles alone.  bf16, us, 256 and 128:
 // 8000 x 1152 x 1024 46.7 / 27.3, 5696 x 384 x 3584 50.8 / 28.8, 3328 x 640 x 5056 65.9 / 35.4, 4096 x 8192 x 2048 171 / 141,
 // 6144 x 1024 x 4096 62.1 / 59.4; 3072^3 71.8 / 77.7, 4096^3 108 / 140, 7808 x 3520 x 4928 279 / 292.  From six slabs on: below, the
 // two are a microsecond or two apart (3072 x 256 x 3072 15.8 / 14.1).
-static bool small_tiles_win(long long tiles256, long long tiles128, int m, int n, int k) {
+static bool small_tiles_win(long long tiles256, long long tiles128, int m, int n, int k, bool both_kc) {
     const int cus = cu_tiles();
     const double slabs = (k + M16_BK - 1) / M16_BK;
     if (slabs < 6) return false;
     const long long most256 = (tiles256 + cus - 1) / cus, most128 = (tiles128 + cus - 1) / cus;
-    const bool hangs_over = m % 256 || n % 256 || k % M16_BK;
+    const bool hangs_over = m % 256 || n % 256 || k % M16_BK, hangs_over128 = m % 128 || n % 128 || k % M16_BK;
+    const double slabs128 = slabs * (!hangs_over128 ? 1 : both_kc ? 1.35 : 1.2) * (most128 >= 5 ? 1.1 : 1);
     const double t256 = 3 + most256 * (slabs * (tiles256 * 4 <= cus * 3ll ? 1.32 : 1.55) + (hangs_over ? 16 : 7));
-    const double t128 = 3 + (most128 == 1 ? slabs * 0.62 + 2 : most128 * (slabs * 0.53 + 1.2));
+    const double t128 = 3 + (most128 == 1 ? slabs128 * 0.62 + 2 : most128 * (slabs128 * 0.53 + 1.2));
     return t128 < 0.95 * t256;
 }
 
@@ -67,7 +71,7 @@ static void choose_tile16(Plan& p, int batch, int m, int k, int n) {
     const long long tiles128 = (long long)((m + 127) / 128) * ((n + 127) / 128) * batch;
     // the 256 x 256 tile runs one block per CU, so it needs a k loop long enough to hide its prologue and
     // epilogue; with fewer than four slabs the smaller tile (two blocks per CU) overlaps them instead
-    if (m >= 256 && n >= 256 && tiles256 >= cu_tiles() / 2 && k >= 4 * M16_BK && (p.ragged || !small_tiles_win(tiles256, tiles128, m, n, k))) { p.bm = 256; p.bn = 256; p.name = "mfma16_256x256"; }
+    if (m >= 256 && n >= 256 && tiles256 >= cu_tiles() / 2 && k >= 4 * M16_BK && (p.ragged || !small_tiles_win(tiles256, tiles128, m, n, k, !p.a_mc && !p.b_mc))) { p.bm = 256; p.bn = 256; p.name = "mfma16_256x256"; }
     // fewer than 128 tiles of 128 x 128 would leave over half the CUs idle: the 64 x 64 tile quadruples the workgroups
     // (1024^3: 10.9 -> 7.3 us)
     // at most 64 rows: a 64 x 256 tile (the same 64 x 64 patch per wave as the 128 x 128 tile, none of it past the last row)

@@ -93,3 +93,19 @@ def test_kernel_selection_of_ragged_rows_and_overlapping_k():
     assert name(1, 1411, 129, 1500, (1, 1411), (1500, 1), (1500, 1), capi.F64) == "mfma64_64x64"
     assert name(1, 3001, 31, 2999, (31, 1), (2999, 1), (2999, 1), capi.F32) == "mfma32_64x64"
     assert name(1, 3001, 129, 2999, (129, 1), (2999, 1), (2999, 1), capi.F32) == "mfma32_128x128"
+
+
+def test_kernel_selection_between_large_and_small_16bit_tiles():
+    """Outputs on either side of the rule for 256 x 256 and 128 x 128 tiles; us with the large and the small one."""
+    layouts = {"nn": lambda m, k, n: ((k, 1), (n, 1)), "nt": lambda m, k, n: ((k, 1), (1, k)), "tn": lambda m, k, n: ((1, m), (n, 1)), "tt": lambda m, k, n: ((1, m), (1, k))}
+    for dt, m, k, n, layout, kernel in [
+            (capi.BF16, 3600, 816, 7904, "nt", "mfma16_256x256"),        # 80 / 109: small tiles that hang over, both operands k-contiguous
+            (capi.F16, 3368, 5960, 3440, "tt", "mfma16_256x256"),        # 175 / 212: that hang over
+            (capi.F16, 7168, 6144, 2944, "tn", "mfma16_256x256"),        # 315 / 386: six whole small tiles a CU
+            (capi.BF16, 4096, 4096, 4096, "nn", "mfma16_256x256"),       # 108 / 140
+            (capi.F16, 4352, 704, 7744, "tn", "mfma16_128x128"),         # 113 / 73
+            (capi.F16, 1472, 832, 5504, "nn", "mfma16_128x128"),         # 47 / 33
+            (capi.BF16, 8000, 1152, 1024, "nn", "mfma16_128x128"),       # 47 / 27
+            (capi.BF16, 4120, 800, 2504, "tn", "mfma16_128x128")]:       # 43 / 34, hanging over
+        a, b = layouts[layout](m, k, n)
+        assert capi.gemm_kernel_name(1, m, k, n, a, b, (n, 1), dt) == kernel, (m, k, n, layout)
