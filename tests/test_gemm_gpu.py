@@ -353,6 +353,25 @@ def test_streaming_rows_finish_repeats_bit_for_bit_over_hundreds_of_launches(m):
     assert oracle.rel_err(oracle.to_f64(first, dt), want) <= tol(dt, k)
 
 
+@pytest.mark.parametrize("dt,m,k,n", [(BF16, 17, 1032, 16648), (F16, 32, 2056, 16904), (F16, 104, 4168, 2312), (BF16, 40, 4104, 4168), (BF16, 96, 2056, 5480)])
+def test_tiled_rows_split_k_with_both_operands_k_contiguous(dt, m, k, n):
+    """More 32 x 32 tiles than the kernel whose waves split k takes: the k split in two launches, k and n ragged against slabs and strips, one
+    to four row tiles, with bias and accumulation, repeated; small integers bit for bit."""
+    rng = np.random.default_rng(45)
+    a, b = _operands(rng, m, k, n, dt, "nt")
+    bias, c0 = rand_storage(rng, (n,), dt), rand_storage(rng, (m, n), dt)
+    first = device_gemm(a, b, dt, bias=bias, c_init=c0, accumulate=True)
+    assert capi.last_gemm_kernel() == "mfma16_skinny_32x128"
+    want = oracle.to_f64(a, dt) @ oracle.to_f64(b, dt) + oracle.to_f64(bias, dt) + oracle.to_f64(c0, dt)
+    assert oracle.rel_err(oracle.to_f64(first, dt), want) <= tol(dt, k)
+    for _ in range(3):
+        assert np.array_equal(first, device_gemm(a, b, dt, bias=bias, c_init=c0, accumulate=True))
+    ai, bi = rng.integers(-2, 3, a.shape).astype(np.float32), rng.integers(-2, 3, b.shape).astype(np.float32)
+    a[...], b[...] = oracle.to_storage(ai.astype(np.float64), dt), oracle.to_storage(bi.astype(np.float64), dt)
+    assert np.array_equal(device_gemm(a, b, dt), oracle.to_storage((ai @ bi).astype(np.float64), dt))
+    assert capi.last_gemm_kernel() == "mfma16_skinny_32x128"
+
+
 @pytest.mark.parametrize("layout", LAYOUTS)
 def test_tiled_rows_split_k_ragged(layout):
     """More rows or another operand layout: the tiled kernel splits k across the grid and a second kernel adds the
@@ -606,6 +625,23 @@ def test_deep_prefetch_small_tiles(m, k, n, dt, layout):
     got = device_gemm(av, bv, dt, bias=bias)
     # sums of at most 1535 products of at most 4 in magnitude whose spread is about 80: rounded to 16 bits once, then the bias once
     assert np.array_equal(got, oracle_gemm(av, bv, dt, bias=bias))
+
+
+@pytest.mark.parametrize("layout", LAYOUTS)
+@pytest.mark.parametrize("dt", HALF, ids=lambda d: NAMES[d])
+@pytest.mark.parametrize("m,k,n", [(576, 704, 512), (576, 768, 512), (576, 832, 512), (576, 896, 512), (520, 712, 504), (520, 776, 504), (520, 840, 504), (520, 904, 504)])
+def test_deep_prefetch_small_tiles_of_every_layout(m, k, n, dt, layout):
+    """The same for outputs of more tiles than the kernel whose waves split k takes, whichever way round A lies: eleven slabs (one at a time)
+    to fifteen (three at a time, every remainder), whole and hanging over."""
+    rng = np.random.default_rng(m + k)
+    a, b = rng.integers(-2, 3, (m, k)).astype(np.float32), rng.integers(-2, 3, (k, n)).astype(np.float32)
+    bias = rng.integers(-3, 4, n).astype(np.float64)
+    sa, sb = (oracle.to_storage(np.ascontiguousarray(v if lay == "n" else v.T).astype(np.float64), dt) for v, lay in zip((a, b), layout))
+    got = device_gemm(sa if layout[0] == "n" else sa.T, sb if layout[1] == "n" else sb.T, dt, bias=oracle.to_storage(bias, dt))
+    assert capi.last_gemm_kernel() == "mfma16_64x64"
+    # sums of at most 904 products of at most 4 in magnitude, exact in fp32; one rounding each for the product and the bias
+    product = oracle.to_f64(oracle.to_storage((a @ b).astype(np.float64), dt), dt)
+    assert np.array_equal(got, oracle.to_storage(product + bias, dt))
 
 
 @pytest.mark.parametrize("dt", ALL, ids=lambda d: NAMES[d])
