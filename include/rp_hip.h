@@ -141,7 +141,8 @@ int rp_hip_gemm_strided_batched_noalloc(void* C, const void* A, const void* B, c
                                         int accumulate, int dtype);
 
 /* Name of the kernel family the dispatcher picks for a problem, for logs and
- * tests ("mfma16_256x256", "skinny", "generic", ...).  No device work. */
+ * tests ("mfma16_256x256", "skinny", "generic", ...).  No device work.  "mfma16_wavek", which stands in for "mfma16_64x64" and
+ * "mfma16_skinny_32x128" where C lies apart from the operands, is named by rp_hip_last_gemm_kernel alone. */
 const char* rp_hip_gemm_kernel_name(int batch, int m, int k, int n,
                                     long long a_rs, long long a_cs,
                                     long long b_rs, long long b_cs,
@@ -252,8 +253,8 @@ int rp_hip_cross_entropy_backward(void* grad_logits, const void* logits, const i
 /* Cross-entropy with every reduction (0 none, 1 mean, 2 sum: ops/ops.h:109-111) on logits (from_logits != 0:
  * log_softmax + softmax inside) or on probabilities (from_logits == 0: log(x), as op_cross_entropy_loss does when its
  * input came out of op_softmax, ops/ops.c:5553-5585).  x [batch, classes], float32 / float64; targets: device
- * int32[batch].  loss_out: batch elements for 'none', one otherwise (the NLL terms summed in batch order in double,
- * ops/ops.c:5342-5352). */
+ * int32[batch].  loss_out: batch elements for 'none', one otherwise (the NLL terms summed in double as in ops/ops.c:5342-5352, there
+ * row after row, here by lanes and workgroups whose sums are added in a fixed order). */
 int rp_hip_cross_entropy_forward(void* loss_out, const void* x, const int* targets, int batch, int classes,
                                  int reduction, int from_logits, int dtype);
 /* Its gradient (backward_cross_entropy_loss_fn, ops/ops.c:5412-5543, which the reference builds on the host):
@@ -288,7 +289,8 @@ int rp_hip_col2im_batched(void* im, const void* col, int batch, int C_in, int H,
  * output size) when the channel count that is summed over is a multiple of 64 (bfloat16 / float16), 32 (float32)
  * or 16 (float64); rp_hip_conv2d_same_supported says whether a shape qualifies, reduced_channels 0 asks about
  * geometry and dtype alone.  x [batch, C_in, H, W], w [C_out, C_in, kH, kW], y / dy [batch, C_out, H, W], all dense.
- * The input is copied once into zero-bordered planes and the GEMM reads every tap from that copy in place; the sum
+ * 16-bit images with taps of k x 3 and k x 5 are read in place where that is the faster way; all others, and an output that
+ * overlaps its image, go by one copy in zero-bordered planes from which the GEMM reads every tap.  Either way the sum
  * over taps and channels is kept in the accumulate type (fp32; fp64 for float64) and rounded once, then the bias
  * is added with its own rounding as in rp_hip_channel_bias_add.  They stand in for the per-sample
  * im2col + matmul (+ col2im) loops of op_conv2d and backward_conv2d_fn (ops/ops.c:4759-4783, 4533-4551). */
@@ -297,11 +299,13 @@ int rp_hip_conv2d_same_forward(void* y, const void* x, const void* w, const void
                                int C_out, int kH, int kW, int dtype);
 int rp_hip_conv2d_same_backward_input(void* dx, const void* dy, const void* w, int batch, int C_in, int H, int W,
                                       int C_out, int kH, int kW, int dtype);
-/* Both gradients from one zero-bordered copy of dy; dx or dw may be NULL (x is read only for dw, w only for dx).
+/* Both gradients; dx or dw may be NULL (x is read only for dw, w only for dx), and a gradient's bits do not depend on whether
+ * the other is asked for unless dx overlaps dy.  dx is stored before dw, which may lie over w.
  * dx needs rp_hip_conv2d_same_supported(C_out, ...); dw [C_out, C_in, kH, kW] needs
  * rp_hip_conv2d_same_supported(0, ...), i.e. only the geometry and the dtype: its reduction runs over the positions
- * of a sample (every (tap, channel) column of the GEMM is a shifted plane of the padded input), the per-sample
- * products are rounded and then summed over the batch in fp32 as in the lowered path (ops/ops.c:4575-4617). */
+ * (every (tap, channel) column of the GEMM is a shifted plane of the image).  dw of 16-bit images read in place ("conv_dw16",
+ * rp_hip_last_gemm_kernel) is summed in fp32 over positions and batch and rounded once; from zero-bordered planes the
+ * products of each sample are rounded to the dtype and then summed over the batch in the accumulate type and rounded, as in the lowered path (ops/ops.c:4575-4617). */
 int rp_hip_conv2d_same_backward(void* dx, void* dw, const void* dy, const void* x, const void* w, int batch, int C_in, int H, int W,
                                 int C_out, int kH, int kW, int dtype);
 

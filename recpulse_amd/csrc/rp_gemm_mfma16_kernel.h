@@ -147,8 +147,8 @@ struct FragMap {
 
 // PF: slabs of both operands that travel in registers at a time, each in a set of its own.  One set gives a load the time of one
 // slab to arrive.  For the 64 x 64 tile that is less than a load from another XCD's memory takes, and with the one or two workgroups
-// per CU of a small product nothing else covers it; three sets do (bf16, us, 1 set and 3: 1024^3 8.9 / 8.0, 256 x 4096 x 256 23.1 / 17.4,
-// 64 x 1024 x 4096 8.4 / 7.5).  The 128 x 128 tile gains nothing (2048^3 20.5 / 20.3: it is bound by what a CU can fetch from its L2,
+// per CU of a small product nothing else covers it; three sets do (bf16, us, 1 set and 3: 1024^3 9.0 / 8.1, 768 x 1024 x 768
+// 9.0 / 7.5, 1024 x 2048 x 512 14.3 / 11.4, with A^T 256 x 4096 x 256 23.4 / 18.2 and 64 x 1024 x 4096 8.4 / 7.4; hanging over 520 x 904 x 504 9.3 / 9.3).  The 128 x 128 tile gains nothing (2048^3 20.5 / 20.3: it is bound by what a CU can fetch from its L2,
 // 32 KB a slab at 39 B a cycle).  The loop runs whole rounds of PF slabs, up to two of them zeros, which a k of few slabs would feel
 // (600 x 264 x 600 6.4 / 6.9): from twelve slabs on.  Two workgroups on a CU cover each other's loads, and the registers of the sets get in
 // their way (fp16, us: 396 tiles of 2304 x 2880 x 704 25.0 / 30.0, 336 of 3584 x 5696 x 384 53.8 / 57.7; 256 of 2048 x 8192 x 512 63.1 / 38.6): up to one

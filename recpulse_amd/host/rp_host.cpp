@@ -1070,8 +1070,8 @@ bool conv_is_pointwise(const ConvSaved& c) {              // 1x1, unit stride, n
 }
 
 // Stride 1, no dilation, odd kernel with padding (k - 1) / 2 and `reduced` channels in whole k slabs of
-// the GEMM: the convolution (reduced = C_in) or its input gradient (reduced = C_out) reads its taps from zero-bordered
-// planes and never builds the lowered matrix.  RP_CONV_NO_DIRECT=1 keeps the lowered path (read at every call).
+// the GEMM: the convolution (reduced = C_in) or its input gradient (reduced = C_out) reads its taps from the image
+// or from zero-bordered planes and never builds the lowered matrix.  RP_CONV_NO_DIRECT=1 keeps the lowered path (read at every call).
 bool conv_direct(const ConvSaved& c, DType dt, int reduced) {
     const char* e = getenv("RP_CONV_NO_DIRECT");
     if (e && e[0] == '1') return false;
@@ -1102,13 +1102,13 @@ void backward_conv2d_fn(GradFn* self, Tensor* grad_output) {         // referenc
     const bool direct_dx = !pointwise && conv_direct(c, dt, c.Co), direct_dw = !pointwise && conv_direct(c, dt, 0);
     if (ok && !pointwise && ((needs_grad(x) && !direct_dx) || (needs_grad(w) && !direct_dw))) ok = rp_hip_malloc(&col, (size_t)chunk * col_n * esz) == 0;
     if (ok && ((needs_grad(x) && direct_dx) || (needs_grad(w) && direct_dw))) {
-        // both gradients from one zero-bordered copy of dy, no lowered matrix
+        // both gradients in one call, no lowered matrix
         Tensor* dx = (needs_grad(x) && direct_dx) ? empty_tensor(dt, x->device_id, x->ndim, x->shape) : nullptr;
         Tensor* dw = (needs_grad(w) && direct_dw) ? empty_tensor(dt, w->device_id, w->ndim, w->shape) : nullptr;
         const bool good = (dx || dw) && rp_hip_conv2d_same_backward(dx ? dx->data : nullptr, dw ? dw->data : nullptr, g->data, xd->data, wd->data,
                                                                     c.N, c.C, c.H, c.W, c.Co, c.kH, c.kW, dt) == 0;
         if (good) { if (dx) accumulate_grad(x, dx); if (dw) accumulate_grad(w, dw); }
-        else { dev_fail("op_conv2d backward (padded planes)"); free_tensor(dx); free_tensor(dw); ok = false; }
+        else { dev_fail("op_conv2d backward (same padding)"); free_tensor(dx); free_tensor(dw); ok = false; }
     }
     if (ok && needs_grad(x) && !direct_dx) {
         // dcol[n] = W^T . dy[n], then each input pixel gathers its taps
