@@ -420,11 +420,12 @@ int* noalloc_arrival_counters() {
     return (int*)g_noalloc_base;
 }
 
-// Rows up to which the column sums of dY join the other gradients of a 16-bit layer: four chunks of 256.  A strip's chunks are a chain
-// that narrow or uneven strips walk at up to 2.2 us a chunk, and a launch of their own costs 3 to 4 us (bf16, us, in the launch and
-// apart: 256 x 256 x 1024 7.0 / 11.4, 1024 x 512 x 512 8.9 / 12.0, 1024 x 8 x 16 11.7 / 11.5, 1280 x 768 x 264 16.4 / 15.1,
-// 1536 x 8 x 16 16.6 / 14.0, 2048 x 40 x 16 21.8 / 16.5, 2048 x 512 x 512 21.2 / 19.3).
-constexpr int LINEAR_DB_ROWS = 1024;
+// Rows up to which the column sums of dY join the other gradients of a 16-bit layer: four chunks of 256, three where a strip of 64 bytes
+// hangs over the columns.  A strip's chunks are a chain that uneven strips walk at up to 2.2 us a chunk, and a launch of their own
+// costs 3 to 4 us (bf16, us, in the launch and apart: 256 x 256 x 1024 7.0 / 11.4, 1024 x 512 x 512 10.0 / 12.5, 1024 x 16 x 64 8.3 / 11.2,
+// 2048 x 512 x 512 21.2 / 19.3; uneven 768 x 16 x 184 10.1 / 10.2, 904 x 16 x 184 12.1 / 11.2, 1024 x 512 x 184 12.9 / 12.0,
+// 1280 x 768 x 264 16.4 / 15.1, 2048 x 40 x 16 21.8 / 16.5).
+constexpr int LINEAR_DB_ROWS = 1024, LINEAR_DB_ROWS_UNEVEN = 768;
 
 // Whether dX and dW of a 16-bit Linear layer go out as one launch: both on the 64 x 64 tile (an output of under half a CU count
 // of 128 x 128 tiles) in the layouts of dense X and W, and neither gradient written over anything that the other product reads
@@ -530,7 +531,7 @@ int rp_hip_linear_backward(void* dx, void* dw, void* db, const void* dy, const v
         // was fine), or its chain of chunks outlasts the products.
         const Span b = span_of(db, 1, n, 0, 1, 2), dys = span_of(dy, m, n, n, 1, 2), ws = span_of(w, k, n, w_rs, w_cs, 2), xs = span_of(x, m, k, x_rs, x_cs, 2);
         const Span dxs = span_of(dx, m, k, dx_rs, dx_cs, 2), dws = span_of(dw, k, n, dw_rs, dw_cs, 2);
-        const bool rides = db && m <= LINEAR_DB_ROWS && !(overlap(b, dys) || overlap(b, ws) || overlap(b, xs) || overlap(b, dxs) || overlap(b, dws));
+        const bool rides = db && m <= (n % 32 ? LINEAR_DB_ROWS_UNEVEN : LINEAR_DB_ROWS) && !(overlap(b, dys) || overlap(b, ws) || overlap(b, xs) || overlap(b, dxs) || overlap(b, dws));
         if (launch_linear_backward16(gx, gw, dx_wavek, rides ? db : nullptr, accumulate_db, edge, dtype) != 0) return -1;
         if (rides) return 0;
     } else {

@@ -785,9 +785,9 @@ def test_linear_backward_pair_whose_dx_splits_k(dt, shape):
 
 
 @pytest.mark.parametrize("dt", HALF, ids=lambda d: NAMES[d])
-@pytest.mark.parametrize("m,n", [(8, 8), (64, 72), (248, 40), (256, 264), (264, 32), (520, 1032), (1024, 136), (1032, 64), (2048, 136), (2056, 64)])
+@pytest.mark.parametrize("m,n", [(8, 8), (64, 72), (248, 40), (256, 264), (264, 32), (520, 1032), (768, 40), (776, 40), (1024, 128), (1024, 136), (1032, 64), (2048, 136), (2056, 64)])
 def test_bias_gradient_beside_the_paired_gradients(dt, m, n):
-    """db in the launch of dX and dW (up to 1024 rows), around its chunks of rows and strips of columns: the bits of
+    """db in the launch of dX and dW (up to 1024 rows, 768 where a strip of columns hangs over), around its chunks of rows and strips of columns: the bits of
     rp_hip_reduce_rows, written and added; over W, which the launch still reads, it comes in a launch of its own."""
     rng = np.random.default_rng(m + n)
     L, k = capi.lib(), 64
