@@ -24,23 +24,27 @@ static inline unsigned grid_for(size_t n, int threads = kThreads, size_t cap = 1
 
 // ---- flat maps ----------------------------------------------------------------
 // out[i] = op(x1[i], x2[i]) in the accumulate type, narrowed once.  When every pointer is 16-byte aligned each
-// thread moves whole 16-byte vectors, four per pass with all four loads in flight; a scalar loop takes the rest.
+// thread moves whole 16-byte vectors, four per pass with all four loads in flight; the elements behind the last whole
+// vector go with the first workgroup's (a launch of their own cost as much as a small map: an MLP step of 589 x 144-815-30-4,
+// two of its four maps with such a tail, 97.7 us, 92.1 now).
 template <typename A> struct AddOp { __device__ __forceinline__ A operator()(A a, A b) const { return a + b; } };
 template <typename A> struct MulScalarOp { A s; __device__ __forceinline__ A operator()(A a, A) const { return a * s; } };
 template <typename A> struct ReluOp { __device__ __forceinline__ A operator()(A a, A) const { return a > (A)0 ? a : (A)0; } };
 template <typename A> struct BackReluOp { __device__ __forceinline__ A operator()(A g, A x) const { return x > (A)0 ? g : (A)0; } };   // (grad, input)
 
 template <typename T, bool TWO, typename Op>
-__global__ void map_scalar_kernel(T* out, const T* x1, const T* x2, Op op, size_t begin, size_t n) {
+__global__ void map_scalar_kernel(T* out, const T* x1, const T* x2, Op op, size_t n) {
     using A = typename traits<T>::acc;
-    for (size_t i = begin + (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
+    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
         out[i] = narrow<T>(op(widen(x1[i]), TWO ? widen(x2[i]) : (A)0));
 }
 
 template <typename T, bool TWO, typename Op>
-__global__ void __launch_bounds__(kThreads) map_vec_kernel(T* out, const T* x1, const T* x2, Op op, size_t nvec) {
+__global__ void __launch_bounds__(kThreads) map_vec_kernel(T* out, const T* x1, const T* x2, Op op, size_t n) {
     using A = typename traits<T>::acc;
     constexpr int VEC = 16 / sizeof(T), U = 4;
+    const size_t nvec = n / VEC, last = nvec * VEC + threadIdx.x;          // fewer than VEC elements are left over
+    if (blockIdx.x == 0 && last < n) out[last] = narrow<T>(op(widen(x1[last]), TWO ? widen(x2[last]) : (A)0));
     const u32x4_t* p1 = (const u32x4_t*)x1;
     const u32x4_t* p2 = (const u32x4_t*)x2;
     u32x4_t* po = (u32x4_t*)out;
@@ -75,15 +79,13 @@ static inline bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 template <typename T, bool TWO, typename Op>
 static void launch_map(T* out, const T* x1, const T* x2, Op op, size_t n) {
     constexpr int VEC = 16 / sizeof(T);
-    size_t nvec = (aligned16(out) && aligned16(x1) && (!TWO || aligned16(x2))) ? n / VEC : 0;
-    if (nvec) {
-        size_t blocks = (nvec + kThreads * 4 - 1) / (kThreads * 4);
-        if (blocks > (1u << 20)) blocks = 1u << 20;
-        hipLaunchKernelGGL((map_vec_kernel<T, TWO, Op>), dim3((unsigned)blocks), dim3(kThreads), 0, current_stream(), out, x1, x2, op, nvec);
+    if (aligned16(out) && aligned16(x1) && (!TWO || aligned16(x2))) {
+        size_t blocks = (n / VEC + kThreads * 4 - 1) / (kThreads * 4);
+        blocks = blocks < 1 ? 1 : blocks > (1u << 20) ? 1u << 20 : blocks;
+        hipLaunchKernelGGL((map_vec_kernel<T, TWO, Op>), dim3((unsigned)blocks), dim3(kThreads), 0, current_stream(), out, x1, x2, op, n);
+    } else {
+        hipLaunchKernelGGL((map_scalar_kernel<T, TWO, Op>), dim3(grid_for(n)), dim3(kThreads), 0, current_stream(), out, x1, x2, op, n);
     }
-    size_t done = nvec * VEC;
-    if (done < n)
-        hipLaunchKernelGGL((map_scalar_kernel<T, TWO, Op>), dim3(grid_for(n - done)), dim3(kThreads), 0, current_stream(), out, x1, x2, op, done, n);
 }
 
 // p[0 .. n) = v with 16-byte stores over the aligned middle (a store of one element per lane fills half a cache line
@@ -212,9 +214,15 @@ template <typename A> __device__ __forceinline__ A lowest();
 template <> __device__ __forceinline__ float lowest<float>() { return -FLT_MAX; }
 template <> __device__ __forceinline__ double lowest<double>() { return -DBL_MAX; }
 
+// Rows of any length, one wave each.  has_scale, here and in the gradient's kernel: softmax_rows_reg_kernel says what it means (one
+// launch instead of two, three with the tail of the multiply: bf16 attention op by op, 100 heads of 95 x 64, 54.7 us, 43.2 now; 150 of 509 x 64 422 and 349).
 template <typename T, bool LOG>
-__global__ void softmax_rows_kernel(T* out, const T* x, size_t rows, size_t dim) {
+__global__ void softmax_rows_kernel(T* out, const T* x, size_t rows, size_t dim, bool has_scale, typename traits<T>::acc scale) {
     using A = typename traits<T>::acc;
+    auto value = [&](const T* p) {
+        const A v = widen(*p);
+        return has_scale ? widen(narrow<T>(v * scale)) : v;
+    };
     int lane = threadIdx.x & 63;
     size_t wave = ((size_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
     size_t nwaves = ((size_t)gridDim.x * blockDim.x) >> 6;
@@ -222,16 +230,16 @@ __global__ void softmax_rows_kernel(T* out, const T* x, size_t rows, size_t dim)
         const T* xr = x + r * dim;
         T* orow = out + r * dim;
         A mx = lowest<A>();
-        for (size_t d = lane; d < dim; d += 64) { A v = widen(xr[d]); mx = v > mx ? v : mx; }
+        for (size_t d = lane; d < dim; d += 64) { A v = value(xr + d); mx = v > mx ? v : mx; }
         mx = wave_max(mx);
         A sum = 0;
-        for (size_t d = lane; d < dim; d += 64) sum += rp_exp(widen(xr[d]) - mx);
+        for (size_t d = lane; d < dim; d += 64) sum += rp_exp(value(xr + d) - mx);
         sum = wave_sum(sum);
         if (LOG) {
             A lse = rp_log(sum);
-            for (size_t d = lane; d < dim; d += 64) orow[d] = narrow<T>(widen(xr[d]) - mx - lse);
+            for (size_t d = lane; d < dim; d += 64) orow[d] = narrow<T>(value(xr + d) - mx - lse);
         } else {
-            for (size_t d = lane; d < dim; d += 64) orow[d] = narrow<T>(rp_exp(widen(xr[d]) - mx) / sum);
+            for (size_t d = lane; d < dim; d += 64) orow[d] = narrow<T>(rp_exp(value(xr + d) - mx) / sum);
         }
     }
 }
@@ -415,7 +423,7 @@ __global__ void softmax_strided_kernel(T* out, const T* x, size_t outer, size_t 
 }
 
 template <typename T>
-__global__ void backwards_softmax_rows_kernel(const T* gc, const T* y, T* gx, size_t rows, size_t dim) {
+__global__ void backwards_softmax_rows_kernel(const T* gc, const T* y, T* gx, size_t rows, size_t dim, bool has_scale, typename traits<T>::acc scale) {
     using A = typename traits<T>::acc;
     int lane = threadIdx.x & 63;
     size_t wave = ((size_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
@@ -426,8 +434,26 @@ __global__ void backwards_softmax_rows_kernel(const T* gc, const T* y, T* gx, si
         A dot = 0;
         for (size_t d = lane; d < dim; d += 64) dot += widen(g[d]) * widen(s[d]);
         dot = wave_sum(dot);
-        for (size_t d = lane; d < dim; d += 64) gx[r * dim + d] = narrow<T>(widen(s[d]) * (widen(g[d]) - dot));
+        for (size_t d = lane; d < dim; d += 64) {
+            const T o = narrow<T>(widen(s[d]) * (widen(g[d]) - dot));
+            gx[r * dim + d] = has_scale ? narrow<T>(widen(o) * scale) : o;
+        }
     }
+}
+
+// Rows one after the other in memory, with a scalar folded in or not: the register kernel where the rows qualify
+template <typename T>
+static void launch_softmax_rows(T* out, const T* x, size_t rows, size_t dim, bool take_log, bool has_scale = false, typename traits<T>::acc scale = 1) {
+    const unsigned blocks = grid_for(rows * 64, kThreads, 1u << 16);
+    if (launch_softmax_reg<T>(out, x, rows, dim, blocks, take_log, has_scale, scale)) return;
+    if (take_log) hipLaunchKernelGGL((softmax_rows_kernel<T, true>), dim3(blocks), dim3(kThreads), 0, current_stream(), out, x, rows, dim, has_scale, scale);
+    else          hipLaunchKernelGGL((softmax_rows_kernel<T, false>), dim3(blocks), dim3(kThreads), 0, current_stream(), out, x, rows, dim, has_scale, scale);
+}
+template <typename T>
+static void launch_bsoftmax_rows(const T* gc, const T* y, T* gx, size_t rows, size_t dim, bool has_scale = false, typename traits<T>::acc scale = 1) {
+    const unsigned blocks = grid_for(rows * 64, kThreads, 1u << 16);
+    if (launch_bsoftmax_reg<T>(gc, y, gx, rows, dim, blocks, has_scale, scale)) return;
+    hipLaunchKernelGGL(backwards_softmax_rows_kernel<T>, dim3(blocks), dim3(kThreads), 0, current_stream(), gc, y, gx, rows, dim, has_scale, scale);
 }
 
 template <typename T>
@@ -950,12 +976,7 @@ int backwards_relu_device(const void* grad_c, const void* x, void* grad_x, size_
 static int softmax_any(void* out, const void* x, size_t outer, size_t dim, size_t inner, int dtype, bool take_log) {
     RP_REQUIRE(out && x && outer && dim && inner, "softmax_kernel_device");
     if (inner == 1) {
-        unsigned blocks = grid_for(outer * 64, kThreads, 1u << 16);
-        RP_DISPATCH_DTYPE(dtype, {
-            if (launch_softmax_reg<T>((T*)out, (const T*)x, outer, dim, blocks, take_log)) {}
-            else if (take_log) hipLaunchKernelGGL((softmax_rows_kernel<T, true>), dim3(blocks), dim3(kThreads), 0, current_stream(), (T*)out, (const T*)x, outer, dim);
-            else          hipLaunchKernelGGL((softmax_rows_kernel<T, false>), dim3(blocks), dim3(kThreads), 0, current_stream(), (T*)out, (const T*)x, outer, dim);
-        });
+        RP_DISPATCH_DTYPE(dtype, launch_softmax_rows<T>((T*)out, (const T*)x, outer, dim, take_log));
     } else {
         unsigned blocks = grid_for(outer * inner);
         RP_DISPATCH_DTYPE(dtype, {
@@ -978,12 +999,7 @@ int backwards_softmax_device(const void* grad_c, const void* softmax_out, void* 
                              size_t outer_size, size_t dim_size, size_t inner_size, int dtype) {
     RP_REQUIRE(grad_c && softmax_out && grad_x && outer_size && dim_size && inner_size, "backwards_softmax_device");
     if (inner_size == 1) {
-        unsigned blocks = grid_for(outer_size * 64, kThreads, 1u << 16);
-        RP_DISPATCH_DTYPE(dtype, {
-            if (launch_bsoftmax_reg<T>((const T*)grad_c, (const T*)softmax_out, (T*)grad_x, outer_size, dim_size, blocks)) {}
-            else hipLaunchKernelGGL(backwards_softmax_rows_kernel<T>, dim3(blocks), dim3(kThreads), 0, current_stream(),
-                                    (const T*)grad_c, (const T*)softmax_out, (T*)grad_x, outer_size, dim_size);
-        });
+        RP_DISPATCH_DTYPE(dtype, launch_bsoftmax_rows<T>((const T*)grad_c, (const T*)softmax_out, (T*)grad_x, outer_size, dim_size));
     } else {
         RP_DISPATCH_DTYPE(dtype, hipLaunchKernelGGL(backwards_softmax_strided_kernel<T>, dim3(grid_for(outer_size * inner_size)), dim3(kThreads), 0,
                                                    current_stream(), (const T*)grad_c, (const T*)softmax_out, (T*)grad_x,
@@ -1014,15 +1030,10 @@ int rp_hip_take_deferred(const void* out, const void** x, double* scalar) {
 int rp_hip_scaled_softmax(void* out, const void* x, const void* scalar, size_t outer_size, size_t dim_size, size_t inner_size, int dtype) {
     RP_REQUIRE(out && x && scalar && outer_size && dim_size && inner_size, "rp_hip_scaled_softmax");
     if (inner_size == 1) {
-        bool done = false;
-        unsigned blocks = grid_for(outer_size * 64, kThreads, 1u << 16);
-        RP_DISPATCH_DTYPE(dtype, {
-            using A = typename traits<T>::acc;
-            done = launch_softmax_reg<T>((T*)out, (const T*)x, outer_size, dim_size, blocks, false, true, *(const A*)scalar);
-        });
-        if (done) return check_launch("softmax kernel") ? 0 : -1;
+        RP_DISPATCH_DTYPE(dtype, launch_softmax_rows<T>((T*)out, (const T*)x, outer_size, dim_size, false, true, *(const typename traits<T>::acc*)scalar));
+        return check_launch("softmax kernel") ? 0 : -1;
     }
-    // rows the one-pass kernel does not take: the two passes, the product going through `out`
+    // an axis that is not the last one: the two passes, the product going through `out`
     if (mul_scalar_kernel_device(out, x, scalar, outer_size * dim_size * inner_size, dtype) != 0) return -1;
     return softmax_kernel_device(out, out, outer_size, dim_size, inner_size, dtype);
 }
@@ -1031,13 +1042,8 @@ int rp_hip_backwards_scaled_softmax(const void* grad_c, const void* softmax_out,
                                     size_t outer_size, size_t dim_size, size_t inner_size, int dtype) {
     RP_REQUIRE(grad_c && softmax_out && grad_x && scalar && outer_size && dim_size && inner_size, "rp_hip_backwards_scaled_softmax");
     if (inner_size == 1) {
-        bool done = false;
-        unsigned blocks = grid_for(outer_size * 64, kThreads, 1u << 16);
-        RP_DISPATCH_DTYPE(dtype, {
-            using A = typename traits<T>::acc;
-            done = launch_bsoftmax_reg<T>((const T*)grad_c, (const T*)softmax_out, (T*)grad_x, outer_size, dim_size, blocks, true, *(const A*)scalar);
-        });
-        if (done) return check_launch("backwards_softmax kernel") ? 0 : -1;
+        RP_DISPATCH_DTYPE(dtype, launch_bsoftmax_rows<T>((const T*)grad_c, (const T*)softmax_out, (T*)grad_x, outer_size, dim_size, true, *(const typename traits<T>::acc*)scalar));
+        return check_launch("backwards_softmax kernel") ? 0 : -1;
     }
     if (backwards_softmax_device(grad_c, softmax_out, grad_x, outer_size, dim_size, inner_size, dtype) != 0) return -1;
     return mul_scalar_kernel_device(grad_x, grad_x, scalar, outer_size * dim_size * inner_size, dtype);

@@ -41,6 +41,21 @@ def test_flat_maps_bit_exact(dt):
 
 
 @pytest.mark.parametrize("dt", ALL, ids=lambda d: NAMES[d])
+@pytest.mark.parametrize("over", [0, 1, -1])
+def test_flat_maps_stop_at_their_last_element(dt, over):
+    """Sizes around whole 16-byte vectors and around whole workgroups of them, in one launch; what lies behind is not written."""
+    rng = np.random.default_rng(39)
+    vec = 16 // np.dtype(capi.NP_STORAGE[dt]).itemsize
+    for n in (vec + over, 1024 * vec + over, 2048 * vec + vec // 2 + over):
+        x = rand_storage(rng, (n,), dt); y = rand_storage(rng, (n,), dt); guard = rand_storage(rng, (n + vec,), dt)
+        dx, dy, do = Dev(x, dt), Dev(y, dt), Dev(guard, dt)
+        capi.check(L().relu_kernel_device(do.ptr, dx.ptr, n, dt), "relu")
+        assert np.array_equal(do.numpy(), np.concatenate([oracle.relu(x, dt), guard[n:]]))
+        capi.check(L().backwards_relu_device(dy.ptr, dx.ptr, do.ptr, n, dt), "backwards_relu")
+        assert np.array_equal(do.numpy(), np.concatenate([oracle.backwards_relu(y, x, dt), guard[n:]]))
+
+
+@pytest.mark.parametrize("dt", ALL, ids=lambda d: NAMES[d])
 def test_broadcasting_add_bit_exact(dt):
     rng = np.random.default_rng(41)
     y = rand_storage(rng, (37, 53), dt); b = rand_storage(rng, (53,), dt)
