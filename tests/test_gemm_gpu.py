@@ -856,6 +856,23 @@ def test_small_fp32_outputs_take_one_launch():
 
 
 
+@pytest.mark.parametrize("layout", LAYOUTS)
+@pytest.mark.parametrize("m,k,n", [(17, 33, 19), (100, 131, 77), (35, 2047, 18), (3, 257, 301)])
+def test_small_fp32_outputs_of_rows_at_any_element(m, k, n, layout):
+    """Rows of odd length that start at an odd element: whole vectors along k are loaded there.  Small integers, so the sums are exact."""
+    rng = np.random.default_rng(44)
+
+    def operand(rows, cols, transposed):
+        shape = (cols, rows + 1) if transposed else (rows, cols + 1)
+        x = rng.integers(-3, 4, shape).astype(np.float32)[:, 1:]
+        return x.T if transposed else x
+
+    a, b = operand(m, k, layout[0] == "t"), operand(k, n, layout[1] == "t")
+    got = device_gemm(a, b, F32)
+    assert capi.last_gemm_kernel() == "tiny32_16x16"
+    assert np.array_equal(got, (a.astype(np.float64) @ b.astype(np.float64)).astype(np.float32))
+
+
 # ---- fp32 products with a short reduction (k <= 64) and many tiles: the resident cross-tile kernel (every layout, ragged
 # extents, k below a whole slab, bias, accumulation) and, for operands with unit stride along their free index, the
 # kernel that multiplies straight out of registers
