@@ -19,8 +19,10 @@
 //   split32  fp32 outputs of 128 x 128 tiles on the bf16 matrix cores, every value split in three (a kernel of family mfmaw).
 //   skinny   m <= 8 against a row-major B: a split-k streaming kernel bound by HBM.
 //   tiny     fp32 outputs of a few hundred 16 x 16 tiles: one launch, k split over the waves of a workgroup.
+//   wavekw   fp32 / fp64 products of few tiles, or a k that is long for them: the waves of a workgroup share k.
 //   generic  any strides, any shape; LDS-tiled scalar FMA.
 #include "rp_gemm.h"
+#include "rp_gemm_wavekw.h"
 
 #include <mutex>
 
@@ -272,6 +274,38 @@ static bool wavek16_takes(const GemmArgs& g, const Plan& p, int dtype) {
            !(g.bias && overlap(c, span_of(g.bias, 1, g.n, 0, 1, 2)));
 }
 
+// fp32 and fp64 products that the waves of a workgroup share (rp_gemm_wavekw.hip, which has figures): those of 64 x 64 tiles, fp64 ones of the generic
+// kernel, and fp32 ones that 16 x 16 tiles of four waves or the row-streaming kernel took.  Stays where it was: fp32 with k up to 512 on 16 x 16 tiles (60 x 443 x 65 3.55 / 3.67 us; 256 x 784 x 256
+// 6.95 / 5.0-6.0); a few rows with k above 1024 (8 x 8192 x 8192 55 / 51, but that kernel's sums are of shorter chains); a k too short for the number of tiles (fp32 2384 x 32 x 368
+// 5.2 / 6.5, 944 x 144 x 1648 14.0 / 16.2; fp64 832 x 48 x 2128 14.6 / 22.7); fp32 outputs of a few tiles whose long k the split deals to more CUs
+// (16 x 5744 x 48 11.5 / 14.4) and sums in shorter chains.  (The k split read all of its operands before it wrote C: outputs over an operand stay there.)
+static bool wavekw_takes(const GemmArgs& g, const Plan& p, int dtype) {
+    const bool f32 = dtype == RP_DTYPE_FLOAT32;
+    if (!(f32 || dtype == RP_DTYPE_FLOAT64) || g.seg_k || g.seg_n || g.bias_by_row || g.c_fold_from || path_disabled("wavekw")) return false;
+    const long long tiles64 = (long long)((g.m + 63) / 64) * ((g.n + 63) / 64) * g.batch, tiles16 = (long long)((g.m + 15) / 16) * ((g.n + 15) / 16) * g.batch;
+    if (p.fam == FAM_MFMAW && p.bm == 64) {
+        if (f32 ? g.k <= 32 || (tiles64 > cu_tiles() && g.k < 256) : g.k <= 48 && tiles64 > cu_tiles() / 2) return false;
+        const bool splits = f32 && (g.n % 4 == 0 || p.ragged), both_kc = g.a_cs == 1 && g.b_rs == 1 && g.b_cs != 1;
+        if (splits && g.k > 2048 && (tiles64 < cu_tiles() / 32 || (!both_kc && tiles16 < cu_tiles() / 4))) return false;
+    } else if (p.fam == FAM_TINY) {
+        if (g.k <= 512) return false;
+    } else if (p.fam == FAM_SKINNY) {
+        if (g.k > 1024) return false;
+    } else if (!(p.fam == FAM_GENERIC && !f32 && !path_disabled("mfma"))) {
+        return false;
+    }
+    if (wavekw_tile(g, dtype) == WKW_NONE) return false;
+    const int esz = (int)dtype_size(dtype);
+    auto span = [&](const void* base, int rows, int cols, long long bs, long long rs, long long cs) {
+        Span s = span_of(base, rows, cols, rs, cs, esz);
+        (bs < 0 ? s.lo : s.hi) += (g.batch - 1) * bs * esz;
+        return s;
+    };
+    const Span c = span(g.C, g.m, g.n, g.c_bs, g.c_rs, g.c_cs);
+    return !overlap(c, span(g.A, g.m, g.k, g.a_bs, g.a_rs, g.a_cs)) && !overlap(c, span(g.B, g.k, g.n, g.b_bs, g.b_rs, g.b_cs)) &&
+           !(g.bias && overlap(c, span_of(g.bias, 1, g.n, 0, 1, esz)));
+}
+
 static thread_local const char* g_last_kernel = "none";      // what rp_hip_last_gemm_kernel reports
 void report_kernel(const char* name) { g_last_kernel = name; }
 
@@ -301,6 +335,10 @@ static int run_gemm(GemmArgs g, int dtype) {
     if (p.fam != FAM_GENERIC && p.fam != FAM_TINY && !p.ragged && !(aligned16(g.A) && aligned16(g.B)))
         p = make_plan(g.batch, g.m, g.k, g.n, g.a_rs, g.a_cs, g.b_rs, g.b_cs, g.c_rs, g.c_cs, g.a_bs, g.b_bs, dtype, false, false);
     if (wavek16_takes(g, p, dtype)) { g_last_kernel = "mfma16_wavek"; return launch_mfma16_wavek(g, dtype); }
+    if (wavekw_takes(g, p, dtype)) {
+        g_last_kernel = p.fam == FAM_MFMAW ? p.name : dtype == RP_DTYPE_FLOAT32 ? "mfma32_wavek" : "mfma64_wavek";      // (among the 64 x 64 tiles it goes by their name)
+        return launch_wavekw(g, dtype);
+    }
     g_last_kernel = p.name;
     switch (p.fam) {
         case FAM_MFMA16:

@@ -1,0 +1,78 @@
+// fp32 / fp64 MFMA GEMM whose waves share k: products of few tiles or a k that is long for them.
+//
+// A workgroup of eight waves owns one tile of 16 x 16 to 64 x 64 of the output, and wave w takes the pieces w, w + 8, ... of k, a cache line
+// of every row that has unit stride along k: straight from memory into registers (16 rows of such an operand through LDS of the wave's own, so
+// that its loads take whole lines), any element the rows may start at.  The eight partial tiles meet in LDS and are added in wave order.  One launch,
+// no workspace.  Bound by what a CU takes in, 35 to 95 GB/s a CU behind 2.7 us of launch and latency, and from 64 x 64 tiles of 1024^3 on by the
+// MFMAs (14.6 us of 25).  What it replaces staged 64 x 64 tiles slab by slab, one wave a SIMD, with a k split and a launch that adds it
+// up in fp32 and without either in fp64.  us, before and here:
+//   fp32 1024^3 30.4 / 25, 512^3 12.9 / 6.2, 935 x 862 x 398 32.0 / 12.9, 25 x 3120 x 2446 38.1 / 13.7, 32 x 8192 x 8192 141 / 60, 17 x 6048 x 173 (B^T)
+//   190 / 11.1, 64 x 4096 x 1024 (B^T) 18.8 / 9.6; fp64 89 x 2787 x 286 390 / 15.5, 2054 x 1064 x 52 (B^T) 120 / 15, 512^3 (A^T) 25.9 / 8.7, 300^3 (B^T) 38 / 5.8.
+// Over 330 drawn fp32 products 0.78 of the time, the slowest 1.03, over 170 fp64 ones 0.19 and 1.01.  The error against 64 bits is smaller than before: k is summed in 8 to 32 chains
+// (1024^3 2.1e-7, 5.8e-7 before; 64 x 4096 x 1024 2.2e-7 and 3.0e-7).
+#include "rp_gemm_wavekw.h"
+
+namespace rp {
+
+// waves a SIMD whose registers have to fit: two workgroups on a CU, one of the 64 x 64 tile
+constexpr int wkw_waves(int tiles) { return tiles <= 4 ? 4 : 2; }
+
+template <typename E, bool A_KC, bool B_KC, int TM, int TN, int NW>
+__global__ void __launch_bounds__(64 * NW, wkw_waves(TM * TN)) gemm_wavekw_kernel(GemmArgs g, int tiles_m, int tiles_n) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char wkw_lds[];
+    gemm_wavekw_block<E, A_KC, B_KC, TM, TN, NW>(g, tiles_m, tiles_n, blockIdx.x, blockIdx.y, wkw_lds);
+}
+
+template <typename E, bool A_KC, bool B_KC, int TM, int TN, int NW>
+static int launch_wavekw_t(const GemmArgs& g) {
+    constexpr size_t smem = wkw_smem<E, A_KC, B_KC, TM, TN, NW>();
+    const int tiles_m = (g.m + 16 * TM - 1) / (16 * TM), tiles_n = (g.n + 16 * TN - 1) / (16 * TN);
+    auto kern = gemm_wavekw_kernel<E, A_KC, B_KC, TM, TN, NW>;
+    if (smem > 64 * 1024 && !check_hip(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem), "hipFuncSetAttribute")) return -1;
+    hipLaunchKernelGGL(kern, dim3((unsigned)((tiles_m * tiles_n + 7) / 8 * 8), g.batch), dim3(64 * NW), smem, current_stream(), g, tiles_m, tiles_n);
+    return check_launch("gemm_wavekw_kernel") ? 0 : -1;
+}
+
+template <typename E, int TM, int TN, int NW>
+static int launch_wavekw_layout(const GemmArgs& g) {
+    const bool a_kc = wkw_a_kc(g), b_kc = wkw_b_kc(g);
+    if (a_kc && !b_kc) return launch_wavekw_t<E, true, false, TM, TN, NW>(g);
+    if (a_kc) return launch_wavekw_t<E, true, true, TM, TN, NW>(g);
+    if (!b_kc) return launch_wavekw_t<E, false, false, TM, TN, NW>(g);
+    return launch_wavekw_t<E, false, true, TM, TN, NW>(g);
+}
+
+// The tile with the least time over the drawn products (2 % from the best of all on the average): 32 x 32 where those occupy three quarters of the CUs (half in
+// fp64), else 16 x 16, or 16 x 32 where an operand's k rows are read (its loads of 16 elements are half a line).  One 64 x 64 tile a CU with a k that is worth
+// its prologue (1024^3 24 us, 28.5 on 32 x 32); 16 x 64 where one fills the chip once with a row-major B, whose lines it takes whole
+// (128 x 5888 x 1600 27.9 us, 33.3 on 16 x 32; 935 x 862 x 398, 413 of them, 14.2 and 12.7 on 32 x 32).
+WkwTile wavekw_tile(const GemmArgs& g, int dtype) {
+    const bool a_kc = wkw_a_kc(g), b_kc = wkw_b_kc(g);
+    if (!(a_kc || g.a_rs == 1) || !(b_kc || g.b_cs == 1) || g.batch > 65535) return WKW_NONE;
+    const long long esz = (long long)dtype_size(dtype), cus = device_cu_count() > 0 ? device_cu_count() : 256, limit = 1ll << 31;
+    // a tile is addressed with 32-bit byte offsets from its first row
+    const auto span = [&](bool kc, long long fs, long long ks) { return ((kc ? 63 * fs + g.k : (long long)(g.k - 1) * ks + 64) * esz); };
+    if (span(a_kc, g.a_rs, g.a_cs) >= limit || span(b_kc, g.b_cs, g.b_rs) >= limit) return WKW_NONE;
+    const auto tiles = [&](int tm, int tn) { return (long long)((g.m + 16 * tm - 1) / (16 * tm)) * ((g.n + 16 * tn - 1) / (16 * tn)) * g.batch; };
+    const auto fits = [&](int tm, int tn) { return (a_kc || g.m >= 16 * tm) && (b_kc || g.n >= 16 * tn); };       // see ms, ns in gemm_wavekw_block
+    if (!fits(1, 1)) return WKW_NONE;
+    if (dtype == RP_DTYPE_FLOAT64) return fits(2, 2) && tiles(2, 2) >= cus / 2 ? WKW_32X32 : WKW_16X16;
+    if (fits(4, 4) && g.k >= 512 && tiles(4, 4) >= cus * 3 / 4 && tiles(4, 4) <= cus) return WKW_64X64;
+    if (a_kc && !b_kc && fits(1, 4) && g.k >= 512 && tiles(1, 4) >= cus / 2 && tiles(1, 4) <= cus) return WKW_16X64;
+    if (fits(2, 2) && tiles(2, 2) >= cus * 3 / 4) return WKW_32X32;
+    return !(a_kc && b_kc) && fits(1, 2) && tiles(1, 2) >= cus / 2 ? WKW_16X32 : WKW_16X16;
+}
+
+int launch_wavekw(const GemmArgs& g, int dtype) {
+    const WkwTile tile = wavekw_tile(g, dtype);
+    if (dtype == RP_DTYPE_FLOAT64) return tile == WKW_32X32 ? launch_wavekw_layout<double, 2, 2, 8>(g) : launch_wavekw_layout<double, 1, 1, 8>(g);
+    switch (tile) {
+        case WKW_64X64: return launch_wavekw_layout<float, 4, 4, 8>(g);
+        case WKW_16X64: return launch_wavekw_t<float, true, false, 1, 4, 8>(g);
+        case WKW_32X32: return launch_wavekw_layout<float, 2, 2, 8>(g);
+        case WKW_16X32: return launch_wavekw_layout<float, 1, 2, 8>(g);
+        default: return launch_wavekw_layout<float, 1, 1, 8>(g);
+    }
+}
+
+}  // namespace rp

@@ -857,7 +857,7 @@ def test_small_fp32_outputs_take_one_launch():
 
 
 @pytest.mark.parametrize("layout", LAYOUTS)
-@pytest.mark.parametrize("m,k,n", [(17, 33, 19), (100, 131, 77), (35, 2047, 18), (3, 257, 301)])
+@pytest.mark.parametrize("m,k,n", [(17, 33, 19), (100, 131, 77), (35, 509, 18), (3, 257, 301)])
 def test_small_fp32_outputs_of_rows_at_any_element(m, k, n, layout):
     """Rows of odd length that start at an odd element: whole vectors along k are loaded there.  Small integers, so the sums are exact."""
     rng = np.random.default_rng(44)
@@ -871,6 +871,51 @@ def test_small_fp32_outputs_of_rows_at_any_element(m, k, n, layout):
     got = device_gemm(a, b, F32)
     assert capi.last_gemm_kernel() == "tiny32_16x16"
     assert np.array_equal(got, (a.astype(np.float64) @ b.astype(np.float64)).astype(np.float32))
+
+
+# fp32 and fp64 products whose waves share k: every tile, k of no whole piece (32 values in fp32, 16 in fp64), of fewer pieces than waves and of many
+# rounds of them, last tiles that start early, batches
+WAVEKW_SHAPES = [(F32, 1, 16, 513, 16, "mfma32_wavek"), (F32, 1, 5, 700, 333, "mfma32_wavek"), (F32, 1, 35, 2047, 18, "mfma32_wavek"), (F32, 1, 70, 545, 300, "mfma32_wavek"),
+                 (F32, 1, 497, 577, 401, "mfma32_wavek"), (F32, 1, 63, 1024, 2113, "mfma32_wavek"), (F32, 1, 3, 1001, 1100, "mfma32_wavek"), (F32, 1, 900, 519, 901, "mfma32_64x64"),
+                 (F32, 3, 67, 1027, 35, "mfma32_wavek"), (F32, 9, 131, 61, 260, "mfma32_64x64"), (F32, 1, 33, 3000, 1100, "mfma32_64x64"), (F64, 1, 16, 1, 16, "mfma64_wavek"),
+                 (F64, 1, 17, 16, 19, "mfma64_wavek"), (F64, 1, 60, 131, 50, "mfma64_wavek"), (F64, 1, 20, 2001, 17, "mfma64_wavek"), (F64, 1, 390, 257, 401, "mfma64_64x64"), (F64, 5, 33, 130, 31, "mfma64_wavek")]
+
+
+@pytest.mark.parametrize("layout", LAYOUTS)
+@pytest.mark.parametrize("dt,batch,m,k,n,kernel", WAVEKW_SHAPES)
+def test_waves_that_share_k_in_fp32_and_fp64(dt, batch, m, k, n, kernel, layout):
+    """The operands are slices, at an odd element, of NaN-filled arrays that end with their last element; small integers, so the bits are known."""
+    rng = np.random.default_rng(m + k + n)
+    es = capi.DTYPE_SIZE[dt]
+    np_t = capi.NP_STORAGE[dt]
+
+    def operand(rows, cols):
+        flat = np.full(1 + batch * rows * (cols + 3) - 3, np.nan, np_t)
+        vals = rng.integers(-2, 3, (batch, rows, cols)).astype(np_t)
+        np.lib.stride_tricks.as_strided(flat[1:], (batch, rows, cols), (rows * (cols + 3) * es, (cols + 3) * es, es))[...] = vals
+        return capi.DeviceBuffer.from_numpy(flat), vals, (rows * (cols + 3), cols + 3, 1)
+
+    da, a, a_st = operand(m, k) if layout[0] == "n" else operand(k, m)
+    db, b, b_st = operand(k, n) if layout[1] == "n" else operand(n, k)
+    if layout[0] == "t":
+        a, a_st = a.transpose(0, 2, 1), (a_st[0], a_st[2], a_st[1])
+    if layout[1] == "t":
+        b, b_st = b.transpose(0, 2, 1), (b_st[0], b_st[2], b_st[1])
+    want = np.matmul(a.astype(np.float64), b.astype(np.float64))
+    bias = rng.integers(-2, 3, n).astype(np_t)
+    dbias = capi.DeviceBuffer.from_numpy(bias)
+    pitch = n + 5
+    c0 = rng.integers(-2, 3, (batch, m, pitch)).astype(np_t)
+    for with_bias, accumulate in ((False, False), (True, True)):
+        dc = capi.DeviceBuffer.from_numpy(c0)
+        capi.gemm(dc.at(es), da.at(es), db.at(es), dbias.ptr if with_bias else None, batch, m, k, n, a_st, b_st, (m * pitch, pitch, 1), accumulate, dt)
+        if not ((layout[0] == "t" and m < 16) or (layout[1] == "n" and n < 16)):       # a row of k shorter than a tile's edge: the kernels of before
+            assert capi.last_gemm_kernel() == kernel
+        expect = c0.reshape(-1).copy()
+        inner = np.lib.stride_tricks.as_strided(expect[1:], (batch, m, n), (m * pitch * es, pitch * es, es))
+        inner[...] = (inner if accumulate else 0) + want + (bias if with_bias else 0)
+        assert np.array_equal(dc.to_numpy(np_t, (expect.size,)), expect)      # C, and nothing around it
+        dc.free()
 
 
 # ---- fp32 products with a short reduction (k <= 64) and many tiles: the resident cross-tile kernel (every layout, ragged
