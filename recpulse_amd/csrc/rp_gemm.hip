@@ -255,15 +255,29 @@ static bool overlap(const Span& a, const Span& b) { return a.lo < b.hi && b.lo <
 // B row-major: up to one 16 x 64 tile per CU, against the k split while k is up to 2048 (64 x 2048 x 2048 9.7 / 6.9, 64 x 4096 x 1024 10.0 / 11.7,
 // 96 x 4096 x 4096 with 384 tiles 16.4 / 19.2).
 // From ten slabs on: the eight of 128 x 512 x 512 take 5.3 and 4.8.  A small layer's dX in one launch with dW follows the same rule.
+// Ragged rows: with any k, and in place of the generic kernel and its k split too, whose loads are of single elements (511 x 4001 x 513 31.8 / 18.1,
+// 53 x 1434 x 14 13.1 / 7.8; 220 drawn ones 0.56 of the time), unless a row-major B of very few tiles has a long k (3 x 3261 x 63 13.0 / 15.1); and of
+// the few rows that the row-streaming kernel took those with k up to 1024 (3 x 281 x 5216 20.5 / 4.7).
 // (The k split with a launch of its own for the sums read all of its operands before it wrote C: outputs over an operand stay there.)
-static bool wavek16_takes(const GemmArgs& g, const Plan& p, int dtype) {
-    if ((dtype != RP_DTYPE_BFLOAT16 && dtype != RP_DTYPE_FLOAT16) || p.ragged || p.a_mc || g.batch != 1 || path_disabled("wavek")) return false;
-    const bool split = p.fam == FAM_MFMA16_SKINNY;
-    if (!split && !(p.fam == FAM_MFMA16 && p.bm == 64 && p.bn == 64)) return false;
-    if (g.k < 10 * M16_BK || g.k >= (1 << 24)) return false;
-    if (p.b_mc) {
-        if ((long long)((g.m + 15) / 16) * ((g.n + 63) / 64) > cu_tiles() || g.k * g.b_rs >= (1ll << 30)) return false;
-        if (split && (g.k > 2048 || stream128_shape(g.batch, g.m, g.k, g.n))) return false;
+static bool wavek16_takes(const GemmArgs& g, const Plan& p, int dtype, bool& ragged) {
+    if ((dtype != RP_DTYPE_BFLOAT16 && dtype != RP_DTYPE_FLOAT16) || g.batch != 1 || path_disabled("wavek")) return false;
+    const bool split = p.fam == FAM_MFMA16_SKINNY, generic = p.fam == FAM_GENERIC || (p.fam == FAM_SKINNY && g.k <= 1024);      // (whose operands no MFMA kernel has looked at)
+    if (!split && !generic && !(p.fam == FAM_MFMA16 && p.bm == 64 && p.bn == 64)) return false;
+    ragged = p.ragged || generic;
+    const bool b_mc = generic ? !(g.b_rs == 1 && g.k >= 8 && (g.b_cs >= g.k || g.n == 1)) : p.b_mc;
+    if (generic) {
+        if (path_disabled("mfma") || path_disabled("ragged") || !(g.a_cs == 1 && g.k >= 8 && (g.a_rs >= g.k || g.m == 1))) return false;
+        if (b_mc && !(g.b_cs == 1 && g.n >= 8 && g.b_rs >= g.n)) return false;
+        if (g.a_rs >= (1ll << 22) || g.b_rs >= (1ll << 22) || g.b_cs >= (1ll << 22)) return false;
+    } else if (p.a_mc) {
+        return false;
+    }
+    if ((!ragged && g.k < 10 * M16_BK) || g.k >= (1 << 24)) return false;
+    if (b_mc) {
+        const long long tiles = (long long)((g.m + 15) / 16) * ((g.n + 63) / 64);
+        if (generic && g.k > 2048 && g.k > 512 * tiles) return false;
+        if (tiles > cu_tiles() || g.k * g.b_rs >= (1ll << 30)) return false;
+        if (split && (g.k > 2048 || (!ragged && stream128_shape(g.batch, g.m, g.k, g.n)))) return false;
     } else {
         const long long tiles = (long long)((g.m + 31) / 32) * ((g.n + 31) / 32);
         if (!(tiles <= cu_tiles() || (split && g.k <= 4096 && tiles <= 2 * cu_tiles()))) return false;
@@ -334,7 +348,11 @@ static int run_gemm(GemmArgs g, int dtype) {
     }
     if (p.fam != FAM_GENERIC && p.fam != FAM_TINY && !p.ragged && !(aligned16(g.A) && aligned16(g.B)))
         p = make_plan(g.batch, g.m, g.k, g.n, g.a_rs, g.a_cs, g.b_rs, g.b_cs, g.c_rs, g.c_cs, g.a_bs, g.b_bs, dtype, false, false);
-    if (wavek16_takes(g, p, dtype)) { g_last_kernel = "mfma16_wavek"; return launch_mfma16_wavek(g, dtype); }
+    bool wavek_ragged = false;
+    if (wavek16_takes(g, p, dtype, wavek_ragged)) {
+        g_last_kernel = wavek_ragged ? p.name : "mfma16_wavek";          // (ragged rows: it goes by the name of the kernel that it stands in for)
+        return launch_mfma16_wavek(g, wavek_ragged, dtype);
+    }
     if (wavekw_takes(g, p, dtype)) {
         g_last_kernel = p.fam == FAM_MFMAW ? p.name : dtype == RP_DTYPE_FLOAT32 ? "mfma32_wavek" : "mfma64_wavek";      // (among the 64 x 64 tiles it goes by their name)
         return launch_wavekw(g, dtype);
@@ -469,13 +487,20 @@ constexpr int LINEAR_DB_ROWS = 1024, LINEAR_DB_ROWS_UNEVEN = 768;
 // of 128 x 128 tiles) in the layouts of dense X and W, and neither gradient written over anything that the other product reads
 // (one launch after the other, dW over W was fine).  Larger tiles fill a CU by themselves and gain nothing from company.
 // dx_wavek: dX by itself would go to the kernel whose waves split k, and does so in the one launch too: the same bits either way.
-static bool linear_backward_pairs(const GemmArgs& gx, const GemmArgs& gw, int dtype, bool& edge, bool& dx_wavek) {
-    if (path_disabled("pair16") || !(aligned16(gx.A) && aligned16(gx.B) && aligned16(gw.A))) return false;
-    const Plan px = make_plan(1, gx.m, gx.k, gx.n, gx.a_rs, gx.a_cs, gx.b_rs, gx.b_cs, gx.c_rs, gx.c_cs, 0, 0, dtype);
-    const Plan pw = make_plan(1, gw.m, gw.k, gw.n, gw.a_rs, gw.a_cs, gw.b_rs, gw.b_cs, gw.c_rs, gw.c_cs, 0, 0, dtype);
-    if (px.fam != FAM_MFMA16 || px.bm != 64 || px.bn != 64 || px.ragged || px.a_mc || px.b_mc) return false;
-    if (pw.fam != FAM_MFMA16 || pw.bm != 64 || pw.bn != 64 || pw.ragged || !pw.a_mc || !pw.b_mc) return false;
-    dx_wavek = wavek16_takes(gx, px, dtype);
+// ragged: rows of either product are; then both take the ragged variants, which do the same with rows of whole vectors.
+static bool linear_backward_pairs(const GemmArgs& gx, const GemmArgs& gw, int dtype, bool& edge, bool& dx_wavek, bool& ragged) {
+    if (path_disabled("pair16")) return false;
+    const auto plan = [&](const GemmArgs& g) {
+        const Plan p = make_plan(1, g.m, g.k, g.n, g.a_rs, g.a_cs, g.b_rs, g.b_cs, g.c_rs, g.c_cs, 0, 0, dtype);
+        if (p.fam == FAM_GENERIC || p.ragged || (aligned16(g.A) && aligned16(g.B))) return p;
+        return make_plan(1, g.m, g.k, g.n, g.a_rs, g.a_cs, g.b_rs, g.b_cs, g.c_rs, g.c_cs, 0, 0, dtype, false, false);
+    };
+    const Plan px = plan(gx), pw = plan(gw);
+    if (pw.fam != FAM_MFMA16 || pw.bm != 64 || pw.bn != 64 || !pw.a_mc || !pw.b_mc) return false;
+    bool dx_ragged = false;
+    dx_wavek = gx.b_rs == 1 && px.fam != FAM_MFMA16_SKINNY && wavek16_takes(gx, px, dtype, dx_ragged);
+    if (!dx_wavek && (px.fam != FAM_MFMA16 || px.bm != 64 || px.bn != 64 || px.a_mc || px.b_mc)) return false;
+    ragged = pw.ragged || px.ragged || (dx_wavek && dx_ragged);
     edge = pw.edge || (px.edge && !dx_wavek);
     const Span dx = span_of(gx.C, gx.m, gx.n, gx.c_rs, gx.c_cs, 2), dw = span_of(gw.C, gw.m, gw.n, gw.c_rs, gw.c_cs, 2);
     const Span dy = span_of(gx.A, gx.m, gx.k, gx.a_rs, gx.a_cs, 2), w = span_of(gx.B, gx.k, gx.n, gx.b_rs, gx.b_cs, 2), x = span_of(gw.A, gw.m, gw.k, gw.a_rs, gw.a_cs, 2);
@@ -562,15 +587,15 @@ int rp_hip_linear_backward(void* dx, void* dw, void* db, const void* dy, const v
         if (!dw) gw.m = 0;
         return launch_linear_backward_tiny(gx, gw, db, dy, m, n, accumulate_db);
     }
-    bool edge = false, dx_wavek = false;
-    if ((dtype == RP_DTYPE_BFLOAT16 || dtype == RP_DTYPE_FLOAT16) && dx && dw && linear_backward_pairs(gx, gw, dtype, edge, dx_wavek)) {
+    bool edge = false, dx_wavek = false, ragged = false;
+    if ((dtype == RP_DTYPE_BFLOAT16 || dtype == RP_DTYPE_FLOAT16) && dx && dw && linear_backward_pairs(gx, gw, dtype, edge, dx_wavek, ragged)) {
         g_last_kernel = "linear_backward16_64x64";
         // The bias gradient rides along unless it would be written over something that is still read (one launch after the other
         // was fine), or its chain of chunks outlasts the products.
         const Span b = span_of(db, 1, n, 0, 1, 2), dys = span_of(dy, m, n, n, 1, 2), ws = span_of(w, k, n, w_rs, w_cs, 2), xs = span_of(x, m, k, x_rs, x_cs, 2);
         const Span dxs = span_of(dx, m, k, dx_rs, dx_cs, 2), dws = span_of(dw, k, n, dw_rs, dw_cs, 2);
         const bool rides = db && m <= (n % 32 ? LINEAR_DB_ROWS_UNEVEN : LINEAR_DB_ROWS) && !(overlap(b, dys) || overlap(b, ws) || overlap(b, xs) || overlap(b, dxs) || overlap(b, dws));
-        if (launch_linear_backward16(gx, gw, dx_wavek, rides ? db : nullptr, accumulate_db, edge, dtype) != 0) return -1;
+        if (launch_linear_backward16(gx, gw, dx_wavek, rides ? db : nullptr, accumulate_db, edge, ragged, dtype) != 0) return -1;
         if (rides) return 0;
     } else {
         if (dx && run_gemm(gx, dtype) != 0) return -1;

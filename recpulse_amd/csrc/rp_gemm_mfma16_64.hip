@@ -71,6 +71,7 @@ struct StripSums {
 // 7.3 us, 7.9 with dX first).  bf16 layer with bias of m x k x n, us, dX on 64 x 64 tiles, in a launch of its own, and here:
 // 64 x 1024 x 1024 6.8 / 7.2 / 4.3, 256 x 256 x 4096 23 / 12 / 8.4, 512 x 512 x 640 6.8 / 11.1 / 6.8, 1024 x 256 x 640 10.9 / 16.1 / 11.7
 // (the column sums' chain, beside more workgroups than before).
+// Ragged rows do the same through the ragged variants (119 x 57 x 245 a layer's forward and backward 22.1 us, 9.6 now; 754 x 43 x 201 23.5 / 14.5; 280 x 610 x 2347 42 / 24).
 constexpr int DX_64X64 = -1;
 template <int DX>
 struct WavekShape {
@@ -88,7 +89,7 @@ __global__ void __launch_bounds__(256) linear_backward16_kernel(GemmArgs gx, Gem
     } else if (WAVEK ? w_slot < w_slots : x_slot >= x_slots) {
         gemm_mfma16_block<T, 64, 64, 2, true, true, EDGE, false, 1>(gw, w_tiles_m, w_tiles_n, nullptr, 0, w_slots, w_slot, 0, w_slots);
     } else if constexpr (WAVEK) {
-        gemm_mfma16_wavek_block<T, WavekShape<DX>::TM, WavekShape<DX>::TN, WavekShape<DX>::NW, false, 4>(gx, x_tiles_m, x_tiles_n, x_slot, smem);
+        gemm_mfma16_wavek_block<T, WavekShape<DX>::TM, WavekShape<DX>::TN, WavekShape<DX>::NW, false, 4, EDGE == M16_RAGGED>(gx, x_tiles_m, x_tiles_n, x_slot, smem);
     } else {
         gemm_mfma16_block<T, 64, 64, 2, false, false, EDGE, false, 1>(gx, x_tiles_m, x_tiles_n, nullptr, 0, x_slots, x_slot, 0, x_slots);
     }
@@ -121,11 +122,17 @@ static int launch_linear_backward16_edge(const GemmArgs& gx, const GemmArgs& gw,
     }
 }
 
-// gx.A is dY [gx.m, gx.k], dense; dx_wavek: the product alone would go to the kernel whose waves split k; edge: of the 64 x 64 tiles;
+template <typename T>
+static int launch_linear_backward16_type(const GemmArgs& gx, const GemmArgs& gw, bool dx_wavek, void* db, int accumulate_db, bool edge, bool ragged) {
+    if (ragged) return launch_linear_backward16_edge<T, M16_RAGGED>(gx, gw, dx_wavek, db, accumulate_db);
+    return edge ? launch_linear_backward16_edge<T, M16_EDGE>(gx, gw, dx_wavek, db, accumulate_db) : launch_linear_backward16_edge<T, M16_WHOLE>(gx, gw, dx_wavek, db, accumulate_db);
+}
+
+// gx.A is dY [gx.m, gx.k], dense; dx_wavek: the product alone would go to the kernel whose waves split k; edge, ragged: of the 64 x 64 tiles;
 // db: gx.k column sums of dY, or null
-int launch_linear_backward16(const GemmArgs& gx, const GemmArgs& gw, bool dx_wavek, void* db, int accumulate_db, bool edge, int dtype) {
-    if (dtype == RP_DTYPE_BFLOAT16) return edge ? launch_linear_backward16_edge<bf16_t, M16_EDGE>(gx, gw, dx_wavek, db, accumulate_db) : launch_linear_backward16_edge<bf16_t, M16_WHOLE>(gx, gw, dx_wavek, db, accumulate_db);
-    return edge ? launch_linear_backward16_edge<f16_t, M16_EDGE>(gx, gw, dx_wavek, db, accumulate_db) : launch_linear_backward16_edge<f16_t, M16_WHOLE>(gx, gw, dx_wavek, db, accumulate_db);
+int launch_linear_backward16(const GemmArgs& gx, const GemmArgs& gw, bool dx_wavek, void* db, int accumulate_db, bool edge, bool ragged, int dtype) {
+    if (dtype == RP_DTYPE_BFLOAT16) return launch_linear_backward16_type<bf16_t>(gx, gw, dx_wavek, db, accumulate_db, edge, ragged);
+    return launch_linear_backward16_type<f16_t>(gx, gw, dx_wavek, db, accumulate_db, edge, ragged);
 }
 
 }  // namespace rp

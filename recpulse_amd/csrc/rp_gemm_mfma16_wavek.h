@@ -38,9 +38,16 @@ constexpr int wk_smem() {
     return stages > parts ? stages : parts;
 }
 
+// `v` with its elements (16 bits each) moved down by `pull` < 8
+__device__ __forceinline__ u32x4_t wk_pull_shift(u32x4_t v, int pull) {
+    return __builtin_bit_cast(u32x4_t, __builtin_bit_cast(unsigned __int128, v) >> (16 * pull));
+}
+
 // Tile `block` of the schedule, by WAVES waves: k goes in NW shares, NW / WAVES of them to a wave one after the other, so
 // that the bits do not depend on how many waves there are.
-template <typename T, int TM, int TN, int NW, bool B_MC, int WAVES>
+// RAGGED: rows of any length that start at any element.  A vector that straddles the end of its row is loaded further back, so that it ends with
+// the row, and shifted into place; at least eight elements along the unit-stride axis.
+template <typename T, int TM, int TN, int NW, bool B_MC, int WAVES, bool RAGGED>
 __device__ __forceinline__ void gemm_mfma16_wavek_block(const GemmArgs& g, int tiles_m, int tiles_n, int block, uint16_t* wk_lds) {
     constexpr int SHARES = NW / WAVES;
     static_assert(NW % WAVES == 0, "whole shares");
@@ -57,9 +64,10 @@ __device__ __forceinline__ void gemm_mfma16_wavek_block(const GemmArgs& g, int t
     uint16_t* const stage = wk_lds + wave * wk_stage<TM, TN, B_MC>(), *const b_stage = stage + 16 * TM * WK_PITCH;
 
     // rows past the end and k past the end read zeros
+    constexpr int BACK = RAGGED && B_MC ? 16 : 0;                        // B's descriptor starts this many bytes early, for vectors moved back
     const int rows_a = g.m - m0 < 16 * TM ? g.m - m0 : 16 * TM, rows_b = g.n - n0 < 16 * TN ? g.n - n0 : 16 * TN;
     const __amdgpu_buffer_rsrc_t a_rsrc = buffer_rsrc((const T*)g.A + m0 * g.a_rs, ((rows_a - 1) * g.a_rs + g.k) * 2);
-    const __amdgpu_buffer_rsrc_t b_rsrc = B_MC ? buffer_rsrc((const T*)g.B + n0, ((g.k - 1) * g.b_rs + rows_b) * 2)
+    const __amdgpu_buffer_rsrc_t b_rsrc = B_MC ? buffer_rsrc((const char*)((const T*)g.B + n0) - BACK, ((g.k - 1) * g.b_rs + rows_b) * 2 + BACK)
                                                : buffer_rsrc((const T*)g.B + n0 * g.b_cs, ((rows_b - 1) * g.b_cs + g.k) * 2);
     uint32_t a_off[2 * TM], b_off[NB];
 #pragma unroll
@@ -67,10 +75,17 @@ __device__ __forceinline__ void gemm_mfma16_wavek_block(const GemmArgs& g, int t
 #pragma unroll
     for (int j = 0; j < NB; j++) {
         const bool live = (B_MC ? load_k : 8 * j + load_row) < rows_b;
-        b_off[j] = live ? (uint32_t)(((8 * j + load_row) * (B_MC ? g.b_rs : g.b_cs) + load_k) * 2) : BUFFER_OOB;
+        b_off[j] = live ? (uint32_t)(((8 * j + load_row) * (B_MC ? g.b_rs : g.b_cs) + load_k) * 2) + BACK : BUFFER_OOB;
     }
+    // elements that this lane's vectors stick out of the columns of a tile at the edge
+    const int b_pull = RAGGED && B_MC && rows_b > load_k && rows_b - load_k < 8 ? 8 - (rows_b - load_k) : 0;
     const uint32_t b_step = B_MC ? (uint32_t)g.b_rs * 2u : 2u;           // bytes from one k to the next
 
+    // elements that this lane's vectors of piece kk stick out of k
+    auto k_pull = [&](int kk) {
+        const int in = g.k - kk - load_k;
+        return in > 0 && in < 8 ? 8 - in : 0;
+    };
     f32x4_t sums[SHARES][TM][TN];
     auto add_up = [&](f32x4_t (&acc)[TM][TN], int share) {
 #pragma unroll
@@ -83,15 +98,30 @@ __device__ __forceinline__ void gemm_mfma16_wavek_block(const GemmArgs& g, int t
             for (int u = 0; u < U; u++) {
                 const int kk = k0 + u * NW * WK_PIECE;
                 const bool live = kk + load_k < g.k;
+                const uint32_t back = RAGGED ? 2u * k_pull(kk) : 0u;
 #pragma unroll
-                for (int i = 0; i < 2 * TM; i++) a[u][i] = __builtin_amdgcn_raw_buffer_load_b128(a_rsrc, (int)(live ? a_off[i] + 2u * kk : BUFFER_OOB), 0, 0);
+                for (int i = 0; i < 2 * TM; i++) a[u][i] = __builtin_amdgcn_raw_buffer_load_b128(a_rsrc, (int)(live && a_off[i] != BUFFER_OOB ? a_off[i] + 2u * kk - back : BUFFER_OOB), 0, 0);
 #pragma unroll
-                for (int j = 0; j < NB; j++)                 // (k is a whole number of eights)
-                    b[u][j] = __builtin_amdgcn_raw_buffer_load_b128(b_rsrc, (int)((B_MC ? kk + 8 * j < g.k : live) && b_off[j] != BUFFER_OOB ? b_off[j] + b_step * kk : BUFFER_OOB), 0, 0);
+                for (int j = 0; j < NB; j++)                 // (unless RAGGED, k is a whole number of eights)
+                    b[u][j] = __builtin_amdgcn_raw_buffer_load_b128(b_rsrc, (int)((B_MC ? kk + 8 * j + (RAGGED ? load_row : 0) < g.k : live) && b_off[j] != BUFFER_OOB ? b_off[j] + b_step * kk - (B_MC ? 2u * b_pull : back) : BUFFER_OOB), 0, 0);
             }
 #pragma unroll
             for (int u = 0; u < U; u++) {
                 if (SHARES > 1 && k0 + u * NW * WK_PIECE >= g.k) break;          // behind k: nothing to add (a wave with one share keeps its loop without branches)
+                if constexpr (RAGGED) {
+                    const int kk = k0 + u * NW * WK_PIECE;
+                    if (kk < g.k && kk + WK_PIECE > g.k) {               // (wave-uniform)
+                        const int pull = k_pull(kk);
+#pragma unroll
+                        for (int i = 0; i < 2 * TM; i++) a[u][i] = wk_pull_shift(a[u][i], pull);
+                        if constexpr (!B_MC)
+#pragma unroll
+                            for (int j = 0; j < NB; j++) b[u][j] = wk_pull_shift(b[u][j], pull);
+                    }
+                    if (B_MC && rows_b < 64)
+#pragma unroll
+                        for (int j = 0; j < NB; j++) b[u][j] = wk_pull_shift(b[u][j], b_pull);
+                }
                 wk_wave_order();
 #pragma unroll
                 for (int i = 0; i < 2 * TM; i++) *(u32x4_t*)(stage + (8 * i + load_row) * WK_PITCH + load_k) = a[u][i];

@@ -805,6 +805,26 @@ def test_bias_gradient_beside_the_paired_gradients(dt, m, n):
     assert np.array_equal(d_dx.numpy(), want_dx) and np.array_equal(d_w.numpy().reshape(-1)[:n], want.numpy())
 
 
+@pytest.mark.parametrize("dt", HALF, ids=lambda d: NAMES[d])
+@pytest.mark.parametrize("m,k,n", [(119, 57, 245), (57, 50, 859), (754, 43, 201), (33, 1033, 71), (9, 1001, 9), (300, 305, 641), (64, 72, 1001), (72, 65, 1024), (1030, 129, 77), (130, 1025, 9)])
+def test_gradients_of_ragged_layers_in_one_launch(m, k, n, dt):
+    """Layers whose rows are no whole vectors: dX, dW and db together have the bits of the three on their own, also accumulated."""
+    rng = np.random.default_rng(m + k + n)
+    L = capi.lib()
+    x, w, dy = rand_storage(rng, (m, k), dt), rand_storage(rng, (k, n), dt), rand_storage(rng, (m, n), dt)
+    d_x, d_w, d_dy = Dev(x, dt), Dev(w, dt), Dev(dy, dt)
+    init = [rand_storage(rng, s, dt) for s in ((m, k), (k, n), (n,))]
+    for acc in (0, 1):
+        want, got = [Dev(i, dt) for i in init], [Dev(i, dt) for i in init]
+        capi.gemm(want[0].ptr, d_dy.ptr, d_w.ptr, None, 1, m, n, k, (0, n, 1), (0, 1, n), (0, k, 1), bool(acc), dt)
+        capi.gemm(want[1].ptr, d_x.ptr, d_dy.ptr, None, 1, k, m, n, (0, 1, k), (0, n, 1), (0, n, 1), bool(acc), dt)
+        capi.check(L.rp_hip_reduce_rows(want[2].ptr, d_dy.ptr, m, n, acc, dt), "reduce_rows")
+        capi.check(L.rp_hip_linear_backward(got[0].ptr, got[1].ptr, got[2].ptr, d_dy.ptr, d_x.ptr, d_w.ptr, m, k, n, k, 1, n, 1, k, 1, n, 1, acc, acc, acc, dt), "linear_backward")
+        assert capi.last_gemm_kernel() == "linear_backward16_64x64"
+        for g, t in zip(got, want):
+            assert np.array_equal(g.numpy(), t.numpy())
+
+
 def test_batch_longer_than_a_grid_axis():
     """70 000 tiny matrices in one call (the batch index rides on a grid axis of at most 65 535 blocks), A shared by
     all of them through a zero batch stride."""
