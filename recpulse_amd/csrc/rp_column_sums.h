@@ -72,4 +72,55 @@ struct ColumnTile {
     }
 };
 
+// Column sums of one strip of 64 bytes' worth of columns by a workgroup, in the order above: a chunk
+// of 256 rows at a time in LDS, its four runs added side by side, the next chunk on its way to registers meanwhile.
+struct BiasGradient {
+    void* out;
+    int cols, accumulate;
+    int blocks;              // workgroups it takes (0: no bias gradient)
+};
+template <typename T, int THREADS>
+struct StripSums {
+    using A = typename traits<T>::acc;
+    using Tile = ColumnTile<T, 64, COLSUM_CHUNK, THREADS, true>;
+    static constexpr int COLS = Tile::COLS, RUNS = COLSUM_CHUNK / COLSUM_RUN;
+    static constexpr size_t LDS = Tile::BYTES + RUNS * COLS * sizeof(A);
+    static __device__ void run(T* out, const T* grad, int rows, int cols, int accumulate, int strip, unsigned char* lds) {
+        T* tile = (T*)lds;
+        A* parts = (A*)(lds + Tile::BYTES);              // [run][column]
+        const int t = threadIdx.x, run = t / COLS, col = t % COLS, c0 = strip * COLS;
+        Tile regs;
+        regs.load(grad, 0, rows, c0, cols, t);
+        A s = 0;
+        for (int r = 0; r < rows; r += COLSUM_CHUNK) {
+            regs.store(tile, t);
+            __syncthreads();
+            if (r + COLSUM_CHUNK < rows) regs.load(grad, r + COLSUM_CHUNK, rows, c0, cols, t);
+            if (rows <= COLSUM_CHUNK) {                  // one chunk: all of its rows top to bottom
+                if (t < COLS)
+                    for (int q = 0; q * COLSUM_RUN < rows; q++)
+                        s = Tile::add(s, tile + Tile::row_offset(q * COLSUM_RUN), col, rows - q * COLSUM_RUN < COLSUM_RUN ? rows - q * COLSUM_RUN : COLSUM_RUN);
+            } else {
+                if (t < RUNS * COLS) {
+                    const int n = rows - r - run * COLSUM_RUN;
+                    parts[t] = n > 0 ? Tile::add(0, tile + Tile::row_offset(run * COLSUM_RUN), col, n < COLSUM_RUN ? n : COLSUM_RUN) : (A)0;
+                }
+                __syncthreads();
+                if (t < COLS) {
+                    A c = parts[t];
+#pragma unroll
+                    for (int q = 1; q < RUNS; q++) c += parts[q * COLS + t];
+                    s += c;
+                }
+            }
+            __syncthreads();
+        }
+        const int j = c0 + t;
+        if (t >= COLS || j >= cols) return;
+        T y = narrow<T>(s);
+        if (accumulate) y = narrow<T>(widen(out[j]) + widen(y));
+        out[j] = y;
+    }
+};
+
 }  // namespace rp

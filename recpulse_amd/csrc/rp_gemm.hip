@@ -483,6 +483,37 @@ int* noalloc_arrival_counters() {
 // 1280 x 768 x 264 16.4 / 15.1, 2048 x 40 x 16 21.8 / 16.5).
 constexpr int LINEAR_DB_ROWS = 1024, LINEAR_DB_ROWS_UNEVEN = 768;
 
+// The plan that a product alone would follow
+static Plan plan_alone(const GemmArgs& g, int dtype) {
+    const Plan p = make_plan(1, g.m, g.k, g.n, g.a_rs, g.a_cs, g.b_rs, g.b_cs, g.c_rs, g.c_cs, 0, 0, dtype);
+    if (p.fam == FAM_GENERIC || p.fam == FAM_TINY || p.ragged || (aligned16(g.A) && aligned16(g.B))) return p;
+    return make_plan(1, g.m, g.k, g.n, g.a_rs, g.a_cs, g.b_rs, g.b_cs, g.c_rs, g.c_cs, 0, 0, dtype, false, false);
+}
+
+// Neither gradient is written over anything that the other product reads (one launch after the other, dW over W was fine)
+static bool gradients_apart(const GemmArgs& gx, const GemmArgs& gw, int dtype) {
+    const int esz = (int)dtype_size(dtype);
+    const Span dx = span_of(gx.C, gx.m, gx.n, gx.c_rs, gx.c_cs, esz), dw = span_of(gw.C, gw.m, gw.n, gw.c_rs, gw.c_cs, esz);
+    const Span dy = span_of(gx.A, gx.m, gx.k, gx.a_rs, gx.a_cs, esz), w = span_of(gx.B, gx.k, gx.n, gx.b_rs, gx.b_cs, esz), x = span_of(gw.A, gw.m, gw.k, gw.a_rs, gw.a_cs, esz);
+    return !(overlap(dx, dw) || overlap(dx, dy) || overlap(dx, x) || overlap(dw, dy) || overlap(dw, w));
+}
+
+// Nor is the bias gradient
+static bool bias_gradient_apart(const void* db, const GemmArgs& gx, const GemmArgs& gw, int dtype) {
+    const int esz = (int)dtype_size(dtype);
+    const Span b = span_of(db, 1, gx.k, 0, 1, esz), dx = span_of(gx.C, gx.m, gx.n, gx.c_rs, gx.c_cs, esz), dw = span_of(gw.C, gw.m, gw.n, gw.c_rs, gw.c_cs, esz);
+    const Span dy = span_of(gx.A, gx.m, gx.k, gx.a_rs, gx.a_cs, esz), w = span_of(gx.B, gx.k, gx.n, gx.b_rs, gx.b_cs, esz), x = span_of(gw.A, gw.m, gw.k, gw.a_rs, gw.a_cs, esz);
+    return !(overlap(b, dy) || overlap(b, w) || overlap(b, x) || overlap(b, dx) || overlap(b, dw));
+}
+
+// The tiles on which a product alone would share k among the waves or run as a tiny one; WKW_NONE: neither, or not with both operands k-contiguous
+// (kc) or both free-index-contiguous
+static WkwTile small_tile_alone(const GemmArgs& g, bool kc, int dtype) {
+    const Plan p = plan_alone(g, dtype);
+    if (wavekw_takes(g, p, dtype)) return wkw_a_kc(g) == kc && wkw_b_kc(g) == kc ? wavekw_tile(g, dtype) : WKW_NONE;
+    return p.fam == FAM_TINY ? WKW_TINY : WKW_NONE;
+}
+
 // Whether dX and dW of a 16-bit Linear layer go out as one launch: both on the 64 x 64 tile (an output of under half a CU count
 // of 128 x 128 tiles) in the layouts of dense X and W, and neither gradient written over anything that the other product reads
 // (one launch after the other, dW over W was fine).  Larger tiles fill a CU by themselves and gain nothing from company.
@@ -490,21 +521,14 @@ constexpr int LINEAR_DB_ROWS = 1024, LINEAR_DB_ROWS_UNEVEN = 768;
 // ragged: rows of either product are; then both take the ragged variants, which do the same with rows of whole vectors.
 static bool linear_backward_pairs(const GemmArgs& gx, const GemmArgs& gw, int dtype, bool& edge, bool& dx_wavek, bool& ragged) {
     if (path_disabled("pair16")) return false;
-    const auto plan = [&](const GemmArgs& g) {
-        const Plan p = make_plan(1, g.m, g.k, g.n, g.a_rs, g.a_cs, g.b_rs, g.b_cs, g.c_rs, g.c_cs, 0, 0, dtype);
-        if (p.fam == FAM_GENERIC || p.ragged || (aligned16(g.A) && aligned16(g.B))) return p;
-        return make_plan(1, g.m, g.k, g.n, g.a_rs, g.a_cs, g.b_rs, g.b_cs, g.c_rs, g.c_cs, 0, 0, dtype, false, false);
-    };
-    const Plan px = plan(gx), pw = plan(gw);
+    const Plan px = plan_alone(gx, dtype), pw = plan_alone(gw, dtype);
     if (pw.fam != FAM_MFMA16 || pw.bm != 64 || pw.bn != 64 || !pw.a_mc || !pw.b_mc) return false;
     bool dx_ragged = false;
     dx_wavek = gx.b_rs == 1 && px.fam != FAM_MFMA16_SKINNY && wavek16_takes(gx, px, dtype, dx_ragged);
     if (!dx_wavek && (px.fam != FAM_MFMA16 || px.bm != 64 || px.bn != 64 || px.a_mc || px.b_mc)) return false;
     ragged = pw.ragged || px.ragged || (dx_wavek && dx_ragged);
     edge = pw.edge || (px.edge && !dx_wavek);
-    const Span dx = span_of(gx.C, gx.m, gx.n, gx.c_rs, gx.c_cs, 2), dw = span_of(gw.C, gw.m, gw.n, gw.c_rs, gw.c_cs, 2);
-    const Span dy = span_of(gx.A, gx.m, gx.k, gx.a_rs, gx.a_cs, 2), w = span_of(gx.B, gx.k, gx.n, gx.b_rs, gx.b_cs, 2), x = span_of(gw.A, gw.m, gw.k, gw.a_rs, gw.a_cs, 2);
-    return !(overlap(dx, dw) || overlap(dx, dy) || overlap(dx, x) || overlap(dw, dy) || overlap(dw, w));
+    return gradients_apart(gx, gw, dtype);
 }
 
 }  // namespace rp
@@ -578,23 +602,29 @@ int rp_hip_linear_backward(void* dx, void* dw, void* db, const void* dy, const v
     GemmArgs gw{dw, x, dy, nullptr, 1, k, m, n, 0, x_cs, x_rs, 0, n, 1, 0, dw_rs, dw_cs, accumulate_dw};
     plain_k_strides(gx.m, gx.k, gx.n, gx.a_rs, gx.a_cs, gx.b_rs, gx.b_cs);
     plain_k_strides(gw.m, gw.k, gw.n, gw.a_rs, gw.a_cs, gw.b_rs, gw.b_cs);
-    bool fused = dtype == RP_DTYPE_FLOAT32 && (dx || dw);
-    if (fused && dx) fused = make_plan(1, gx.m, gx.k, gx.n, gx.a_rs, gx.a_cs, gx.b_rs, gx.b_cs, gx.c_rs, gx.c_cs, 0, 0, dtype).fam == FAM_TINY;
-    if (fused && dw) fused = make_plan(1, gw.m, gw.k, gw.n, gw.a_rs, gw.a_cs, gw.b_rs, gw.b_cs, gw.c_rs, gw.c_cs, 0, 0, dtype).fam == FAM_TINY;
-    if (fused) {
-        // small layer: one launch does all three, block for block what the separate launches would do
-        if (!dx) gx.m = 0;
-        if (!dw) gw.m = 0;
-        return launch_linear_backward_tiny(gx, gw, db, dy, m, n, accumulate_db);
+    if (dtype == RP_DTYPE_FLOAT32 || dtype == RP_DTYPE_FLOAT64) {
+        const WkwTile tx = dx ? small_tile_alone(gx, true, dtype) : WKW_TINY, tw = dw ? small_tile_alone(gw, false, dtype) : WKW_TINY;
+        if (dtype == RP_DTYPE_FLOAT32 && (dx || dw) && tx == WKW_TINY && tw == WKW_TINY) {
+            // small layer: one launch does all three, block for block what the separate launches would do
+            if (!dx) gx.m = 0;
+            if (!dw) gw.m = 0;
+            return launch_linear_backward_tiny(gx, gw, db, dy, m, n, accumulate_db);
+        }
+        // (more than two rounds of 16 x 16 tiles need the registers and the LDS that they have alone: fp32 2659 x 49 x 3731 70.3 us apart, 73.4 in one launch)
+        const auto rounds16 = [&](const GemmArgs& g, WkwTile t) { return t == WKW_16X16 && (long long)((g.m + 15) / 16) * ((g.n + 15) / 16) > 2 * cu_tiles(); };
+        if (dx && dw && linear_backward_wavekw_takes(tx, tw, dtype) && (tx == tw || !(rounds16(gx, tx) || rounds16(gw, tw))) && gradients_apart(gx, gw, dtype)) {
+            g_last_kernel = "linear_backward_wavek";
+            const bool rides = db && m <= LINEAR_DB_ROWS && bias_gradient_apart(db, gx, gw, dtype);
+            if (launch_linear_backward_wavekw(gx, gw, tx, tw, rides ? db : nullptr, accumulate_db, dtype) != 0) return -1;
+            return db && !rides ? rp_hip_reduce_rows(db, dy, m, n, accumulate_db, dtype) : 0;
+        }
     }
     bool edge = false, dx_wavek = false, ragged = false;
     if ((dtype == RP_DTYPE_BFLOAT16 || dtype == RP_DTYPE_FLOAT16) && dx && dw && linear_backward_pairs(gx, gw, dtype, edge, dx_wavek, ragged)) {
         g_last_kernel = "linear_backward16_64x64";
         // The bias gradient rides along unless it would be written over something that is still read (one launch after the other
         // was fine), or its chain of chunks outlasts the products.
-        const Span b = span_of(db, 1, n, 0, 1, 2), dys = span_of(dy, m, n, n, 1, 2), ws = span_of(w, k, n, w_rs, w_cs, 2), xs = span_of(x, m, k, x_rs, x_cs, 2);
-        const Span dxs = span_of(dx, m, k, dx_rs, dx_cs, 2), dws = span_of(dw, k, n, dw_rs, dw_cs, 2);
-        const bool rides = db && m <= (n % 32 ? LINEAR_DB_ROWS_UNEVEN : LINEAR_DB_ROWS) && !(overlap(b, dys) || overlap(b, ws) || overlap(b, xs) || overlap(b, dxs) || overlap(b, dws));
+        const bool rides = db && m <= (n % 32 ? LINEAR_DB_ROWS_UNEVEN : LINEAR_DB_ROWS) && bias_gradient_apart(db, gx, gw, dtype);
         if (launch_linear_backward16(gx, gw, dx_wavek, rides ? db : nullptr, accumulate_db, edge, ragged, dtype) != 0) return -1;
         if (rides) return 0;
     } else {

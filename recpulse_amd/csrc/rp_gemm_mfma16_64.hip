@@ -7,57 +7,6 @@ namespace rp {
 
 int launch_mfma16_64(const GemmArgs& g, const Plan& p, int dtype) { return m16_launch_tile_dtype<64, 64, 2>(g, p, dtype); }
 
-// Column sums of one strip of 64 bytes' worth of columns by a workgroup of 256 threads, in the order of rp_column_sums.h: a chunk
-// of 256 rows at a time in LDS, its four runs added side by side, the next chunk on its way to registers meanwhile.
-struct BiasGradient {
-    void* out;
-    int cols, accumulate;
-    int blocks;              // workgroups it takes (0: no bias gradient)
-};
-template <typename T>
-struct StripSums {
-    using A = typename traits<T>::acc;
-    using Tile = ColumnTile<T, 64, COLSUM_CHUNK, 256, true>;
-    static constexpr int COLS = Tile::COLS, RUNS = COLSUM_CHUNK / COLSUM_RUN;
-    static constexpr size_t LDS = Tile::BYTES + RUNS * COLS * sizeof(A);
-    static __device__ void run(T* out, const T* grad, int rows, int cols, int accumulate, int strip, unsigned char* lds) {
-        T* tile = (T*)lds;
-        A* parts = (A*)(lds + Tile::BYTES);              // [run][column]
-        const int t = threadIdx.x, run = t / COLS, col = t % COLS, c0 = strip * COLS;
-        Tile regs;
-        regs.load(grad, 0, rows, c0, cols, t);
-        A s = 0;
-        for (int r = 0; r < rows; r += COLSUM_CHUNK) {
-            regs.store(tile, t);
-            __syncthreads();
-            if (r + COLSUM_CHUNK < rows) regs.load(grad, r + COLSUM_CHUNK, rows, c0, cols, t);
-            if (rows <= COLSUM_CHUNK) {                  // one chunk: all of its rows top to bottom
-                if (t < COLS)
-                    for (int q = 0; q * COLSUM_RUN < rows; q++)
-                        s = Tile::add(s, tile + Tile::row_offset(q * COLSUM_RUN), col, rows - q * COLSUM_RUN < COLSUM_RUN ? rows - q * COLSUM_RUN : COLSUM_RUN);
-            } else {
-                if (t < RUNS * COLS) {
-                    const int n = rows - r - run * COLSUM_RUN;
-                    parts[t] = n > 0 ? Tile::add(0, tile + Tile::row_offset(run * COLSUM_RUN), col, n < COLSUM_RUN ? n : COLSUM_RUN) : (A)0;
-                }
-                __syncthreads();
-                if (t < COLS) {
-                    A c = parts[t];
-#pragma unroll
-                    for (int q = 1; q < RUNS; q++) c += parts[q * COLS + t];
-                    s += c;
-                }
-            }
-            __syncthreads();
-        }
-        const int j = c0 + t;
-        if (t >= COLS || j >= cols) return;
-        T y = narrow<T>(s);
-        if (accumulate) y = narrow<T>(widen(out[j]) + widen(y));
-        out[j] = y;
-    }
-};
-
 // All gradients of a Linear layer in one launch: the first workgroups add up the columns of dY (their chain of chunks is the longest of
 // any), the next ones compute dX = dY . W^T (k-contiguous operands), the others dW = X^T . dY (free-index-contiguous ones), tile for
 // tile and chunk for chunk what separate launches would do, so the same bits.
@@ -85,7 +34,7 @@ __global__ void __launch_bounds__(256) linear_backward16_kernel(GemmArgs gx, Gem
     const int b = (int)blockIdx.x - db.blocks, x_slot = WAVEK ? b - w_slots : b, w_slot = WAVEK ? b : b - x_slots;
     extern __shared__ __attribute__((aligned(16))) uint16_t smem[];
     if (b < 0) {
-        if ((int)blockIdx.x * StripSums<T>::COLS < db.cols) StripSums<T>::run((T*)db.out, (const T*)gx.A, gx.m, db.cols, db.accumulate, blockIdx.x, (unsigned char*)smem);
+        if ((int)blockIdx.x * StripSums<T, 256>::COLS < db.cols) StripSums<T, 256>::run((T*)db.out, (const T*)gx.A, gx.m, db.cols, db.accumulate, blockIdx.x, (unsigned char*)smem);
     } else if (WAVEK ? w_slot < w_slots : x_slot >= x_slots) {
         gemm_mfma16_block<T, 64, 64, 2, true, true, EDGE, false, 1>(gw, w_tiles_m, w_tiles_n, nullptr, 0, w_slots, w_slot, 0, w_slots);
     } else if constexpr (WAVEK) {
@@ -103,9 +52,9 @@ static int launch_linear_backward16_t(const GemmArgs& gx, const GemmArgs& gw, vo
     const int x_slots = wavek ? (xm * xn + 7) / 8 * 8 : scheduled_grid(xm, xn), w_slots = scheduled_grid(wm, wn);
     constexpr size_t x_smem = wavek ? WavekShape<DX>::SMEM : m16_smem_bytes(64, 64, 2, false, false, 2, 32), w_smem = m16_smem_bytes(64, 64, 2, true, true, 2, 32);
     constexpr size_t smem = x_smem > w_smem ? x_smem : w_smem;
-    static_assert(StripSums<T>::LDS <= smem, "the column sums use the tiles' LDS");
+    static_assert(StripSums<T, 256>::LDS <= smem, "the column sums use the tiles' LDS");
     // whole rounds of the XCDs, so that the tiles' workgroups stay where the schedule wants them
-    const BiasGradient sums{db, gx.k, accumulate_db, db ? ((gx.k - 1) / StripSums<T>::COLS + 8) / 8 * 8 : 0};
+    const BiasGradient sums{db, gx.k, accumulate_db, db ? ((gx.k - 1) / StripSums<T, 256>::COLS + 8) / 8 * 8 : 0};
     static_assert(smem <= 64 * 1024, "no attribute needed");
     hipLaunchKernelGGL((linear_backward16_kernel<T, EDGE, DX>), dim3(sums.blocks + x_slots + w_slots), dim3(256), smem, current_stream(), gx, gw, sums, xm, xn, wm, wn, x_slots, w_slots);
     return check_launch("linear_backward16_kernel") ? 0 : -1;

@@ -315,8 +315,11 @@ __device__ __forceinline__ void gemm_wavekw_block(const GemmArgs& g, int tiles_m
 }
 
 // Tiles of a product, and whether the operands can be addressed that way; WKW_NONE: not at all
-enum WkwTile { WKW_NONE, WKW_16X16, WKW_16X32, WKW_32X32, WKW_16X64, WKW_64X64 };
+enum WkwTile { WKW_NONE, WKW_16X16, WKW_16X32, WKW_32X32, WKW_16X64, WKW_64X64, WKW_TINY };       // WKW_TINY: the 16 x 16 tiles of rp_gemm_tiny.h, two a workgroup
 WkwTile wavekw_tile(const GemmArgs& g, int dtype);
+// All gradients of a Linear layer in one launch, each product on the tiles that it would get alone; gx.A is dY [gx.m, gx.k], dense; db: gx.k column sums of dY, or null
+bool linear_backward_wavekw_takes(WkwTile x, WkwTile w, int dtype);
+int launch_linear_backward_wavekw(const GemmArgs& gx, const GemmArgs& gw, WkwTile x, WkwTile w, void* db, int accumulate_db, int dtype);
 static inline bool wkw_a_kc(const GemmArgs& g) { return g.a_cs == 1; }
 static inline bool wkw_b_kc(const GemmArgs& g) { return g.b_rs == 1 && (g.b_cs != 1 || g.n == 1); }
 

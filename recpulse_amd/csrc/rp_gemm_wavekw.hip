@@ -10,6 +10,8 @@
 //   190 / 11.1, 64 x 4096 x 1024 (B^T) 18.8 / 9.6; fp64 89 x 2787 x 286 390 / 15.5, 2054 x 1064 x 52 (B^T) 120 / 15, 512^3 (A^T) 25.9 / 8.7, 300^3 (B^T) 38 / 5.8.
 // Over 330 drawn fp32 products 0.78 of the time, the slowest 1.03, over 170 fp64 ones 0.19 and 1.01.  The error against 64 bits is smaller than before: k is summed in 8 to 32 chains
 // (1024^3 2.1e-7, 5.8e-7 before; 64 x 4096 x 1024 2.2e-7 and 3.0e-7).
+#include "rp_column_sums.h"
+#include "rp_gemm_tiny.h"
 #include "rp_gemm_wavekw.h"
 
 namespace rp {
@@ -72,6 +74,83 @@ int launch_wavekw(const GemmArgs& g, int dtype) {
         case WKW_32X32: return launch_wavekw_layout<float, 2, 2, 8>(g);
         case WKW_16X32: return launch_wavekw_layout<float, 1, 2, 8>(g);
         default: return launch_wavekw_layout<float, 1, 1, 8>(g);
+    }
+}
+
+// All gradients of a Linear layer in one launch: the first workgroups add up the columns of dY, then come the tiles of the product with the longer k,
+// then the other's, each doing what it would do in a launch of its own, so the same bits.  What goes away is two launches of three, 4.7 us each
+// behind another one.  fp32 layers with bias, forward and backward, us, apart and here: 512^3 22.1 / 17.4,
+// 935 x 213 x 862 34.5 / 28.8, 64 x 4544 x 128 25.8 / 21.4; fp64 208 x 299 x 482 18.9 / 12.7.
+// Either product may be on the 16 x 16 tiles of four waves, two of which share a workgroup.
+template <WkwTile K> struct WkwShape { static constexpr int TM = K == WKW_32X32 ? 2 : 1, TN = K == WKW_32X32 || K == WKW_16X32 ? 2 : 1; };
+
+template <typename E, WkwTile K, bool KC>
+constexpr size_t wkw_part_smem() {
+    if constexpr (K == WKW_TINY) return 2 * 3 * 256 * sizeof(float);
+    else return wkw_smem<E, KC, KC, WkwShape<K>::TM, WkwShape<K>::TN, 8>();
+}
+// Slot `block` of one product: KC, KC for dX = dY . W^T, MC, MC for dW = X^T . dY
+template <typename E, WkwTile K, bool KC>
+__device__ __forceinline__ void wkw_part(const GemmArgs& g, int tiles_m, int tiles_n, int block, int vec_flags, unsigned char* lds) {
+    if constexpr (K == WKW_TINY) {
+        const int half = threadIdx.x >> 8, tile = 2 * block + half, tiles = tiles_m * tiles_n;
+        if (2 * block >= tiles) return;
+        tiny_tile_any(g, vec_flags & 1, vec_flags & 2, tile < tiles ? tile : tiles - 1, (float (*)[256])lds + 3 * half, threadIdx.x & 255, tile < tiles);
+    } else {
+        gemm_wavekw_block<E, KC, KC, WkwShape<K>::TM, WkwShape<K>::TN, 8>(g, tiles_m, tiles_n, block, 0, lds);
+    }
+}
+
+template <typename E, WkwTile X, WkwTile W>
+__global__ void __launch_bounds__(512, 4) linear_backward_wavekw_kernel(GemmArgs gx, GemmArgs gw, BiasGradient db, int x_tiles_m, int x_tiles_n, int w_tiles_m, int w_tiles_n, int x_slots, int w_slots, int x_first, int vec_flags) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char wkw_lds[];
+    const int b = (int)blockIdx.x - db.blocks, first = x_first ? x_slots : w_slots;
+    if (b < 0) {
+        if ((int)blockIdx.x * StripSums<E, 512>::COLS < db.cols) StripSums<E, 512>::run((E*)db.out, (const E*)gx.A, gx.m, db.cols, db.accumulate, blockIdx.x, wkw_lds);
+    } else if ((b < first) == (x_first != 0)) {
+        wkw_part<E, X, true>(gx, x_tiles_m, x_tiles_n, b < first ? b : b - first, vec_flags, wkw_lds);
+    } else {
+        wkw_part<E, W, false>(gw, w_tiles_m, w_tiles_n, b < first ? b : b - first, vec_flags >> 2, wkw_lds);
+    }
+}
+
+template <typename E, WkwTile X, WkwTile W>
+static int launch_linear_backward_wavekw_t(const GemmArgs& gx, const GemmArgs& gw, void* db, int accumulate_db) {
+    const int xm = (gx.m + 16 * WkwShape<X>::TM - 1) / (16 * WkwShape<X>::TM), xn = (gx.n + 16 * WkwShape<X>::TN - 1) / (16 * WkwShape<X>::TN);
+    const int wm = (gw.m + 16 * WkwShape<W>::TM - 1) / (16 * WkwShape<W>::TM), wn = (gw.n + 16 * WkwShape<W>::TN - 1) / (16 * WkwShape<W>::TN);
+    // whole rounds of the XCDs, so that the tiles' workgroups stay where their schedules want them
+    const auto slots = [](WkwTile k, int tiles) { return ((k == WKW_TINY ? (tiles + 1) / 2 : tiles) + 7) / 8 * 8; };
+    const BiasGradient sums{db, gx.k, accumulate_db, db ? ((gx.k - 1) / StripSums<E, 512>::COLS + 8) / 8 * 8 : 0};
+    constexpr size_t xs = wkw_part_smem<E, X, true>(), ws = wkw_part_smem<E, W, false>(), part = xs > ws ? xs : ws, smem = part > StripSums<E, 512>::LDS ? part : StripSums<E, 512>::LDS;
+    static_assert(smem <= 64 * 1024, "no attribute needed");
+    const int x_slots = slots(X, xm * xn), w_slots = slots(W, wm * wn);
+    const int flags = (tiny_a_vec(gx) ? 1 : 0) | (tiny_b_vec(gx) ? 2 : 0) | (tiny_a_vec(gw) ? 4 : 0) | (tiny_b_vec(gw) ? 8 : 0);
+    hipLaunchKernelGGL((linear_backward_wavekw_kernel<E, X, W>), dim3(sums.blocks + x_slots + w_slots), dim3(512), smem, current_stream(), gx, gw, sums, xm, xn, wm, wn, x_slots, w_slots, gx.k >= gw.k, flags);
+    return check_launch("linear_backward_wavekw_kernel") ? 0 : -1;
+}
+
+bool linear_backward_wavekw_takes(WkwTile x, WkwTile w, int dtype) {
+    const bool f32 = dtype == RP_DTYPE_FLOAT32;
+    const auto small = [&](WkwTile k) { return k == WKW_16X16 || k == WKW_32X32 || (f32 && k == WKW_TINY); };
+    return small(x) && (small(w) || (f32 && w == WKW_16X32)) && !(x == WKW_TINY && w == WKW_TINY);
+}
+
+template <typename E, WkwTile X>
+static int launch_linear_backward_wavekw_x(const GemmArgs& gx, const GemmArgs& gw, WkwTile w, void* db, int accumulate_db) {
+    if constexpr (sizeof(E) == 4) {
+        if (w == WKW_16X32) return launch_linear_backward_wavekw_t<E, X, WKW_16X32>(gx, gw, db, accumulate_db);
+        if constexpr (X != WKW_TINY)
+            if (w == WKW_TINY) return launch_linear_backward_wavekw_t<E, X, WKW_TINY>(gx, gw, db, accumulate_db);
+    }
+    return w == WKW_32X32 ? launch_linear_backward_wavekw_t<E, X, WKW_32X32>(gx, gw, db, accumulate_db) : launch_linear_backward_wavekw_t<E, X, WKW_16X16>(gx, gw, db, accumulate_db);
+}
+
+int launch_linear_backward_wavekw(const GemmArgs& gx, const GemmArgs& gw, WkwTile x, WkwTile w, void* db, int accumulate_db, int dtype) {
+    if (dtype == RP_DTYPE_FLOAT64) return x == WKW_32X32 ? launch_linear_backward_wavekw_x<double, WKW_32X32>(gx, gw, w, db, accumulate_db) : launch_linear_backward_wavekw_x<double, WKW_16X16>(gx, gw, w, db, accumulate_db);
+    switch (x) {
+        case WKW_TINY: return launch_linear_backward_wavekw_x<float, WKW_TINY>(gx, gw, w, db, accumulate_db);
+        case WKW_32X32: return launch_linear_backward_wavekw_x<float, WKW_32X32>(gx, gw, w, db, accumulate_db);
+        default: return launch_linear_backward_wavekw_x<float, WKW_16X16>(gx, gw, w, db, accumulate_db);
     }
 }
 

@@ -825,6 +825,34 @@ def test_gradients_of_ragged_layers_in_one_launch(m, k, n, dt):
             assert np.array_equal(g.numpy(), t.numpy())
 
 
+@pytest.mark.parametrize("dt,m,k,n", [(F32,) + s for s in ((935, 213, 862), (20, 100, 700), (700, 30, 40), (600, 250, 600), (600, 900, 50), (513, 64, 2000), (33, 1200, 600), (600, 130, 500),
+                                                          (520, 420, 500), (64, 1024, 1024), (1100, 40, 600))]
+                         + [(F64,) + s for s in ((89, 2787, 286), (64, 60, 70), (500, 40, 600), (200, 1000, 33), (33, 100, 2000), (1030, 64, 96))])
+def test_gradients_whose_waves_share_k_in_one_launch(dt, m, k, n):
+    """fp32 and fp64 layers, every pair of tiles that the two products can be on: dX, dW and db together have the bits of the three on their own, also
+    accumulated; dW written over W (which dX reads) is the three one after the other."""
+    rng = np.random.default_rng(m + k + n)
+    L = capi.lib()
+    x, w, dy = rand_storage(rng, (m, k), dt), rand_storage(rng, (k, n), dt), rand_storage(rng, (m, n), dt)
+    d_x, d_w, d_dy = Dev(x, dt), Dev(w, dt), Dev(dy, dt)
+    init = [rand_storage(rng, s, dt) for s in ((m, k), (k, n), (n,))]
+    for acc in (0, 1):
+        want, got = [Dev(i, dt) for i in init], [Dev(i, dt) for i in init]
+        capi.gemm(want[0].ptr, d_dy.ptr, d_w.ptr, None, 1, m, n, k, (0, n, 1), (0, 1, n), (0, k, 1), bool(acc), dt)
+        capi.gemm(want[1].ptr, d_x.ptr, d_dy.ptr, None, 1, k, m, n, (0, 1, k), (0, n, 1), (0, n, 1), bool(acc), dt)
+        capi.check(L.rp_hip_reduce_rows(want[2].ptr, d_dy.ptr, m, n, acc, dt), "reduce_rows")
+        capi.check(L.rp_hip_linear_backward(got[0].ptr, got[1].ptr, got[2].ptr, d_dy.ptr, d_x.ptr, d_w.ptr, m, k, n, k, 1, n, 1, k, 1, n, 1, acc, acc, acc, dt), "linear_backward")
+        assert capi.last_gemm_kernel() == "linear_backward_wavek"
+        for g, t in zip(got, want):
+            assert np.array_equal(g.numpy(), t.numpy())
+    want, got = [Dev(i, dt) for i in init[:2]], Dev(init[0], dt)
+    capi.gemm(want[0].ptr, d_dy.ptr, d_w.ptr, None, 1, m, n, k, (0, n, 1), (0, 1, n), (0, k, 1), False, dt)
+    capi.gemm(want[1].ptr, d_x.ptr, d_dy.ptr, None, 1, k, m, n, (0, 1, k), (0, n, 1), (0, n, 1), False, dt)
+    capi.check(L.rp_hip_linear_backward(got.ptr, d_w.ptr, None, d_dy.ptr, d_x.ptr, d_w.ptr, m, k, n, k, 1, n, 1, k, 1, n, 1, 0, 0, 0, dt), "dW over W")
+    assert capi.last_gemm_kernel() != "linear_backward_wavek"
+    assert np.array_equal(got.numpy(), want[0].numpy()) and np.array_equal(d_w.numpy(), want[1].numpy())
+
+
 def test_batch_longer_than_a_grid_axis():
     """70 000 tiny matrices in one call (the batch index rides on a grid axis of at most 65 535 blocks), A shared by
     all of them through a zero batch stride."""
