@@ -87,6 +87,14 @@ __device__ __forceinline__ void attn_add_parts(T* out, const float* parts, const
     }
 }
 
+// Eight 16-bit values, negated or not
+__device__ __forceinline__ s16x8_t attn_signed(u32x4_t v, bool negate) {
+    const uint32_t sign = negate ? 0x80008000u : 0u;
+#pragma unroll
+    for (int e = 0; e < 4; e++) v[e] ^= sign;
+    return __builtin_bit_cast(s16x8_t, v);
+}
+
 // The larger of this lane's value and that of the lane 32 away
 __device__ __forceinline__ float attn_pair_max(float x) {
     const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
@@ -129,7 +137,8 @@ __global__ void __launch_bounds__(256, D > 64 || SPLIT ? 2 : 3) attention_fwd16_
     const uint16_t* K = (const uint16_t*)g.K + (long long)z * g.k_bs;
     const uint16_t* V = (const uint16_t*)g.V + (long long)z * g.v_bs;
     // exp(scale * s - max) = exp2(s * sc - max * sc) with sc = |scale| log2 e: one fused multiply-add per score; a
-    // negative scale flips the sign of the scores first, so that the running maximum can be kept on the raw scores
+    // negative scale flips the sign of Q, so that the running maximum can be kept on the raw scores (of the scores, a select each even
+    // where the scale is not negative: forward [10, 1565, 1565, 64] in fp16 18.3 us, 17.8 this way)
     const float sc = fabsf(g.scale) * 1.44269504088896341f;
     const bool flip = g.scale < 0.f;
 
@@ -140,7 +149,7 @@ __global__ void __launch_bounds__(256, D > 64 || SPLIT ? 2 : 3) attention_fwd16_
     s16x8_t qf[KS];
 #pragma unroll
     for (int ks = 0; ks < KS; ks++)
-        qf[ks] = __builtin_bit_cast(s16x8_t, __builtin_amdgcn_raw_buffer_load_b128(q_rsrc, (int)(((long long)c * g.q_rs + 16 * ks + 8 * h) * 2), 0, 0));
+        qf[ks] = attn_signed(__builtin_amdgcn_raw_buffer_load_b128(q_rsrc, (int)(((long long)c * g.q_rs + 16 * ks + 8 * h) * 2), 0, 0), flip);
 
     // K and V blocks [32 keys][D] go to LDS, 16 bytes per thread and piece, in whole rows (every cache line is
     // requested once per workgroup; fragment loads straight from global memory would touch 32 lines per instruction
@@ -244,12 +253,6 @@ __global__ void __launch_bounds__(256, D > 64 || SPLIT ? 2 : 3) attention_fwd16_
         if constexpr (SPLIT) attn_wave_order();
         else read_vs(0);
 
-        if (flip) {
-#pragma unroll
-            for (int b = 0; b < NB; b++)
-#pragma unroll
-                for (int v = 0; v < 16; v++) st[b][v] = -st[b][v];
-        }
         const bool ragged = kb + KEYS > g.sk;               // the last block of a ragged sk
         if (ragged) {
 #pragma unroll
