@@ -325,6 +325,52 @@ __global__ void channel_sums_finish_kernel(T* out, const typename traits<T>::acc
     out[c] = r;
 }
 
+// The same in one launch, a workgroup per channel: the (plane, 64 vectors) pieces of the channel are dealt to its waves, eight of them requested at
+// a time, whatever element a plane starts at.  Bound by what a CU takes in, 25 GB/s behind 2.7 us, against two launches of 4.7 us at least and a workgroup
+// per plane, however small: taken while a channel holds no more than CHANNEL_SUM_BYTES.  bf16, us, two launches and one: 64 x 256 x 14^2 17.8 / 5.8,
+// 64 x 256 x 7^2 15.7 / 5.4, 1 x 64 x 7^2 6.3 / 3.5, 12 x 192 x 53^2 (67 KB a channel) 11.0 / 5.9; 16 x 128 x 56^2 (100 KB) 6.4 / 6.6, 64 x 64 x 56^2 9.3 / 19.
+constexpr size_t CHANNEL_SUM_BYTES = 72 * 1024;
+template <typename T>
+__global__ void __launch_bounds__(1024) channel_sums_kernel(T* out, const T* g, int batch, int channels, int hw, int accumulate) {
+    using A = typename traits<T>::acc;
+    constexpr int VEC = 16 / (int)sizeof(T), U = 8, WAVES = 16;
+    __shared__ A part[WAVES];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), c = blockIdx.x;
+    const int per_plane = (hw + 64 * VEC - 1) / (64 * VEC), pieces = batch * per_plane;
+    A s = 0;
+    for (int p0 = wave; p0 < pieces; p0 += U * WAVES) {
+        T v[U][VEC];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int piece = p0 + u * WAVES, n = piece / per_plane, at = ((piece - n * per_plane) * 64 + lane) * VEC;
+            memset(v[u], 0, 16);
+            if (piece >= pieces) continue;
+            const T* p = g + ((size_t)n * channels + c) * hw + at;
+            if (at + VEC <= hw) memcpy(v[u], p, 16);
+            else
+#pragma unroll
+                for (int e = 0; e < VEC; e++) if (at + e < hw) v[u][e] = p[e];
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            A q = widen(v[u][0]);
+#pragma unroll
+            for (int e = 1; e < VEC; e++) q += widen(v[u][e]);
+            s += q;
+        }
+    }
+    for (int half = 32; half > 0; half >>= 1) s += __shfl_xor(s, half, 64);
+    if (lane == 0) part[wave] = s;
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    A sum = part[0];
+#pragma unroll
+    for (int w = 1; w < WAVES; w++) sum += part[w];
+    T r = narrow<T>(sum);
+    if (accumulate) r = narrow<T>(widen(out[c]) + widen(r));
+    out[c] = r;
+}
+
 // ---- convolution without a lowered matrix (stride 1, "same" padding) ----
 // 16-bit images go to the kernels that read them in place (rp_conv_direct.hip) where those take the shape; what follows is for
 // fp32 and fp64, wide rows, taps other than k x 3 and k x 5, and outputs that overlap their input.
@@ -836,6 +882,10 @@ int rp_hip_channel_sums(void* out, const void* grad, int batch, int channels, in
         return -1;
     }
     if (!dtype_size(dtype)) { set_error("rp_hip_channel_sums: unsupported dtype %d", dtype); return -1; }
+    if ((size_t)batch * hw * dtype_size(dtype) <= CHANNEL_SUM_BYTES) {
+        RP_DISPATCH_DTYPE(dtype, hipLaunchKernelGGL(channel_sums_kernel<T>, dim3((unsigned)channels), dim3(1024), 0, current_stream(), (T*)out, (const T*)grad, batch, channels, hw, accumulate));
+        return check_launch("channel_sums_kernel") ? 0 : -1;
+    }
     void* partial = nullptr;                 // one accumulate-type value per (n, c) plane, from the stream-ordered pool
     if (rp_hip_malloc(&partial, (size_t)batch * channels * 8) != 0) return -1;
     RP_DISPATCH_DTYPE(dtype, launch_channel_sums<T>(out, grad, partial, batch, channels, hw, accumulate));

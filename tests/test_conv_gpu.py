@@ -94,6 +94,17 @@ def test_channel_bias_add_and_channel_sums(dt):
     assert np.array_equal(ds.numpy(), oracle.add(got0, got0, dt))
 
 
+@pytest.mark.parametrize("dt", ALL, ids=lambda d: NAMES[d])
+@pytest.mark.parametrize("N,C,HW", [(1, 1, 1), (3, 2, 513), (33, 5, 49), (4, 3, 4607), (5, 3, 8001), (5, 2, 18500)])
+def test_channel_sums_of_every_size(dt, N, C, HW):
+    """Planes that start at any element, channels on either side of what one workgroup sums; small integers, so the sums are exact before they are rounded once."""
+    rng = np.random.default_rng(N + HW)
+    g = rng.integers(-2, 3, (N, C, HW)).astype(np.float64)
+    ds = Dev.empty((C,), dt)
+    capi.check(capi.lib().rp_hip_channel_sums(ds.ptr, Dev(oracle.to_storage(g, dt), dt).ptr, N, C, HW, 0, dt), "rp_hip_channel_sums")
+    assert np.array_equal(ds.numpy(), oracle.to_storage(g.sum(axis=(0, 2)), dt))
+
+
 def test_lowering_rejects_inconsistent_geometry():
     d = capi.DeviceBuffer(1 << 16)
     L = capi.lib()
