@@ -454,6 +454,36 @@ def test_allocator_reuses_blocks_and_reports_errors():
     assert e0.elapsed_ms(e1) >= 0.0
 
 
+def test_copies_to_the_host_of_every_size_and_start():
+    """Copies that go through pinned memory and larger ones, from any byte, by several threads at once and again after the blocks were given back."""
+    rng = np.random.default_rng(49)
+    data = rng.integers(0, 256, 1 << 20, dtype=np.uint8)
+    buf = capi.DeviceBuffer.from_numpy(data)
+    bad = []
+
+    def check(at, n):
+        got = np.full(n + 2, 7, np.uint8)
+        rc = L().rp_hip_memcpy_d2h(got.ctypes.data + 1, buf.ptr + at, n)
+        if rc != 0 or got[0] != 7 or got[-1] != 7 or not np.array_equal(got[1:-1], data[at:at + n]):
+            bad.append((at, n))
+
+    sizes = (1, 15, 16, 17, 4095, 10240, 65537, 256 * 1024 - 16, 256 * 1024 - 15, 256 * 1024, 256 * 1024 + 1, 700001)
+    for _ in range(2):
+        for n in sizes:
+            for at in (0, 1, 15, 16, 4097):
+                check(at, n)
+        check(len(data) - 1, 1)
+        check(len(data) - 4099, 4099)
+        capi.check(L().rp_hip_empty_cache(), "empty_cache")
+    threads = [threading.Thread(target=lambda i=i: [check(i * 4096 + r, 3000 * i + 5) for r in range(40)]) for i in range(1, 9)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad
+    assert L().rp_hip_memcpy_d2h(data.ctypes.data, None, 4) == -1
+
+
 def test_graph_replay_matches_eager():
     """A recorded GEMM + bias-gradient + relu sequence replays to the eager result every time (no memset nodes inside)."""
     rng = np.random.default_rng(48)
