@@ -368,6 +368,33 @@ static int run_gemm(GemmArgs g, int dtype) {
     }
 }
 
+// fp32 products with segments that the waves of a workgroup share; WKW_NONE: the 64 x 64 and 128 x 128 tiles of four waves that share the output.
+// us of the products of layers [batch, C_in, H, W, C_out, k], before and here; a convolution is one product per image, so what counts is the tiles of all of them.
+// Segments along k (forward and input gradient: m = C_out, n = positions, k = taps C_in): 16 x 32 tiles, 16 x 16 where those are fewer than the CUs,
+// [1, 128, 28, 28, 64, 5] 105.7 / 16.4, [2, 256, 15, 15, 64, 3] 88.9 / 15.2, [8, 192, 14, 14, 128, 5] 185 / 64, [40, 128, 28, 28, 64, 3] 95 / 83.  They read A and B once per
+// 16 x 32 values, so with enough 64 x 64 tiles to fill the chip they are left behind, sooner where k is short: 64 channels of 3 x 3, 64 -> 64 at 28 x 28,
+// 26 images (364 tiles) 42.6 / 41.5, 33 45.0 / 50.4, 54 58.6 / 74.9; from 1024 on [60, 128, 28, 28, 64, 3] (840 tiles) 109 / 112.
+// From 192 rows on the 64 x 64 tile with k shared takes over there: [12, 64, 55, 55, 192, 3] 186 / 134 (16 x 32: 156), [9, 192, 28, 28, 256, 3] 111 / 87 (96).
+// Segments along n (weight gradients: m = C_out, n = taps C_in, k = positions): 32 x 32 up to one 64 x 64 tile a CU ([1, 128, 28, 28, 64, 5] 40.1 / 19.4, [5, 64, 56, 15, 64, 3]
+// 48.7 / 22.7, [22, 64, 48, 48, 64, 3] 96 / 85).  With nearly that many and a long k those of more than 64 rows are 64 x 64 tiles, [1, 256, 56, 56, 128, 5] 123 / 86 (32 x 32: 116), and
+// those of 64 stay what they were, [10, 64, 56, 56, 64, 5] 121 / 139.  Up to four a CU where C_out is more than 64
+// and the positions many ([18, 128, 28, 28, 192, 3] 152 / 107, but [31, 256, 26, 26, 64, 3] 109 / 143, [13, 192, 7, 7, 256, 3] 45.5 / 56.5).
+static WkwTile segmented_wavek_tile(const GemmArgs& g) {
+    if (path_disabled("wavekw") || g.a_cs != 1 || g.n < 64 || g.accumulate || g.batch > 65535 || g.b_extent * 4 >= (1ll << 31) || (63 * g.a_rs + g.k) * 4 >= (1ll << 31)) return WKW_NONE;
+    const long long cus = cu_tiles(), tiles64 = (long long)((g.m + 63) / 64) * ((g.n + 63) / 64) * g.batch;
+    if (g.seg_k > 0) {
+        if (g.seg_k % 32) return WKW_NONE;
+        if (g.m >= 192) { if (tiles64 * 4 >= cus * 7) return WKW_64X64; }
+        else if (g.k < 1024 ? tiles64 * 4 > cus * 5 : tiles64 > cus * 3) return WKW_NONE;
+        return (long long)((g.m + 15) / 16) * ((g.n + 31) / 32) * g.batch >= cus ? WKW_16X32 : WKW_16X16;
+    }
+    if (tiles64 <= cus) {
+        if (g.k < 2048 || tiles64 * 4 < cus * 3) return WKW_32X32;
+        return g.m > 64 ? WKW_64X64 : tiles64 * 8 > cus * 7 ? WKW_NONE : WKW_32X32;
+    }
+    return g.m > 64 && g.k >= 640 && tiles64 <= 4 * cus ? WKW_32X32 : WKW_NONE;
+}
+
 // C_z = A_z . B_z with B's k axis or its n axis given as segments (GemmArgs::seg_*): the MFMA kernels read every
 // segment in place, at any alignment of whole elements.  For callers inside the library (the convolution), which
 // guarantee: A with unit stride along k or m, B with unit stride along n and k a whole number of segments of whole
@@ -395,6 +422,10 @@ int launch_gemm_segmented_b(const GemmArgs& g, int dtype) {
         Plan p{FAM_MFMA16, 64, 64, !a_kc, g.seg_k > 0, true, "mfma16"};
         choose_tile16(p, g.batch, g.m, g.k, g.n);
         return launch_mfma16(g, p, dtype);
+    }
+    if (dtype == RP_DTYPE_FLOAT32) {
+        const WkwTile tile = segmented_wavek_tile(g);
+        if (tile != WKW_NONE) return launch_wavekw_segmented(g, tile);
     }
     Plan p{FAM_MFMAW, 64, 64, !a_kc, g.seg_k > 0, true, "mfmaw"};
     const long long tiles128 = (long long)((g.m + 127) / 128) * ((g.n + 127) / 128) * g.batch;

@@ -53,9 +53,21 @@ __device__ __forceinline__ wkw_vec_t<E, N> wkw_fetch(__amdgpu_buffer_rsrc_t rsrc
 template <typename E, int T>
 struct WkwFragments { wkw_vec_t<E, wkw_cfg<E>::KV> v[WKW_CHUNKS][T]; };
 
+// Byte offset of row `first + r` of an operand with unit stride along k, from the tile's first row (SEG: from the operand)
+template <typename E, bool SEG>
+__device__ __forceinline__ uint32_t wkw_row_offset(const GemmArgs& g, long long fs, int first, int extent, int r) {
+    const int row = first + r < extent ? first + r : extent - 1;
+    if constexpr (SEG) {
+        const int seg = row / g.seg_n, c = row - seg * g.seg_n;
+        return (uint32_t)((seg / g.seg_w * g.seg_sh + seg % g.seg_w * g.seg_sw + c * fs) * (long long)sizeof(E));
+    }
+    return (uint32_t)((row - first) * fs * (long long)sizeof(E));
+}
+
 // Pieces of one operand on their way, and where a lane finds its part of them.
 // Unit stride along k, 16 rows: a load takes whole lines of eight rows, and LDS of the wave's own turns rows into fragments.
-template <typename E, bool KC, int T>
+// SEG: B's k or n axis is a list of segments (GemmArgs::seg_*), for convolutions.
+template <typename E, bool KC, int T, bool SEG>
 struct WkwOperand {
     static_assert(KC && T == 1, "the others are below");
     static constexpr int KV = wkw_cfg<E>::KV, SZ = (int)sizeof(E);
@@ -65,14 +77,11 @@ struct WkwOperand {
     struct Piece { wkw_vec_t<E, KV> raw[2]; };
 
     // first: the tile's first row; rows past the last one read the last one
-    __device__ __forceinline__ void init(const E* base, long long fs, long long ks, int first, int extent, int lane) {
-        rsrc = buffer_rsrc(base + (long long)first * fs, 0x7fffffffll);
+    __device__ __forceinline__ void init(const GemmArgs& g, const E* base, long long fs, long long ks, int first, int extent, int lane) {
+        rsrc = buffer_rsrc(base + (SEG ? 0 : (long long)first * fs), 0x7fffffffll);
         k_lane = lane % 8 * KV;
 #pragma unroll
-        for (int i = 0; i < 2; i++) {
-            const int r = 8 * i + lane / 8;
-            off[i] = (uint32_t)((first + r < extent ? r : extent - 1 - first) * fs * SZ) + k_lane * SZ;
-        }
+        for (int i = 0; i < 2; i++) off[i] = wkw_row_offset<E, SEG>(g, fs, first, extent, 8 * i + lane / 8) + k_lane * SZ;
         lds_write = lane / 8 * WKW_ROW_PITCH + lane % 8 * 16;
         lds_read = lane % 16 * WKW_ROW_PITCH + lane / 16 * 16;
     }
@@ -99,7 +108,7 @@ struct WkwOperand {
 };
 
 // Unit stride along k, more rows: fragment t holds rows 16 t + r, loaded as it is.
-template <typename E, int T>
+template <typename E, int T, bool SEG>
 struct WkwOperandRows {
     static constexpr int KV = wkw_cfg<E>::KV, SZ = (int)sizeof(E);
     __amdgpu_buffer_rsrc_t rsrc;
@@ -107,14 +116,11 @@ struct WkwOperandRows {
     int k_lane;
     struct Piece { wkw_vec_t<E, KV> v[WKW_CHUNKS][T]; };
 
-    __device__ __forceinline__ void init(const E* base, long long fs, long long ks, int first, int extent, int lane) {
-        rsrc = buffer_rsrc(base + (long long)first * fs, 0x7fffffffll);
+    __device__ __forceinline__ void init(const GemmArgs& g, const E* base, long long fs, long long ks, int first, int extent, int lane) {
+        rsrc = buffer_rsrc(base + (SEG ? 0 : (long long)first * fs), 0x7fffffffll);
         k_lane = lane / 16 * KV;
 #pragma unroll
-        for (int t = 0; t < T; t++) {
-            const int r = 16 * t + lane % 16;
-            off[t] = (uint32_t)((first + r < extent ? r : extent - 1 - first) * fs * SZ) + k_lane * SZ;
-        }
+        for (int t = 0; t < T; t++) off[t] = wkw_row_offset<E, SEG>(g, fs, first, extent, 16 * t + lane % 16) + k_lane * SZ;
     }
     __device__ __forceinline__ void load(Piece& p, int piece) const {
 #pragma unroll
@@ -138,27 +144,39 @@ struct WkwOperandRows {
 
 // Unit stride along the free index: fragment t holds rows T r + t, so that a lane's T values of a k row are neighbours and 16 lanes load a
 // stretch of it, which is a fragment as it is.
-template <typename E, int T>
-struct WkwOperand<E, false, T> {
+template <typename E, int T, bool SEG>
+struct WkwOperand<E, false, T, SEG> {
     static constexpr int KV = wkw_cfg<E>::KV, SZ = (int)sizeof(E);
     __amdgpu_buffer_rsrc_t rsrc;
     uint32_t off[KV], k_bytes;                           // bytes; from one k to the next
     int k_lane;
     struct Piece { wkw_vec_t<E, T> row[WKW_CHUNKS][KV]; };
 
+    int seg_k, seg_w;
+    uint32_t seg_sh, seg_sw;                             // bytes
+
     // first: at most extent - 16 T
-    __device__ __forceinline__ void init(const E* base, long long fs, long long ks, int first, int extent, int lane) {
+    __device__ __forceinline__ void init(const GemmArgs& g, const E* base, long long fs, long long ks, int first, int extent, int lane) {
         rsrc = buffer_rsrc(base + first, 0x7fffffffll);
+        if constexpr (SEG) { seg_k = g.seg_k; seg_w = g.seg_w; seg_sh = (uint32_t)(g.seg_sh * SZ); seg_sw = (uint32_t)(g.seg_sw * SZ); }
         k_bytes = (uint32_t)ks * SZ;
         k_lane = lane / 16 * KV;
 #pragma unroll
         for (int j = 0; j < KV; j++) off[j] = (uint32_t)(k_lane + j) * k_bytes + lane % 16 * T * SZ;
     }
+    // a piece lies inside a segment (whole pieces long)
     __device__ __forceinline__ void load(Piece& p, int piece) const {
+        uint32_t start = 0, k0 = (uint32_t)piece * wkw_piece<E>();
+        if constexpr (SEG) {
+            const uint32_t seg = k0 / (uint32_t)seg_k, row = seg / (uint32_t)seg_w;
+            k0 -= seg * (uint32_t)seg_k;
+            start = row * seg_sh + (seg - row * (uint32_t)seg_w) * seg_sw;
+        }
+        start += k0 * k_bytes;
 #pragma unroll
         for (int c = 0; c < WKW_CHUNKS; c++)
 #pragma unroll
-            for (int j = 0; j < KV; j++) p.row[c][j] = wkw_fetch<E, T>(rsrc, off[j], (uint32_t)(piece * WKW_CHUNKS + c) * 4 * KV * k_bytes);
+            for (int j = 0; j < KV; j++) p.row[c][j] = wkw_fetch<E, T>(rsrc, off[j], start + (uint32_t)c * 4 * KV * k_bytes);
     }
     __device__ __forceinline__ void load_end(Piece& p, int piece, int left) const {
 #pragma unroll
@@ -172,16 +190,16 @@ struct WkwOperand<E, false, T> {
     __device__ __forceinline__ void fragments(WkwFragments<E, T>&, const unsigned char*) const {}
 };
 
-template <typename E, bool KC, int T>
-using wkw_operand = std::conditional_t<KC && (T > 1), WkwOperandRows<E, T>, WkwOperand<E, KC, T == 1 || !KC ? T : 1>>;
+template <typename E, bool KC, int T, bool SEG>
+using wkw_operand = std::conditional_t<KC && (T > 1), WkwOperandRows<E, T, SEG>, WkwOperand<E, KC, T == 1 || !KC ? T : 1, SEG>>;
 
 // The 16 TM x 16 TN tile `block` of matrix z, by NW waves.  k goes in pieces, dealt to the waves in turn: a wave multiplies one piece out of
 // registers while the next is on its way there, and the partial tiles meet in LDS, where they are added in a fixed order.
-template <typename E, bool A_KC, bool B_KC, int TM, int TN, int NW>
+template <typename E, bool A_KC, bool B_KC, int TM, int TN, int NW, bool SEG = false>
 __device__ __forceinline__ void gemm_wavekw_block(const GemmArgs& g, int tiles_m, int tiles_n, int block, int z, unsigned char* lds) {
     using cfg = wkw_cfg<E>;
-    using OpA = wkw_operand<E, A_KC, TM>;
-    using OpB = wkw_operand<E, B_KC, TN>;
+    using OpA = wkw_operand<E, A_KC, TM, false>;
+    using OpB = wkw_operand<E, B_KC, TN, SEG>;
     constexpr int PK = wkw_piece<E>(), KV = cfg::KV;
     constexpr bool STAGED = wkw_staged(A_KC, TM) || wkw_staged(B_KC, TN);
     // block b runs on XCD b % 8: a run of tiles along the shorter side of the output for each XCD, whose L2 then serves what they share
@@ -194,8 +212,8 @@ __device__ __forceinline__ void gemm_wavekw_block(const GemmArgs& g, int tiles_m
     const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
     OpA opa;
     OpB opb;
-    opa.init((const E*)g.A + (long long)z * g.a_bs, g.a_rs, g.a_cs, ms, g.m, lane);
-    opb.init((const E*)g.B + (long long)z * g.b_bs, g.b_cs, g.b_rs, ns, g.n, lane);
+    opa.init(g, (const E*)g.A + (long long)z * g.a_bs, g.a_rs, g.a_cs, ms, g.m, lane);
+    opb.init(g, (const E*)g.B + (long long)z * g.b_bs, g.b_cs, g.b_rs, ns, g.n, lane);
     unsigned char* const a_stage = lds + wave * wkw_stage<A_KC, B_KC, TM, TN>(), * const b_stage = a_stage + (wkw_staged(A_KC, TM) ? 16 * WKW_ROW_PITCH : 0);
 
     // Two pieces on their way at a time.  Sets of accumulators: where there are registers for them a piece's chunks, and pieces in turn, have their
@@ -309,6 +327,16 @@ __device__ __forceinline__ void gemm_wavekw_block(const GemmArgs& g, int tiles_m
 #pragma unroll
         for (int w = 1; w < SHARES; w++) sum += parts[w * SHARE + at];
         if (gm < m0 || gm >= g.m || gn < n0 || gn >= g.n) continue;
+        if constexpr (SEG) {                             // folded output, bias per row: see GemmArgs
+            int at_col = gn;
+            if (g.c_fold_from > 0) {
+                const int run = gn / g.c_fold_from, within = gn - run * g.c_fold_from;
+                if (within >= g.c_fold_to) continue;
+                at_col = run * g.c_fold_to + within;
+            }
+            C[gm * g.c_rs + at_col * g.c_cs] = finish<E>(sum, bias != nullptr, bias ? bias[g.bias_by_row ? gm : gn] : (E)0, false, (E)0);
+            continue;
+        }
         E* out = C + gm * g.c_rs + gn * g.c_cs;
         *out = finish<E>(sum, bias != nullptr, bias ? bias[gn] : (E)0, g.accumulate != 0, g.accumulate ? *out : (E)0);
     }
@@ -317,6 +345,7 @@ __device__ __forceinline__ void gemm_wavekw_block(const GemmArgs& g, int tiles_m
 // Tiles of a product, and whether the operands can be addressed that way; WKW_NONE: not at all
 enum WkwTile { WKW_NONE, WKW_16X16, WKW_16X32, WKW_32X32, WKW_16X64, WKW_64X64, WKW_TINY };       // WKW_TINY: the 16 x 16 tiles of rp_gemm_tiny.h, two a workgroup
 WkwTile wavekw_tile(const GemmArgs& g, int dtype);
+int launch_wavekw_segmented(const GemmArgs& g, WkwTile tile);       // fp32, A with unit stride along k, B in segments
 // All gradients of a Linear layer in one launch, each product on the tiles that it would get alone; gx.A is dY [gx.m, gx.k], dense; db: gx.k column sums of dY, or null
 bool linear_backward_wavekw_takes(WkwTile x, WkwTile w, int dtype);
 int launch_linear_backward_wavekw(const GemmArgs& gx, const GemmArgs& gw, WkwTile x, WkwTile w, void* db, int accumulate_db, int dtype);

@@ -19,17 +19,17 @@ namespace rp {
 // waves a SIMD whose registers have to fit: two workgroups on a CU, one of the 64 x 64 tile
 constexpr int wkw_waves(int tiles) { return tiles <= 4 ? 4 : 2; }
 
-template <typename E, bool A_KC, bool B_KC, int TM, int TN, int NW>
+template <typename E, bool A_KC, bool B_KC, int TM, int TN, int NW, bool SEG>
 __global__ void __launch_bounds__(64 * NW, wkw_waves(TM * TN)) gemm_wavekw_kernel(GemmArgs g, int tiles_m, int tiles_n) {
     extern __shared__ __attribute__((aligned(16))) unsigned char wkw_lds[];
-    gemm_wavekw_block<E, A_KC, B_KC, TM, TN, NW>(g, tiles_m, tiles_n, blockIdx.x, blockIdx.y, wkw_lds);
+    gemm_wavekw_block<E, A_KC, B_KC, TM, TN, NW, SEG>(g, tiles_m, tiles_n, blockIdx.x, blockIdx.y, wkw_lds);
 }
 
-template <typename E, bool A_KC, bool B_KC, int TM, int TN, int NW>
+template <typename E, bool A_KC, bool B_KC, int TM, int TN, int NW, bool SEG = false>
 static int launch_wavekw_t(const GemmArgs& g) {
     constexpr size_t smem = wkw_smem<E, A_KC, B_KC, TM, TN, NW>();
     const int tiles_m = (g.m + 16 * TM - 1) / (16 * TM), tiles_n = (g.n + 16 * TN - 1) / (16 * TN);
-    auto kern = gemm_wavekw_kernel<E, A_KC, B_KC, TM, TN, NW>;
+    auto kern = gemm_wavekw_kernel<E, A_KC, B_KC, TM, TN, NW, SEG>;
     if (smem > 64 * 1024 && !check_hip(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem), "hipFuncSetAttribute")) return -1;
     hipLaunchKernelGGL(kern, dim3((unsigned)((tiles_m * tiles_n + 7) / 8 * 8), g.batch), dim3(64 * NW), smem, current_stream(), g, tiles_m, tiles_n);
     return check_launch("gemm_wavekw_kernel") ? 0 : -1;
@@ -74,6 +74,19 @@ int launch_wavekw(const GemmArgs& g, int dtype) {
         case WKW_32X32: return launch_wavekw_layout<float, 2, 2, 8>(g);
         case WKW_16X32: return launch_wavekw_layout<float, 1, 2, 8>(g);
         default: return launch_wavekw_layout<float, 1, 1, 8>(g);
+    }
+}
+
+template <int TM, int TN>
+static int launch_wavekw_segmented_t(const GemmArgs& g) {
+    return g.seg_k > 0 ? launch_wavekw_t<float, true, false, TM, TN, 8, true>(g) : launch_wavekw_t<float, true, true, TM, TN, 8, true>(g);
+}
+int launch_wavekw_segmented(const GemmArgs& g, WkwTile tile) {
+    switch (tile) {
+        case WKW_64X64: return launch_wavekw_segmented_t<4, 4>(g);
+        case WKW_32X32: return launch_wavekw_segmented_t<2, 2>(g);
+        case WKW_16X32: return launch_wavekw_segmented_t<1, 2>(g);
+        default: return launch_wavekw_segmented_t<1, 1>(g);
     }
 }
 

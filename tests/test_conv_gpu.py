@@ -226,6 +226,32 @@ def test_same_convolution_from_the_image_is_exact_on_integers(dt, case, forward,
     assert np.array_equal(oracle.to_f64(gw.numpy(), dt), oracle.to_f64(want, dt))
 
 
+SHARED_CASES = [  # fp32 (batch, C_in, H, W, C_out, kH, kW) on 256 CUs.  Forward and input gradient: 16 x 16 tiles, 16 x 32, 64 x 64, the tiles without
+                  # shared k; weight gradient: 32 x 32 up to one 64 x 64 tile a CU, 64 x 64, 32 x 32 above; whole and folded rows, ragged channels
+    (1, 64, 9, 9, 64, 3, 3), (1, 96, 6, 11, 40, 5, 3), (4, 64, 28, 28, 96, 3, 3), (7, 192, 41, 40, 192, 3, 3), (6, 64, 53, 39, 200, 3, 3),
+    (28, 64, 28, 28, 64, 3, 3), (22, 64, 48, 48, 64, 3, 3), (3, 64, 50, 51, 128, 5, 5), (17, 32, 28, 28, 128, 3, 3)]
+
+
+@pytest.mark.parametrize("case", SHARED_CASES, ids=lambda c: "x".join(map(str, c)))
+def test_same_convolution_in_fp32_is_exact_on_integers(case):
+    """Small integers: every sum is an integer below 2^24, exact in any order of additions."""
+    import torch
+    N, Ci, H, W, Co, kH, kW = case
+    L = capi.lib()
+    rng = np.random.default_rng(H + W)
+    ints = lambda *shape: rng.integers(-3, 4, shape).astype(np.float32)          # noqa: E731
+    x, w, b, g = ints(N, Ci, H, W), ints(Co, Ci, kH, kW), ints(Co), ints(N, Co, H, W)
+    dx_, dw_, db_, dg_ = (Dev(v, F32) for v in (x, w, b, g))
+    y, gx, gw = Dev.empty((N, Co, H, W), F32), Dev.empty((N, Ci, H, W), F32), Dev.empty((Co, Ci, kH, kW), F32)
+    xt, wt, gt, pad = torch.tensor(x), torch.tensor(w), torch.tensor(g), (kH // 2, kW // 2)
+    capi.check(L.rp_hip_conv2d_same_forward(y.ptr, dx_.ptr, dw_.ptr, db_.ptr, N, Ci, H, W, Co, kH, kW, F32), "same forward")
+    assert np.array_equal(y.numpy(), torch.nn.functional.conv2d(xt, wt, torch.tensor(b), padding=pad).numpy())
+    with_dx = L.rp_hip_conv2d_same_supported(Co, H, W, kH, kW, F32) == 1
+    capi.check(L.rp_hip_conv2d_same_backward(gx.ptr if with_dx else None, gw.ptr, dg_.ptr, dx_.ptr, dw_.ptr, N, Ci, H, W, Co, kH, kW, F32), "same backward")
+    if with_dx: assert np.array_equal(gx.numpy(), torch.nn.grad.conv2d_input((N, Ci, H, W), wt, gt, padding=pad).numpy())
+    assert np.array_equal(gw.numpy(), torch.nn.grad.conv2d_weight(xt, (Co, Ci, kH, kW), gt, padding=pad).numpy())
+
+
 @pytest.mark.parametrize("dt", [F16, BF16], ids=lambda d: NAMES[d])
 @pytest.mark.parametrize("case", [(23, 64, 56, 52, 64, 3), (29, 64, 48, 48, 64, 5), (2, 128, 12, 40, 64, 3), (1, 64, 53, 53, 128, 5)], ids=lambda c: "x".join(map(str, c)))
 def test_weight_gradient_does_not_depend_on_the_input_gradient(dt, case):
