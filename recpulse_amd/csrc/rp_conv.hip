@@ -860,6 +860,8 @@ int rp_hip_conv2d_same_backward(void* dx, void* dw, const void* dy, const void* 
     const bool apart = !dx || images_apart(dx, C_in, dy, C_out, batch, H, W, dtype);
     const bool direct_dx = dx && apart && conv_taps16_takes(batch, C_out, C_in, H, W, kH, kW, dtype);
     const bool direct_dw = dw && apart && conv_dw16_takes(batch, C_in, C_out, H, W, kH, kW, dtype);
+    int both = 0;
+    if (direct_dx && direct_dw && launch_conv_gradients16(dx, dw, dy, x, w, batch, C_in, C_out, H, W, kH, kW, dtype, both)) return both;
     void *const planes_dx = direct_dx ? nullptr : dx, *const planes_dw = direct_dw ? nullptr : dw;
     if (direct_dx && launch_conv_taps16(dx, dy, w, nullptr, batch, C_out, C_in, H, W, kH, kW, true, dtype) != 0) return -1;
     if (planes_dx || planes_dw) {

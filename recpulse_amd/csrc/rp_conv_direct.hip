@@ -76,20 +76,68 @@ __device__ __forceinline__ u32x4_t gather_position(const V (&v)[8]) {
 
 // Blocks that read the same part of an image go to one XCD side by side, and so do neighbouring parts: block b runs on XCD b % 8,
 // every XCD owns a run of consecutive parts, and a part's `shared` blocks follow each other.  False: nothing left to do.
-__device__ __forceinline__ bool shared_block(int parts, int shared, int& part, int& which) {
-    const int per = (parts + 7) / 8, slot = (int)blockIdx.x / 8;
-    part = (int)(blockIdx.x % 8) * per + slot / shared;
+__device__ __forceinline__ bool shared_block(int block, int parts, int shared, int& part, int& which) {
+    const int per = (parts + 7) / 8, slot = block / 8;
+    part = block % 8 * per + slot / shared;
     which = slot % shared;
     return slot / shared < per && part < parts;
 }
 static unsigned shared_grid(int parts, int shared) { return 8u * (unsigned)((parts + 7) / 8) * (unsigned)shared; }
 
 // ---- weights: [C_out][C_in][tap] -> [C_from / 32][tap][C_to][32], for the input gradient transposed and the taps reversed ----
-__global__ void __launch_bounds__(256) conv_weights_by_tap_kernel(uint16_t* wt, const uint16_t* w, int C_from, int C_to, int taps, int total, int for_input_grad) {
+struct ConvSort {
+    uint16_t* wt;
+    const uint16_t* w;
+    int C_from, C_to, taps, total, for_input_grad;
+    int blocks;                                  // of CD_SORT values, beside other work: a whole number of eights (0: none)
+};
+constexpr int CD_SORT = 2048;
+__device__ __forceinline__ uint16_t weight_by_tap(const ConvSort& s, int i) {
+    const int row = i / 32, to = row % s.C_to, tap = row / s.C_to % s.taps, from = row / (s.C_to * s.taps) * 32 + i % 32;
+    return s.for_input_grad ? s.w[((size_t)from * s.C_to + to) * s.taps + s.taps - 1 - tap] : s.w[((size_t)to * s.C_from + from) * s.taps + tap];
+}
+__global__ void __launch_bounds__(256) conv_weights_by_tap_kernel(ConvSort s) {
     const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= total) return;
-    const int row = i / 32, to = row % C_to, tap = row / C_to % taps, from = row / (C_to * taps) * 32 + i % 32;
-    wt[i] = for_input_grad ? w[((size_t)from * C_to + to) * taps + taps - 1 - tap] : w[((size_t)to * C_from + from) * taps + tap];
+    if (i < s.total) s.wt[i] = weight_by_tap(s, i);
+}
+
+// ---- weight gradient, second half ----
+struct ConvFinish {
+    void* dw;
+    const float* part;                           // [split][tap][C_out][C_in]
+    int splits, channels, taps;
+    int first, blocks;                           // beside other work: the first of these blocks, and how many (0: none)
+};
+// dw[co][ci][tap] = sum over the splits, in their order (four runs of them side by side, then the runs in order), rounded once;
+// 64 V neighbouring sums for 256 threads
+template <typename T, int V>
+__device__ __forceinline__ void conv_dw_finish(const ConvFinish& f, int unit, float (*runs)[64 * V]) {
+    typedef float __attribute__((ext_vector_type(V))) sums_t;
+    const int total = f.channels * f.taps, lane = threadIdx.x & 63, i = (unit * 64 + lane) * V, run = threadIdx.x >> 6;
+    const int per = (f.splits + 3) / 4, s0 = run * per, s1 = s0 + per < f.splits ? s0 + per : f.splits;
+    sums_t sum = (sums_t)(0.f);
+    if (i < total) {
+        int s = s0;
+        for (; s + 8 <= s1; s += 8) {
+            sums_t v[8];
+#pragma unroll
+            for (int u = 0; u < 8; u++) v[u] = *(const sums_t*)(f.part + (size_t)(s + u) * total + i);
+#pragma unroll
+            for (int u = 0; u < 8; u++) sum += v[u];
+        }
+        for (; s < s1; s++) sum += *(const sums_t*)(f.part + (size_t)s * total + i);
+    }
+    if (run > 0) *(sums_t*)(runs[run - 1] + lane * V) = sum;
+    __syncthreads();
+    if (run == 0 && i < total) {
+#pragma unroll
+        for (int r = 0; r < 3; r++) sum += *(const sums_t*)(runs[r] + lane * V);
+#pragma unroll
+        for (int e = 0; e < V; e++) {
+            const int tap = (i + e) / f.channels, c = i + e - tap * f.channels;          // c = co * C_in + ci
+            ((T*)f.dw)[(size_t)c * f.taps + tap] = narrow<T>(sum[e]);
+        }
+    }
 }
 
 // ---- forward / input gradient ----
@@ -108,6 +156,7 @@ struct ConvTapsArgs {
     int cells;                                   // room for the strip with its borders
     int groups;                                  // of positions
     int by_channel;                              // wt is [C_to][C_from][tap], as the caller keeps weights (3 x 3 taps only)
+    ConvFinish finish;                           // the last blocks add up a weight gradient
 };
 
 // A workgroup computes 64 channels of `positions` consecutive positions (over all samples), four waves side by side: NPOS = 256 gives
@@ -128,9 +177,16 @@ __global__ void __launch_bounds__(256, 2) conv_taps16_kernel(ConvTapsArgs g) {
     uint16_t* cells = cd_smem;
     uint16_t* wts = cd_smem + (size_t)g.cells * CD_PITCH;
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6, wn = wave % WN, wm = wave / WN;
+    if (g.finish.blocks > 0 && (int)blockIdx.x >= g.finish.first) {
+        for (int u = (int)blockIdx.x - g.finish.first; u * 256 < g.finish.channels * g.finish.taps; u += g.finish.blocks) {
+            conv_dw_finish<T, 4>(g.finish, u, (float (*)[256])cd_smem);
+            __syncthreads();
+        }
+        return;
+    }
     const int H = g.H, W = g.W, HW = H * W, total = g.batch * HW, ph = g.kH / 2, Wc = W + KW - 1, taps = g.kH * KW;
     int group, c_tile;
-    if (!shared_block(g.groups, (g.C_to + CD_CO - 1) / CD_CO, group, c_tile)) return;
+    if (!shared_block(blockIdx.x, g.groups, (g.C_to + CD_CO - 1) / CD_CO, group, c_tile)) return;
     const int q0 = group * g.positions, q1 = q0 + g.positions < total ? q0 + g.positions : total;
     const int co0 = c_tile * CD_CO;
     // Samples n_lo .. n_hi have rows here.  LDS holds, sample by sample, the image rows that the output rows reach.
@@ -363,6 +419,7 @@ struct ConvDwArgs {
     int rows;                                    // image rows of a strip
     int strips, per_split;                       // strips of the whole batch (over all samples), and of one split
     int c_in_tiles, splits;
+    ConvSort sort;                               // the first blocks sort the weights of an input gradient
 };
 
 // A workgroup owns 64 x 64 channels of one tap row and walks the strips of its split; the sums stay in registers.  k is the
@@ -375,13 +432,20 @@ template <typename T, int KW, int VW>
 __global__ void __launch_bounds__(256, 2) conv_dw16_kernel(ConvDwArgs g) {
     extern __shared__ __attribute__((aligned(16))) uint16_t cd_smem[];
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6, half = wave & 1, parity = wave >> 1;
+    if ((int)blockIdx.x < g.sort.blocks) {
+        const int first = (int)blockIdx.x * CD_SORT + t;
+#pragma unroll
+        for (int i = 0; i < CD_SORT / 256; i++)
+            if (first + 256 * i < g.sort.total) g.sort.wt[first + 256 * i] = weight_by_tap(g.sort, first + 256 * i);
+        return;
+    }
     const int H = g.H, W = g.W, HW = H * W, Wc = W + KW - 1, Wk = (W + 3) & ~3, npos = g.rows * Wk, steps = (npos + 15) / 16;
     const int cells = g.rows * Wc + KW;          // the last KW cells stay zero
     uint16_t* xs = cd_smem;
     uint16_t* ds = cd_smem + (size_t)cells * CW_XP;
     const int tiles = g.c_in_tiles * ((g.C_out + 63) / 64);
     int part, kh;                                // the tap rows of a part read the same rows of the images
-    if (!shared_block(g.splits * tiles, g.kH, part, kh)) return;
+    if (!shared_block((int)blockIdx.x - g.sort.blocks, g.splits * tiles, g.kH, part, kh)) return;
     const int split = part / tiles, tile = part % tiles, co0 = (tile / g.c_in_tiles) * 64, ci0 = (tile % g.c_in_tiles) * 64;
     const int strip0 = split * g.per_split, strip1 = strip0 + g.per_split < g.strips ? strip0 + g.per_split : g.strips;
     const int all_rows = g.batch * H, shift = kh - g.kH / 2;
@@ -503,32 +567,10 @@ __global__ void __launch_bounds__(256, 2) conv_dw16_kernel(ConvDwArgs g) {
     }
 }
 
-// dw[co][ci][tap] = sum over the splits, in their order (four runs of them side by side, then the runs in order), rounded once
 template <typename T>
-__global__ void __launch_bounds__(256) conv_dw_finish_kernel(T* dw, const float* part, int splits, int channels, int taps) {
+__global__ void __launch_bounds__(256) conv_dw_finish_kernel(ConvFinish f) {
     __shared__ float runs[3][64];
-    const int total = channels * taps, i = (int)blockIdx.x * 64 + (threadIdx.x & 63), run = threadIdx.x >> 6;
-    const int per = (splits + 3) / 4, s0 = run * per, s1 = s0 + per < splits ? s0 + per : splits;
-    float sum = 0.f;
-    if (i < total) {
-        int s = s0;
-        for (; s + 8 <= s1; s += 8) {
-            float v[8];
-#pragma unroll
-            for (int u = 0; u < 8; u++) v[u] = part[(size_t)(s + u) * total + i];
-#pragma unroll
-            for (int u = 0; u < 8; u++) sum += v[u];
-        }
-        for (; s < s1; s++) sum += part[(size_t)s * total + i];
-    }
-    if (run > 0) runs[run - 1][threadIdx.x & 63] = sum;
-    __syncthreads();
-    if (run == 0 && i < total) {
-#pragma unroll
-        for (int r = 0; r < 3; r++) sum += runs[r][threadIdx.x];
-        const int tap = i / channels, c = i - tap * channels;          // c = co * C_in + ci
-        dw[(size_t)c * taps + tap] = narrow<T>(sum);
-    }
+    conv_dw_finish<T, 1>(f, blockIdx.x, runs);
 }
 
 // ---- host side ----
@@ -609,7 +651,7 @@ static int launch_taps_t(const ConvTapsArgs& g) {
     const size_t smem = taps_smem(NPOS, g.cells, g.kH, KW);
     auto kern = conv_taps16_kernel<T, KW, ROWS, VW, NPOS>;
     if (smem > 64 * 1024 && !check_hip(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem), "hipFuncSetAttribute")) return -1;
-    hipLaunchKernelGGL(kern, dim3(shared_grid(g.groups, (g.C_to + CD_CO - 1) / CD_CO)), dim3(256), smem, current_stream(), g);
+    hipLaunchKernelGGL(kern, dim3(shared_grid(g.groups, (g.C_to + CD_CO - 1) / CD_CO) + (unsigned)g.finish.blocks), dim3(256), smem, current_stream(), g);
     return check_launch("conv_taps16_kernel") ? 0 : -1;
 }
 
@@ -619,30 +661,42 @@ static int launch_taps_k(const ConvTapsArgs& g, int npos, int vw) {
     return vw >= 4 ? launch_taps_t<T, KW, ROWS, 4, 64>(g) : launch_taps_t<T, KW, ROWS, 0, 64>(g);
 }
 
+static int launch_taps(const ConvTapsArgs& g, int npos, int kW, int dtype) {
+    const bool bf = dtype == RP_DTYPE_BFLOAT16;
+    const int vw = group_width(g.W, g.in, g.out);
+    if (kW == 3 && g.kH == 3) return bf ? launch_taps_k<bf16_t, 3, 3>(g, npos, vw) : launch_taps_k<f16_t, 3, 3>(g, npos, vw);
+    if (kW == 3) return bf ? launch_taps_k<bf16_t, 3, 1>(g, npos, vw) : launch_taps_k<f16_t, 3, 1>(g, npos, vw);
+    return bf ? launch_taps_k<bf16_t, 5, 1>(g, npos, vw) : launch_taps_k<f16_t, 5, 1>(g, npos, vw);
+}
+
+static ConvTapsArgs taps_args(void* out, const void* in, const void* bias, int batch, int C_from, int C_to, int H, int W, int kH, int kW, int npos) {
+    const int positions = positions_per_group(npos, batch, H, W, kH, kW), groups = (int)(((long long)batch * H * W + positions - 1) / positions);
+    return ConvTapsArgs{out, in, nullptr, bias, batch, C_from, C_to, H, W, kH, positions, (int)strip_cells(positions, batch, H, W, kH, kW), groups, 0, ConvFinish{}};
+}
+
+static bool ranges_apart(const void* a, size_t a_bytes, const void* b, size_t b_bytes) {
+    return (const char*)a + a_bytes <= (const char*)b || (const char*)b + b_bytes <= (const char*)a;
+}
+
 // out[batch, C_to, H, W] from in[batch, C_from, H, W] and w [C_out, C_in, kH, kW] (for_input_grad: C_from = C_out); bias per output channel or null
 int launch_conv_taps16(void* out, const void* in, const void* w, const void* bias, int batch, int C_from, int C_to, int H, int W, int kH, int kW, bool for_input_grad, int dtype) {
-    const int taps = kH * kW, total = C_from * C_to * taps;
-    const int npos = taps_npos(batch, C_to, H, W), positions = positions_per_group(npos, batch, H, W, kH, kW);
-    const int groups = (int)(((long long)batch * H * W + positions - 1) / positions), vw = group_width(W, in, out);
+    const int taps = kH * kW, total = C_from * C_to * taps, npos = taps_npos(batch, C_to, H, W);
+    ConvTapsArgs g = taps_args(out, in, bias, batch, C_from, C_to, H, W, kH, kW, npos);
     // Workgroups that sort the weights themselves save a launch and take longer each (us, sorted by a launch and in the workgroups: 49
     // of them 11.4 / 8.9, 196 24 / 21, 784 26 / 30): as long as there is not more than one per CU.
     // An output over the weights: a workgroup reads them for every 32 channels while others already store, so they are copied first.
-    const char *out0 = (const char*)out, *w0 = (const char*)w;
-    const bool apart = out0 + (size_t)batch * C_to * H * W * 2 <= w0 || w0 + (size_t)total * 2 <= out0;
-    const bool by_channel = kH == 3 && kW == 3 && !for_input_grad && apart && ((uintptr_t)w & 15) == 0 && (long long)groups * ((C_to + CD_CO - 1) / CD_CO) <= cus_of_device();
+    const bool apart = ranges_apart(out, (size_t)batch * C_to * H * W * 2, w, (size_t)total * 2);
+    g.by_channel = kH == 3 && kW == 3 && !for_input_grad && apart && ((uintptr_t)w & 15) == 0 && (long long)g.groups * ((C_to + CD_CO - 1) / CD_CO) <= cus_of_device();
     void* wt = nullptr;
-    if (!by_channel && rp_hip_malloc(&wt, (size_t)total * 2) != 0) return -1;
-    if (!by_channel) hipLaunchKernelGGL(conv_weights_by_tap_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, current_stream(), (uint16_t*)wt, (const uint16_t*)w, C_from, C_to, taps, total,
-                       for_input_grad ? 1 : 0);
-    ConvTapsArgs g{out, in, by_channel ? w : wt, bias, batch, C_from, C_to, H, W, kH, positions, (int)strip_cells(positions, batch, H, W, kH, kW),
-                   groups, by_channel ? 1 : 0};
-    int rc = check_launch("conv_weights_by_tap_kernel") ? 0 : -1;
-    if (rc == 0) {
-        const bool bf = dtype == RP_DTYPE_BFLOAT16;
-        if (kW == 3 && kH == 3) rc = bf ? launch_taps_k<bf16_t, 3, 3>(g, npos, vw) : launch_taps_k<f16_t, 3, 3>(g, npos, vw);
-        else if (kW == 3) rc = bf ? launch_taps_k<bf16_t, 3, 1>(g, npos, vw) : launch_taps_k<f16_t, 3, 1>(g, npos, vw);
-        else rc = bf ? launch_taps_k<bf16_t, 5, 1>(g, npos, vw) : launch_taps_k<f16_t, 5, 1>(g, npos, vw);
+    int rc = 0;
+    if (!g.by_channel) {
+        if (rp_hip_malloc(&wt, (size_t)total * 2) != 0) return -1;
+        const ConvSort sort{(uint16_t*)wt, (const uint16_t*)w, C_from, C_to, taps, total, for_input_grad ? 1 : 0, 0};
+        hipLaunchKernelGGL(conv_weights_by_tap_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, current_stream(), sort);
+        rc = check_launch("conv_weights_by_tap_kernel") ? 0 : -1;
     }
+    g.wt = g.by_channel ? w : wt;
+    if (rc == 0) rc = launch_taps(g, npos, kW, dtype);
     report_kernel(npos == 256 ? "conv_taps16_256x64" : "conv_taps16_64x64");
     if (wt) rp_hip_free(wt);                     // back to the pool while the kernels are still queued: safe for later work on this stream
     return rc;
@@ -669,23 +723,23 @@ static int launch_dw_t(const ConvDwArgs& g) {
     const size_t smem = dw_smem(g.W, KW);
     auto kern = conv_dw16_kernel<T, KW, VW>;
     if (smem > 64 * 1024 && !check_hip(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem), "hipFuncSetAttribute")) return -1;
-    hipLaunchKernelGGL(kern, dim3(shared_grid(g.splits * g.c_in_tiles * ((g.C_out + 63) / 64), g.kH)), dim3(256), smem, current_stream(), g);
+    hipLaunchKernelGGL(kern, dim3(shared_grid(g.splits * g.c_in_tiles * ((g.C_out + 63) / 64), g.kH) + (unsigned)g.sort.blocks), dim3(256), smem, current_stream(), g);
     return check_launch("conv_dw16_kernel") ? 0 : -1;
 }
 
-template <typename T>
-static int launch_dw(const ConvDwArgs& g, int kW, int vw, void* dw) {
-    int rc;
-    if (kW == 3) rc = vw == 8 ? launch_dw_t<T, 3, 8>(g) : vw == 4 ? launch_dw_t<T, 3, 4>(g) : launch_dw_t<T, 3, 0>(g);
-    else rc = vw >= 4 ? launch_dw_t<T, 5, 4>(g) : launch_dw_t<T, 5, 0>(g);           // (its accumulators leave no room for groups of eight)
-    if (rc != 0) return rc;
-    const int taps = g.kH * kW, channels = g.C_out * g.C_in;
-    hipLaunchKernelGGL(conv_dw_finish_kernel<T>, dim3((unsigned)(((long long)channels * taps + 63) / 64)), dim3(256), 0, current_stream(), (T*)dw, (const float*)g.part, g.splits, channels, taps);
-    return check_launch("conv_dw_finish_kernel") ? 0 : -1;
+static int launch_dw(const ConvDwArgs& g, int kW, int dtype) {
+    const bool bf = dtype == RP_DTYPE_BFLOAT16;
+    const int vw = group_width(g.W, g.dy, g.x);
+    if (kW == 3) {
+        if (vw == 8) return bf ? launch_dw_t<bf16_t, 3, 8>(g) : launch_dw_t<f16_t, 3, 8>(g);
+        if (vw == 4) return bf ? launch_dw_t<bf16_t, 3, 4>(g) : launch_dw_t<f16_t, 3, 4>(g);
+        return bf ? launch_dw_t<bf16_t, 3, 0>(g) : launch_dw_t<f16_t, 3, 0>(g);
+    }
+    if (vw >= 4) return bf ? launch_dw_t<bf16_t, 5, 4>(g) : launch_dw_t<f16_t, 5, 4>(g);           // (its accumulators leave no room for groups of eight)
+    return bf ? launch_dw_t<bf16_t, 5, 0>(g) : launch_dw_t<f16_t, 5, 0>(g);
 }
 
-// dw [C_out, C_in, kH, kW] from dy [batch, C_out, H, W] and x [batch, C_in, H, W]
-int launch_conv_dw16(void* dw, const void* dy, const void* x, int batch, int C_in, int C_out, int H, int W, int kH, int kW, int dtype) {
+static ConvDwArgs dw_args(const void* dy, const void* x, int batch, int C_in, int C_out, int H, int W, int kH) {
     const int rows = dw_rows(W);
     const int strips = (int)(((long long)batch * H + rows - 1) / rows);
     const int tiles = ((C_in + 63) / 64) * ((C_out + 63) / 64);
@@ -693,14 +747,58 @@ int launch_conv_dw16(void* dw, const void* dy, const void* x, int batch, int C_i
     splits = splits < 1 ? 1 : (splits > strips ? strips : splits);
     const int per_split = (strips + splits - 1) / splits;
     splits = (strips + per_split - 1) / per_split;
+    return ConvDwArgs{nullptr, dy, x, batch, C_in, C_out, H, W, kH, rows, strips, per_split, (C_in + 63) / 64, splits, ConvSort{}};
+}
+static size_t dw_part_bytes(const ConvDwArgs& g, int kW) { return (size_t)g.splits * g.C_in * g.C_out * g.kH * kW * sizeof(float); }
+
+// dw [C_out, C_in, kH, kW] from dy [batch, C_out, H, W] and x [batch, C_in, H, W]
+int launch_conv_dw16(void* dw, const void* dy, const void* x, int batch, int C_in, int C_out, int H, int W, int kH, int kW, int dtype) {
+    ConvDwArgs g = dw_args(dy, x, batch, C_in, C_out, H, W, kH);
     void* part = nullptr;
-    if (rp_hip_malloc(&part, (size_t)splits * C_in * C_out * kH * kW * sizeof(float)) != 0) return -1;
-    ConvDwArgs g{(float*)part, dy, x, batch, C_in, C_out, H, W, kH, rows, strips, per_split, (C_in + 63) / 64, splits};
-    const int vw = group_width(W, dy, x);
-    const int rc = dtype == RP_DTYPE_BFLOAT16 ? launch_dw<bf16_t>(g, kW, vw, dw) : launch_dw<f16_t>(g, kW, vw, dw);
+    if (rp_hip_malloc(&part, dw_part_bytes(g, kW)) != 0) return -1;
+    g.part = (float*)part;
+    int rc = launch_dw(g, kW, dtype);
+    if (rc == 0) {
+        const ConvFinish f{dw, g.part, g.splits, C_out * C_in, kH * kW, 0, 0};
+        const dim3 grid((unsigned)(((long long)f.channels * f.taps + 63) / 64));
+        if (dtype == RP_DTYPE_BFLOAT16) hipLaunchKernelGGL(conv_dw_finish_kernel<bf16_t>, grid, dim3(256), 0, current_stream(), f);
+        else hipLaunchKernelGGL(conv_dw_finish_kernel<f16_t>, grid, dim3(256), 0, current_stream(), f);
+        rc = check_launch("conv_dw_finish_kernel") ? 0 : -1;
+    }
     report_kernel("conv_dw16");
     rp_hip_free(part);
     return rc;
+}
+
+// Both gradients, each as above (the same bits), in two launches of four: the weights of dX are sorted beside the partial sums of dW, which are
+// added up beside dX.  Behind one another a launch costs 4.7 us whatever it does, and both of these small ones are done before the large ones' last
+// workgroups are.  us, forward, both gradients and bias gradient, four launches and two: bf16 64 x 64 x 56 x 56 -> 64 3 x 3 101.5 / 95.3, 5 x 64 x 28 x 28 -> 256
+// 59.4 / 49.9, 11 x 64 x 28 x 28 -> 64 5 x 5 62.3 / 50.3, f16 14 x 64 x 14 x 14 -> 64 3 x 3 42.8 / 34.6; 53 x 128 x 38 x 38 -> 128 194.6 / 195.8.
+// Sums are added four to a thread here, not one: a workgroup holds the LDS of the one beside it, which leaves few of them on a CU.
+// False: not taken (a gradient over what the other reads, or no memory for both at once).
+bool launch_conv_gradients16(void* dx, void* dw, const void* dy, const void* x, const void* w, int batch, int C_in, int C_out, int H, int W, int kH, int kW, int dtype, int& rc) {
+    const int taps = kH * kW, total = C_in * C_out * taps;
+    const size_t w_bytes = (size_t)total * 2, hw = (size_t)H * W * 2;
+    // dW is stored while dX is read from dY and stored; x is read before dX is stored
+    if (!ranges_apart(dw, w_bytes, dy, (size_t)batch * C_out * hw) || !ranges_apart(dw, w_bytes, dx, (size_t)batch * C_in * hw) ||
+        !ranges_apart(dx, (size_t)batch * C_in * hw, x, (size_t)batch * C_in * hw)) return false;
+    ConvDwArgs gw = dw_args(dy, x, batch, C_in, C_out, H, W, kH);
+    const int npos = taps_npos(batch, C_in, H, W);
+    ConvTapsArgs gx = taps_args(dx, dy, nullptr, batch, C_out, C_in, H, W, kH, kW, npos);
+    void *wt = nullptr, *part = nullptr;
+    if (rp_hip_malloc(&part, dw_part_bytes(gw, kW)) != 0) return false;
+    if (rp_hip_malloc(&wt, w_bytes) != 0) { rp_hip_free(part); return false; }
+    gw.part = (float*)part;
+    gw.sort = ConvSort{(uint16_t*)wt, (const uint16_t*)w, C_out, C_in, taps, total, 1, ((total + CD_SORT - 1) / CD_SORT + 7) / 8 * 8};
+    gx.wt = wt;
+    const int units = (total + 255) / 256, most = 4 * cus_of_device();          // (C_out is whole 32s: total is whole fours)
+    gx.finish = ConvFinish{dw, gw.part, gw.splits, C_out * C_in, taps, (int)shared_grid(gx.groups, (C_in + CD_CO - 1) / CD_CO), units < most ? units : most};
+    rc = launch_dw(gw, kW, dtype);
+    if (rc == 0) rc = launch_taps(gx, npos, kW, dtype);
+    report_kernel("conv_dw16");
+    rp_hip_free(part);
+    rp_hip_free(wt);
+    return true;
 }
 
 }  // namespace rp

@@ -240,6 +240,7 @@ bool conv_taps16_takes(int batch, int C_from, int C_to, int H, int W, int kH, in
 int launch_conv_taps16(void* out, const void* in, const void* w, const void* bias, int batch, int C_from, int C_to, int H, int W, int kH, int kW, bool for_input_grad, int dtype);
 bool conv_dw16_takes(int batch, int C_in, int C_out, int H, int W, int kH, int kW, int dtype);
 int launch_conv_dw16(void* dw, const void* dy, const void* x, int batch, int C_in, int C_out, int H, int W, int kH, int kW, int dtype);
+bool launch_conv_gradients16(void* dx, void* dw, const void* dy, const void* x, const void* w, int batch, int C_in, int C_out, int H, int W, int kH, int kW, int dtype, int& rc);
 int launch_linear_backward_tiny(const GemmArgs& gx, const GemmArgs& gw, void* db, const void* dy, int rows, int cols, int accumulate_db);
 // adds k-split partials [g.batch][nsplit][part_rows][n] (fp32, rows beyond g.m unused) in split order and runs the epilogue into C
 int launch_splitk_combine(const GemmArgs& g, const float* partials, int nsplit, int part_rows, int dtype);

@@ -280,6 +280,30 @@ def test_weight_gradient_does_not_depend_on_the_input_gradient(dt, case):
 
 
 @pytest.mark.parametrize("dt", [F16, BF16], ids=lambda d: NAMES[d])
+@pytest.mark.parametrize("case", [(2, 5, 9, 12, 64, 3, 3), (3, 40, 14, 14, 128, 3, 3), (1, 64, 8, 24, 64, 5, 5), (40, 64, 28, 28, 192, 3, 3), (3, 7, 3, 6, 64, 1, 3)],
+                         ids=lambda c: "x".join(map(str, c)))
+def test_both_gradients_in_one_call_are_those_of_two_calls(dt, case):
+    """Bit for bit, apart and with dW over W, dW over x or dX over W (the last of them read before the gradient is stored)."""
+    N, Ci, H, W, Co, kH, kW = case
+    L = capi.lib()
+    rng = np.random.default_rng(N + Ci)
+    x, w, g = rand_storage(rng, (N, Ci, H, W), dt), oracle.to_storage(rng.standard_normal((Co, Ci, kH, kW)) * 0.2, dt), rand_storage(rng, (N, Co, H, W), dt)
+    dx_, dw_, dg_ = Dev(x, dt), Dev(w, dt), Dev(g, dt)
+    gx, gw = Dev.empty((N, Ci, H, W), dt), Dev.empty((Co, Ci, kH, kW), dt)
+    capi.check(L.rp_hip_conv2d_same_backward(gx.ptr, None, dg_.ptr, None, dw_.ptr, N, Ci, H, W, Co, kH, kW, dt), "input gradient")
+    capi.check(L.rp_hip_conv2d_same_backward(None, gw.ptr, dg_.ptr, dx_.ptr, None, N, Ci, H, W, Co, kH, kW, dt), "weight gradient")
+    want = gx.numpy(), gw.numpy()
+    size = max(x.size, w.size)
+    for over_x, over_w in ((None, None), (None, "w"), (None, "x"), ("w", None)):
+        bx, bw = Dev.empty((size,), dt), Dev.empty((size,), dt)
+        pad = lambda a: Dev(np.concatenate([a.ravel(), np.zeros(size - a.size, a.dtype)]), dt)          # noqa: E731
+        bufs = {"x": pad(x), "w": pad(w)}
+        ox, ow = bufs.get(over_x, bx), bufs.get(over_w, bw)
+        capi.check(L.rp_hip_conv2d_same_backward(ox.ptr, ow.ptr, dg_.ptr, bufs["x"].ptr, bufs["w"].ptr, N, Ci, H, W, Co, kH, kW, dt), "both")
+        assert np.array_equal(ox.numpy()[:x.size], want[0].ravel()) and np.array_equal(ow.numpy()[:w.size], want[1].ravel()), (over_x, over_w)
+
+
+@pytest.mark.parametrize("dt", [F16, BF16], ids=lambda d: NAMES[d])
 def test_same_convolution_over_its_own_input(dt):
     """An output that overlaps the image it is computed from: the image is copied first, as for any other convolution."""
     N, C, H, W = 2, 64, 9, 12
