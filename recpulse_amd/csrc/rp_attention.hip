@@ -138,7 +138,9 @@ __global__ void __launch_bounds__(256, D > 64 || SPLIT ? 2 : 3) attention_fwd16_
     const uint16_t* V = (const uint16_t*)g.V + (long long)z * g.v_bs;
     // exp(scale * s - max) = exp2(s * sc - max * sc) with sc = |scale| log2 e: one fused multiply-add per score; a
     // negative scale flips the sign of Q, so that the running maximum can be kept on the raw scores (of the scores, a select each even
-    // where the scale is not negative: forward [10, 1565, 1565, 64] in fp16 18.3 us, 17.8 this way)
+    // where the scale is not negative: forward [10, 1565, 1565, 64] in fp16 18.3 us, 17.8 this way).  d = 128 split is out of registers: five
+    // spilled with Q flipped, one query of 32 heads against 4096 keys 48 us, and 36 with the scores flipped.
+    constexpr bool FLIP_Q = !(SPLIT && D > 64);
     const float sc = fabsf(g.scale) * 1.44269504088896341f;
     const bool flip = g.scale < 0.f;
 
@@ -149,7 +151,7 @@ __global__ void __launch_bounds__(256, D > 64 || SPLIT ? 2 : 3) attention_fwd16_
     s16x8_t qf[KS];
 #pragma unroll
     for (int ks = 0; ks < KS; ks++)
-        qf[ks] = attn_signed(__builtin_amdgcn_raw_buffer_load_b128(q_rsrc, (int)(((long long)c * g.q_rs + 16 * ks + 8 * h) * 2), 0, 0), flip);
+        qf[ks] = attn_signed(__builtin_amdgcn_raw_buffer_load_b128(q_rsrc, (int)(((long long)c * g.q_rs + 16 * ks + 8 * h) * 2), 0, 0), FLIP_Q && flip);
 
     // K and V blocks [32 keys][D] go to LDS, 16 bytes per thread and piece, in whole rows (every cache line is
     // requested once per workgroup; fragment loads straight from global memory would touch 32 lines per instruction
@@ -253,6 +255,12 @@ __global__ void __launch_bounds__(256, D > 64 || SPLIT ? 2 : 3) attention_fwd16_
         if constexpr (SPLIT) attn_wave_order();
         else read_vs(0);
 
+        if (!FLIP_Q && flip) {
+#pragma unroll
+            for (int b = 0; b < NB; b++)
+#pragma unroll
+                for (int v = 0; v < 16; v++) st[b][v] = -st[b][v];
+        }
         const bool ragged = kb + KEYS > g.sk;               // the last block of a ragged sk
         if (ragged) {
 #pragma unroll

@@ -292,12 +292,16 @@ static bool wavek16_takes(const GemmArgs& g, const Plan& p, int dtype, bool& rag
 // kernel, and fp32 ones that 16 x 16 tiles of four waves or the row-streaming kernel took.  Stays where it was: fp32 with k up to 512 on 16 x 16 tiles (60 x 443 x 65 3.55 / 3.67 us; 256 x 784 x 256
 // 6.95 / 5.0-6.0); a few rows with k above 1024 (8 x 8192 x 8192 55 / 51, but that kernel's sums are of shorter chains); a k too short for the number of tiles (fp32 2384 x 32 x 368
 // 5.2 / 6.5, 944 x 144 x 1648 14.0 / 16.2; fp64 832 x 48 x 2128 14.6 / 22.7); fp32 outputs of a few tiles whose long k the split deals to more CUs
-// (16 x 5744 x 48 11.5 / 14.4) and sums in shorter chains.  (The k split read all of its operands before it wrote C: outputs over an operand stay there.)
+// (16 x 5744 x 48 11.5 / 14.4) and sums in shorter chains; batches of more than one 64 x 64 tile a CU that fill those as well as 32 x 32 ones (fp32
+// 128 x 512 x 128 100 of them 26.8 / 33.2, 60 21.2 / 14.9; 20 x 600 x 20 1000 of them 50.8 / 26.1; fp64 40 x 100 x 40 3000 of them 84 / 124) or, in fp32, of a k up
+// to 64 (128 x 64 x 128, 50 of them 6.2 / 7.6).  (The k split read all of its operands before it wrote C: outputs over an operand stay there.)
 static bool wavekw_takes(const GemmArgs& g, const Plan& p, int dtype) {
     const bool f32 = dtype == RP_DTYPE_FLOAT32;
     if (!(f32 || dtype == RP_DTYPE_FLOAT64) || g.seg_k || g.seg_n || g.bias_by_row || g.c_fold_from || path_disabled("wavekw")) return false;
     const long long tiles64 = (long long)((g.m + 63) / 64) * ((g.n + 63) / 64) * g.batch, tiles16 = (long long)((g.m + 15) / 16) * ((g.n + 15) / 16) * g.batch;
     if (p.fam == FAM_MFMAW && p.bm == 64) {
+        const long long tiles32 = (long long)((g.m + 31) / 32) * ((g.n + 31) / 32) * g.batch;
+        if (g.batch > 1 && ((tiles64 > cu_tiles() && tiles32 * 2 >= tiles64 * 7) || (f32 && g.k <= 64 && tiles64 > cu_tiles() / 2))) return false;
         if (f32 ? g.k <= 32 || (tiles64 > cu_tiles() && g.k < 256) : g.k <= 48 && tiles64 > cu_tiles() / 2) return false;
         const bool splits = f32 && (g.n % 4 == 0 || p.ragged), both_kc = g.a_cs == 1 && g.b_rs == 1 && g.b_cs != 1;
         if (splits && g.k > 2048 && (tiles64 < cu_tiles() / 32 || (!both_kc && tiles16 < cu_tiles() / 4))) return false;
@@ -380,7 +384,7 @@ static int run_gemm(GemmArgs g, int dtype) {
 // those of 64 stay what they were, [10, 64, 56, 56, 64, 5] 121 / 139.  Up to four a CU where C_out is more than 64
 // and the positions many ([18, 128, 28, 28, 192, 3] 152 / 107, but [31, 256, 26, 26, 64, 3] 109 / 143, [13, 192, 7, 7, 256, 3] 45.5 / 56.5).
 static WkwTile segmented_wavek_tile(const GemmArgs& g) {
-    if (path_disabled("wavekw") || g.a_cs != 1 || g.n < 64 || g.accumulate || g.batch > 65535 || g.b_extent * 4 >= (1ll << 31) || (63 * g.a_rs + g.k) * 4 >= (1ll << 31)) return WKW_NONE;
+    if (path_disabled("wavekw") || g.a_cs != 1 || g.n < 64 || g.accumulate || (long long)((g.m + 15) / 16) * ((g.n + 15) / 16) * g.batch >= 1ll << 24 || g.b_extent * 4 >= (1ll << 31) || (63 * g.a_rs + g.k) * 4 >= (1ll << 31)) return WKW_NONE;
     const long long cus = cu_tiles(), tiles64 = (long long)((g.m + 63) / 64) * ((g.n + 63) / 64) * g.batch;
     if (g.seg_k > 0) {
         if (g.seg_k % 32) return WKW_NONE;

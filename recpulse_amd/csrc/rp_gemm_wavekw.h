@@ -193,18 +193,20 @@ struct WkwOperand<E, false, T, SEG> {
 template <typename E, bool KC, int T, bool SEG>
 using wkw_operand = std::conditional_t<KC && (T > 1), WkwOperandRows<E, T, SEG>, WkwOperand<E, KC, T == 1 || !KC ? T : 1, SEG>>;
 
-// The 16 TM x 16 TN tile `block` of matrix z, by NW waves.  k goes in pieces, dealt to the waves in turn: a wave multiplies one piece out of
+// A 16 TM x 16 TN tile, number `block` of the schedule of `batch` matrices, by NW waves.  k goes in pieces, dealt to the waves in turn: a wave multiplies one piece out of
 // registers while the next is on its way there, and the partial tiles meet in LDS, where they are added in a fixed order.
 template <typename E, bool A_KC, bool B_KC, int TM, int TN, int NW, bool SEG = false>
-__device__ __forceinline__ void gemm_wavekw_block(const GemmArgs& g, int tiles_m, int tiles_n, int block, int z, unsigned char* lds) {
+__device__ __forceinline__ void gemm_wavekw_block(const GemmArgs& g, int tiles_m, int tiles_n, int block, int batch, unsigned char* lds) {
     using cfg = wkw_cfg<E>;
     using OpA = wkw_operand<E, A_KC, TM, false>;
     using OpB = wkw_operand<E, B_KC, TN, SEG>;
     constexpr int PK = wkw_piece<E>(), KV = cfg::KV;
     constexpr bool STAGED = wkw_staged(A_KC, TM) || wkw_staged(B_KC, TN);
-    // block b runs on XCD b % 8: a run of tiles along the shorter side of the output for each XCD, whose L2 then serves what they share
-    const int total = tiles_m * tiles_n, per = (total + 7) / 8, idx = block % 8 * per + block / 8;
-    if (block / 8 >= per || idx >= total) return;
+    // block b runs on XCD b % 8: a run of matrices, and of tiles along the shorter side of an output, for each XCD, whose L2 then serves what they share.
+    // (With a run of every matrix's tiles for each XCD, 250 matrices of one tile each were all on the first: 64 x 512 x 64 114 us, 25.)
+    const int tiles = tiles_m * tiles_n, total = tiles * batch, per = (total + 7) / 8, at = block % 8 * per + block / 8;
+    if (block / 8 >= per || at >= total) return;
+    const int z = at / tiles, idx = at - z * tiles;
     const bool tall = tiles_m > tiles_n;
     const int m0 = (tall ? idx / tiles_n : idx % tiles_m) * 16 * TM, n0 = (tall ? idx % tiles_n : idx / tiles_m) * 16 * TN;
     // where a row of an operand is a row of k the last tile starts early, so that it ends with the operand; only its own part is stored

@@ -22,7 +22,7 @@ constexpr int wkw_waves(int tiles) { return tiles <= 4 ? 4 : 2; }
 template <typename E, bool A_KC, bool B_KC, int TM, int TN, int NW, bool SEG>
 __global__ void __launch_bounds__(64 * NW, wkw_waves(TM * TN)) gemm_wavekw_kernel(GemmArgs g, int tiles_m, int tiles_n) {
     extern __shared__ __attribute__((aligned(16))) unsigned char wkw_lds[];
-    gemm_wavekw_block<E, A_KC, B_KC, TM, TN, NW, SEG>(g, tiles_m, tiles_n, blockIdx.x, blockIdx.y, wkw_lds);
+    gemm_wavekw_block<E, A_KC, B_KC, TM, TN, NW, SEG>(g, tiles_m, tiles_n, blockIdx.x, g.batch, wkw_lds);
 }
 
 template <typename E, bool A_KC, bool B_KC, int TM, int TN, int NW, bool SEG = false>
@@ -31,7 +31,7 @@ static int launch_wavekw_t(const GemmArgs& g) {
     const int tiles_m = (g.m + 16 * TM - 1) / (16 * TM), tiles_n = (g.n + 16 * TN - 1) / (16 * TN);
     auto kern = gemm_wavekw_kernel<E, A_KC, B_KC, TM, TN, NW, SEG>;
     if (smem > 64 * 1024 && !check_hip(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem), "hipFuncSetAttribute")) return -1;
-    hipLaunchKernelGGL(kern, dim3((unsigned)((tiles_m * tiles_n + 7) / 8 * 8), g.batch), dim3(64 * NW), smem, current_stream(), g, tiles_m, tiles_n);
+    hipLaunchKernelGGL(kern, dim3((unsigned)(((long long)tiles_m * tiles_n * g.batch + 7) / 8 * 8)), dim3(64 * NW), smem, current_stream(), g, tiles_m, tiles_n);
     return check_launch("gemm_wavekw_kernel") ? 0 : -1;
 }
 
@@ -57,7 +57,7 @@ WkwTile wavekw_tile(const GemmArgs& g, int dtype) {
     if (span(a_kc, g.a_rs, g.a_cs) >= limit || span(b_kc, g.b_cs, g.b_rs) >= limit) return WKW_NONE;
     const auto tiles = [&](int tm, int tn) { return (long long)((g.m + 16 * tm - 1) / (16 * tm)) * ((g.n + 16 * tn - 1) / (16 * tn)) * g.batch; };
     const auto fits = [&](int tm, int tn) { return (a_kc || g.m >= 16 * tm) && (b_kc || g.n >= 16 * tn); };       // see ms, ns in gemm_wavekw_block
-    if (!fits(1, 1)) return WKW_NONE;
+    if (!fits(1, 1) || tiles(1, 1) >= 1ll << 24) return WKW_NONE;
     if (dtype == RP_DTYPE_FLOAT64) return fits(2, 2) && tiles(2, 2) >= cus / 2 ? WKW_32X32 : WKW_16X16;
     if (fits(4, 4) && g.k >= 512 && tiles(4, 4) >= cus * 3 / 4 && tiles(4, 4) <= cus) return WKW_64X64;
     if (a_kc && !b_kc && fits(1, 4) && g.k >= 512 && tiles(1, 4) >= cus / 2 && tiles(1, 4) <= cus) return WKW_16X64;
@@ -110,7 +110,7 @@ __device__ __forceinline__ void wkw_part(const GemmArgs& g, int tiles_m, int til
         if (2 * block >= tiles) return;
         tiny_tile_any(g, vec_flags & 1, vec_flags & 2, tile < tiles ? tile : tiles - 1, (float (*)[256])lds + 3 * half, threadIdx.x & 255, tile < tiles);
     } else {
-        gemm_wavekw_block<E, KC, KC, WkwShape<K>::TM, WkwShape<K>::TN, 8>(g, tiles_m, tiles_n, block, 0, lds);
+        gemm_wavekw_block<E, KC, KC, WkwShape<K>::TM, WkwShape<K>::TN, 8>(g, tiles_m, tiles_n, block, 1, lds);
     }
 }
 

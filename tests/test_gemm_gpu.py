@@ -926,7 +926,8 @@ def test_small_fp32_outputs_of_rows_at_any_element(m, k, n, layout):
 WAVEKW_SHAPES = [(F32, 1, 16, 513, 16, "mfma32_wavek"), (F32, 1, 5, 700, 333, "mfma32_wavek"), (F32, 1, 35, 2047, 18, "mfma32_wavek"), (F32, 1, 70, 545, 300, "mfma32_wavek"),
                  (F32, 1, 497, 577, 401, "mfma32_wavek"), (F32, 1, 63, 1024, 2113, "mfma32_wavek"), (F32, 1, 3, 1001, 1100, "mfma32_wavek"), (F32, 1, 900, 519, 901, "mfma32_64x64"),
                  (F32, 3, 67, 1027, 35, "mfma32_wavek"), (F32, 9, 131, 61, 260, "mfma32_64x64"), (F32, 1, 33, 3000, 1100, "mfma32_64x64"), (F64, 1, 16, 1, 16, "mfma64_wavek"),
-                 (F64, 1, 17, 16, 19, "mfma64_wavek"), (F64, 1, 60, 131, 50, "mfma64_wavek"), (F64, 1, 20, 2001, 17, "mfma64_wavek"), (F64, 1, 390, 257, 401, "mfma64_64x64"), (F64, 5, 33, 130, 31, "mfma64_wavek")]
+                 (F64, 1, 17, 16, 19, "mfma64_wavek"), (F64, 1, 60, 131, 50, "mfma64_wavek"), (F64, 1, 20, 2001, 17, "mfma64_wavek"), (F64, 1, 390, 257, 401, "mfma64_64x64"), (F64, 5, 33, 130, 31, "mfma64_wavek"),
+                 (F32, 253, 64, 512, 64, "mfma32_64x64"), (F32, 301, 20, 600, 24, "mfma32_64x64"), (F64, 130, 64, 70, 130, "mfma64_64x64")]
 
 
 @pytest.mark.parametrize("layout", LAYOUTS)
