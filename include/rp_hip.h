@@ -58,6 +58,7 @@ int rp_hip_empty_cache(void);
 int rp_hip_memory_stats(long long* malloc_requests, long long* device_mallocs, long long* live_blocks, long long* cached_blocks);
 int rp_hip_memset(void* ptr, int value, size_t bytes);
 int rp_hip_memcpy_h2d(void* dst_device, const void* src_host, size_t bytes);
+/* Returns when dst_host holds the bytes; up to 256 KB go through pinned host memory that a kernel writes. */
 int rp_hip_memcpy_d2h(void* dst_host, const void* src_device, size_t bytes);
 int rp_hip_memcpy_d2d(void* dst_device, const void* src_device, size_t bytes);
 int rp_hip_synchronize(void);
@@ -142,7 +143,9 @@ int rp_hip_gemm_strided_batched_noalloc(void* C, const void* A, const void* B, c
 
 /* Name of the kernel family the dispatcher picks for a problem, for logs and
  * tests ("mfma16_256x256", "skinny", "generic", ...).  No device work.  "mfma16_wavek", which stands in for "mfma16_64x64" and
- * "mfma16_skinny_32x128" where C lies apart from the operands, is named by rp_hip_last_gemm_kernel alone. */
+ * "mfma16_skinny_32x128" where C lies apart from the operands, "mfma32_wavek" and "mfma64_wavek", which stand in for "tiny32_16x16", "skinny" and (float64)
+ * "generic" there, and "linear_backward_wavek" are named by rp_hip_last_gemm_kernel alone.  In the place of "mfma32_64x64", "mfma64_64x64" and
+ * any 16-bit kernel for rows of arbitrary length, waves that share k go by the name of the kernel that they stand in for. */
 const char* rp_hip_gemm_kernel_name(int batch, int m, int k, int n,
                                     long long a_rs, long long a_cs,
                                     long long b_rs, long long b_cs,
@@ -217,8 +220,8 @@ int rp_hip_convert(void* dst, int dst_dtype, const void* src, int src_dtype, siz
  * db [n] = column sums of dy (as rp_hip_reduce_rows).  dy [m, n] is dense; x [m, k], w [k, n],
  * dx and dw carry (row, column) strides in elements; any of dx, dw, db may be NULL; accumulate_* = 1 adds to what the
  * output holds.  Same values, bit for bit, as two rp_hip_gemm_strided_batched calls with the transposes as swapped
- * strides (backward_matmul_fn, ops/ops.c:6759-6814) and rp_hip_reduce_rows; for small float32 layers (the
- * one-launch 16 x 16-tile kernel's range) the three run as ONE launch, which is most of such a layer's time. */
+ * strides (backward_matmul_fn, ops/ops.c:6759-6814) and rp_hip_reduce_rows; for layers of few output tiles (float32's
+ * one-launch 16 x 16-tile kernel, and every dtype's workgroups whose waves share k) the three run as ONE launch. */
 int rp_hip_linear_backward(void* dx, void* dw, void* db, const void* dy, const void* x, const void* w, int m, int k, int n,
                            long long x_rs, long long x_cs, long long w_rs, long long w_cs,
                            long long dx_rs, long long dx_cs, long long dw_rs, long long dw_cs,
@@ -300,7 +303,7 @@ int rp_hip_conv2d_same_forward(void* y, const void* x, const void* w, const void
 int rp_hip_conv2d_same_backward_input(void* dx, const void* dy, const void* w, int batch, int C_in, int H, int W,
                                       int C_out, int kH, int kW, int dtype);
 /* Both gradients; dx or dw may be NULL (x is read only for dw, w only for dx), and a gradient's bits do not depend on whether
- * the other is asked for unless dx overlaps dy.  dx is stored before dw, which may lie over w.
+ * the other is asked for unless dx overlaps dy.  dw may lie over w.
  * dx needs rp_hip_conv2d_same_supported(C_out, ...); dw [C_out, C_in, kH, kW] needs
  * rp_hip_conv2d_same_supported(0, ...), i.e. only the geometry and the dtype: its reduction runs over the positions
  * (every (tap, channel) column of the GEMM is a shifted plane of the image).  dw of 16-bit images read in place ("conv_dw16",
