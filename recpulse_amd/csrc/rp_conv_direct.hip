@@ -89,7 +89,7 @@ struct ConvSort {
     uint16_t* wt;
     const uint16_t* w;
     int C_from, C_to, taps, total, for_input_grad;
-    int blocks;                                  // of CD_SORT values, beside other work: a whole number of eights (0: none)
+    int first, blocks;                           // of CD_SORT values, beside other work: the first of these blocks, and how many (0: none)
 };
 constexpr int CD_SORT = 2048;
 __device__ __forceinline__ uint16_t weight_by_tap(const ConvSort& s, int i) {
@@ -419,7 +419,7 @@ struct ConvDwArgs {
     int rows;                                    // image rows of a strip
     int strips, per_split;                       // strips of the whole batch (over all samples), and of one split
     int c_in_tiles, splits;
-    ConvSort sort;                               // the first blocks sort the weights of an input gradient
+    ConvSort sort;                               // the last blocks sort the weights of an input gradient
 };
 
 // A workgroup owns 64 x 64 channels of one tap row and walks the strips of its split; the sums stay in registers.  k is the
@@ -432,8 +432,8 @@ template <typename T, int KW, int VW>
 __global__ void __launch_bounds__(256, 2) conv_dw16_kernel(ConvDwArgs g) {
     extern __shared__ __attribute__((aligned(16))) uint16_t cd_smem[];
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6, half = wave & 1, parity = wave >> 1;
-    if ((int)blockIdx.x < g.sort.blocks) {
-        const int first = (int)blockIdx.x * CD_SORT + t;
+    if (g.sort.blocks > 0 && (int)blockIdx.x >= g.sort.first) {
+        const int first = ((int)blockIdx.x - g.sort.first) * CD_SORT + t;
 #pragma unroll
         for (int i = 0; i < CD_SORT / 256; i++)
             if (first + 256 * i < g.sort.total) g.sort.wt[first + 256 * i] = weight_by_tap(g.sort, first + 256 * i);
@@ -445,7 +445,7 @@ __global__ void __launch_bounds__(256, 2) conv_dw16_kernel(ConvDwArgs g) {
     uint16_t* ds = cd_smem + (size_t)cells * CW_XP;
     const int tiles = g.c_in_tiles * ((g.C_out + 63) / 64);
     int part, kh;                                // the tap rows of a part read the same rows of the images
-    if (!shared_block((int)blockIdx.x - g.sort.blocks, g.splits * tiles, g.kH, part, kh)) return;
+    if (!shared_block(blockIdx.x, g.splits * tiles, g.kH, part, kh)) return;
     const int split = part / tiles, tile = part % tiles, co0 = (tile / g.c_in_tiles) * 64, ci0 = (tile % g.c_in_tiles) * 64;
     const int strip0 = split * g.per_split, strip1 = strip0 + g.per_split < g.strips ? strip0 + g.per_split : g.strips;
     const int all_rows = g.batch * H, shift = kh - g.kH / 2;
@@ -691,7 +691,7 @@ int launch_conv_taps16(void* out, const void* in, const void* w, const void* bia
     int rc = 0;
     if (!g.by_channel) {
         if (rp_hip_malloc(&wt, (size_t)total * 2) != 0) return -1;
-        const ConvSort sort{(uint16_t*)wt, (const uint16_t*)w, C_from, C_to, taps, total, for_input_grad ? 1 : 0, 0};
+        const ConvSort sort{(uint16_t*)wt, (const uint16_t*)w, C_from, C_to, taps, total, for_input_grad ? 1 : 0, 0, 0};
         hipLaunchKernelGGL(conv_weights_by_tap_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, current_stream(), sort);
         rc = check_launch("conv_weights_by_tap_kernel") ? 0 : -1;
     }
@@ -772,8 +772,9 @@ int launch_conv_dw16(void* dw, const void* dy, const void* x, int batch, int C_i
 
 // Both gradients, each as above (the same bits), in two launches of four: the weights of dX are sorted beside the partial sums of dW, which are
 // added up beside dX.  Behind one another a launch costs 4.7 us whatever it does, and both of these small ones are done before the large ones' last
-// workgroups are.  us, forward, both gradients and bias gradient, four launches and two: bf16 64 x 64 x 56 x 56 -> 64 3 x 3 101.5 / 95.3, 5 x 64 x 28 x 28 -> 256
+// workgroups are.  us, forward, both gradients and bias gradient, four launches and two: bf16 64 x 64 x 56 x 56 -> 64 3 x 3 99.8 / 93.9, 5 x 64 x 28 x 28 -> 256
 // 59.4 / 49.9, 11 x 64 x 28 x 28 -> 64 5 x 5 62.3 / 50.3, f16 14 x 64 x 14 x 14 -> 64 3 x 3 42.8 / 34.6; 53 x 128 x 38 x 38 -> 128 194.6 / 195.8.
+// (The sorting blocks last: dW's leave some places of the chip's 512 free, and in front of them they took 1.4 us more.)
 // Sums are added four to a thread here, not one: a workgroup holds the LDS of the one beside it, which leaves few of them on a CU.
 // False: not taken (a gradient over what the other reads, or no memory for both at once).
 bool launch_conv_gradients16(void* dx, void* dw, const void* dy, const void* x, const void* w, int batch, int C_in, int C_out, int H, int W, int kH, int kW, int dtype, int& rc) {
@@ -789,7 +790,7 @@ bool launch_conv_gradients16(void* dx, void* dw, const void* dy, const void* x, 
     if (rp_hip_malloc(&part, dw_part_bytes(gw, kW)) != 0) return false;
     if (rp_hip_malloc(&wt, w_bytes) != 0) { rp_hip_free(part); return false; }
     gw.part = (float*)part;
-    gw.sort = ConvSort{(uint16_t*)wt, (const uint16_t*)w, C_out, C_in, taps, total, 1, ((total + CD_SORT - 1) / CD_SORT + 7) / 8 * 8};
+    gw.sort = ConvSort{(uint16_t*)wt, (const uint16_t*)w, C_out, C_in, taps, total, 1, (int)shared_grid(gw.splits * gw.c_in_tiles * ((C_out + 63) / 64), kH), (total + CD_SORT - 1) / CD_SORT};
     gx.wt = wt;
     const int units = (total + 255) / 256, most = 4 * cus_of_device();          // (C_out is whole 32s: total is whole fours)
     gx.finish = ConvFinish{dw, gw.part, gw.splits, C_out * C_in, taps, (int)shared_grid(gx.groups, (C_in + CD_CO - 1) / CD_CO), units < most ? units : most};
