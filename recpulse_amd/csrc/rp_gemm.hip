@@ -525,7 +525,8 @@ static Plan plan_alone(const GemmArgs& g, int dtype) {
     return make_plan(1, g.m, g.k, g.n, g.a_rs, g.a_cs, g.b_rs, g.b_cs, g.c_rs, g.c_cs, 0, 0, dtype, false, false);
 }
 
-// Neither gradient is written over anything that the other product reads (one launch after the other, dW over W was fine)
+// Neither gradient is written over anything that the other product (or the bias gradient) reads: one launch after the other, dW over W was fine.
+// (An absent gradient is at address 0, apart from everything.)
 static bool gradients_apart(const GemmArgs& gx, const GemmArgs& gw, int dtype) {
     const int esz = (int)dtype_size(dtype);
     const Span dx = span_of(gx.C, gx.m, gx.n, gx.c_rs, gx.c_cs, esz), dw = span_of(gw.C, gw.m, gw.n, gw.c_rs, gw.c_cs, esz);
@@ -533,7 +534,7 @@ static bool gradients_apart(const GemmArgs& gx, const GemmArgs& gw, int dtype) {
     return !(overlap(dx, dw) || overlap(dx, dy) || overlap(dx, x) || overlap(dw, dy) || overlap(dw, w));
 }
 
-// Nor is the bias gradient
+// Nor does the bias gradient lie over an operand or a gradient of theirs
 static bool bias_gradient_apart(const void* db, const GemmArgs& gx, const GemmArgs& gw, int dtype) {
     const int esz = (int)dtype_size(dtype);
     const Span b = span_of(db, 1, gx.k, 0, 1, esz), dx = span_of(gx.C, gx.m, gx.n, gx.c_rs, gx.c_cs, esz), dw = span_of(gw.C, gw.m, gw.n, gw.c_rs, gw.c_cs, esz);
@@ -639,15 +640,18 @@ int rp_hip_linear_backward(void* dx, void* dw, void* db, const void* dy, const v
     plain_k_strides(gw.m, gw.k, gw.n, gw.a_rs, gw.a_cs, gw.b_rs, gw.b_cs);
     if (dtype == RP_DTYPE_FLOAT32 || dtype == RP_DTYPE_FLOAT64) {
         const WkwTile tx = dx ? small_tile_alone(gx, true, dtype) : WKW_TINY, tw = dw ? small_tile_alone(gw, false, dtype) : WKW_TINY;
-        if (dtype == RP_DTYPE_FLOAT32 && (dx || dw) && tx == WKW_TINY && tw == WKW_TINY) {
+        const bool apart = gradients_apart(gx, gw, dtype);
+        if (dtype == RP_DTYPE_FLOAT32 && (dx || dw) && tx == WKW_TINY && tw == WKW_TINY && apart) {
             // small layer: one launch does all three, block for block what the separate launches would do
+            const bool rides = db && bias_gradient_apart(db, gx, gw, dtype);
             if (!dx) gx.m = 0;
             if (!dw) gw.m = 0;
-            return launch_linear_backward_tiny(gx, gw, db, dy, m, n, accumulate_db);
+            if (launch_linear_backward_tiny(gx, gw, rides ? db : nullptr, dy, m, n, accumulate_db) != 0) return -1;
+            return db && !rides ? rp_hip_reduce_rows(db, dy, m, n, accumulate_db, dtype) : 0;
         }
         // (more than two rounds of 16 x 16 tiles need the registers and the LDS that they have alone: fp32 2659 x 49 x 3731 70.3 us apart, 73.4 in one launch)
         const auto rounds16 = [&](const GemmArgs& g, WkwTile t) { return t == WKW_16X16 && (long long)((g.m + 15) / 16) * ((g.n + 15) / 16) > 2 * cu_tiles(); };
-        if (dx && dw && linear_backward_wavekw_takes(tx, tw, dtype) && (tx == tw || !(rounds16(gx, tx) || rounds16(gw, tw))) && gradients_apart(gx, gw, dtype)) {
+        if (dx && dw && linear_backward_wavekw_takes(tx, tw, dtype) && (tx == tw || !(rounds16(gx, tx) || rounds16(gw, tw))) && apart) {
             g_last_kernel = "linear_backward_wavek";
             const bool rides = db && m <= LINEAR_DB_ROWS && bias_gradient_apart(db, gx, gw, dtype);
             if (launch_linear_backward_wavekw(gx, gw, tx, tw, rides ? db : nullptr, accumulate_db, dtype) != 0) return -1;

@@ -853,6 +853,33 @@ def test_gradients_whose_waves_share_k_in_one_launch(dt, m, k, n):
     assert np.array_equal(got.numpy(), want[0].numpy()) and np.array_equal(d_w.numpy(), want[1].numpy())
 
 
+@pytest.mark.parametrize("m,k,n", [(37, 50, 21), (256, 128, 10), (200, 240, 160)])
+def test_gradients_of_small_layers_over_operands(m, k, n):
+    """Small fp32 layers, whose gradients go out in one launch: a gradient over what another product reads gives what the calls
+    one after the other give.  Small integers, so the bits do not depend on the kernels."""
+    rng = np.random.default_rng(m + k + n)
+    L = capi.lib()
+    x, w, dy = (rng.integers(-2, 3, s).astype(np.float32) for s in ((m, k), (k, n), (m, n)))
+    dx_, dw_, db_ = dy @ w.T, x.T @ dy, dy.sum(0)
+
+    def call(over):
+        d_x, d_w, d_dy = Dev(x, F32), Dev(w, F32), Dev(dy, F32)
+        out = {"dx": Dev.empty((m, k), F32), "dw": Dev.empty((k, n), F32), "db": Dev.empty((n,), F32)}
+        place = dict(out)
+        for name, operand in over.items():
+            place[name] = {"x": d_x, "w": d_w}[operand]
+        capi.check(L.rp_hip_linear_backward(place["dx"].ptr, place["dw"].ptr, place["db"].ptr, d_dy.ptr, d_x.ptr, d_w.ptr, m, k, n,
+                                            k, 1, n, 1, k, 1, n, 1, 0, 0, 0, F32), str(over))
+        return {name: d.numpy() for name, d in place.items()}
+
+    got = call({"dw": "w"})
+    assert np.array_equal(got["dx"], dx_) and np.array_equal(got["dw"], dw_) and np.array_equal(got["db"], db_)
+    got = call({"dx": "x"})                             # (dX is stored before dW is computed from what then stands there)
+    assert np.array_equal(got["dx"], dx_) and np.array_equal(got["dw"], (dx_.T.astype(np.float64) @ dy).astype(np.float32)) and np.array_equal(got["db"], db_)
+    got = call({"db": "w"})
+    assert np.array_equal(got["dx"], dx_) and np.array_equal(got["dw"], dw_) and np.array_equal(got["db"].reshape(-1)[:n], db_)
+
+
 def test_batch_longer_than_a_grid_axis():
     """70 000 tiny matrices in one call (the batch index rides on a grid axis of at most 65 535 blocks), A shared by
     all of them through a zero batch stride."""
