@@ -508,9 +508,9 @@ static bool same_conv_ok(int reduced_channels, int H, int W, int kH, int kW, int
 // out[nb, C_to, H, W] (dense) = sum over taps and C_from of wt[C_to][tap][C_from] . padded[nb, C_from, planes of pg], (+ bias per
 // channel): the GEMM whose k axis walks the taps as segments.  When image rows are whole 16-byte vectors its epilogue
 // stores only the valid columns, folded into dense planes, and adds the bias; otherwise the product goes to `product`
-// ([nb, C_to, H * Wp]) and a copy kernel drops the unused columns.
+// ([nb, C_to, H * Wp]) and a copy kernel drops the unused columns.  batch: samples of the whole call, of which these are nb.
 template <typename T>
-static int taps_gemm(T* out, void* product, const void* wt, const void* padded, const void* bias, int nb, int C_from, int C_to,
+static int taps_gemm(T* out, void* product, const void* wt, const void* padded, const void* bias, int nb, int batch, int C_from, int C_to,
                      const PadGeom& pg, int kH, int kW, int dtype) {
     constexpr int VEC = 16 / (int)sizeof(T);
     const int H = pg.H, W = pg.W;
@@ -529,7 +529,7 @@ static int taps_gemm(T* out, void* product, const void* wt, const void* padded, 
     } else {
         g.C = product; g.c_bs = (long long)C_to * cols; g.c_rs = cols;
     }
-    if (launch_gemm_segmented_b(g, dtype) != 0) return -1;
+    if (launch_gemm_segmented_b(g, batch, dtype) != 0) return -1;
     if (!fold) {
         const unsigned elems = (unsigned)((long long)nb * C_to * H * W);
         hipLaunchKernelGGL((unpad_planes_kernel<T, 1>), dim3((elems + 255) / 256), dim3(256), 0, current_stream(), out, (const T*)product, (const T*)bias, C_to, H, W, pg.Wp, elems);
@@ -565,7 +565,7 @@ static int same_conv_run(void* out, const void* in, const void* wt, const void* 
         const unsigned pad_vecs = (unsigned)((long long)nb * C_from * (pg.P / VEC));
         launch_pad<T>((T*)padded, in0, pg, pad_vecs, job);          // the first chunk's launch reorders the weights too
         job.blocks = 0;
-        rc = taps_gemm<T>(out0, product, wt, padded, bias, nb, C_from, C_to, pg, kH, kW, dtype);
+        rc = taps_gemm<T>(out0, product, wt, padded, bias, nb, batch, C_from, C_to, pg, kH, kW, dtype);
     }
     if (rc == 0 && !check_launch("padded-plane convolution kernels")) rc = -1;
     rp_hip_free(product);
@@ -659,7 +659,7 @@ static int same_conv_backward(void* dx, void* dw, const void* dy, const void* x,
         job.blocks = 0;
         if (dx) {
             T* dx0 = (T*)dx + (size_t)b0 * C_in * H * W;
-            ok = taps_gemm<T>(dx0, product, wt, dy_pad, nullptr, nb, C_out, C_in, pg, kH, kW, dtype) == 0;
+            ok = taps_gemm<T>(dx0, product, wt, dy_pad, nullptr, nb, batch, C_out, C_in, pg, kH, kW, dtype) == 0;
             if (!ok) break;
         }
         if (dw) {
@@ -675,7 +675,7 @@ static int same_conv_backward(void* dx, void* dw, const void* dy, const void* x,
             g.b_bs = (long long)C_in * pg.P; g.b_rs = 1; g.b_cs = pg.P;
             g.c_bs = w_n; g.c_rs = (long long)taps * C_in; g.c_cs = 1;
             g.seg_n = C_in; g.seg_w = kW; g.seg_sh = pg.Wp; g.seg_sw = 1; g.b_extent = (long long)C_in * pg.P;
-            ok = launch_gemm_segmented_b(g, dtype) == 0;
+            ok = launch_gemm_segmented_b(g, batch, dtype) == 0;
             if (ok) hipLaunchKernelGGL(conv_dw_from_samples_kernel<T>, dim3((unsigned)((w_n + 255) / 256)), dim3(256), 0, current_stream(),
                                        (T*)dw, (const T*)product, nb, C_out, C_in, taps, b0 > 0 ? 1 : 0);
         }

@@ -233,7 +233,7 @@ bool pipe16k_takes(const GemmArgs& g);         // the 16-bit kernel for outputs 
 int launch_pipe16k(const GemmArgs& g, int dtype);
 bool pipe32k_takes(const GemmArgs& g);         // and its fp32 twin
 int launch_pipe32k(const GemmArgs& g);
-int launch_gemm_segmented_b(const GemmArgs& g, int dtype);
+int launch_gemm_segmented_b(const GemmArgs& g, int samples, int dtype);
 void report_kernel(const char* name);          // what rp_hip_last_gemm_kernel names next (a string of static lifetime)
 // 16-bit same-padding convolutions straight from the image (rp_conv_direct.hip); outputs must not overlap the images they are read from
 bool conv_taps16_takes(int batch, int C_from, int C_to, int H, int W, int kH, int kW, int dtype);

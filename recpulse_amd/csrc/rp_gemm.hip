@@ -383,14 +383,15 @@ static int run_gemm(GemmArgs g, int dtype) {
 // 48.7 / 22.7, [22, 64, 48, 48, 64, 3] 96 / 85).  With nearly that many and a long k those of more than 64 rows are 64 x 64 tiles, [1, 256, 56, 56, 128, 5] 123 / 86 (32 x 32: 116), and
 // those of 64 stay what they were, [10, 64, 56, 56, 64, 5] 121 / 139.  Up to four a CU where C_out is more than 64
 // and the positions many ([18, 128, 28, 28, 192, 3] 152 / 107, but [31, 256, 26, 26, 64, 3] 109 / 143, [13, 192, 7, 7, 256, 3] 45.5 / 56.5).
-static WkwTile segmented_wavek_tile(const GemmArgs& g) {
-    if (path_disabled("wavekw") || g.a_cs != 1 || g.n < 64 || g.accumulate || (long long)((g.m + 15) / 16) * ((g.n + 15) / 16) * g.batch >= 1ll << 24 || g.b_extent * 4 >= (1ll << 31) || (63 * g.a_rs + g.k) * 4 >= (1ll << 31)) return WKW_NONE;
-    const long long cus = cu_tiles(), tiles64 = (long long)((g.m + 63) / 64) * ((g.n + 63) / 64) * g.batch;
+// samples: how many the whole call has, of which g.batch go out now.  The tile follows all of them, so that the bits do not depend on how the batch is cut.
+static WkwTile segmented_wavek_tile(const GemmArgs& g, long long samples) {
+    if (path_disabled("wavekw") || g.a_cs != 1 || g.n < 64 || g.accumulate || (long long)((g.m + 15) / 16) * ((g.n + 15) / 16) * samples >= 1ll << 24 || g.b_extent * 4 >= (1ll << 31) || (63 * g.a_rs + g.k) * 4 >= (1ll << 31)) return WKW_NONE;
+    const long long cus = cu_tiles(), tiles64 = (long long)((g.m + 63) / 64) * ((g.n + 63) / 64) * samples;
     if (g.seg_k > 0) {
         if (g.seg_k % 32) return WKW_NONE;
         if (g.m >= 192) { if (tiles64 * 4 >= cus * 7) return WKW_64X64; }
         else if (g.k < 1024 ? tiles64 * 4 > cus * 5 : tiles64 > cus * 3) return WKW_NONE;
-        return (long long)((g.m + 15) / 16) * ((g.n + 31) / 32) * g.batch >= cus ? WKW_16X32 : WKW_16X16;
+        return (long long)((g.m + 15) / 16) * ((g.n + 31) / 32) * samples >= cus ? WKW_16X32 : WKW_16X16;
     }
     if (tiles64 <= cus) {
         if (g.k < 2048 || tiles64 * 4 < cus * 3) return WKW_32X32;
@@ -402,8 +403,8 @@ static WkwTile segmented_wavek_tile(const GemmArgs& g) {
 // C_z = A_z . B_z with B's k axis or its n axis given as segments (GemmArgs::seg_*): the MFMA kernels read every
 // segment in place, at any alignment of whole elements.  For callers inside the library (the convolution), which
 // guarantee: A with unit stride along k or m, B with unit stride along n and k a whole number of segments of whole
-// slabs, or B with unit stride along k and n a whole number of segments.
-int launch_gemm_segmented_b(const GemmArgs& g, int dtype) {
+// slabs, or B with unit stride along k and n a whole number of segments.  samples: matrices of the whole call, of which g is a part.
+int launch_gemm_segmented_b(const GemmArgs& g, int samples, int dtype) {
     const bool is16 = dtype == RP_DTYPE_FLOAT16 || dtype == RP_DTYPE_BFLOAT16;
     const int vec = 16 / (int)dtype_size(dtype);
     const int bk = is16 ? M16_BK : (dtype == RP_DTYPE_FLOAT32 ? 32 : 16);           // k slab of the kernel that will run
@@ -428,7 +429,7 @@ int launch_gemm_segmented_b(const GemmArgs& g, int dtype) {
         return launch_mfma16(g, p, dtype);
     }
     if (dtype == RP_DTYPE_FLOAT32) {
-        const WkwTile tile = segmented_wavek_tile(g);
+        const WkwTile tile = segmented_wavek_tile(g, samples);
         if (tile != WKW_NONE) return launch_wavekw_segmented(g, tile);
     }
     Plan p{FAM_MFMAW, 64, 64, !a_kc, g.seg_k > 0, true, "mfmaw"};

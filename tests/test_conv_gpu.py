@@ -370,6 +370,34 @@ def test_same_convolution_in_chunks_of_the_batch(monkeypatch):
     assert np.array_equal(whole[0], run()[0])
 
 
+@pytest.mark.parametrize("N,Ci,H,W,Co", [(24, 64, 28, 28, 64), (11, 192, 28, 28, 192), (5, 64, 9, 11, 96)])
+def test_fp32_same_convolution_in_chunks_of_the_batch(monkeypatch, N, Ci, H, W, Co):
+    """fp32 images of random values: y and dX have the same bits whether the batch goes in one piece or in several, and dX whether
+    dW is asked for or not (the workspace of dW makes its chunks smaller).  The whole batches of the first two shapes have too many tiles for
+    the kernel that their parts would go to."""
+    L = capi.lib()
+    rng = np.random.default_rng(85)
+    x, w, g = rand_storage(rng, (N, Ci, H, W), F32), oracle.to_storage(rng.standard_normal((Co, Ci, 3, 3)) * 0.05, F32), rand_storage(rng, (N, Co, H, W), F32)
+    dx_, dw_, dg_ = Dev(x, F32), Dev(w, F32), Dev(g, F32)
+
+    def run(with_dw):
+        y, gx, gw = Dev.empty((N, Co, H, W), F32), Dev.empty((N, Ci, H, W), F32), Dev.empty((Co, Ci, 3, 3), F32)
+        capi.check(L.rp_hip_conv2d_same_forward(y.ptr, dx_.ptr, dw_.ptr, None, N, Ci, H, W, Co, 3, 3, F32), "same forward")
+        capi.check(L.rp_hip_conv2d_same_backward(gx.ptr, gw.ptr if with_dw else None, dg_.ptr, dx_.ptr, dw_.ptr, N, Ci, H, W, Co, 3, 3, F32), "same backward")
+        return y.numpy(), gx.numpy(), gw.numpy()
+
+    whole = run(True)
+    assert np.array_equal(whole[1], run(False)[1])
+    plane = (H + 2) * ((W + 2 + 3) // 4 * 4) + 16                     # a zero-bordered plane and its slack, elements
+    for samples in (2, N // 2):
+        # (what a sample takes with dW: planes of dY and X and the larger product; without, and in the forward, more of them fit)
+        monkeypatch.setenv("RP_CONV_WORKSPACE_BYTES", str(samples * 4 * ((Ci + Co) * plane + max(Ci * plane, Co * Ci * 9)) + 64))
+        parts, without = run(True), run(False)
+        assert np.array_equal(whole[0], parts[0]) and np.array_equal(whole[1], parts[1]) and np.array_equal(whole[1], without[1])
+        assert oracle.rel_err(parts[2].astype(np.float64), whole[2].astype(np.float64)) <= 1e-5
+    monkeypatch.delenv("RP_CONV_WORKSPACE_BYTES")
+
+
 def test_same_convolution_rejects_other_shapes():
     L = capi.lib()
     assert L.rp_hip_conv2d_same_supported(48, 8, 8, 3, 3, BF16) == 0           # channels in whole k slabs: 64 for 16-bit types,
