@@ -222,7 +222,6 @@ __device__ __forceinline__ void batched_block(int tiles_m, int tiles_n, int& slo
 bool direct32_takes(const GemmArgs& g);          // pointer alignment and spans the short-k fp32 kernel can address
 int launch_direct32(const GemmArgs& g);
 size_t skinny16_workspace(int batch, int m, int k, int n);          // bytes of partial sums that the tiled 16-bit k split needs
-int launch_wavekw(const GemmArgs& g, int dtype);              // fp32 / fp64 products that the waves of a workgroup share, see wavekw_takes
 int launch_mfma16_wavek(const GemmArgs& g, bool ragged, int dtype);       // few tiles, deep k, A k-contiguous; see wavek16_takes
 int launch_linear_backward16(const GemmArgs& gx, const GemmArgs& gw, bool dx_wavek, void* db, int accumulate_db, bool edge, bool ragged, int dtype);      // both on 64 x 64 tiles or dX's waves splitting k, whole or ending in whole 16-byte vectors, see linear_backward_pairs
 bool pipe32_takes(const GemmArgs& g);          // options, alignment and spans the k-contiguous short-k fp32 kernel can address

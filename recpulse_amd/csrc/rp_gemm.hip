@@ -290,29 +290,36 @@ static bool wavek16_takes(const GemmArgs& g, const Plan& p, int dtype, bool& rag
 
 // fp32 and fp64 products that the waves of a workgroup share (rp_gemm_wavekw.hip, which has figures): those of 64 x 64 tiles, fp64 ones of the generic
 // kernel, and fp32 ones that 16 x 16 tiles of four waves or the row-streaming kernel took.  Stays where it was: fp32 with k up to 512 on 16 x 16 tiles (60 x 443 x 65 3.55 / 3.67 us; 256 x 784 x 256
-// 6.95 / 5.0-6.0); a few rows with k above 1024 (8 x 8192 x 8192 55 / 51, but that kernel's sums are of shorter chains); a k too short for the number of tiles (fp32 2384 x 32 x 368
+// 6.95 / 5.0-6.0); a k too short for the number of tiles (fp32 2384 x 32 x 368
 // 5.2 / 6.5, 944 x 144 x 1648 14.0 / 16.2; fp64 832 x 48 x 2128 14.6 / 22.7); fp32 outputs of a few tiles whose long k the split deals to more CUs
 // (16 x 5744 x 48 11.5 / 14.4) and sums in shorter chains; batches of more than one 64 x 64 tile a CU that fill those as well as 32 x 32 ones (fp32
 // 128 x 512 x 128 100 of them 26.8 / 33.2, 60 21.2 / 14.9; 20 x 600 x 20 1000 of them 50.8 / 26.1; fp64 40 x 100 x 40 3000 of them 84 / 124) or, in fp32, of a k up
 // to 64 (128 x 64 x 128, 50 of them 6.2 / 7.6).  (The k split read all of its operands before it wrote C: outputs over an operand stay there.)
-static bool wavekw_takes(const GemmArgs& g, const Plan& p, int dtype) {
+// Of the row-streaming kernel's products (up to 8 rows), which sums chains of 32 values: those with 168 <= k <= 1024, on 16 x 32 tiles alone, whose waves'
+// chains are no longer (relative error of 8 x k x 16384, there and here: k = 128 8.7e-8 / 8.9e-8, 168 9.5e-8 / 9.2e-8, 256 1.13e-7 / 9.6e-8, 640 1.15e-7 / 1.13e-7, 1024 1.19e-7 / 1.13e-7
+// with 16 waves, 1.25e-7 with 8; the larger tiles' chains are of k / 16 and k / 8: 1024 1.6e-7 and 2.1e-7), us there and here: 8 x 256 x 8192 22.0 / 5.0, 1 x 1024 x 8192 11.4 / 5.8, 8 x 1024 x 16384 24.2 / 14.2.
+// Up to four rows of very many columns stay where k is short or takes 16 waves: 1 x 200 x 49152 7.9 / 10.6, 4 x 200 x 65000 13.1 / 15.0, 1 x 1000 x 32768 23.6 / 25.2 (1 x 200 x 24576 7.1 / 6.0,
+// 1 x 384 x 49152 16.7 / 14.7, 1 x 1000 x 16384 15.5 / 13.9, 5 x 176 x 65000 16.6 / 14.0).
+static WkwTile wavekw_takes(const GemmArgs& g, const Plan& p, int dtype) {
     const bool f32 = dtype == RP_DTYPE_FLOAT32;
-    if (!(f32 || dtype == RP_DTYPE_FLOAT64) || g.seg_k || g.seg_n || g.bias_by_row || g.c_fold_from || path_disabled("wavekw")) return false;
+    if (!(f32 || dtype == RP_DTYPE_FLOAT64) || g.seg_k || g.seg_n || g.bias_by_row || g.c_fold_from || path_disabled("wavekw")) return WKW_NONE;
     const long long tiles64 = (long long)((g.m + 63) / 64) * ((g.n + 63) / 64) * g.batch, tiles16 = (long long)((g.m + 15) / 16) * ((g.n + 15) / 16) * g.batch;
     if (p.fam == FAM_MFMAW && p.bm == 64) {
         const long long tiles32 = (long long)((g.m + 31) / 32) * ((g.n + 31) / 32) * g.batch;
-        if (g.batch > 1 && ((tiles64 > cu_tiles() && tiles32 * 2 >= tiles64 * 7) || (f32 && g.k <= 64 && tiles64 > cu_tiles() / 2))) return false;
-        if (f32 ? g.k <= 32 || (tiles64 > cu_tiles() && g.k < 256) : g.k <= 48 && tiles64 > cu_tiles() / 2) return false;
+        if (g.batch > 1 && ((tiles64 > cu_tiles() && tiles32 * 2 >= tiles64 * 7) || (f32 && g.k <= 64 && tiles64 > cu_tiles() / 2))) return WKW_NONE;
+        if (f32 ? g.k <= 32 || (tiles64 > cu_tiles() && g.k < 256) : g.k <= 48 && tiles64 > cu_tiles() / 2) return WKW_NONE;
         const bool splits = f32 && (g.n % 4 == 0 || p.ragged), both_kc = g.a_cs == 1 && g.b_rs == 1 && g.b_cs != 1;
-        if (splits && g.k > 2048 && (tiles64 < cu_tiles() / 32 || (!both_kc && tiles16 < cu_tiles() / 4))) return false;
+        if (splits && g.k > 2048 && (tiles64 < cu_tiles() / 32 || (!both_kc && tiles16 < cu_tiles() / 4))) return WKW_NONE;
     } else if (p.fam == FAM_TINY) {
-        if (g.k <= 512) return false;
+        if (g.k <= 512) return WKW_NONE;
     } else if (p.fam == FAM_SKINNY) {
-        if (g.k > 1024) return false;
+        if (!f32 || g.k < 168 || g.k > 1024) return WKW_NONE;
+        if (g.m <= 4 && (g.k > 640 ? g.n > 16384 : g.n > 24576 && g.k < 384)) return WKW_NONE;
     } else if (!(p.fam == FAM_GENERIC && !f32 && !path_disabled("mfma"))) {
-        return false;
+        return WKW_NONE;
     }
-    if (wavekw_tile(g, dtype) == WKW_NONE) return false;
+    const WkwTile tile = wavekw_tile(g, dtype);
+    if (tile == WKW_NONE) return WKW_NONE;
     const int esz = (int)dtype_size(dtype);
     auto span = [&](const void* base, int rows, int cols, long long bs, long long rs, long long cs) {
         Span s = span_of(base, rows, cols, rs, cs, esz);
@@ -320,8 +327,9 @@ static bool wavekw_takes(const GemmArgs& g, const Plan& p, int dtype) {
         return s;
     };
     const Span c = span(g.C, g.m, g.n, g.c_bs, g.c_rs, g.c_cs);
-    return !overlap(c, span(g.A, g.m, g.k, g.a_bs, g.a_rs, g.a_cs)) && !overlap(c, span(g.B, g.k, g.n, g.b_bs, g.b_rs, g.b_cs)) &&
-           !(g.bias && overlap(c, span_of(g.bias, 1, g.n, 0, 1, esz)));
+    const bool apart = !overlap(c, span(g.A, g.m, g.k, g.a_bs, g.a_rs, g.a_cs)) && !overlap(c, span(g.B, g.k, g.n, g.b_bs, g.b_rs, g.b_cs)) &&
+                       !(g.bias && overlap(c, span_of(g.bias, 1, g.n, 0, 1, esz)));
+    return !apart ? WKW_NONE : p.fam == FAM_SKINNY ? WKW_FEW_ROWS : tile;
 }
 
 static thread_local const char* g_last_kernel = "none";      // what rp_hip_last_gemm_kernel reports
@@ -357,9 +365,10 @@ static int run_gemm(GemmArgs g, int dtype) {
         g_last_kernel = wavek_ragged ? p.name : "mfma16_wavek";          // (ragged rows: it goes by the name of the kernel that it stands in for)
         return launch_mfma16_wavek(g, wavek_ragged, dtype);
     }
-    if (wavekw_takes(g, p, dtype)) {
+    const WkwTile shared_k = wavekw_takes(g, p, dtype);
+    if (shared_k != WKW_NONE) {
         g_last_kernel = p.fam == FAM_MFMAW ? p.name : dtype == RP_DTYPE_FLOAT32 ? "mfma32_wavek" : "mfma64_wavek";      // (among the 64 x 64 tiles it goes by their name)
-        return launch_wavekw(g, dtype);
+        return launch_wavekw(g, shared_k, dtype);
     }
     g_last_kernel = p.name;
     switch (p.fam) {
@@ -547,7 +556,8 @@ static bool bias_gradient_apart(const void* db, const GemmArgs& gx, const GemmAr
 // (kc) or both free-index-contiguous
 static WkwTile small_tile_alone(const GemmArgs& g, bool kc, int dtype) {
     const Plan p = plan_alone(g, dtype);
-    if (wavekw_takes(g, p, dtype)) return wkw_a_kc(g) == kc && wkw_b_kc(g) == kc ? wavekw_tile(g, dtype) : WKW_NONE;
+    const WkwTile tile = wavekw_takes(g, p, dtype);
+    if (tile != WKW_NONE) return wkw_a_kc(g) == kc && wkw_b_kc(g) == kc ? tile : WKW_NONE;
     return p.fam == FAM_TINY ? WKW_TINY : WKW_NONE;
 }
 

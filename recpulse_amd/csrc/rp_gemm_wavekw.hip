@@ -8,8 +8,8 @@
 // up in fp32 and without either in fp64.  us, before and here:
 //   fp32 1024^3 30.4 / 25, 512^3 12.9 / 6.2, 935 x 862 x 398 32.0 / 12.9, 25 x 3120 x 2446 38.1 / 13.7, 32 x 8192 x 8192 141 / 60, 17 x 6048 x 173 (B^T)
 //   190 / 11.1, 64 x 4096 x 1024 (B^T) 18.8 / 9.6; fp64 89 x 2787 x 286 390 / 15.5, 2054 x 1064 x 52 (B^T) 120 / 15, 512^3 (A^T) 25.9 / 8.7, 300^3 (B^T) 38 / 5.8.
-// Over 330 drawn fp32 products 0.78 of the time, the slowest 1.03, over 170 fp64 ones 0.19 and 1.01.  The error against 64 bits is smaller than before: k is summed in 8 to 32 chains
-// (1024^3 2.1e-7, 5.8e-7 before; 64 x 4096 x 1024 2.2e-7 and 3.0e-7).
+// Over 330 drawn fp32 products 0.78 of the time, the slowest 1.03, over 170 fp64 ones 0.19 and 1.01.  k is summed in 8 to 64 chains, so the error against 64 bits is smaller than in one
+// (1024^3 2.1e-7, 5.8e-7 before; 64 x 4096 x 1024 2.2e-7 and 3.0e-7); wavekw_takes leaves products alone whose kernel sums shorter chains.
 #include "rp_column_sums.h"
 #include "rp_gemm_tiny.h"
 #include "rp_gemm_wavekw.h"
@@ -65,14 +65,14 @@ WkwTile wavekw_tile(const GemmArgs& g, int dtype) {
     return !(a_kc && b_kc) && fits(1, 2) && tiles(1, 2) >= cus / 2 ? WKW_16X32 : WKW_16X16;
 }
 
-int launch_wavekw(const GemmArgs& g, int dtype) {
-    const WkwTile tile = wavekw_tile(g, dtype);
+int launch_wavekw(const GemmArgs& g, WkwTile tile, int dtype) {
     if (dtype == RP_DTYPE_FLOAT64) return tile == WKW_32X32 ? launch_wavekw_layout<double, 2, 2, 8>(g) : launch_wavekw_layout<double, 1, 1, 8>(g);
     switch (tile) {
         case WKW_64X64: return launch_wavekw_layout<float, 4, 4, 8>(g);
         case WKW_16X64: return launch_wavekw_t<float, true, false, 1, 4, 8>(g);
         case WKW_32X32: return launch_wavekw_layout<float, 2, 2, 8>(g);
         case WKW_16X32: return launch_wavekw_layout<float, 1, 2, 8>(g);
+        case WKW_FEW_ROWS: return g.k <= 640 ? launch_wavekw_t<float, true, false, 1, 2, 8>(g) : launch_wavekw_t<float, true, false, 1, 2, 16>(g);
         default: return launch_wavekw_layout<float, 1, 1, 8>(g);
     }
 }
