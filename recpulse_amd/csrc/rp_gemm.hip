@@ -394,7 +394,7 @@ static int run_gemm(GemmArgs g, int dtype) {
 // and the positions many ([18, 128, 28, 28, 192, 3] 152 / 107, but [31, 256, 26, 26, 64, 3] 109 / 143, [13, 192, 7, 7, 256, 3] 45.5 / 56.5).
 // samples: how many the whole call has, of which g.batch go out now.  The tile follows all of them, so that the bits do not depend on how the batch is cut.
 static WkwTile segmented_wavek_tile(const GemmArgs& g, long long samples) {
-    if (path_disabled("wavekw") || g.a_cs != 1 || g.n < 64 || g.accumulate || (long long)((g.m + 15) / 16) * ((g.n + 15) / 16) * samples >= 1ll << 24 || g.b_extent * 4 >= (1ll << 31) || (63 * g.a_rs + g.k) * 4 >= (1ll << 31)) return WKW_NONE;
+    if (path_disabled("wavekw") || g.a_cs != 1 || g.n < 64 || g.accumulate || (long long)((g.m + 15) / 16) * ((g.n + 15) / 16) * samples >= (1ll << 23) - 8 || g.b_extent * 4 >= (1ll << 31) || (63 * g.a_rs + g.k) * 4 >= (1ll << 31)) return WKW_NONE;
     const long long cus = cu_tiles(), tiles64 = (long long)((g.m + 63) / 64) * ((g.n + 63) / 64) * samples;
     if (g.seg_k > 0) {
         if (g.seg_k % 32) return WKW_NONE;
@@ -662,7 +662,7 @@ int rp_hip_linear_backward(void* dx, void* dw, void* db, const void* dy, const v
         }
         // (more than two rounds of 16 x 16 tiles need the registers and the LDS that they have alone: fp32 2659 x 49 x 3731 70.3 us apart, 73.4 in one launch)
         const auto rounds16 = [&](const GemmArgs& g, WkwTile t) { return t == WKW_16X16 && (long long)((g.m + 15) / 16) * ((g.n + 15) / 16) > 2 * cu_tiles(); };
-        if (dx && dw && linear_backward_wavekw_takes(tx, tw, dtype) && (tx == tw || !(rounds16(gx, tx) || rounds16(gw, tw))) && apart) {
+        if (dx && dw && linear_backward_wavekw_takes(gx, gw, tx, tw, dtype) && (tx == tw || !(rounds16(gx, tx) || rounds16(gw, tw))) && apart) {
             g_last_kernel = "linear_backward_wavek";
             const bool rides = db && m <= LINEAR_DB_ROWS && bias_gradient_apart(db, gx, gw, dtype);
             if (launch_linear_backward_wavekw(gx, gw, tx, tw, rides ? db : nullptr, accumulate_db, dtype) != 0) return -1;

@@ -351,7 +351,7 @@ WkwTile wavekw_tile(const GemmArgs& g, int dtype);
 int launch_wavekw(const GemmArgs& g, WkwTile tile, int dtype);      // fp32 / fp64 products that the waves of a workgroup share, see wavekw_takes
 int launch_wavekw_segmented(const GemmArgs& g, WkwTile tile);       // fp32, A with unit stride along k, B in segments
 // All gradients of a Linear layer in one launch, each product on the tiles that it would get alone; gx.A is dY [gx.m, gx.k], dense; db: gx.k column sums of dY, or null
-bool linear_backward_wavekw_takes(WkwTile x, WkwTile w, int dtype);
+bool linear_backward_wavekw_takes(const GemmArgs& gx, const GemmArgs& gw, WkwTile x, WkwTile w, int dtype);
 int launch_linear_backward_wavekw(const GemmArgs& gx, const GemmArgs& gw, WkwTile x, WkwTile w, void* db, int accumulate_db, int dtype);
 static inline bool wkw_a_kc(const GemmArgs& g) { return g.a_cs == 1; }
 static inline bool wkw_b_kc(const GemmArgs& g) { return g.b_rs == 1 && (g.b_cs != 1 || g.n == 1); }

@@ -48,6 +48,7 @@ static int launch_wavekw_layout(const GemmArgs& g) {
 // fp64), else 16 x 16, or 16 x 32 where an operand's k rows are read (its loads of 16 elements are half a line).  One 64 x 64 tile a CU with a k that is worth
 // its prologue (1024^3 24 us, 28.5 on 32 x 32); 16 x 64 where one fills the chip once with a row-major B, whose lines it takes whole
 // (128 x 5888 x 1600 27.9 us, 33.3 on 16 x 32; 935 x 862 x 398, 413 of them, 14.2 and 12.7 on 32 x 32).
+constexpr long long WKW_MAX_SLOTS = (1ll << 32) / 512 - 8;       // workgroups of 512 threads in a launch of fewer than 2^32 threads, less what rounds them up to eights
 WkwTile wavekw_tile(const GemmArgs& g, int dtype) {
     const bool a_kc = wkw_a_kc(g), b_kc = wkw_b_kc(g);
     if (!(a_kc || g.a_rs == 1) || !(b_kc || g.b_cs == 1) || g.batch > 65535) return WKW_NONE;
@@ -58,11 +59,14 @@ WkwTile wavekw_tile(const GemmArgs& g, int dtype) {
     const auto tiles = [&](int tm, int tn) { return (long long)((g.m + 16 * tm - 1) / (16 * tm)) * ((g.n + 16 * tn - 1) / (16 * tn)) * g.batch; };
     const auto fits = [&](int tm, int tn) { return (a_kc || g.m >= 16 * tm) && (b_kc || g.n >= 16 * tn); };       // see ms, ns in gemm_wavekw_block
     if (!fits(1, 1) || tiles(1, 1) >= 1ll << 24) return WKW_NONE;
-    if (dtype == RP_DTYPE_FLOAT64) return fits(2, 2) && tiles(2, 2) >= cus / 2 ? WKW_32X32 : WKW_16X16;
-    if (fits(4, 4) && g.k >= 512 && tiles(4, 4) >= cus * 3 / 4 && tiles(4, 4) <= cus) return WKW_64X64;
-    if (a_kc && !b_kc && fits(1, 4) && g.k >= 512 && tiles(1, 4) >= cus / 2 && tiles(1, 4) <= cus) return WKW_16X64;
-    if (fits(2, 2) && tiles(2, 2) >= cus * 3 / 4) return WKW_32X32;
-    return !(a_kc && b_kc) && fits(1, 2) && tiles(1, 2) >= cus / 2 ? WKW_16X32 : WKW_16X16;
+    if (dtype == RP_DTYPE_FLOAT64 && fits(2, 2) && tiles(2, 2) >= cus / 2) return WKW_32X32;
+    if (dtype != RP_DTYPE_FLOAT64) {
+        if (fits(4, 4) && g.k >= 512 && tiles(4, 4) >= cus * 3 / 4 && tiles(4, 4) <= cus) return WKW_64X64;
+        if (a_kc && !b_kc && fits(1, 4) && g.k >= 512 && tiles(1, 4) >= cus / 2 && tiles(1, 4) <= cus) return WKW_16X64;
+        if (fits(2, 2) && tiles(2, 2) >= cus * 3 / 4) return WKW_32X32;
+        if (!(a_kc && b_kc) && fits(1, 2) && tiles(1, 2) >= cus / 2) return tiles(1, 2) <= WKW_MAX_SLOTS ? WKW_16X32 : WKW_NONE;
+    }
+    return tiles(1, 1) <= WKW_MAX_SLOTS ? WKW_16X16 : WKW_NONE;       // (many tiles where an operand is only 16 to 31 wide)
 }
 
 int launch_wavekw(const GemmArgs& g, WkwTile tile, int dtype) {
@@ -142,7 +146,9 @@ static int launch_linear_backward_wavekw_t(const GemmArgs& gx, const GemmArgs& g
     return check_launch("linear_backward_wavekw_kernel") ? 0 : -1;
 }
 
-bool linear_backward_wavekw_takes(WkwTile x, WkwTile w, int dtype) {
+bool linear_backward_wavekw_takes(const GemmArgs& gx, const GemmArgs& gw, WkwTile x, WkwTile w, int dtype) {
+    const auto tiles16 = [](const GemmArgs& g) { return (long long)((g.m + 15) / 16) * ((g.n + 15) / 16); };
+    if (tiles16(gx) + tiles16(gw) + gx.k / 8 + 16 > WKW_MAX_SLOTS) return false;
     const bool f32 = dtype == RP_DTYPE_FLOAT32;
     const auto small = [&](WkwTile k) { return k == WKW_16X16 || k == WKW_32X32 || (f32 && k == WKW_TINY); };
     return small(x) && (small(w) || (f32 && w == WKW_16X32)) && !(x == WKW_TINY && w == WKW_TINY);

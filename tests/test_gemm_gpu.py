@@ -894,6 +894,21 @@ def test_batch_longer_than_a_grid_axis():
     assert oracle.rel_err(got[69999].astype(np.float64), oracle.matmul(a, np.ascontiguousarray(b[69999]), F32).astype(np.float64)) <= tol(F32, k)
 
 
+def test_more_tiles_than_workgroups_fit_a_launch():
+    """2^23 tiles of 16 x 16, whose workgroups of 512 threads are more than a launch holds: fp64 with a row-major B of 24 columns (A's rows are one
+    row, expanded; 1.3e10 bytes of C, of which a few rows are looked at)."""
+    rng = np.random.default_rng(47)
+    m, k, n = 1 << 26, 50, 24
+    a, b = rng.integers(-3, 4, k).astype(np.float64), rng.integers(-3, 4, (k, n)).astype(np.float64)
+    da, db, dc = capi.DeviceBuffer.from_numpy(a), capi.DeviceBuffer.from_numpy(b), capi.DeviceBuffer(m * n * 8)
+    capi.gemm(dc.ptr, da.ptr, db.ptr, None, 1, m, k, n, (0, 0, 1), (0, n, 1), (0, n, 1), False, F64)
+    got = np.empty((2, n))
+    for row in (0, 12345678, m // 2 - 1, m - 2):
+        capi.check(capi.lib().rp_hip_memcpy_d2h(got.ctypes.data, dc.at(row * n * 8), got.nbytes), "memcpy_d2h")
+        assert np.array_equal(got, np.stack([a @ b] * 2))
+    dc.free()
+
+
 def test_rejects_bad_arguments():
     lib = capi.lib()
     d = capi.DeviceBuffer(64)
