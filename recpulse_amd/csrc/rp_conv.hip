@@ -884,7 +884,10 @@ int rp_hip_channel_sums(void* out, const void* grad, int batch, int channels, in
         return -1;
     }
     if (!dtype_size(dtype)) { set_error("rp_hip_channel_sums: unsupported dtype %d", dtype); return -1; }
-    if ((size_t)batch * hw * dtype_size(dtype) <= CHANNEL_SUM_BYTES) {
+    // (A launch holds fewer than 2^32 threads.  A sum stored over values that another channel's workgroup still reads: the two launches read them all first.)
+    const size_t esz = dtype_size(dtype), per_channel = (size_t)batch * hw * esz;
+    const bool apart = (const char*)out + channels * esz <= (const char*)grad || (const char*)grad + per_channel * channels <= (const char*)out;
+    if (per_channel <= CHANNEL_SUM_BYTES && channels < 1 << 22 && apart) {
         RP_DISPATCH_DTYPE(dtype, hipLaunchKernelGGL(channel_sums_kernel<T>, dim3((unsigned)channels), dim3(1024), 0, current_stream(), (T*)out, (const T*)grad, batch, channels, hw, accumulate));
         return check_launch("channel_sums_kernel") ? 0 : -1;
     }

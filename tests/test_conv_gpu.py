@@ -105,6 +105,27 @@ def test_channel_sums_of_every_size(dt, N, C, HW):
     assert np.array_equal(ds.numpy(), oracle.to_storage(g.sum(axis=(0, 2)), dt))
 
 
+@pytest.mark.parametrize("dt", ALL, ids=lambda d: NAMES[d])
+def test_channel_sums_over_the_gradient_and_of_very_many_channels(dt):
+    """Sums written over values that other channels' sums read, and more channels than workgroups of 1024 threads fit a launch; small integers."""
+    rng = np.random.default_rng(82)
+    L = capi.lib()
+    es = capi.DTYPE_SIZE[dt]
+    for N, C, HW in ((5, 600, 49), (1, 3000, 7)):
+        g = rng.integers(-2, 3, (N, C, HW)).astype(np.float64)
+        want = oracle.to_storage(g.sum(axis=(0, 2)), dt)
+        for at in (0, C * HW - C):                       # over the first planes, over the last ones of the first sample
+            flat = oracle.to_storage(g, dt).reshape(-1)
+            d = capi.DeviceBuffer.from_numpy(flat)
+            capi.check(L.rp_hip_channel_sums(d.at(at * es), d.ptr, N, C, HW, 0, dt), "rp_hip_channel_sums")
+            assert np.array_equal(d.to_numpy(flat.dtype, (flat.size,))[at:at + C], want)
+    C = 1 << 22
+    g = oracle.to_storage(rng.integers(-2, 3, (1, C, 2)).astype(np.float64), dt)
+    ds = Dev.empty((C,), dt)
+    capi.check(L.rp_hip_channel_sums(ds.ptr, Dev(g, dt).ptr, 1, C, 2, 0, dt), "rp_hip_channel_sums")
+    assert np.array_equal(ds.numpy(), oracle.to_storage(oracle.to_f64(g, dt).sum(axis=(0, 2)), dt))
+
+
 def test_lowering_rejects_inconsistent_geometry():
     d = capi.DeviceBuffer(1 << 16)
     L = capi.lib()
