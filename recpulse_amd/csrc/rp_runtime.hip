@@ -189,7 +189,7 @@ public:
         std::lock_guard<std::mutex> lk(g_readback_mu);
         std::vector<void*>& kept = readback_blocks();
         if (!kept.empty()) { ptr = kept.back(); kept.pop_back(); }
-        else if (g_readback_out >= READBACK_BLOCKS || hipHostMalloc(&ptr, READBACK_BYTES, hipHostMallocPortable | hipHostMallocMapped) != hipSuccess) { (void)hipGetLastError(); ptr = nullptr; return; }
+        else if (g_readback_out >= READBACK_BLOCKS || !allocate()) { ptr = nullptr; return; }
         g_readback_out++;
     }
     ~ReadbackBlock() {
@@ -201,6 +201,18 @@ public:
     ReadbackBlock(const ReadbackBlock&) = delete;
     ReadbackBlock& operator=(const ReadbackBlock&) = delete;
     void* ptr = nullptr;
+
+private:
+    // While another thread records a graph in the runtime's default mode, an allocation by any thread is refused and spoils that recording,
+    // unless the thread is in the relaxed mode.  (The copy that this replaces allocated nothing.)
+    bool allocate() {
+        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+        if (hipThreadExchangeStreamCaptureMode(&mode) != hipSuccess) { (void)hipGetLastError(); return false; }
+        const bool ok = hipHostMalloc(&ptr, READBACK_BYTES, hipHostMallocPortable | hipHostMallocMapped) == hipSuccess;
+        if (!ok) (void)hipGetLastError();
+        (void)hipThreadExchangeStreamCaptureMode(&mode);         // back to what it was
+        return ok;
+    }
 };
 
 __global__ void __launch_bounds__(256) readback_kernel(uint4* dst, const uint4* src, int n) {

@@ -484,6 +484,42 @@ def test_copies_to_the_host_of_every_size_and_start():
     assert L().rp_hip_memcpy_d2h(data.ctypes.data, None, 4) == -1
 
 
+def test_first_copy_to_the_host_beside_another_threads_recording():
+    """A graph recorded in the runtime's default mode, in which no thread may allocate: another thread's first small copy to the host leaves it whole."""
+    hip = L()                                                    # (its handle finds the runtime's functions too)
+    data = np.arange(3000, dtype=np.float32)
+    buf, out = capi.DeviceBuffer.from_numpy(data), Dev(np.zeros(512, np.float32), F32)
+    stream, graph, executable = ctypes.c_void_p(), ctypes.c_void_p(), ctypes.c_void_p()
+    capi.check(L().rp_hip_stream_create(ctypes.byref(stream)), "stream")
+    capi.synchronize()
+    capi.check(L().rp_hip_empty_cache(), "empty_cache")          # (the pinned blocks too)
+    got = np.zeros_like(data)
+    status = []
+
+    def copy():
+        status.append(L().rp_hip_memcpy_d2h(got.ctypes.data, buf.ptr, got.nbytes))
+
+    capi.check(L().rp_hip_set_stream(stream), "set stream")
+    try:
+        assert hip.hipStreamBeginCapture(stream, 0) == 0         # hipStreamCaptureModeGlobal
+        capi.check(L().rp_hip_fill(out.ptr, 3.0, 512, F32), "fill")
+        thread = threading.Thread(target=copy)
+        thread.start()
+        thread.join()
+        assert hip.hipStreamEndCapture(stream, ctypes.byref(graph)) == 0
+    finally:
+        L().rp_hip_set_stream(None)
+    assert status == [0] and np.array_equal(got, data)
+    assert hip.hipGraphInstantiate(ctypes.byref(executable), graph, None, None, ctypes.c_size_t(0)) == 0
+    for _ in range(3):
+        capi.check(L().rp_hip_memset(out.ptr, 0, 2048), "memset")
+        capi.synchronize()
+        assert hip.hipGraphLaunch(executable, stream) == 0 and hip.hipStreamSynchronize(stream) == 0
+        assert np.array_equal(out.numpy(), np.full(512, 3.0, np.float32))
+    assert hip.hipGraphExecDestroy(executable) == 0 and hip.hipGraphDestroy(graph) == 0
+    capi.check(L().rp_hip_stream_destroy(stream), "stream")
+
+
 def test_graph_replay_matches_eager():
     """A recorded GEMM + bias-gradient + relu sequence replays to the eager result every time (no memset nodes inside)."""
     rng = np.random.default_rng(48)
