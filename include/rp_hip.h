@@ -144,18 +144,22 @@ int rp_hip_gemm_strided_batched_noalloc(void* C, const void* A, const void* B, c
 /* Name of the kernel family the dispatcher picks for a problem, for logs and
  * tests ("mfma16_256x256", "skinny", "generic", ...).  No device work.  "mfma16_wavek", which stands in for "mfma16_64x64" and
  * "mfma16_skinny_32x128" where C lies apart from the operands, "mfma32_wavek" and "mfma64_wavek", which stand in for "tiny32_16x16", "skinny" and (float64)
- * "generic" there, and "linear_backward_wavek" are named by rp_hip_last_gemm_kernel alone.  In the place of "mfma32_64x64", "mfma64_64x64" and
- * any 16-bit kernel for rows of arbitrary length, waves that share k go by the name of the kernel that they stand in for. */
+ * "generic" there, and "linear_backward_wavek" are named by rp_hip_last_gemm_kernel alone. */
 const char* rp_hip_gemm_kernel_name(int batch, int m, int k, int n,
                                     long long a_rs, long long a_cs,
                                     long long b_rs, long long b_cs,
                                     long long c_rs, long long c_cs, int dtype);
 /* Name of the kernel family and tile that the calling thread's most recent GEMM entry-point call dispatched ("none"
  * before the first): unlike rp_hip_gemm_kernel_name it reflects the bias, the accumulate flag and the pointers of that
- * call.  The rp_hip_conv2d_same_* entries report theirs too: "conv_taps16_256x64" or "_64x64" (a workgroup's positions x channels)
+ * call.  Waves that share k in the place of "mfma32_64x64", "mfma64_64x64" or any 16-bit kernel for rows of arbitrary length go by
+ * the name of the kernel that they stand in for; rp_hip_last_gemm_launch tells them apart.  The rp_hip_conv2d_same_* entries report theirs too: "conv_taps16_256x64" or "_64x64" (a workgroup's positions x channels)
  * and "conv_dw16" for 16-bit images read in place, "conv_planes" for zero-bordered copies; a call with both gradients names the
  * weight gradient's.  No counterpart in the reference (whose device GEMM is one cuBLAS call). */
 const char* rp_hip_last_gemm_kernel(void);
+/* Name of the kernel that this call launched: the same, except for what stands in for another one.  "mfma16_wavek" and "mfma16_wavek_ragged";
+ * "mfma32_wavek_" and "mfma64_wavek_" with the tile (16x16, 16x32, 16x64, 32x32, 64x64, few_rows); "linear_backward16_ragged"; "conv_gradients16" for both
+ * gradients of a 16-bit convolution in two launches; for fp32 "conv_planes" the tile of the call's last product where its waves share k.  No counterpart in the reference. */
+const char* rp_hip_last_gemm_launch(void);
 
 /* ------------------------------------------------------------------------
  * The other device entry points the benchmark configurations touch.  Names and

@@ -796,7 +796,7 @@ bool launch_conv_gradients16(void* dx, void* dw, const void* dy, const void* x, 
     gx.finish = ConvFinish{dw, gw.part, gw.splits, C_out * C_in, taps, (int)shared_grid(gx.groups, (C_in + CD_CO - 1) / CD_CO), units < most ? units : most};
     rc = launch_dw(gw, kW, dtype);
     if (rc == 0) rc = launch_taps(gx, npos, kW, dtype);
-    report_kernel("conv_dw16");
+    report_kernel("conv_dw16", "conv_gradients16");
     rp_hip_free(part);
     rp_hip_free(wt);
     return true;

@@ -233,7 +233,9 @@ int launch_pipe16k(const GemmArgs& g, int dtype);
 bool pipe32k_takes(const GemmArgs& g);         // and its fp32 twin
 int launch_pipe32k(const GemmArgs& g);
 int launch_gemm_segmented_b(const GemmArgs& g, int samples, int dtype);
-void report_kernel(const char* name);          // what rp_hip_last_gemm_kernel names next (a string of static lifetime)
+// What rp_hip_last_gemm_kernel names next and, where another kernel stands in for that one, rp_hip_last_gemm_launch (strings of static lifetime)
+void report_kernel(const char* name, const char* launched = nullptr);
+void report_launch(const char* launched);       // the latter alone
 // 16-bit same-padding convolutions straight from the image (rp_conv_direct.hip); outputs must not overlap the images they are read from
 bool conv_taps16_takes(int batch, int C_from, int C_to, int H, int W, int kH, int kW, int dtype);
 int launch_conv_taps16(void* out, const void* in, const void* w, const void* bias, int batch, int C_from, int C_to, int H, int W, int kH, int kW, bool for_input_grad, int dtype);

@@ -332,45 +332,46 @@ static WkwTile wavekw_takes(const GemmArgs& g, const Plan& p, int dtype) {
     return !apart ? WKW_NONE : p.fam == FAM_SKINNY ? WKW_FEW_ROWS : tile;
 }
 
-static thread_local const char* g_last_kernel = "none";      // what rp_hip_last_gemm_kernel reports
-void report_kernel(const char* name) { g_last_kernel = name; }
+static thread_local const char *g_last_kernel = "none", *g_last_launch = "none";      // what rp_hip_last_gemm_kernel and rp_hip_last_gemm_launch report
+void report_kernel(const char* name, const char* launched) { g_last_kernel = name; g_last_launch = launched ? launched : name; }
+void report_launch(const char* launched) { g_last_launch = launched; }
 
 static int run_gemm(GemmArgs g, int dtype) {
     plain_k_strides(g.m, g.k, g.n, g.a_rs, g.a_cs, g.b_rs, g.b_cs);
     Plan p = make_plan(g.batch, g.m, g.k, g.n, g.a_rs, g.a_cs, g.b_rs, g.b_cs, g.c_rs, g.c_cs, g.a_bs, g.b_bs, dtype);
     if (p.fam == FAM_PIPE32) {
-        if (pipe32_takes(g)) { g_last_kernel = p.name; return launch_pipe32(g); }
+        if (pipe32_takes(g)) { report_kernel(p.name); return launch_pipe32(g); }
         p = make_plan(g.batch, g.m, g.k, g.n, g.a_rs, g.a_cs, g.b_rs, g.b_cs, g.c_rs, g.c_cs, g.a_bs, g.b_bs, dtype, false);     // options, base pointers or spans it does not take
     }
     if (p.fam == FAM_PIPE16) {
-        if (pipe16_takes(g)) { g_last_kernel = p.name; return launch_pipe16(g, dtype); }
+        if (pipe16_takes(g)) { report_kernel(p.name); return launch_pipe16(g, dtype); }
         p = make_plan(g.batch, g.m, g.k, g.n, g.a_rs, g.a_cs, g.b_rs, g.b_cs, g.c_rs, g.c_cs, g.a_bs, g.b_bs, dtype, false);
     }
     if (p.fam == FAM_PIPE16K) {
-        if (pipe16k_takes(g)) { g_last_kernel = p.name; return launch_pipe16k(g, dtype); }
+        if (pipe16k_takes(g)) { report_kernel(p.name); return launch_pipe16k(g, dtype); }
         p = make_plan(g.batch, g.m, g.k, g.n, g.a_rs, g.a_cs, g.b_rs, g.b_cs, g.c_rs, g.c_cs, g.a_bs, g.b_bs, dtype, false);
     }
     if (p.fam == FAM_PIPE32K) {
-        if (pipe32k_takes(g)) { g_last_kernel = p.name; return launch_pipe32k(g); }
+        if (pipe32k_takes(g)) { report_kernel(p.name); return launch_pipe32k(g); }
         p = make_plan(g.batch, g.m, g.k, g.n, g.a_rs, g.a_cs, g.b_rs, g.b_cs, g.c_rs, g.c_cs, g.a_bs, g.b_bs, dtype, false);
     }
     if (p.fam == FAM_DIRECT32) {
-        if (direct32_takes(g)) { g_last_kernel = p.name; return launch_direct32(g); }
+        if (direct32_takes(g)) { report_kernel(p.name); return launch_direct32(g); }
         p = make_plan(g.batch, g.m, g.k, g.n, g.a_rs, g.a_cs, g.b_rs, g.b_cs, g.c_rs, g.c_cs, g.a_bs, g.b_bs, dtype, false);     // base pointers or spans it cannot address
     }
     if (p.fam != FAM_GENERIC && p.fam != FAM_TINY && !p.ragged && !(aligned16(g.A) && aligned16(g.B)))
         p = make_plan(g.batch, g.m, g.k, g.n, g.a_rs, g.a_cs, g.b_rs, g.b_cs, g.c_rs, g.c_cs, g.a_bs, g.b_bs, dtype, false, false);
     bool wavek_ragged = false;
     if (wavek16_takes(g, p, dtype, wavek_ragged)) {
-        g_last_kernel = wavek_ragged ? p.name : "mfma16_wavek";          // (ragged rows: it goes by the name of the kernel that it stands in for)
+        report_kernel(wavek_ragged ? p.name : "mfma16_wavek", wavek_ragged ? "mfma16_wavek_ragged" : "mfma16_wavek");      // (ragged rows: by the name of the kernel that it stands in for)
         return launch_mfma16_wavek(g, wavek_ragged, dtype);
     }
     const WkwTile shared_k = wavekw_takes(g, p, dtype);
     if (shared_k != WKW_NONE) {
-        g_last_kernel = p.fam == FAM_MFMAW ? p.name : dtype == RP_DTYPE_FLOAT32 ? "mfma32_wavek" : "mfma64_wavek";      // (among the 64 x 64 tiles it goes by their name)
+        report_kernel(p.fam == FAM_MFMAW ? p.name : dtype == RP_DTYPE_FLOAT32 ? "mfma32_wavek" : "mfma64_wavek", wavekw_name(shared_k, dtype));      // (among the 64 x 64 tiles by their name)
         return launch_wavekw(g, shared_k, dtype);
     }
-    g_last_kernel = p.name;
+    report_kernel(p.name);
     switch (p.fam) {
         case FAM_MFMA16:
         case FAM_MFMA16_SKINNY: return launch_mfma16(g, p, dtype);
@@ -439,7 +440,7 @@ int launch_gemm_segmented_b(const GemmArgs& g, int samples, int dtype) {
     }
     if (dtype == RP_DTYPE_FLOAT32) {
         const WkwTile tile = segmented_wavek_tile(g, samples);
-        if (tile != WKW_NONE) return launch_wavekw_segmented(g, tile);
+        if (tile != WKW_NONE) { report_launch(wavekw_name(tile, dtype)); return launch_wavekw_segmented(g, tile); }
     }
     Plan p{FAM_MFMAW, 64, 64, !a_kc, g.seg_k > 0, true, "mfmaw"};
     const long long tiles128 = (long long)((g.m + 127) / 128) * ((g.n + 127) / 128) * g.batch;
@@ -663,7 +664,7 @@ int rp_hip_linear_backward(void* dx, void* dw, void* db, const void* dy, const v
         // (more than two rounds of 16 x 16 tiles need the registers and the LDS that they have alone: fp32 2659 x 49 x 3731 70.3 us apart, 73.4 in one launch)
         const auto rounds16 = [&](const GemmArgs& g, WkwTile t) { return t == WKW_16X16 && (long long)((g.m + 15) / 16) * ((g.n + 15) / 16) > 2 * cu_tiles(); };
         if (dx && dw && linear_backward_wavekw_takes(gx, gw, tx, tw, dtype) && (tx == tw || !(rounds16(gx, tx) || rounds16(gw, tw))) && apart) {
-            g_last_kernel = "linear_backward_wavek";
+            report_kernel("linear_backward_wavek");
             const bool rides = db && m <= LINEAR_DB_ROWS && bias_gradient_apart(db, gx, gw, dtype);
             if (launch_linear_backward_wavekw(gx, gw, tx, tw, rides ? db : nullptr, accumulate_db, dtype) != 0) return -1;
             return db && !rides ? rp_hip_reduce_rows(db, dy, m, n, accumulate_db, dtype) : 0;
@@ -671,7 +672,7 @@ int rp_hip_linear_backward(void* dx, void* dw, void* db, const void* dy, const v
     }
     bool edge = false, dx_wavek = false, ragged = false;
     if ((dtype == RP_DTYPE_BFLOAT16 || dtype == RP_DTYPE_FLOAT16) && dx && dw && linear_backward_pairs(gx, gw, dtype, edge, dx_wavek, ragged)) {
-        g_last_kernel = "linear_backward16_64x64";
+        report_kernel("linear_backward16_64x64", ragged ? "linear_backward16_ragged" : nullptr);
         // The bias gradient rides along unless it would be written over something that is still read (one launch after the other
         // was fine), or its chain of chunks outlasts the products.
         const bool rides = db && m <= (n % 32 ? LINEAR_DB_ROWS_UNEVEN : LINEAR_DB_ROWS) && bias_gradient_apart(db, gx, gw, dtype);
@@ -686,6 +687,7 @@ int rp_hip_linear_backward(void* dx, void* dw, void* db, const void* dy, const v
 }
 
 const char* rp_hip_last_gemm_kernel(void) { return g_last_kernel; }
+const char* rp_hip_last_gemm_launch(void) { return g_last_launch; }
 
 const char* rp_hip_gemm_kernel_name(int batch, int m, int k, int n, long long a_rs, long long a_cs,
                                     long long b_rs, long long b_cs, long long c_rs, long long c_cs, int dtype) {

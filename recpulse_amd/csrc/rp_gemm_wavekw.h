@@ -348,6 +348,7 @@ __device__ __forceinline__ void gemm_wavekw_block(const GemmArgs& g, int tiles_m
 // WKW_FEW_ROWS: 16 x 32 with chains of at most 32 values; WKW_TINY: the 16 x 16 tiles of rp_gemm_tiny.h, two a workgroup
 enum WkwTile { WKW_NONE, WKW_16X16, WKW_16X32, WKW_32X32, WKW_16X64, WKW_64X64, WKW_FEW_ROWS, WKW_TINY };
 WkwTile wavekw_tile(const GemmArgs& g, int dtype);
+const char* wavekw_name(WkwTile tile, int dtype);                   // what rp_hip_last_gemm_launch says of it
 int launch_wavekw(const GemmArgs& g, WkwTile tile, int dtype);      // fp32 / fp64 products that the waves of a workgroup share, see wavekw_takes
 int launch_wavekw_segmented(const GemmArgs& g, WkwTile tile);       // fp32, A with unit stride along k, B in segments
 // All gradients of a Linear layer in one launch, each product on the tiles that it would get alone; gx.A is dY [gx.m, gx.k], dense; db: gx.k column sums of dY, or null

@@ -69,6 +69,18 @@ WkwTile wavekw_tile(const GemmArgs& g, int dtype) {
     return tiles(1, 1) <= WKW_MAX_SLOTS ? WKW_16X16 : WKW_NONE;       // (many tiles where an operand is only 16 to 31 wide)
 }
 
+const char* wavekw_name(WkwTile tile, int dtype) {
+    if (dtype == RP_DTYPE_FLOAT64) return tile == WKW_32X32 ? "mfma64_wavek_32x32" : "mfma64_wavek_16x16";
+    switch (tile) {
+        case WKW_64X64: return "mfma32_wavek_64x64";
+        case WKW_16X64: return "mfma32_wavek_16x64";
+        case WKW_32X32: return "mfma32_wavek_32x32";
+        case WKW_16X32: return "mfma32_wavek_16x32";
+        case WKW_FEW_ROWS: return "mfma32_wavek_few_rows";
+        default: return "mfma32_wavek_16x16";
+    }
+}
+
 int launch_wavekw(const GemmArgs& g, WkwTile tile, int dtype) {
     if (dtype == RP_DTYPE_FLOAT64) return tile == WKW_32X32 ? launch_wavekw_layout<double, 2, 2, 8>(g) : launch_wavekw_layout<double, 1, 1, 8>(g);
     switch (tile) {

@@ -273,6 +273,26 @@ def test_same_convolution_in_fp32_is_exact_on_integers(case):
     assert np.array_equal(gw.numpy(), torch.nn.grad.conv2d_weight(xt, (Co, Ci, kH, kW), gt, padding=pad).numpy())
 
 
+@pytest.mark.parametrize("case,forward,input_grad,weight_grad", zip(SHARED_CASES, *zip(
+    ("16x16", "16x16", "32x32"), ("16x16", None, "32x32"), ("16x32", "16x32", "32x32"), ("64x64", "64x64", "32x32"), ("64x64", None, "64x64"),
+    (None, None, "32x32"), (None, None, "32x32"), ("16x32", "16x32", "32x32"), (None, "16x32", "32x32"))), ids=lambda c: "x".join(map(str, c)) if isinstance(c, tuple) else str(c))
+def test_tiles_of_same_convolution_in_fp32(case, forward, input_grad, weight_grad):
+    """The tiles that the cases above are for (on 256 CUs); None: those whose waves do not share k."""
+    N, Ci, H, W, Co, kH, kW = case
+    L = capi.lib()
+    d = Dev(np.zeros((N, max(Ci, Co), H, W), np.float32), F32)
+    out, w = Dev.empty((N, max(Ci, Co), H, W), F32), Dev(np.zeros((Co, Ci, kH, kW), np.float32), F32)
+    name = lambda tile: f"mfma32_wavek_{tile}" if tile else "conv_planes"          # noqa: E731
+    capi.check(L.rp_hip_conv2d_same_forward(out.ptr, d.ptr, w.ptr, None, N, Ci, H, W, Co, kH, kW, F32), "same forward")
+    assert capi.last_gemm_launch() == name(forward) and capi.last_gemm_kernel() == "conv_planes"
+    if L.rp_hip_conv2d_same_supported(Co, H, W, kH, kW, F32) == 1:
+        capi.check(L.rp_hip_conv2d_same_backward(out.ptr, None, d.ptr, None, w.ptr, N, Ci, H, W, Co, kH, kW, F32), "dX")
+        assert capi.last_gemm_launch() == name(input_grad) and capi.last_gemm_kernel() == "conv_planes"
+    capi.check(L.rp_hip_conv2d_same_backward(None, w.ptr, d.ptr, out.ptr, None, N, Ci, H, W, Co, kH, kW, F32), "dW")
+    assert capi.last_gemm_launch() == name(weight_grad) and capi.last_gemm_kernel() == "conv_planes"
+    capi.synchronize()
+
+
 @pytest.mark.parametrize("dt", [F16, BF16], ids=lambda d: NAMES[d])
 @pytest.mark.parametrize("case", [(23, 64, 56, 52, 64, 3), (29, 64, 48, 48, 64, 5), (2, 128, 12, 40, 64, 3), (1, 64, 53, 53, 128, 5)], ids=lambda c: "x".join(map(str, c)))
 def test_weight_gradient_does_not_depend_on_the_input_gradient(dt, case):

@@ -611,6 +611,21 @@ def test_ragged_rows(dt, batch, m, k, n, kernel, layout):
         dc.free()
 
 
+# (dtype, batch, m, k, n, name, launched, layouts): ragged rows on waves that share k in the place of the kernel named, and those that are left to it
+RAGGED_LAUNCHES = [(BF16, 1, 5, 4099, 1027, "mfma16_skinny_32x128", "mfma16_wavek_ragged", ["nt"]), (F16, 1, 65, 2561, 127, "generic", "mfma16_wavek_ragged", ["nn", "nt"]),
+                   (F32, 1, 530, 261, 527, "mfma32_64x64", "mfma32_wavek_32x32", LAYOUTS), (F64, 1, 131, 5, 67, "mfma64_64x64", "mfma64_wavek_16x16", LAYOUTS),
+                   (F32, 1, 16, 5745, 49, "mfma32_64x64", "mfma32_64x64", LAYOUTS), (F32, 1, 60, 2049, 131, "mfma32_64x64", "mfma32_64x64", LAYOUTS),
+                   (F32, 1, 1450, 31, 1403, "mfma32_64x64", "mfma32_64x64", LAYOUTS), (F64, 1, 1450, 33, 1403, "mfma64_64x64", "mfma64_64x64", LAYOUTS),
+                   (F64, 2, 1100, 41, 563, "mfma64_64x64", "mfma64_64x64", LAYOUTS), (BF16, 1, 105, 4165, 2311, "mfma16_skinny_32x128", "mfma16_skinny_32x128", ["nt"]),
+                   (F16, 1, 105, 4165, 2311, "mfma16_skinny_32x128", "mfma16_skinny_32x128", ["nt"]), (BF16, 1, 11, 3261, 63, "generic", "generic", ["nn"])]
+
+
+@pytest.mark.parametrize("dt,batch,m,k,n,kernel,launched,layout", [c[:-1] + (layout,) for c in RAGGED_LAUNCHES for layout in c[-1]])
+def test_ragged_rows_by_the_kernel_launched(dt, batch, m, k, n, kernel, launched, layout):
+    test_ragged_rows(dt, batch, m, k, n, kernel, layout)
+    assert capi.last_gemm_launch() == launched
+
+
 @pytest.mark.parametrize("layout", LAYOUTS)
 @pytest.mark.parametrize("dt", HALF, ids=lambda d: NAMES[d])
 @pytest.mark.parametrize("m,k,n", [(64, 704, 128), (64, 768, 128), (128, 832, 64), (64, 896, 192), (72, 712, 136), (136, 776, 200), (200, 840, 72), (8, 904, 72), (64, 961, 129), (130, 1535, 66)])
@@ -1007,6 +1022,55 @@ def test_waves_that_share_k_in_fp32_and_fp64(dt, batch, m, k, n, kernel, layout)
         inner[...] = (inner if accumulate else 0) + want + (bias if with_bias else 0)
         assert np.array_equal(dc.to_numpy(np_t, (expect.size,)), expect)      # C, and nothing around it
         dc.free()
+
+
+@pytest.mark.parametrize("dt,batch,m,k,n,tile", [(F32, 1, 16, 513, 16, "16x16"), (F32, 1, 70, 545, 300, "16x16"), (F32, 1, 497, 577, 401, "16x64"), (F32, 1, 900, 519, 901, "64x64"), (F32, 9, 131, 77, 260, "32x32"),
+                                                 (F32, 253, 64, 512, 64, "64x64"), (F32, 1, 63, 1024, 2113, "16x64"), (F32, 1, 3, 1001, 1100, "few_rows"), (F32, 1, 33, 3000, 1500, "16x32"),
+                                                 (F64, 1, 60, 131, 50, "16x16"), (F64, 1, 390, 257, 401, "32x32"), (F64, 130, 64, 70, 130, "32x32")])
+def test_tiles_of_waves_that_share_k(dt, batch, m, k, n, tile):
+    """Which of the tiles shapes like those above are on (A and B row-major, on 256 CUs)."""
+    es = capi.DTYPE_SIZE[dt]
+    da, db, dc = (capi.DeviceBuffer(batch * size * es) for size in (m * k, k * n, m * n))
+    capi.gemm(dc.ptr, da.ptr, db.ptr, None, batch, m, k, n, (m * k, k, 1), (k * n, n, 1), (m * n, n, 1), False, dt)
+    assert capi.last_gemm_launch() == f"mfma{8 * es}_wavek_{tile}"
+    capi.synchronize()
+
+
+@pytest.mark.parametrize("dt,m,k,n", [(F32, 935, 213, 862), (F32, 64, 1024, 1024), (F32, 600, 900, 50), (F64, 89, 287, 286), (F64, 500, 40, 600), (BF16, 119, 57, 245), (F16, 300, 305, 641), (F32, 37, 50, 21)])
+def test_gradients_in_one_launch_with_pitches_and_over_operands(dt, m, k, n):
+    """x, w, dx and dw with pitches of their own, dx and dw also transposed: the bits of the three on their own and nothing around them written; and gradients
+    over what the launch still reads, which come one after the other."""
+    rng = np.random.default_rng(m + k + n)
+    L = capi.lib()
+    dy = rand_storage(rng, (m, n), dt)
+    x, w = rand_storage(rng, (m, k + 3), dt), rand_storage(rng, (k, n + 5), dt)
+    d_dy, d_x, d_w = Dev(dy, dt), Dev(x, dt), Dev(w, dt)
+    want_b, got_b = Dev.empty((n,), dt), Dev.empty((n,), dt)
+    capi.check(L.rp_hip_reduce_rows(want_b.ptr, d_dy.ptr, m, n, 0, dt), "reduce_rows")
+    for transposed in (False, True):
+        shape_x, st_x = ((k, m + 2), (1, m + 2)) if transposed else ((m, k + 7), (k + 7, 1))
+        shape_w, st_w = ((n, k + 1), (1, k + 1)) if transposed else ((k, n + 9), (n + 9, 1))
+        init_x, init_w = rand_storage(rng, shape_x, dt), rand_storage(rng, shape_w, dt)
+        want, got = [Dev(v, dt) for v in (init_x, init_w)], [Dev(v, dt) for v in (init_x, init_w)]
+        capi.gemm(want[0].ptr, d_dy.ptr, d_w.ptr, None, 1, m, n, k, (0, n, 1), (0, 1, n + 5), (0,) + st_x, False, dt)
+        capi.gemm(want[1].ptr, d_x.ptr, d_dy.ptr, None, 1, k, m, n, (0, 1, k + 3), (0, n, 1), (0,) + st_w, False, dt)
+        capi.check(L.rp_hip_linear_backward(got[0].ptr, got[1].ptr, got_b.ptr, d_dy.ptr, d_x.ptr, d_w.ptr, m, k, n, k + 3, 1, n + 5, 1, *st_x, *st_w, 0, 0, 0, dt), "linear_backward")
+        for g, t in zip(got + [got_b], want + [want_b]):
+            assert np.array_equal(g.numpy(), t.numpy())
+    # db over W: written after dX has read W; dX over X: dW is computed from what then stands there; dW over W, as deep as the pitches
+    want = [Dev.empty((m, k), dt), Dev(rand_storage(rng, (k, n + 5), dt), dt)]
+    xs, ws = np.ascontiguousarray(x[:, :k]), np.ascontiguousarray(w)
+    for over in ("db", "dx", "dw"):
+        d_x, d_w = Dev(xs, dt), Dev(ws, dt)
+        place = {"dx": Dev.empty((m, k), dt), "dw": Dev(w, dt), "db": Dev.empty((n,), dt)}
+        place[over] = d_x if over == "dx" else d_w
+        capi.check(L.rp_hip_linear_backward(place["dx"].ptr, place["dw"].ptr, place["db"].ptr, d_dy.ptr, d_x.ptr, d_w.ptr, m, k, n, k, 1, n + 5, 1, k, 1, n + 5, 1, 0, 0, 0, dt), over)
+        e_x, e_w = Dev(xs, dt), Dev(ws, dt)
+        capi.gemm(want[0].ptr, d_dy.ptr, e_w.ptr, None, 1, m, n, k, (0, n, 1), (0, 1, n + 5), (0, k, 1), False, dt)
+        capi.gemm(want[1].ptr, want[0].ptr if over == "dx" else e_x.ptr, d_dy.ptr, None, 1, k, m, n, (0, 1, k), (0, n, 1), (0, n + 5, 1), False, dt)
+        assert np.array_equal(place["dx"].numpy(), want[0].numpy()), over
+        assert np.array_equal(place["dw"].numpy()[:, :n], want[1].numpy()[:, :n]), over
+        assert np.array_equal(place["db"].numpy().reshape(-1)[:n], want_b.numpy()), over
 
 
 def _sums_of_short_chains(a, b):
