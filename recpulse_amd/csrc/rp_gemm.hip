@@ -288,6 +288,19 @@ static bool wavek16_takes(const GemmArgs& g, const Plan& p, int dtype, bool& rag
            !(g.bias && overlap(c, span_of(g.bias, 1, g.n, 0, 1, 2)));
 }
 
+// Of the generic kernel's fp64 products (expanded or overlapping rows, very small outputs): not those of few slabs of 16 values of k and many tiles.  A tile of
+// 32 x 32 costs the chip 5.8 ns here whatever k is, one of 16 x 16 half of that; a 64 x 64 one costs 6 (nearly empty) to 12 ns there with one slab, 15 with two,
+// 21 with three, 27 with four.  us there and here: 3000 x 64 x 5 x 64 36.7 / 71.9, 3000 x 33 x 5 x 65 46.3 / 103.8, 400 x 64 x 5 x 64 10.7 / 13.6, 3001 x 3 x 2001 23.7 / 37.4, 3000 x 20 x 5 x 20
+// 24.7 / 34.2, but 8000 x 1 x 3 x 1 49.8 / 41.4, 100 x 64 x 5 x 64 6.9 / 4.9; 3000 x 64 x 17 x 64 45.3 / 75.5, 3000 x 20 x 17 x 20 41.6 / 35.4, 400 x 33 x 17 x 65 18.5 / 17.9; 3000 x 64 x 48 x 64
+// 62.9 / 78.0, 3001 x 40 x 2001 35.7 / 40.3, 3000 x 33 x 33 x 65 113 / 112, 400 x 64 x 48 x 64 16.8 / 14.2; 3000 x 64 x 64 x 64 81 / 82; 3000 x 64 x 130 x 64 171 / 121, 8000 x 1 x 1001 x 1 2999 / 256.
+static bool generic64_wins(const GemmArgs& g, WkwTile tile) {
+    const long long cus = cu_tiles(), tiles64 = (long long)((g.m + 63) / 64) * ((g.n + 63) / 64) * g.batch;
+    const long long work = tile == WKW_32X32 ? (long long)((g.m + 31) / 32) * ((g.n + 31) / 32) * g.batch : (long long)((g.m + 15) / 16) * ((g.n + 15) / 16) * g.batch / 2;       // in tiles of 32 x 32
+    if (g.k <= 16) return work >= 4 * cus && work * 2 >= tiles64 * 3;
+    if (g.k <= 32) return work >= 10 * cus && work * 2 >= tiles64 * 5;
+    return g.k <= 48 && work >= 16 * cus && work * 2 >= tiles64 * 7;
+}
+
 // fp32 and fp64 products that the waves of a workgroup share (rp_gemm_wavekw.hip, which has figures): those of 64 x 64 tiles, fp64 ones of the generic
 // kernel, and fp32 ones that 16 x 16 tiles of four waves or the row-streaming kernel took.  Stays where it was: fp32 with k up to 512 on 16 x 16 tiles (60 x 443 x 65 3.55 / 3.67 us; 256 x 784 x 256
 // 6.95 / 5.0-6.0); a k too short for the number of tiles (fp32 2384 x 32 x 368
@@ -319,7 +332,7 @@ static WkwTile wavekw_takes(const GemmArgs& g, const Plan& p, int dtype) {
         return WKW_NONE;
     }
     const WkwTile tile = wavekw_tile(g, dtype);
-    if (tile == WKW_NONE) return WKW_NONE;
+    if (tile == WKW_NONE || (p.fam == FAM_GENERIC && generic64_wins(g, tile))) return WKW_NONE;
     const int esz = (int)dtype_size(dtype);
     auto span = [&](const void* base, int rows, int cols, long long bs, long long rs, long long cs) {
         Span s = span_of(base, rows, cols, rs, cs, esz);

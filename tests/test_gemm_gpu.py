@@ -1073,6 +1073,20 @@ def test_gradients_in_one_launch_with_pitches_and_over_operands(dt, m, k, n):
         assert np.array_equal(place["db"].numpy().reshape(-1)[:n], want_b.numpy()), over
 
 
+@pytest.mark.parametrize("batch,m,k,n,launched", [(3000, 64, 5, 64, "generic"), (3000, 33, 5, 65, "generic"), (1, 3001, 3, 2001, "generic"), (3000, 20, 5, 20, "generic"), (3000, 64, 17, 64, "generic"),
+                                                  (3000, 64, 48, 64, "generic"), (100, 64, 5, 64, "mfma64_wavek_32x32"), (3000, 20, 17, 20, "mfma64_wavek_16x16"), (400, 64, 48, 64, "mfma64_wavek_32x32"),
+                                                  (3000, 33, 33, 65, "mfma64_wavek_32x32"), (400, 64, 130, 64, "mfma64_wavek_32x32"), (1, 300, 17, 301, "mfma64_wavek_16x16")])
+def test_overlapping_rows_in_fp64(batch, m, k, n, launched):
+    """A's rows are windows that move on by one value (on 256 CUs: few slabs of k and many tiles on the generic kernel); small integers, so the bits are known."""
+    rng = np.random.default_rng(m + k)
+    a, b = rng.integers(-2, 3, (batch, k + m)).astype(np.float64), rng.integers(-2, 3, (batch, k, n)).astype(np.float64)
+    da, db, dc = Dev(a, F64), Dev(b, F64), Dev.empty((batch, m, n), F64)
+    capi.gemm(dc.ptr, da.ptr, db.ptr, None, batch, m, k, n, (k + m, 1, 1), (k * n, n, 1), (m * n, n, 1), False, F64)
+    assert capi.last_gemm_launch() == launched
+    windows = np.lib.stride_tricks.as_strided(a, (batch, m, k), (a.strides[0], 8, 8))
+    assert np.array_equal(dc.numpy(), np.matmul(np.ascontiguousarray(windows), b))
+
+
 def _sums_of_short_chains(a, b):
     """a @ b in float32 as the row-streaming kernel sums it: chains of 32 products with fused multiply-adds (a float64 step holds a product and
     its sum, rounded once), eight chains to a block of 256, blocks one after the other."""
