@@ -541,6 +541,10 @@ int* noalloc_arrival_counters() {
 // 2048 x 512 x 512 21.2 / 19.3; uneven 768 x 16 x 184 10.1 / 10.2, 904 x 16 x 184 12.1 / 11.2, 1024 x 512 x 184 12.9 / 12.0,
 // 1280 x 768 x 264 16.4 / 15.1, 2048 x 40 x 16 21.8 / 16.5).
 constexpr int LINEAR_DB_ROWS = 1024, LINEAR_DB_ROWS_UNEVEN = 768;
+// The same for fp32 and fp64 layers whose waves share k: a chunk of a strip takes 1.5 us there, 2.1 us of an uneven one.  us, in the launch and apart: fp32 1248 x 48 x 1488
+// 11.8 / 16.2, 1200 x 128 x 448 11.4 / 15.1, 1536 x 112 x 64 9.2 / 10.1, 1296 x 64 x 320 9.8 / 9.5, 1648 x 176 x 272 12.7 / 11.9; uneven 1150 x 160 x 373 10.7 / 14.8, 1225 x 127 x 77
+// 8.8 / 9.9, 1444 x 23 x 847 13.4 / 11.9, 1570 x 22 x 263 12.1 / 10.7; fp64 1280 x 96 x 512 13.9 / 15.7, 1399 x 689 x 151 27.0 / 30.9, 1648 x 272 x 464 32.5 / 28.9.
+constexpr int LINEAR_DB_ROWS_WAVEKW = 1536, LINEAR_DB_ROWS_WAVEKW_UNEVEN = 1280;
 
 // The plan that a product alone would follow
 static Plan plan_alone(const GemmArgs& g, int dtype) {
@@ -674,11 +678,12 @@ int rp_hip_linear_backward(void* dx, void* dw, void* db, const void* dy, const v
             if (launch_linear_backward_tiny(gx, gw, rides ? db : nullptr, dy, m, n, accumulate_db) != 0) return -1;
             return db && !rides ? rp_hip_reduce_rows(db, dy, m, n, accumulate_db, dtype) : 0;
         }
-        // (more than two rounds of 16 x 16 tiles need the registers and the LDS that they have alone: fp32 2659 x 49 x 3731 70.3 us apart, 73.4 in one launch)
-        const auto rounds16 = [&](const GemmArgs& g, WkwTile t) { return t == WKW_16X16 && (long long)((g.m + 15) / 16) * ((g.n + 15) / 16) > 2 * cu_tiles(); };
+        // (many rounds of 16 x 16 tiles need the registers and the LDS that they have alone: three of them (us apart and in one launch: fp32 832 x 160 x 800 14.9 / 10.3,
+        // 876 x 191 x 812 19.2 / 13.4), beside the 32 x 32 tiles of a long dW two (2659 x 49 x 3731 70.3 / 73.4, 1200 x 144 x 1408 24.7 / 26.1))
+        const auto rounds16 = [&](const GemmArgs& g, WkwTile t) { return t == WKW_16X16 && (long long)((g.m + 15) / 16) * ((g.n + 15) / 16) > (tw == WKW_32X32 && m > 1024 ? 2 : 3) * cu_tiles(); };
         if (dx && dw && linear_backward_wavekw_takes(gx, gw, tx, tw, dtype) && (tx == tw || !(rounds16(gx, tx) || rounds16(gw, tw))) && apart) {
             report_kernel("linear_backward_wavek");
-            const bool rides = db && m <= LINEAR_DB_ROWS && bias_gradient_apart(db, gx, gw, dtype);
+            const bool rides = db && m <= (n * dtype_size(dtype) % 64 ? LINEAR_DB_ROWS_WAVEKW_UNEVEN : LINEAR_DB_ROWS_WAVEKW) && bias_gradient_apart(db, gx, gw, dtype);
             if (launch_linear_backward_wavekw(gx, gw, tx, tw, rides ? db : nullptr, accumulate_db, dtype) != 0) return -1;
             return db && !rides ? rp_hip_reduce_rows(db, dy, m, n, accumulate_db, dtype) : 0;
         }

@@ -868,6 +868,24 @@ def test_gradients_whose_waves_share_k_in_one_launch(dt, m, k, n):
     assert np.array_equal(got.numpy(), want[0].numpy()) and np.array_equal(d_w.numpy(), want[1].numpy())
 
 
+@pytest.mark.parametrize("dt,m,k,n", [(F32, 1040, 160, 272), (F32, 1536, 32, 512), (F32, 1537, 32, 512), (F32, 1280, 33, 130), (F32, 1281, 33, 130), (F32, 832, 160, 800), (F32, 272, 544, 624), (F32, 720, 256, 2100),
+                                      (F64, 1536, 64, 72), (F64, 1280, 64, 75), (F64, 1281, 64, 75), (F64, 1540, 64, 72)])
+def test_gradients_in_one_launch_of_more_rows_and_tiles(dt, m, k, n):
+    """The bias gradient beside the others around the rows up to which it rides, and two to three rounds of 16 x 16 tiles beside another product: the bits of the three on their own."""
+    rng = np.random.default_rng(m + k + n)
+    L = capi.lib()
+    x, w, dy = rand_storage(rng, (m, k), dt), rand_storage(rng, (k, n), dt), rand_storage(rng, (m, n), dt)
+    d_x, d_w, d_dy = Dev(x, dt), Dev(w, dt), Dev(dy, dt)
+    want, got = ([Dev.empty(s, dt) for s in ((m, k), (k, n), (n,))] for _ in range(2))
+    capi.gemm(want[0].ptr, d_dy.ptr, d_w.ptr, None, 1, m, n, k, (0, n, 1), (0, 1, n), (0, k, 1), False, dt)
+    capi.gemm(want[1].ptr, d_x.ptr, d_dy.ptr, None, 1, k, m, n, (0, 1, k), (0, n, 1), (0, n, 1), False, dt)
+    capi.check(L.rp_hip_reduce_rows(want[2].ptr, d_dy.ptr, m, n, 0, dt), "reduce_rows")
+    capi.check(L.rp_hip_linear_backward(got[0].ptr, got[1].ptr, got[2].ptr, d_dy.ptr, d_x.ptr, d_w.ptr, m, k, n, k, 1, n, 1, k, 1, n, 1, 0, 0, 0, dt), "linear_backward")
+    assert capi.last_gemm_kernel() == "linear_backward_wavek"
+    for g, t in zip(got, want):
+        assert np.array_equal(g.numpy(), t.numpy())
+
+
 @pytest.mark.parametrize("m,k,n", [(37, 50, 21), (256, 128, 10), (200, 240, 160)])
 def test_gradients_of_small_layers_over_operands(m, k, n):
     """Small fp32 layers, whose gradients go out in one launch: a gradient over what another product reads gives what the calls
