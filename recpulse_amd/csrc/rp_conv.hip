@@ -15,6 +15,8 @@
 // host path computes (functional/functional.c:885-912, functional_host.c:1291-1313) and is repeatable.
 #include "rp_gemm.h"
 
+#include <cmath>
+
 namespace rp {
 
 struct ConvGeom {
@@ -330,6 +332,16 @@ __global__ void channel_sums_finish_kernel(T* out, const typename traits<T>::acc
 // per plane, however small: taken while a channel holds no more than CHANNEL_SUM_BYTES.  bf16, us, two launches and one: 64 x 256 x 14^2 17.8 / 5.8,
 // 64 x 256 x 7^2 15.7 / 5.4, 1 x 64 x 7^2 6.3 / 3.5, 12 x 192 x 53^2 (67 KB a channel) 11.0 / 5.9; 16 x 128 x 56^2 (100 KB) 6.4 / 6.6, 64 x 64 x 56^2 9.3 / 19.
 constexpr size_t CHANNEL_SUM_BYTES = 72 * 1024;
+// Price of both in us, fitted to 1500 drawn sums: a workgroup a channel pays for its wave slots, for a piece however short the plane, and for its bytes;
+// two launches pay for a workgroup a plane and for the chain over the samples.  us, two launches and one: bf16 1035 x 2 x 14 19.8 / 42.3, 1 x 2587 x 1024 6.9 / 13.3,
+// 6 x 570 x 4139 8.8 / 12.0, fp32 1887 x 1 x 9 32.7 / 50.0.  Of 1000 others 2 run more than 5 % slower than in two launches, 18 % at most; all of them together take 0.49 of the time.
+static bool one_launch_wins(int batch, int channels, int hw, int esz) {
+    const bool is16 = esz == 2;
+    const int per_plane = (hw + 64 * (16 / esz) - 1) / (64 * (16 / esz));
+    const double n = batch, c = channels, pieces = n * per_plane, mb = n * c * hw * esz * 1e-6;
+    const double one = 3 + fmax(fmax(c * (is16 ? 0.0038 : 0.0022), pieces * (is16 ? 0.037 : 0.024)), mb * (!is16 ? 0.1 : channels > 512 ? 0.3 : 0.2));      // (512: as many as are on the chip at a time)
+    return one <= 5.2 + 0.016 * n + 0.0008 * n * c + 0.12 * mb;
+}
 template <typename T>
 __global__ void __launch_bounds__(1024) channel_sums_kernel(T* out, const T* g, int batch, int channels, int hw, int accumulate) {
     using A = typename traits<T>::acc;
@@ -887,7 +899,7 @@ int rp_hip_channel_sums(void* out, const void* grad, int batch, int channels, in
     // (A launch holds fewer than 2^32 threads.  A sum stored over values that another channel's workgroup still reads: the two launches read them all first.)
     const size_t esz = dtype_size(dtype), per_channel = (size_t)batch * hw * esz;
     const bool apart = (const char*)out + channels * esz <= (const char*)grad || (const char*)grad + per_channel * channels <= (const char*)out;
-    if (per_channel <= CHANNEL_SUM_BYTES && channels < 1 << 22 && apart) {
+    if (per_channel <= CHANNEL_SUM_BYTES && channels < 1 << 22 && apart && one_launch_wins(batch, channels, hw, (int)esz)) {
         RP_DISPATCH_DTYPE(dtype, hipLaunchKernelGGL(channel_sums_kernel<T>, dim3((unsigned)channels), dim3(1024), 0, current_stream(), (T*)out, (const T*)grad, batch, channels, hw, accumulate));
         return check_launch("channel_sums_kernel") ? 0 : -1;
     }

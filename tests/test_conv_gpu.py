@@ -126,6 +126,13 @@ def test_channel_sums_over_the_gradient_and_of_very_many_channels(dt):
     assert np.array_equal(ds.numpy(), oracle.to_storage(oracle.to_f64(g, dt).sum(axis=(0, 2)), dt))
 
 
+@pytest.mark.parametrize("dt", ALL, ids=lambda d: NAMES[d])
+@pytest.mark.parametrize("N,C,HW", [(1035, 2, 14), (300, 5, 21), (1887, 1, 9), (1, 2587, 1024), (3, 2102, 86), (200, 64, 11)])
+def test_channel_sums_of_many_samples_or_channels(dt, N, C, HW):
+    """Channels that one workgroup could sum, on either side of the line where two launches are the faster; small integers."""
+    test_channel_sums_of_every_size(dt, N, C, HW)
+
+
 def test_lowering_rejects_inconsistent_geometry():
     d = capi.DeviceBuffer(1 << 16)
     L = capi.lib()
