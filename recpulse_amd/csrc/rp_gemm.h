@@ -223,7 +223,7 @@ bool direct32_takes(const GemmArgs& g);          // pointer alignment and spans 
 int launch_direct32(const GemmArgs& g);
 size_t skinny16_workspace(int batch, int m, int k, int n);          // bytes of partial sums that the tiled 16-bit k split needs
 int launch_mfma16_wavek(const GemmArgs& g, bool ragged, int dtype);       // few tiles, deep k, A k-contiguous; see wavek16_takes
-int launch_linear_backward16(const GemmArgs& gx, const GemmArgs& gw, bool dx_wavek, void* db, int accumulate_db, bool edge, bool ragged, int dtype);      // both on 64 x 64 tiles or dX's waves splitting k, whole or ending in whole 16-byte vectors, see linear_backward_pairs
+int launch_linear_backward16(const GemmArgs& gx, const GemmArgs& gw, bool dx_wavek, void* db, int accumulate_db, bool edge, bool ragged, int dtype);      // both on 64 x 64 tiles or dX's waves splitting k, rows of any length, see linear_backward_pairs
 bool pipe32_takes(const GemmArgs& g);          // options, alignment and spans the k-contiguous short-k fp32 kernel can address
 int launch_pipe32(const GemmArgs& g);
 bool pipe16_takes(const GemmArgs& g);          // the same for the 16-bit kernel (C row-major in whole 8-byte quads)

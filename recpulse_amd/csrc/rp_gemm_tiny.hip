@@ -5,7 +5,8 @@
 // waves each take a quarter of k with v_mfma_f32_16x16x4_f32, and the four partial tiles meet in LDS: one launch, a
 // fixed order of additions, up to about a thousand workgroups in flight.  Operands are read straight from global
 // memory with any strides (16-byte loads along k where k is the unit-stride axis, at any element: four loads of a value each, which
-// rows of no whole vectors had before, made a backward of 935 x 213 x 862 take 44.6 us, 24.4 now); nothing is staged, every value is
+// rows of no whole vectors had before, made a backward of 935 x 213 x 862 take 44.6 us here, 24.4 with vectors; waves that share k have
+// it now, 19.8); nothing is staged, every value is
 // used once per workgroup.
 #include "rp_column_sums.h"
 #include "rp_gemm_tiny.h"

@@ -174,9 +174,9 @@ NullStreamScratch::NullStreamScratch(size_t bytes) {
 NullStreamScratch::~NullStreamScratch() { if (ptr) g_null_stream_mu.unlock(); }
 
 // Pinned host memory that a copy to the host goes through: a kernel writes it across the bus and the calling thread copies it on once the stream is
-// done.  hipMemcpyAsync to pageable memory takes 14 us behind a chain of kernels for 10 KB and 34 for 64 KB, this 3.1 and 4.8, without its checks
-// (at 400 KB 24 and 18: larger copies stay with it).  MLP inference 784-256-128-10 of 256, read back, 44.3 us, 36.4 now.  A block belongs to one call at a time, so threads and streams never share one; at most READBACK_BLOCKS
-// are kept, until rp_hip_empty_cache.
+// done.  us behind a chain of six kernels, hipMemcpyAsync to pageable memory and this: 10 KB 12.8 / 3.9, 64 KB 10.7 / 5.6, 128 KB 13.5 / 8.3, 255 KB 18.9 / 13.2; the limit is one of pinned
+// memory, a megabyte in all.  MLP inference 784-256-128-10 of 256, read back, 40.9 us, 33.9 now.  A block belongs to one call at a time, so threads and streams never share one; at most
+// READBACK_BLOCKS are kept, until rp_hip_empty_cache.
 constexpr size_t READBACK_BYTES = 256 * 1024;
 constexpr size_t READBACK_BLOCKS = 4;
 static std::mutex g_readback_mu;
